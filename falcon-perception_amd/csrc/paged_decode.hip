@@ -988,22 +988,23 @@ constexpr int kPhasePartial = 1;
 constexpr int kPhaseMerge = 2;
 constexpr int kPhasePlan = 4;  // alone: write the step's plan instead of launching the passes
 
-// Workgroups of the even-cut kernel the current device holds at once (asked once per kernel and device).
-template <typename E, int D, int G, bool kAligned, bool kPerHeadK>
-int resident_workgroups() {
-  const auto kernel = paged_decode_kernel<E, D, G, false, kAligned, kPerHeadK, true>;
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cached[dev] == 0) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, 0) != hipSuccess || per_cu <= 0) {
-      (void)hipGetLastError();  // not an error of the launch that follows: the launch goes split by split
-      cached[dev] = -1;
-    } else
-      cached[dev] = per_cu * fp::compute_units();
-  }
-  return cached[dev] > 0 ? cached[dev] : 0;
+// The even cut leaves about chunks / B partial results per sequence to a merge pass of one wavefront per row, which
+// takes them eight at a time: beyond eight, a launch that fits the GPU in one go is cheaper split by split (one
+// sequence of 711 tokens 9.7 us a layer against 10.5 us, four of 5 k to 16 k tokens 22.8 against 23.7 us).
+bool few_sequences(int64_t chunks, int B) { return chunks > 8 * static_cast<int64_t>(B); }
+
+// Chunks per cache head of the even cut of a launch, 0 where it goes split by split: two per CU, as many as the
+// workspace of the launch's split count has rows for (one per chunk + sequence), but at least one per CU.
+int even_cut_chunks(int Hc, int B, int n_splits, int max_context, int page_size) {
+  const int cus = fp::compute_units();
+  const int64_t wanted = 2 * cus / Hc, rows = static_cast<int64_t>(B) * (n_splits - 1);
+  const int64_t chunks = wanted < rows ? wanted : rows;
+  const bool positions_fit = static_cast<int64_t>(B) * (max_context + 64) < (1ll << 30);  // the flat axis is int
+  if (chunks < 1 || 2 * chunks < wanted || B > kFlatMaxB || !positions_fit) return 0;
+  if (few_sequences(wanted, B) && static_cast<int64_t>(Hc) * B * n_splits <= 2 * cus) return 0;
+  // a chunk's pages have to fit the page-id table
+  if ((static_cast<int64_t>(B) * (max_context + 64) / chunks + 128) / page_size + 2 > kMaxSplitPages) return 0;
+  return static_cast<int>(chunks);
 }
 
 template <typename E, int D, int G, bool kPerHeadK = false>
@@ -1020,7 +1021,10 @@ void launch_decode(const DecodeArgs& a, int B, int phases, hipStream_t st) {
     else
       hipLaunchKernelGGL((paged_decode_kernel<E, D, G, true, false, kPerHeadK>), grid, dim3(kThreads), 0, st, a);
   } else {
-    // A launch with more workgroups than the GPU holds at once is cut evenly instead: two chunks
+    // Cut evenly: the work of a workgroup then follows from the lengths of the sequences and not from max_context,
+    // which an engine sets to the longest sequence it may ever hold (16 padded rows of 350 to 4620 tokens under a
+    // limit of 8192, 16 q heads / 8 kv heads with shared V: 57.4 us a layer split by split, one workgroup to a CU,
+    // against 38.8 us).  Two chunks
     // per CU, all of the same length, all resident from the start, so that every CU streams the same
     // number of rows (split by split, the CUs end up with loads 25 % apart at 64 sequences of 1 k to
     // 4 k tokens, and workgroups queue behind busy shader engines).  Measured at 64 sequences of 16 q /
@@ -1033,18 +1037,7 @@ void launch_decode(const DecodeArgs& a, int B, int phases, hipStream_t st) {
     // step for 1 / 2 / 3 chunks per CU: D 128 110.4 / 111.3 / 112.2; D 64 61.7 / 61.3 / 62.1; page size 64, 32
     // sequences 89.2 / 90.9 / 90.4: two stays.  The even cut needs the lengths of at most kFlatMaxB sequences in LDS, a workspace row per (chunk + sequence),
     // and chunks within the page-id table.
-    int n_chunks = 0;
-    {
-      const int resident = aligned ? resident_workgroups<E, D, G, true, kPerHeadK>()
-                                   : resident_workgroups<E, D, G, false, kPerHeadK>();
-      const int64_t wgs = static_cast<int64_t>(a.Hc) * B * a.n_splits;
-      const int chunks = 2 * fp::compute_units() / a.Hc;
-      const bool rows_fit = chunks + B <= static_cast<int64_t>(B) * a.n_splits;  // workspace rows: one per (chunk + sequence)
-      const bool positions_fit = static_cast<int64_t>(B) * (a.max_context + 64) < (1ll << 30);  // the flat axis is int
-      if (chunks >= 1 && wgs > resident && B <= kFlatMaxB && rows_fit && positions_fit &&
-          (static_cast<int64_t>(B) * (a.max_context + 64) / chunks + 128) / a.pd.page_size + 2 <= kMaxSplitPages)
-        n_chunks = chunks;
-    }
+    const int n_chunks = even_cut_chunks(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size);
     DecodeArgs af = a;
     af.B = B;
     af.n_chunks = n_chunks;
@@ -1113,6 +1106,11 @@ int default_split_tokens(int B, int Hc, int max_context, int page_size) {
   target = target < 512 ? 512 : target > 2048 ? 2048 : target;
   int split = 2048;
   while (split > 128 && static_cast<int64_t>(B) * Hc * ((max_context + split - 1) / split) < target) split >>= 1;
+  // the workspace has B rows per split: enough of them for the even cut, where it can have them
+  const int64_t chunks = 2 * fp::compute_units() / Hc;
+  auto rows = [&](int s) { return static_cast<int64_t>(B) * ((max_context + s - 1) / s - 1); };
+  if (2 * rows(64) >= chunks && !few_sequences(chunks, B))
+    while (split > 64 && rows(split) < chunks) split >>= 1;
   while (split / page_size + 2 > kMaxSplitPages) split >>= 1;
   return split < 64 ? 64 : split;
 }
