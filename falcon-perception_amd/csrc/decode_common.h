@@ -1,0 +1,263 @@
+// Shared by the decode kernels (paged_decode.hip, paged_decode_mfma.hip): their arguments, the plan of a step, the even
+// cut of a launch, the sink gate and lane exchanges.
+#pragma once
+
+#include "fp_common.h"
+
+#include <math.h>
+
+namespace fp_decode {
+
+constexpr int kMaxSplitPages = 1024;  // page ids of one split held in LDS
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLn2 = 0.6931471805599453f;
+
+struct DecodeArgs {
+  const char* q;
+  int64_t qs_b, qs_h;  // bytes
+  const char* pool_k;
+  const char* pool_v;
+  const int64_t* page_table;
+  int64_t pt_row_stride;
+  const int64_t* batch_idx;
+  const void* input_pos;
+  int pos_i64;
+  char* out;
+  int64_t os_b, os_h;  // bytes
+  float* lse;
+  const float* sinks;  // optional [Hq]: out is multiplied by sigmoid(lse - sinks[h])
+  float* ws_acc;  // [B, Hq, n_splits, D]
+  float* ws_ml;   // [B, Hq, n_splits, 2]
+  int Hq, Hc;
+  fp::PageDiv pd;
+  int n_pages, max_batch;
+  int64_t n_slots;
+  int max_context;
+  int split_tokens;
+  int n_splits;
+  float qscale;  // scale * log2(e)
+  // fused append (optional): the row of the newest token of every sequence, [B, Hc, 1, D]
+  const char* k_new;
+  const char* v_new;
+  int64_t kn_b, kn_h, vn_b, vn_h;  // bytes
+  int B;         // sequences of the launch
+  int n_chunks;  // even cut (kFlat): workgroups per cache head
+  int* plan;     // optional: the step's plan of the even cut (fp_paged_decode_plan), kPlanInts ints per chunk
+};
+
+// The plan of a decode step: what every workgroup of the even cut needs before it can ask for its first K row,
+// computed once per step instead of once per layer and workgroup.  Per chunk (workgroup of a cache head):
+//   rec[0]            pieces of the chunk, or -1: no plan for this chunk (more pieces or pages than a record
+//                     holds), the workgroup works everything out itself
+//   rec[1 .. 3]       B, n_chunks, max_context of the launch the plan was made for: a workgroup that finds other
+//                     values ignores the plan
+//   rec[4 + 6 k ..]   piece k: sequence, first token, tokens, raw length (position + 1), row of the page table
+//                     (-1: not a valid slot), offset of its page ids in the chunk's list
+//   pages[..]         page ids of the pieces, piece after piece (unmapped or foreign pages as 0, like the kernel
+//                     stages them)
+//   chunk 0, rec[126]  a hash of the positions and slots the plan was made from (plan_hash_term)
+// The positions, the slots and the page table must not change between the plan and the launches that use it.
+// What the launches do if they did: the merge pass recomputes the hash from the step's positions and slots
+// (it reads them anyway) and stores NaN in every row of out and lse when it differs, so a stale plan fails
+// loudly.  The split-K pass itself does not look (a check of its own position before the fused append's store
+// measured 1.2 us per launch): with a stale plan the fresh rows of the sequences that moved land where the plan
+// says.
+constexpr int kPlanPieces = 20;
+constexpr int kPlanHashAt = 126;
+constexpr int kPlanRec = 128;            // 4 + 6 * kPlanPieces, rounded up
+constexpr int kPlanPages = kMaxSplitPages;
+constexpr int kPlanInts = kPlanRec + kPlanPages;
+static_assert(4 + 6 * kPlanPieces <= kPlanHashAt && kPlanHashAt < kPlanRec, "a record holds its pieces and the hash");
+
+// Contribution of sequence b to the hash of a step's positions and slots (summed over the sequences, mod 2^32).
+__device__ __forceinline__ uint32_t plan_hash_term(int b, int64_t L, int64_t trow) {
+  const uint32_t w = 2u * static_cast<uint32_t>(b) + 1u;
+  return (static_cast<uint32_t>(L) + static_cast<uint32_t>(trow) * 0x9E3779B1u) * w;
+}
+
+// Attention-sink gate of the caller's post-attention step (model.py:122-128), applied where the
+// output row and its lse are final: the reference multiplies the attention output, already rounded
+// to the model dtype, by sigmoid(lse - sinks[h]) in fp32 and rounds again.
+template <typename E>
+__device__ __forceinline__ float sink_gate(float o, float lse_nat, const float* sinks, int hq) {
+  if (sinks == nullptr) return o;
+  const float g = 1.f / (1.f + __expf(sinks[hq] - lse_nat));
+  return E::round(o) * g;
+}
+
+// ---- cross-lane helpers ---------------------------------------------------
+template <int kCtrl>
+__device__ __forceinline__ float dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xf, 0xf, true));
+}
+
+// Sum over the kLanes consecutive lanes that share a row; every lane gets the total.
+// All kN values advance one butterfly step at a time, so back-to-back DPP
+// instructions are independent of each other.
+template <int kLanes, int kN>
+__device__ __forceinline__ void row_sum(float (&x)[kN]) {
+#pragma unroll
+  for (int i = 0; i < kN; ++i) if (kLanes >= 2) x[i] += dpp<0xB1>(x[i]);   // quad_perm [1,0,3,2]
+#pragma unroll
+  for (int i = 0; i < kN; ++i) if (kLanes >= 4) x[i] += dpp<0x4E>(x[i]);   // quad_perm [2,3,0,1]
+#pragma unroll
+  for (int i = 0; i < kN; ++i) if (kLanes >= 8) x[i] += dpp<0x141>(x[i]);  // row_half_mirror
+#pragma unroll
+  for (int i = 0; i < kN; ++i) if (kLanes >= 16) x[i] += dpp<0x140>(x[i]); // row_mirror
+#pragma unroll
+  for (int i = 0; i < kN; ++i) if (kLanes >= 32) x[i] += __shfl_xor(x[i], 16);
+#pragma unroll
+  for (int i = 0; i < kN; ++i) if (kLanes >= 64) x[i] += __shfl_xor(x[i], 32);
+}
+
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+__device__ __forceinline__ float safe_max(float m) { return m == -INFINITY ? 0.f : m; }
+
+// tokens per split of a context of L tokens: L is divided evenly over ceil(L / split_tokens)
+// splits, rounded up to 64 tokens (so every split starts on a wavefront-iteration boundary)
+__device__ __forceinline__ int split_part(int L, int split_tokens) {
+  if (L <= 0) return split_tokens;
+  const int n = (L + split_tokens - 1) / split_tokens;
+  const int even = (L + n - 1) / n;
+  return (even + 63) & ~63;
+}
+
+// Even cut of a launch (kFlat): the contexts of the launch, each rounded up to 64 tokens, are laid end
+// to end and cut into n_chunks pieces of equal length.  Sequence b starts at flat_start[b]; chunk c covers
+// [c * len, (c + 1) * len); a chunk that spans several sequences works through them one after another.
+constexpr int kFlatMaxB = 1024;
+
+// Start of every sequence on the flat axis -> s_start[0 .. B] (s_start[B] = total), by one wavefront.
+__device__ __forceinline__ void flat_starts(const DecodeArgs& a, int* s_start) {
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    const int per = (a.B + 63) / 64;  // consecutive sequences per lane
+    int sum = 0;
+    for (int i = 0; i < per; ++i) {
+      const int b = lane * per + i;
+      int Lr = 0;
+      if (b < a.B) {
+        int64_t L = fp::load_index(a.input_pos, b, a.pos_i64) + 1;
+        const int64_t trow = a.batch_idx[b];
+        if (trow < 0 || trow >= a.max_batch || L < 0) L = 0;
+        if (L > a.max_context) L = a.max_context;
+        Lr = (static_cast<int>(L) + 63) & ~63;
+      }
+      sum += Lr;
+    }
+    int incl = sum;  // inclusive scan over the lanes
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(incl, off);
+      if (lane >= off) incl += up;
+    }
+    int run = incl - sum;
+    for (int i = 0; i < per; ++i) {
+      const int b = lane * per + i;
+      if (b > a.B) break;
+      s_start[b] = run;
+      if (b < a.B) {
+        int64_t L = fp::load_index(a.input_pos, b, a.pos_i64) + 1;
+        const int64_t trow = a.batch_idx[b];
+        if (trow < 0 || trow >= a.max_batch || L < 0) L = 0;
+        if (L > a.max_context) L = a.max_context;
+        run += (static_cast<int>(L) + 63) & ~63;
+      }
+    }
+    if (lane == 63 && a.B == 64 * per) s_start[a.B] = incl;
+  }
+}
+
+// tokens per chunk of the even cut
+__device__ __forceinline__ int flat_chunk_len(int total, int n_chunks) {
+  const int len = (total + n_chunks - 1) / n_chunks;
+  return len < 64 ? 64 : (len + 63) & ~63;
+}
+
+// What a workgroup does with its cut: piece(sequence, first token, tokens, whether it is the sequence's first piece, and
+// where its partial result goes: workspace row head * part_mul + part_add; then the record and the page ids of a planned piece).
+
+// Grid (workgroup heads, B, splits).
+template <class Piece>
+__device__ __forceinline__ void walk_split(const DecodeArgs& a, const Piece& piece) {
+  // A context of L tokens is cut into ceil(L / split_tokens) parts of equal
+  // size (a multiple of 64 tokens), so the workgroups of one sequence carry the same load instead of
+  // leaving a short tail split.
+  // The workgroup dispatcher deals consecutive workgroups of an XCD to its four shader engines in turn
+  // and starts them in order, so with grid y = sequence every split of a sequence would land on the
+  // same engine and an engine's load would be the lengths of "its" sequences (12 % apart at 64
+  // sequences of 1 k to 4 k tokens).  Rotating the sequences by the split index spreads each sequence
+  // over the engines.
+  const int split = blockIdx.z;
+  const int b = static_cast<int>((blockIdx.y + blockIdx.z) % gridDim.y);
+  int64_t L = fp::load_index(a.input_pos, b, a.pos_i64) + 1;
+  if (L > a.max_context) L = a.max_context;
+  const int part = split_part(static_cast<int>(L < 0 ? 0 : L), a.split_tokens);
+  piece(b, split * part, part, split == 0, a.n_splits, static_cast<int64_t>(b) * a.Hq * a.n_splits + split);
+}
+
+// Grid (workgroup heads, n_chunks): every workgroup streams the same number of rows, whatever the lengths are.  `s_start`
+// holds kFlatMaxB + 1 ints, `s_pages` kMaxSplitPages.
+template <int kThreads, class Piece>
+__device__ __forceinline__ void walk_even_cut(const DecodeArgs& a, int* s_start, int* s_pages, const Piece& piece) {
+  const int tid = threadIdx.x;
+  if (a.plan) {
+    // the chunk's record goes where the sequence starts would go, its page ids where a piece stages its own:
+    // one trip to memory instead of positions -> cut -> page table
+    const int* src = a.plan + static_cast<int64_t>(blockIdx.y) * kPlanInts;
+    if (tid < kPlanRec) s_start[tid] = src[tid];
+    s_pages[tid] = src[kPlanRec + tid];  // the first kThreads page ids; more only for very long chunks
+    __syncthreads();
+    const int n = s_start[0];
+    if (n >= 0 && n <= kPlanPieces && s_start[1] == a.B && s_start[2] == a.n_chunks && s_start[3] == a.max_context) {
+      int n_pages_used = 0;
+      if (n > 0) {
+        const int* last = s_start + 4 + 6 * (n - 1);
+        n_pages_used = last[5] + last[2] / a.pd.page_size + 2;  // an upper bound of the list's length
+      }
+      if (n_pages_used > kThreads) {
+        for (int i = kThreads + tid; i < n_pages_used && i < kPlanPages; i += kThreads) s_pages[i] = src[kPlanRec + i];
+        __syncthreads();
+      }
+      const int c = blockIdx.y;
+      // the records are read from registers of a copy: a piece reuses s_start's LDS for nothing, but keeps s_pages
+      for (int k = 0; k < n; ++k) {
+        int r[6];
+#pragma unroll
+        for (int j = 0; j < 6; ++j) r[j] = s_start[4 + 6 * k + j];
+        piece(r[0], r[1], r[2], false, 1, static_cast<int64_t>(c + r[0]) * a.Hq, r, s_pages + r[5]);
+        __syncthreads();  // the LDS of the piece is free again
+      }
+      return;
+    }
+    __syncthreads();  // no usable plan: s_start and s_pages are written anew below
+  }
+  flat_starts(a, s_start);
+  __syncthreads();
+  const int total = s_start[a.B];
+  const int len = flat_chunk_len(total, a.n_chunks);
+  const int c = blockIdx.y;
+  const int64_t lo = static_cast<int64_t>(c) * len;
+  const int64_t hi = lo + len < total ? lo + len : total;
+  if (lo >= total) return;
+  // first sequence that ends after lo
+  int b = 0;
+  {
+    int left = 0, right = a.B - 1;
+    while (left < right) {
+      const int mid = (left + right) >> 1;
+      if (s_start[mid + 1] > lo) right = mid; else left = mid + 1;
+    }
+    b = left;
+  }
+  for (; b < a.B && s_start[b] < hi; ++b) {
+    const int begin = s_start[b], end = s_start[b + 1];
+    if (end == begin) continue;  // a sequence without keys has no piece; the merge pass writes its zeros
+    const int t0 = lo > begin ? static_cast<int>(lo - begin) : 0;
+    const int t1 = static_cast<int>((hi < end ? hi : end) - begin);
+    piece(b, t0, t1 - t0, false, 1, static_cast<int64_t>(c + b) * a.Hq);
+    __syncthreads();  // the LDS of the piece is free again
+  }
+}
+
+}  // namespace fp_decode

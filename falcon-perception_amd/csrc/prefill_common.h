@@ -26,6 +26,18 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, c
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(m0v), "v"(offset), "s"(base) : "memory");
 }
 
+// Both forms for rows that are read once (non-temporal, so that they do not displace what the caches hold).
+__device__ __forceinline__ void load_to_lds_nt(const char* src, char* lds) {
+  const uint32_t base = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" : : "s"(base), "v"(src) : "memory");
+}
+__device__ __forceinline__ void load_to_lds_nt(const char* base, uint32_t offset, char* lds) {
+  const uint32_t m0v = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" : : "s"(m0v), "v"(offset), "s"(base) : "memory");
+}
+
 // max(x of lane l, x of lane l ^ 32) in both lanes, without the trip through LDS a shuffle takes:
 // v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second, so
 // from (x, x) it leaves the lower halves' values in one register and the upper halves' in the other.

@@ -1,0 +1,52 @@
+"""GPU parity: the matrix-core decode kernel (16-bit caches, four or eight query heads per cache head) against the float64
+oracle, at the edges of its stages (16 tokens at head_dim 128, 32 at 64), on pages that hold whole stages and pages that do
+not, for every way a launch is cut."""
+
+import numpy as np
+import pytest
+import torch
+
+from falcon_perception_amd import ops
+from oracle import paged_kv_oracle as O
+from tests.gpu_cases import DEV, PagedState, f64, randn
+
+pytestmark = pytest.mark.gpu
+
+# A result is rounded once to the type (half a unit in the last place: at most 2^-8 of the value in bf16, 2^-11 in f16).  The probabilities keep 16
+# (bf16) or 22 (f16) bits, so the sum before that rounding is off by at most 2^-16 of the largest |v| (below 6 here), and
+# the hardware's exp2 and log2 add about 2^-20.
+TOL = {torch.bfloat16: (2.0 ** -8 * 1.01, 6 * 2.0 ** -16 + 2e-5), torch.float16: (2.0 ** -11 * 1.01, 6 * 2.0 ** -21 + 2e-5)}
+
+EDGES = [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 257]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("G,P", [(4, 32), (4, 24), (8, 64), (8, 16)])
+@pytest.mark.parametrize("cut", ["one split", "split by split", "even"])
+@pytest.mark.parametrize("spread", [1.0, 6.0], ids=["scores-N01", "scores-spread"])
+def test_matrix_core_decode(dtype, D, G, P, cut, spread):
+    Hc = 2
+    lens = EDGES if cut != "even" else EDGES * 18  # tokens with the new one; 288 sequences fill the 256 chunks' rows
+    split, limit = {"one split": (512, 288), "split by split": (64, 288), "even": (128, 384)}[cut]
+    B = len(lens)
+    limit = -(-limit // P) * P
+    st = PagedState(300 + D + G, n_pages=max(limit // P, sum(-(-L // P) for L in lens)) + 4, page_size=P, max_batch=B + 2,
+                    Hc=Hc, D=D, dtype=dtype)
+    for L in lens:
+        st.add_sequence(L)
+    st.prefill_random()
+    q = (randn(st.gen, (B, Hc * G, 1, D), torch.float32) * spread).to(dtype).to(DEV)
+    k_new, v_new = (randn(st.gen, (B, Hc, 1, D), dtype).to(DEV) for _ in range(2))
+    pos = torch.tensor(lens, dtype=torch.int32, device=DEV) - 1
+    bidx = torch.tensor(st.slots, dtype=torch.int64, device=DEV)
+    pk, pv = st.pool_planes()
+    out, lse = ops.paged_decode(q, pk, pv, st.cache.page_table, bidx, pos, P, limit, split_tokens=split, k_new=k_new,
+                                v_new=v_new)
+    for b, L in enumerate(lens):  # the fresh rows are in their slots
+        slot = int(st.cache.page_table[st.slots[b], (L - 1) // P]) * P + (L - 1) % P
+        assert torch.equal(pk[:, slot], k_new[b, :, 0]) and torch.equal(pv[:, slot], v_new[b, :, 0])
+    eo, el = O.decode_attention(f64(q), f64(pk), f64(pv), st.mirror.page_table, st.slots, np.array(lens) - 1, P)
+    rtol, atol = TOL[dtype]
+    np.testing.assert_allclose(f64(out), eo, rtol=rtol, atol=atol)
+    np.testing.assert_allclose(f64(lse), el, rtol=1e-5, atol=1e-5)
