@@ -40,6 +40,9 @@ constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 constexpr int kTileN = 64;  // keys per tile
 constexpr int kSlotTable = 2048;  // tiles of a run whose first pool slot is looked up ahead of the tile loop
+constexpr int kMinShareTiles = 8;  // key tiles a key share has at least
+constexpr float kRowFinished = -1.f;  // in the place of share 0's denominator: the row is stored, the merge pass leaves it alone
+constexpr int kTailSlot = -2;     // table entries at or below it: a tile that ends past the run's last key
 constexpr float kMaxSlack = 6.f;  // the running maximum may lag a row's true maximum by this much (log2)
 constexpr int kPrefetchK = 4; // K operand reads in flight ahead of the MFMA that uses them
 constexpr int kPrefetchV = 4; // V^T operand read pairs in flight ahead of their MFMA
@@ -153,28 +156,32 @@ struct Swizzle {
 // 32 query rows: every head of the group works from the same staged K/V tile, so the bytes that
 // travel from L2 into LDS (64 B per cycle and CU, and a wavefront waits at its load instructions
 // while that path is busy) are shared by all of them.
-template <typename E, int D, int G, bool kPow2, int W = kWaves, bool kBounded = false>
+//
+// KG = 2: the two halves of the workgroup have the same query rows (half as many) and take the key tiles in turn, each half from
+// buffers of its own; their states meet in LDS at the end.  See launch_group for the launches that go out so.
+template <typename E, int D, int G, bool kPow2, int W = kWaves, bool kBounded = false, int KG = 1>
 __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_prefill_kernel(const PrefillArgs a) {
   constexpr int kThreads = W * 64;  // shadows the file-scope constant: W wavefronts per workgroup
   using SW = Swizzle<D>;
   constexpr int MB = 1;                    // 32-row blocks per wavefront
-  constexpr int RB = W / G;                // 32-row blocks per workgroup
+  constexpr int ITEMS = W / KG;            // (row block, query head) pairs; so many wavefronts stage a tile
+  constexpr int RB = ITEMS / G;            // 32-row blocks per workgroup
   constexpr int BM = RB * 32;              // query rows per workgroup
   constexpr int ROWB = D * 2;              // bytes of a K/V row
   constexpr int CPR = SW::CPR;
   constexpr int R32 = SW::R32;
   constexpr int RPI = 64 / CPR;            // rows one wavefront load instruction brings in
-  constexpr int NI = kTileN / (RPI * W);   // load instructions per wavefront, tile and tensor
+  constexpr int NI = kTileN / (RPI * ITEMS);  // load instructions per wavefront, tile and tensor
   constexpr int DS = D / 16;               // MFMA k-steps over head_dim
   constexpr int DB = D / 32;               // 32-wide blocks of head_dim in O^T
   constexpr int TILE_BYTES = kTileN * ROWB;
 
   // four separate arrays (not one indexed array) so that a load into one buffer is known not to
   // alias the reads of the other
-  __shared__ __attribute__((aligned(1024))) char s_k0[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char s_k1[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char s_v0[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char s_v1[TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char s_k0[KG * TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char s_k1[KG * TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char s_v0[KG * TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char s_v1[KG * TILE_BYTES];
   __shared__ int s_bidx[BM];
   __shared__ int s_red[W];
   __shared__ int s_tslot[kSlotTable];
@@ -192,8 +199,10 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   }
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int hq = hc * G + wave % G;  // query head of this wavefront
-  const int rblock = wave / G;       // its block of 32 rows inside the tile
+  const int kg = KG == 1 ? 0 : wave / ITEMS;  // key group
+  const int item = KG == 1 ? wave : wave % ITEMS;
+  const int hq = hc * G + item % G;  // query head of this wavefront
+  const int rblock = item / G;       // its block of 32 rows inside the tile
   const int lane = tid & 63;
   const int half = lane >> 5;   // which 8 of 16 k-values / which 4 of 8 rows this lane holds
   const int ln = lane & 31;     // query column (S^T, O^T) or key row (K operand)
@@ -243,11 +252,11 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   const char* vplane = a.pool_v + static_cast<int64_t>(hc) * a.n_slots * ROWB;
 
   // ---- per-lane constants of the staging loads and of the operand reads ----
-  // load instruction i of this wavefront fills LDS rows (i * W + wave) * RPI .. + RPI; this lane
+  // load instruction i of this wavefront fills LDS rows (i * ITEMS + item) * RPI .. + RPI; this lane
   // fills position lp of row lrow in that group.  kswz / vrot of the row do not depend on i.
   const int lrow = lane / CPR;
   const int lp = lane % CPR;
-  const int st_row0 = wave * RPI + lrow;  // row of load instruction 0; instruction i adds i * W * RPI
+  const int st_row0 = item * RPI + lrow;  // row of load instruction 0; instruction i adds i * ITEMS * RPI
   const int k_src_off = (lp ^ SW::kswz(st_row0)) * 16;
   const int v_src_off = ((((lp >> 1) + R32 - SW::vrot(st_row0)) % R32) * 2 + (lp & 1)) * 16;
   // K operand: row kb * 32 + ln, chunk 2 * ds + half at position (2 * ds) ^ ksel
@@ -289,19 +298,15 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       // padding rows: out = 0, lse = -inf
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        if (!active[mb]) continue;
-        if (gridDim.z > 1) {  // an empty share; the merge pass then writes out = 0, lse = -inf
-          const int64_t p = (static_cast<int64_t>(blockIdx.z) * a.Lq + row[mb]) * a.Hq + hq;
-#pragma unroll
-          for (int c = 0; c < D / 8; ++c) *reinterpret_cast<uint2*>(a.ws_acc + p * D + half * (D / 2) + c * 4) = uint2{0, 0};
-          if (half == 0) *reinterpret_cast<float2*>(a.ws_ml + p * 2) = float2{-INFINITY, 0.f};
-          continue;
-        }
+        if (!active[mb] || kg != 0 || blockIdx.z != 0) continue;
         // a row is 2 * D bytes; each lane half clears D of them
         char* o = a.out + row[mb] * a.os_row + hq * a.os_h + half * D;
 #pragma unroll
         for (int c = 0; c < D / 8; ++c) *reinterpret_cast<uint2*>(o + c * 8) = uint2{0, 0};
-        if (half == 0) a.lse[static_cast<int64_t>(hq) * a.Lq + row[mb]] = -INFINITY;
+        if (half == 0) {
+          a.lse[static_cast<int64_t>(hq) * a.Lq + row[mb]] = -INFINITY;
+          if (gridDim.z > 1) a.ws_ml[(static_cast<int64_t>(row[mb]) * a.Hq + hq) * 2 + 1] = kRowFinished;
+        }
       }
       run0 = run1;
       continue;
@@ -327,10 +332,24 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     for (int w = 0; w < W; ++w) kv_max = max(kv_max, s_red[w]);
     kv_max = __builtin_amdgcn_readfirstlane(kv_max);
     const int n_run_tiles = (kv_max + kTileN - 1) / kTileN;
+    // Key shares of the run: the grid has as many as may pay, but only the kernel knows how long the run's range is
+    const int z = blockIdx.z;
+    int n_shares = 1;
+    if (gridDim.z > 1) {
+      n_shares = min(max(n_run_tiles / kMinShareTiles, 1), static_cast<int>(gridDim.z));
+      if (z >= n_shares) {
+        if (n_shares > 1 && active[0] && kg == 0 && half == 0)  // a share without keys
+          *reinterpret_cast<float2*>(a.ws_ml + ((static_cast<int64_t>(z) * a.Lq + row[0]) * a.Hq + hq) * 2) =
+              float2{-INFINITY, 0.f};
+        run0 = run1;
+        continue;
+      }
+    }
     // this workgroup's share of the run's key tiles: [kt_lo, n_kv_tiles)
-    const int kt_lo = static_cast<int>(static_cast<int64_t>(n_run_tiles) * blockIdx.z / gridDim.z);
-    const int n_kv_tiles = static_cast<int>(static_cast<int64_t>(n_run_tiles) * (blockIdx.z + 1) / gridDim.z);
-    const int n_my = n_kv_tiles - kt_lo;
+    const int kt_lo = static_cast<int>(static_cast<int64_t>(n_run_tiles) * z / n_shares);
+    const int n_kv_tiles = static_cast<int>(static_cast<int64_t>(n_run_tiles) * (z + 1) / n_shares);
+    const int n_my = (n_kv_tiles - kt_lo + KG - 1) / KG;  // steps
+    const int kt_my = kt_lo + kg;                           // step i of this wavefront works on key tile kt_my + KG * i
 
     f32x16 o_acc[MB][DB];
     float m_run[MB], l_run[MB];
@@ -344,29 +363,33 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
 
     // ---- K/V fetch pipeline ----
     // Every wavefront stages NI groups of RPI rows of each tile.  Where a page holds whole tiles
-    // (page size a power of two, at least the tile), a tile that lies before the run's last key in a
-    // mapped page is contiguous in the pool: its first slot is looked up once per run into s_tslot,
-    // and a staging load is then a scalar base plus a fixed offset per lane.  Any other tile (the
-    // last one of a run, small or odd page sizes, unmapped pages, runs longer than the table) is
-    // staged row by row: a key that does not exist (past the run's last key, or an unmapped page)
-    // reads slot 0, finite bytes, and every such key is masked.
+    // (page size a power of two, at least the tile), a tile in a mapped page is contiguous in the
+    // pool: its first slot is looked up once per run into s_tslot, and a staging load is then a
+    // scalar base plus a fixed offset per lane.  In the last tile of a run the rows past the last key
+    // read that key's row again: a page behind the last key may hold anything, and these keys are masked,
+    // but 0 x inf is not 0.  (Staged row by row, every load instruction of such a tile waits for a page
+    // id of its own, about 5000 cycles a run.)  Any other tile (small or odd page sizes, unmapped pages,
+    // runs longer than the table) is staged row by row: a key that does not exist (past the run's
+    // last key, or an unmapped page) reads slot 0, finite bytes, and every such key is masked.
     const int64_t* pt_row = a.page_table + static_cast<int64_t>(sq) * a.pt_row_stride;
     const int64_t pool_pages = a.n_slots / a.pd.page_size;
     const bool page_holds_tile = kPow2 && a.pd.page_size % kTileN == 0;
+    const int tail_row = (kv_max - 1) % kTileN;  // row of the last key in the last tile
     for (int t = kt_lo + tid; t < n_kv_tiles && t - kt_lo < kSlotTable; t += kThreads) {
       int slot = -1;
-      if (page_holds_tile && (t + 1) * kTileN <= kv_max) {
+      if (page_holds_tile) {
         const int key0 = t * kTileN;
         const int blk = key0 >> a.pd.shift;
         if (blk < a.n_pages) {
           const int64_t pg = pt_row[blk];
           if (pg >= 0 && pg < pool_pages) slot = static_cast<int>(pg) * a.pd.page_size + (key0 & (a.pd.page_size - 1));
+          if (slot >= 0 && key0 + kTileN > kv_max) slot = kTailSlot - slot;
         }
       }
       s_tslot[t - kt_lo] = slot;
     }
     __syncthreads();
-    // first pool slot of tile kt, or -1: wavefront-uniform
+    // first pool slot of tile kt, kTailSlot minus it for the tile with the last key, or -1: wavefront-uniform
     auto tile_slot = [&](int kt) {
       return __builtin_amdgcn_readfirstlane((kt >= kt_lo && kt < n_kv_tiles && kt - kt_lo < kSlotTable) ? s_tslot[kt - kt_lo] : -1);
     };
@@ -385,21 +408,26 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     uint32_t lane_k[NI], lane_v[NI];  // byte offset of this lane's 16 bytes from the first row of a tile
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      lane_k[i] = (i * W * RPI + st_row0) * ROWB + k_src_off;
-      lane_v[i] = (i * W * RPI + st_row0) * ROWB + v_src_off;
+      lane_k[i] = (i * ITEMS * RPI + st_row0) * ROWB + k_src_off;
+      lane_v[i] = (i * ITEMS * RPI + st_row0) * ROWB + v_src_off;
     }
-    // One staging load of tile kt, whose first slot is ts (or -1): pieces 0 .. NI - 1 are the V loads
+    // One staging load of tile kt, whose table entry is ts: pieces 0 .. NI - 1 are the V loads
     // of the row groups, NI .. 2 NI - 1 the K loads.  Tiles past the run's last one are not staged.
     auto fetch_piece = [&](int piece, int kt, int ts, char* dst) {
       if (kt >= n_kv_tiles) return;
       const int i = piece % NI;
       const bool is_k = piece >= NI;
-      char* lds = dst + (i * W + wave) * RPI * ROWB;  // wavefront-uniform
+      char* lds = dst + kg * TILE_BYTES + (i * ITEMS + item) * RPI * ROWB;  // wavefront-uniform
       if (ts >= 0) {
         load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(ts) * ROWB, is_k ? lane_k[i] : lane_v[i], lds);
+      } else if (ts <= kTailSlot) {
+        asm volatile("");  // once per run
+        const int past = i * ITEMS * RPI + st_row0 - tail_row;
+        const uint32_t off = (is_k ? lane_k[i] : lane_v[i]) - (past > 0 ? past : 0) * ROWB;
+        load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(kTailSlot - ts) * ROWB, off, lds);
       } else {
         asm volatile("");  // rare: keep it out of the way as a branch
-        const int kpos = kt * kTileN + i * W * RPI + st_row0;
+        const int kpos = kt * kTileN + i * ITEMS * RPI + st_row0;
         int blkid, off;
         key_block(kpos, blkid, off);
         const bool in_range = kpos < kv_max && blkid < a.n_pages;
@@ -413,10 +441,10 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     // per-lane LDS offsets of the operand reads, the same for every tile and buffer
     int kofs[DS], vofs[DB];
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) kofs[ds] = ln * ROWB + (((2 * ds) ^ ksel) * 16);
+    for (int ds = 0; ds < DS; ++ds) kofs[ds] = kg * TILE_BYTES + ln * ROWB + (((2 * ds) ^ ksel) * 16);
 #pragma unroll
     for (int db = 0; db < DB; ++db)
-      vofs[db] = (half * 4 + (bi >> 2)) * ROWB + (bi & 3) * 8 + ((2 * db + vsel) % R32) * 32;
+      vofs[db] = kg * TILE_BYTES + (half * 4 + (bi >> 2)) * ROWB + (bi & 3) * 8 + ((2 * db + vsel) % R32) * 32;
 
     // ---- schedule ----
     // Step i of a wavefront is M(i) = { O^T += V^T P^T of tile i - 1;  S^T = K Q^T of tile i } on the
@@ -430,9 +458,9 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     // begins.  (A second barrier between the two parts of the interval kept the halves in step more
     // strictly and cost 2 %.)  K(i) lives in K buffer i % 2, V(i) in V buffer i % 2.
     {
-      const int ts0 = tile_slot(kt_lo);
+      const int ts0 = tile_slot(kt_my);
 #pragma unroll
-      for (int piece = NI; piece < 2 * NI; ++piece) fetch_piece(piece, kt_lo, ts0, s_k0);  // K of the first tile
+      for (int piece = NI; piece < 2 * NI; ++piece) fetch_piece(piece, kt_my, ts0, s_k0);  // K of the first tile
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's rows have landed in LDS
 
@@ -456,15 +484,15 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       const char* vprev = kBuf ? s_v0 : s_v1;  // V(i - 1)
       char* knext = kBuf ? s_k0 : s_k1;        // K(i + 1) goes here
       char* vcur = kBuf ? s_v1 : s_v0;         // V(i) goes here
-      const int key0 = (kt_lo + i) * kTileN;  // step i works on key tile kt_lo + i
-      const bool work_cur = i < n_my && key0 < wave_max;
-      const bool work_prev = i > 0 && key0 - kTileN < wave_max;
+      const int key0 = (kt_my + KG * i) * kTileN;
+      const bool work_cur = (KG == 1 ? i < n_my : kt_my + KG * i < n_kv_tiles) && key0 < wave_max;
+      const bool work_prev = i > 0 && (KG == 1 || kt_my + KG * (i - 1) < n_kv_tiles) && key0 - KG * kTileN < wave_max;
 
-      // the staging step this wavefront issues during the step: K of tile kt_k, V of tile kt_k - 1.
+      // the staging step this wavefront issues during the step: K of tile kt_k, V of the tile one step before it.
       // The table is read ahead of the barrier, whose wait hides the LDS latency.
-      const int kt_k = kt_lo + (kSecond ? i + 2 : i + 1);
+      const int kt_k = kt_my + KG * (kSecond ? i + 2 : i + 1);
       const int ts_k = tile_slot(kt_k);
-      const int ts_v = tile_slot(kt_k - 1);
+      const int ts_v = tile_slot(kt_k - KG);
       if (!kSecond) __builtin_amdgcn_s_waitcnt(0x0F70);  // staging step i - 1 of this wavefront has landed
       if (!kSecond) __builtin_amdgcn_s_barrier();
 
@@ -498,7 +526,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
         for (int t = 0; t < 4 * DB; ++t) {
           const s16x4 lo = rlo[t % kPrefetchV], hi = rhi[t % kPrefetchV];
           const s16x8 va = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          if (!kSecond && t % kPvEvery == 0) fetch_piece(t / kPvEvery, kt_k - 1, ts_v, vcur);
+          if (!kSecond && t % kPvEvery == 0) fetch_piece(t / kPvEvery, kt_k - KG, ts_v, vcur);
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) o_acc[mb][t % DB] = E::mfma(va, p_op[mb][t / DB], o_acc[mb][t % DB]);
           if (t + kPrefetchV < 4 * DB) read_v(t + kPrefetchV, rlo[t % kPrefetchV], rhi[t % kPrefetchV]);
@@ -506,7 +534,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
         }
       } else if (!kSecond) {
 #pragma unroll
-        for (int piece = 0; piece < NI; ++piece) fetch_piece(piece, kt_k - 1, ts_v, vcur);
+        for (int piece = 0; piece < NI; ++piece) fetch_piece(piece, kt_k - KG, ts_v, vcur);
       }
 
       // ---- M(i), second part: S^T = K Q^T for the two 32-key blocks of tile i ----
@@ -544,7 +572,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
         // staging step i + 1: K(i + 2) into the buffer of K(i), V(i + 1) into that of V(i - 1)
 #pragma unroll
         for (int piece = 0; piece < 2 * NI; ++piece)
-          fetch_piece(piece, piece < NI ? kt_k - 1 : kt_k, piece < NI ? ts_v : ts_k,
+          fetch_piece(piece, piece < NI ? kt_k - KG : kt_k, piece < NI ? ts_v : ts_k,
                       const_cast<char*>(piece < NI ? vprev : kcur));
       }
 
@@ -640,10 +668,10 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     } else {
       __builtin_amdgcn_s_barrier();  // B(0): the first half starts M(0)
       {  // staging step 0: K(1), V(0)
-        const int ts1 = tile_slot(kt_lo + 1), ts0 = tile_slot(kt_lo);
+        const int ts1 = tile_slot(kt_my + KG), ts0 = tile_slot(kt_my);
 #pragma unroll
         for (int piece = 0; piece < 2 * NI; ++piece)
-          fetch_piece(piece, piece < NI ? kt_lo : kt_lo + 1, piece < NI ? ts0 : ts1, piece < NI ? s_v0 : s_k1);
+          fetch_piece(piece, piece < NI ? kt_my : kt_my + KG, piece < NI ? ts0 : ts1, piece < NI ? s_v0 : s_k1);
       }
       for (int i = 0; i <= n_my; i += 2) {
         step(IntC<1>{}, IntC<0>{}, i);
@@ -652,109 +680,161 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // no staging load is in flight when the LDS tiles are reused
 
-    // ---- finish the run: normalise and store ----
+    // ---- finish the run ----
+    float l_tot = l_run[0] + __shfl_xor(l_run[0], 32);
+    float m_tot = m_run[0];
+    constexpr int PB = DB / KG;  // blocks of O^T a wavefront finishes
+    if constexpr (KG == 2) {
+      // the two states of a row meet: each wavefront hands the blocks it does not finish, at the common reference point, to the
+      // other one of its item
+      __shared__ float s_m[W][32], s_l[W][32];
+      if (half == 0) {
+        s_m[wave][ln] = m_tot;
+        s_l[wave][ln] = l_tot;
+      }
+      __syncthreads();  // and every tile has been read
+      const int other = kg == 0 ? wave + ITEMS : wave - ITEMS;
+      const float m_other = s_m[other][ln];
+      const float m_both = fmaxf(m_tot, m_other), m_safe = m_both == -INFINITY ? 0.f : m_both;
+      const float mine = fast_exp2(m_tot - m_safe);
+      l_tot = fmaf(l_tot, mine, s_l[other][ln] * fast_exp2(m_other - m_safe));
+      m_tot = m_both;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const float l_tot = l_run[mb] + __shfl_xor(l_run[mb], 32);
+      for (int db = 0; db < DB; ++db) o_acc[0][db] *= mine;
+      static_assert(PB * 4096 * ITEMS <= KG * TILE_BYTES, "a half's blocks fit one buffer");
+      f32x4* const give = reinterpret_cast<f32x4*>((kg == 0 ? s_k0 : s_v0) + item * (PB * 4096)) + lane;
+      f32x4* const take = reinterpret_cast<f32x4*>((kg == 0 ? s_v0 : s_k0) + item * (PB * 4096)) + lane;
+      if (kg == 0) {
+#pragma unroll
+        for (int j = 0; j < PB * 4; ++j) {
+          const f32x16& o = o_acc[0][PB + j / 4];
+          give[j * 64] = f32x4{o[j % 4 * 4], o[j % 4 * 4 + 1], o[j % 4 * 4 + 2], o[j % 4 * 4 + 3]};
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < PB * 4; ++j) {
+          const f32x16& o = o_acc[0][j / 4];
+          give[j * 64] = f32x4{o[j % 4 * 4], o[j % 4 * 4 + 1], o[j % 4 * 4 + 2], o[j % 4 * 4 + 3]};
+        }
+#pragma unroll
+        for (int db = 0; db < PB; ++db) o_acc[0][db] = o_acc[0][PB + db];  // the blocks to finish come first
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < PB * 4; ++j) {
+        const f32x4 x = take[j * 64];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o_acc[0][j / 4][j % 4 * 4 + c] += x[c];
+      }
+    }
+    const int d0 = kg * PB * 32;  // first element of the blocks of this wavefront
+    if (active[0]) {
       const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-      if (!active[mb]) continue;
-      if (gridDim.z > 1) {
-        // one of several key shares: the unnormalised state goes to the merge pass
-        const int64_t p = (static_cast<int64_t>(blockIdx.z) * a.Lq + row[mb]) * a.Hq + hq;
-        short* po = a.ws_acc + p * D;
+      const bool writes_ml = half == 0 && kg == 0;
+      if (n_shares > 1) {
+        // one of several key shares: the state goes to the merge pass
+        const int64_t p = (static_cast<int64_t>(z) * a.Lq + row[0]) * a.Hq + hq;
+        short* po = a.ws_acc + p * D + d0;
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < PB; ++db)
 #pragma unroll
           for (int i4 = 0; i4 < 4; ++i4)
             *reinterpret_cast<uint2*>(po + db * 32 + i4 * 8 + half * 4) =
-                uint2{E::pack2(o_acc[mb][db][i4 * 4] * inv, o_acc[mb][db][i4 * 4 + 1] * inv),
-                      E::pack2(o_acc[mb][db][i4 * 4 + 2] * inv, o_acc[mb][db][i4 * 4 + 3] * inv)};
-        if (half == 0) *reinterpret_cast<float2*>(a.ws_ml + p * 2) = float2{m_run[mb], l_tot};
-        continue;
-      }
-      char* o = a.out + row[mb] * a.os_row + hq * a.os_h;
-      const float lse_nat = l_tot > 0.f ? (m_run[mb] + log2f(l_tot)) * kLn2 : -INFINITY;
-      // attention-sink gate of the caller's post-attention step (model.py:122-128): the output,
-      // rounded to the model dtype, times sigmoid(lse - sinks[h]) in fp32, rounded again
-      const bool gated = a.sinks != nullptr;
-      const float gate = gated ? 1.f / (1.f + __expf(a.sinks[hq] - lse_nat)) : 1.f;
-      auto fin = [&](float x) { return gated ? E::round(x * inv) * gate : x * inv; };
+                uint2{E::pack2(o_acc[0][db][i4 * 4] * inv, o_acc[0][db][i4 * 4 + 1] * inv),
+                      E::pack2(o_acc[0][db][i4 * 4 + 2] * inv, o_acc[0][db][i4 * 4 + 3] * inv)};
+        if (writes_ml) *reinterpret_cast<float2*>(a.ws_ml + p * 2) = float2{m_tot, l_tot};
+      } else {
+        char* o = a.out + row[0] * a.os_row + hq * a.os_h + d0 * 2;
+        const float lse_nat = l_tot > 0.f ? (m_tot + log2f(l_tot)) * kLn2 : -INFINITY;
+        // attention-sink gate of the caller's post-attention step (model.py:122-128): the output,
+        // rounded to the model dtype, times sigmoid(lse - sinks[h]) in fp32, rounded again
+        const bool gated = a.sinks != nullptr;
+        const float gate = gated ? 1.f / (1.f + __expf(a.sinks[hq] - lse_nat)) : 1.f;
+        auto fin = [&](float x) { return gated ? E::round(x * inv) * gate : x * inv; };
 #pragma unroll
-      for (int db = 0; db < DB; ++db) {
+        for (int db = 0; db < PB; ++db) {
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          // registers 4*i4 .. 4*i4+3 hold d = db*32 + i4*8 + half*4 + 0..3
-          const int d = db * 32 + i4 * 8 + half * 4;
-          const uint32_t w0 = E::pack2(fin(o_acc[mb][db][i4 * 4 + 0]), fin(o_acc[mb][db][i4 * 4 + 1]));
-          const uint32_t w1 = E::pack2(fin(o_acc[mb][db][i4 * 4 + 2]), fin(o_acc[mb][db][i4 * 4 + 3]));
-          *reinterpret_cast<uint2*>(o + d * 2) = uint2{w0, w1};
+          for (int i4 = 0; i4 < 4; ++i4) {
+            // registers 4*i4 .. 4*i4+3 hold d = db*32 + i4*8 + half*4 + 0..3
+            const int d = db * 32 + i4 * 8 + half * 4;
+            const uint32_t w0 = E::pack2(fin(o_acc[0][db][i4 * 4 + 0]), fin(o_acc[0][db][i4 * 4 + 1]));
+            const uint32_t w1 = E::pack2(fin(o_acc[0][db][i4 * 4 + 2]), fin(o_acc[0][db][i4 * 4 + 3]));
+            *reinterpret_cast<uint2*>(o + d * 2) = uint2{w0, w1};
+          }
+        }
+        if (writes_ml) {
+          a.lse[static_cast<int64_t>(hq) * a.Lq + row[0]] = lse_nat;
+          if (gridDim.z > 1) a.ws_ml[(static_cast<int64_t>(row[0]) * a.Hq + hq) * 2 + 1] = kRowFinished;
         }
       }
-      if (half == 0) a.lse[static_cast<int64_t>(hq) * a.Lq + row[mb]] = lse_nat;
     }
     run0 = run1;
   }
 }
 
 // ---- merge of the key shares ----
-// One wavefront per (query row, query head): combines the shares' results, each weighted by its
-// denominator at the common maximum, applies the sink gate, stores out and lse.
-constexpr int kMergeRows = 4;  // (row, head) pairs per workgroup
+// Combines the shares' results of a (query row, query head), each weighted by its denominator at the common maximum, applies the
+// sink gate, stores out and lse.  D / 8 lanes to an item, 16 bytes of its row each, every share requested at once: the pass is a
+// single trip to memory, so few wavefronts with wide loads (640 rows x 16 heads, D 128, five shares: the launch 28.6 us with a wavefront per
+// item, 25.0 us so).
+constexpr int kMergeThreads = 256;
 
 template <typename E, int D>
-__global__ __launch_bounds__(kMergeRows * 64) void paged_prefill_merge_kernel(const PrefillArgs a, int n_shares) {
-  constexpr int EPL = D / 64;  // output elements per lane
-  const int lane = threadIdx.x & 63;
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * kMergeRows + (threadIdx.x >> 6);
+__global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(const PrefillArgs a, int n_shares) {
+  constexpr int TPI = D / 8;  // lanes per item
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * (kMergeThreads / TPI) + threadIdx.x / TPI;
   if (item >= static_cast<int64_t>(a.Lq) * a.Hq) return;
+  const int col = threadIdx.x % TPI;
   const int row = static_cast<int>(item / a.Hq), hq = static_cast<int>(item % a.Hq);
   const int64_t share_stride = static_cast<int64_t>(a.Lq) * a.Hq;
   constexpr int kBatch = 8;  // the launcher never makes more shares
-  float m_s[kBatch], l_s[kBatch], acc_s[kBatch][EPL];
+  float2 ml[kBatch];
+  uint2 acc[kBatch][2];
 #pragma unroll
   for (int s = 0; s < kBatch; ++s) {
     const bool on = s < n_shares;
     const int64_t p = s * share_stride + item;
-    m_s[s] = on ? a.ws_ml[p * 2] : -INFINITY;
-    l_s[s] = on ? a.ws_ml[p * 2 + 1] : 0.f;
-    if (EPL == 2) {
-      const uint32_t w = on ? *reinterpret_cast<const uint32_t*>(a.ws_acc + p * D + lane * 2) : 0u;
-      acc_s[s][0] = E::to_float(static_cast<short>(w & 0xffffu));
-      acc_s[s][EPL - 1] = E::to_float(static_cast<short>(w >> 16));
-    } else {
-      acc_s[s][0] = on ? E::to_float(a.ws_acc[p * D + lane]) : 0.f;
-    }
+    ml[s] = on ? *reinterpret_cast<const float2*>(a.ws_ml + p * 2) : float2{-INFINITY, 0.f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      acc[s][h] = on ? *reinterpret_cast<const uint2*>(a.ws_acc + p * D + col * 8 + h * 4) : uint2{0u, 0u};
   }
+  if (ml[0].y == kRowFinished) return;
   float mn = -INFINITY;
 #pragma unroll
-  for (int s = 0; s < kBatch; ++s) mn = fmaxf(mn, m_s[s]);
+  for (int s = 0; s < kBatch; ++s) mn = fmaxf(mn, ml[s].x);
   const float ms = mn == -INFINITY ? 0.f : mn;
-  float den = 0.f, num[EPL];
+  float den = 0.f, num[8];
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) num[e] = 0.f;
+  for (int e = 0; e < 8; ++e) num[e] = 0.f;
 #pragma unroll
   for (int s = 0; s < kBatch; ++s) {
-    const float wgt = l_s[s] * fast_exp2(m_s[s] - ms);  // 0 for a share that saw no key
+    const float wgt = ml[s].y * fast_exp2(ml[s].x - ms);
     den += wgt;
+    if (ml[s].y == 0.f) continue;  // a share without keys: whatever its place in the workspace held stays out
+    const uint32_t w[4] = {acc[s][0].x, acc[s][0].y, acc[s][1].x, acc[s][1].y};
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) num[e] += acc_s[s][e] * wgt;
+    for (int e = 0; e < 8; ++e)
+      num[e] += E::to_float(static_cast<short>((e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu)) * wgt;
   }
   const float inv = den > 0.f ? 1.f / den : 0.f;
   const float lse_nat = den > 0.f ? (mn + log2f(den)) * kLn2 : -INFINITY;
   const bool gated = a.sinks != nullptr;
   const float gate = gated ? 1.f / (1.f + __expf(a.sinks[hq] - lse_nat)) : 1.f;
   auto fin = [&](float x) { return gated ? E::round(x * inv) * gate : x * inv; };
-  char* o = a.out + row * a.os_row + hq * a.os_h + lane * EPL * 2;
-  if (EPL == 2)
-    *reinterpret_cast<uint32_t*>(o) = E::pack2(fin(num[0]), fin(num[EPL - 1]));
-  else
-    *reinterpret_cast<short*>(o) = E::from_float(fin(num[0]));
-  if (lane == 0) a.lse[static_cast<int64_t>(hq) * a.Lq + row] = lse_nat;
+  char* o = a.out + row * a.os_row + hq * a.os_h + col * 16;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    *reinterpret_cast<uint2*>(o + h * 8) = uint2{E::pack2(fin(num[4 * h]), fin(num[4 * h + 1])),
+                                                 E::pack2(fin(num[4 * h + 2]), fin(num[4 * h + 3]))};
+  if (col == 0) a.lse[static_cast<int64_t>(hq) * a.Lq + row] = lse_nat;
 }
 
 constexpr int kMaxKeyShares = 8;
 
-// Key shares for a launch of `wgs` workgroups.  bf16 / f16: a launch that would leave at least half of the
+// Key shares for a launch of `wgs` workgroups, at most: the kernel makes fewer of a run without kMinShareTiles for each, down
+// to none (a share costs its partial results and the launch their merge; 613 keys of 16 heads: 28.6 us in five shares, 22.9 us
+// uncut).  bf16 / f16: a launch that would leave at least half of the
 // CUs idle is cut along the keys until every CU has a workgroup.  (With about one workgroup per CU
 // already, a cut in two costs more in partial results and their merge than the shorter critical path
 // saves: 138 us against 111 us at 8 sequences x 512 rows.)  fp32: the kernel takes about eight times as
@@ -782,23 +862,31 @@ bool bounded_path(float score_bound) {
   return std::is_same<E, BF16>::value && score_bound > 0.f && score_bound <= kMaxScoreBound;
 }
 
-template <typename E, int D, int G, bool kPow2, int W, bool kBounded>
+template <typename E, int D, int G, bool kPow2, int W, bool kBounded, int KG>
 void launch_instance(const PrefillArgs& a, dim3 grid, hipStream_t st) {
-  hipLaunchKernelGGL((paged_prefill_kernel<E, D, G, kPow2, W, kBounded>), grid, dim3(W * 64), 0, st, a);
+  hipLaunchKernelGGL((paged_prefill_kernel<E, D, G, kPow2, W, kBounded, KG>), grid, dim3(W * 64), 0, st, a);
 }
 
-template <typename E, int D, int G, int W>
+template <typename E, int D, int G, int W, int KG = 1>
 void launch_main(const PrefillArgs& a, dim3 grid, bool bounded, hipStream_t st) {
   const bool pow2 = a.pd.shift >= 0;
   if constexpr (std::is_same<E, BF16>::value) {
     if (bounded) {
-      if (pow2) launch_instance<E, D, G, true, W, true>(a, grid, st);
-      else launch_instance<E, D, G, false, W, true>(a, grid, st);
+      if (pow2) launch_instance<E, D, G, true, W, true, KG>(a, grid, st);
+      else launch_instance<E, D, G, false, W, true, KG>(a, grid, st);
       return;
     }
   }
-  if (pow2) launch_instance<E, D, G, true, W, false>(a, grid, st);
-  else launch_instance<E, D, G, false, W, false>(a, grid, st);
+  if (pow2) launch_instance<E, D, G, true, W, false, KG>(a, grid, st);
+  else launch_instance<E, D, G, false, W, false, KG>(a, grid, st);
+}
+
+template <typename E, int D>
+void launch_merge(const PrefillArgs& a, int shares, hipStream_t st) {
+  const int64_t items = static_cast<int64_t>(a.Lq) * a.Hq;
+  constexpr int kItems = kMergeThreads / (D / 8);
+  hipLaunchKernelGGL((paged_prefill_merge_kernel<E, D>), dim3(static_cast<unsigned>((items + kItems - 1) / kItems)),
+                     dim3(kMergeThreads), 0, st, a, shares);
 }
 
 template <typename E, int D, int G>
@@ -809,9 +897,33 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   a.n_tiles = (a.Lq + BM - 1) / BM;
   int shares = workspace ? key_shares_for(static_cast<int64_t>(a.Hc) * a.n_tiles, FP_DTYPE_BF16) : 1;  // f16 alike
   while (shares > 1 && share_bytes(shares, a.Lq, a.Hq, D, 2) > workspace_bytes) --shares;  // what the workspace holds
-  if (shares > 1) {
+  auto set_workspace = [&] {
+    if (shares <= 1) return;
     a.ws_ml = static_cast<float*>(workspace);
     a.ws_acc = reinterpret_cast<short*>(a.ws_ml + static_cast<int64_t>(shares) * a.Lq * a.Hq * 2);
+  };
+  // Launches of few rows, where a workgroup's chain of key tiles sets the time, go out as workgroups of half as many rows whose
+  // halves take the key tiles in turn: half the chain, twice the workgroups, no partial results in memory.  They have to fit the
+  // GPU in one go (K and V travel to LDS twice as often: 2700 rows, 352 workgroups, 88 us against 73 us).  us a launch, 16 q heads
+  // on 16, D 128, before (256 rows a workgroup, up to 8 key shares and their merge) and now: 59 rows 13.1 / 10.8, 170 rows
+  // 18.8 / 13.0, 613 rows 24.3 / 18.4, 1060 rows 31.8 / 25.8, 1600 rows 39.8 / 34.1; D 64 10.5 / 8.0, 13.7 / 9.4, 16.7 / 13.3,
+  // 21.0 / 17.5, 26.8 / 22.6.  Key shares go on top where four or more fit (512 rows over 2048 and 4096 cached tokens, 8 kv heads:
+  // 32.4 / 27.9 and 38.4 / 37.1); where two or three would, a caller that brings a workspace for them has long ranges, and
+  // there the staging costs more than the merge (2 x 512 rows over 4096: 52 against 58).
+  if constexpr (G <= 4) {
+    constexpr int BM2 = (kWaves / 2 / G) * 32;
+    const int tiles = (a.Lq + BM2 - 1) / BM2;
+    const int64_t wgs = static_cast<int64_t>(a.Hc) * tiles;
+    const int64_t fit = fp::compute_units() / (wgs < 1 ? 1 : wgs);
+    if (fit >= 4 || fit == 1 || (fit >= 1 && shares == 1)) {
+      a.n_tiles = tiles;
+      shares = shares < fit ? shares : static_cast<int>(fit);
+      set_workspace();
+      a.order = nullptr;  // every workgroup starts at once
+      launch_main<E, D, G, kWaves, 2>(a, dim3(a.Hc, a.n_tiles, shares), bounded, st);
+      if (shares > 1) launch_merge<E, D>(a, shares, st);
+      return;
+    }
   }
   // head_dim 64: a launch that is not cut along the keys goes out as workgroups of four wavefronts, up to
   // three to a CU.  A staged K/V tile then serves half as many query rows, but at 128-byte rows the staging is
@@ -831,13 +943,10 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
       return;
     }
   }
+  set_workspace();
   if (a.order_rows != BM) a.order = nullptr;
   launch_main<E, D, G, kWaves>(a, dim3(a.Hc, a.n_tiles, shares), bounded, st);
-  if (shares > 1) {
-    const int64_t items = static_cast<int64_t>(a.Lq) * a.Hq;
-    hipLaunchKernelGGL((paged_prefill_merge_kernel<E, D>), dim3(static_cast<unsigned>((items + kMergeRows - 1) / kMergeRows)),
-                       dim3(kMergeRows * 64), 0, st, a, shares);
-  }
+  if (shares > 1) launch_merge<E, D>(a, shares, st);
 }
 
 template <typename E, int D>
@@ -852,7 +961,8 @@ int launch(const PrefillArgs& a, float score_bound, void* ws, int64_t ws_bytes, 
 }
 
 // Rows per query tile of the launch fp_paged_prefill makes for this shape with a workspace of this size (the
-// same decisions as launch_group); 0 for the fp32 kernel, which takes no order.
+// same decisions as launch_group, but for launches of few rows, whose workgroups all start at once and which
+// take no order); 0 for the fp32 kernel, which takes no order either.
 int tile_rows_for(int Lq, int Hq, int Hc, int D, int dtype, int64_t workspace_bytes) {
   if (dtype == FP_DTYPE_F32) return 0;
   const int g = Hq / Hc;

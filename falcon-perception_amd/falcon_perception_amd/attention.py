@@ -131,6 +131,7 @@ class HybridPrefillMask:
         self._step_key = None  # (address, shape) of the positions whose row limits are kept below
         self._step_layer = -1  # layer that asked last: a layer id that does not grow starts a new step
         self._row_limit = None
+        self.most_keys = 0  # no row of the step sees more keys than this (host bookkeeping of the cache)
         self._tile_orders: dict[int, tuple[Tensor, int]] = {}  # rows per tile -> tile order of the step's limits
 
     def _limits_from_ids(self, open_spans, validate) -> Tensor:
@@ -176,6 +177,7 @@ class HybridPrefillMask:
             self._row_limit = (input_pos.reshape(-1) + reach).to(torch.int32)
             self._step_key = key
             self._tile_orders = {}
+            self.most_keys = max(self.cache.capacity)
         self._step_layer = layer_id
         return self._row_limit
 
@@ -316,6 +318,10 @@ def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, 
         rows = cache.prefill_tile_rows(Lq, Hq, D, pool_k.shape[0], q.dtype, workspace.numel() if workspace is not False else 0)
         if rows and -(-Lq // rows) <= 4096:
             order = block_mask.tile_order(step.batch_idx, rows)
+    # Key shares and their merge pay from about 1500 keys on where two or three of them fit the GPU, and later where more
+    # do: without a workspace the 16-bit launch is not cut and has no merge pass behind it.
+    if block_mask.most_keys <= 23 * 64 and q.dtype != torch.float32:
+        workspace = False
     out, lse = ops.paged_prefill(
         q, pool_k, pool_v, cache.page_table, step.batch_idx, limits, cache.page_size, scale=scale, sinks=sinks,
         workspace=workspace, score_bound=cache.score_bound(D, scale), tile_order=order,

@@ -1,0 +1,69 @@
+"""GPU: prefill launches of few rows, whose workgroups split the key tiles between their two halves, and the tail tile of a
+run, against the oracle.  The tolerances are those of the other prefill tests: the rounding of the results and of the
+probabilities to the dtype."""
+
+import numpy as np
+import pytest
+import torch
+
+from falcon_perception_amd import ops
+from oracle import paged_kv_oracle as O
+from tests.gpu_cases import DEV, f64
+from tests.test_gpu_prefill_key_shares import TOL, make_case
+
+pytestmark = pytest.mark.gpu
+
+
+def check(st, q, bidx, lim, P, dtype, **kw):
+    pk, pv = st.pool_planes()
+    out, lse = ops.paged_prefill(q.to(DEV), pk, pv, st.cache.page_table, bidx, lim, P, **kw)
+    eo, el = O.prefill_attention_paged(f64(q), f64(pk), f64(pv), st.mirror.page_table, bidx.cpu().numpy(), None,
+                                       lim.cpu().numpy(), P)
+    atol, rtol = TOL[dtype]
+    np.testing.assert_allclose(f64(out), eo, atol=atol, rtol=rtol)
+    np.testing.assert_allclose(f64(lse), el, atol=max(atol * 0.1, 1e-4), rtol=rtol)
+    return out, lse
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("D,G,P", [(128, 1, 128), (64, 2, 64), (128, 4, 16), (64, 1, 24), (128, 2, 256), (64, 4, 128)])
+@pytest.mark.parametrize("lens,pads", [([1], [0]), ([63, 64, 65], [1, 0, 2]), ([127], [1]), ([129, 3], [0, 60]), ([192, 1], [0, 0])], ids=str)
+def test_sizes_around_the_tiles(dtype, D, G, P, lens, pads):
+    """One key tile (the second half of the workgroup has none), odd and even numbers of them, tails of one key."""
+    st, q, bidx, lim = make_case(dtype, D, G, P, lens=lens, pads=pads)
+    check(st, q, bidx, lim, P, dtype, workspace=False)
+
+
+@pytest.mark.parametrize("lens", [[960], [961, 40], [1025, 20]], ids=str)
+@pytest.mark.parametrize("D,G", [(128, 1), (64, 4), (128, 8)])
+def test_ranges_around_the_first_second_share(lens, D, G):
+    """15, 16 and 17 key tiles: the launch has key shares, a run of fewer than 16 tiles is not cut, and a launch holds
+    cut and uncut runs side by side.  The workspace starts as NaN: nothing that no share wrote may come through."""
+    dtype, P = torch.bfloat16, 64
+    st, q, bidx, lim = make_case(dtype, D, G, P, lens=lens, pads=[5] + [0] * (len(lens) - 1))
+    need = ops.prefill_workspace_bytes(q.shape[2], q.shape[1], 2, D, dtype)
+    assert need > 0
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV)
+    check(st, q, bidx, lim, P, dtype, workspace=ws)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("rows", [100, 2 * 128 * 140])
+def test_rows_behind_the_last_key_stay_out(dtype, rows):
+    """The page rows behind a sequence's last key hold NaN: launches of few rows and of many (one sequence repeated
+    as rows over the same keys)."""
+    D, G, P = 128, 1, 128
+    st, q, bidx, lim = make_case(dtype, D, G, P, lens=[100], pads=[0])
+    pk, pv = st.pool_planes()
+    page = int(st.cache.page_table[st.slots[0], 0])
+    pk[:, page * P + 100:(page + 1) * P] = float("nan")
+    pv[:, page * P + 100:(page + 1) * P] = float("nan")
+    n = -(-rows // 100)
+    out, lse = ops.paged_prefill(q.repeat(1, 1, n, 1).to(DEV), pk, pv, st.cache.page_table, bidx.repeat(n), lim.repeat(n), P,
+                                 workspace=False)
+    assert torch.isfinite(out).all() and torch.isfinite(lse).all()
+    for part in (pk, pv):
+        part[:, page * P + 100:(page + 1) * P] = 0.0
+    ref, _ = check(st, q, bidx, lim, P, dtype, workspace=False)
+    atol, rtol = TOL[dtype]
+    np.testing.assert_allclose(f64(out[:, :, -100:]), f64(ref), atol=atol, rtol=rtol)
