@@ -269,11 +269,12 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
     # The plan of the step: the reference converts its mask once per step and every layer consumes it
     # (paged_inference.py:847-848, model.py:689-699); here the first attention call that meets this mask object
     # has the decode kernel's per-step work done once, and the layers after it start from the result.
-    plan = cache.decode_plan()
+    # (The plan saves a layer 1.3 to 2.5 us and takes 4 to 5 us: a model of one or two layers goes without.)
+    plan = cache.decode_plan() if len(cache._planes) > 2 else None
     args = (q, pool_k, pool_v, cache.page_table, block_mask.batch_idx, step.input_pos, cache.page_size,
             block_mask.max_context)
     shape = (q.shape[0], q.shape[1], q.shape[3], k.shape[1], kv_rep, split_tokens, step.input_pos.data_ptr())
-    if cache._decode_plan_owner is not block_mask or block_mask._plan_shape != shape:
+    if plan is not None and (cache._decode_plan_owner is not block_mask or block_mask._plan_shape != shape):
         ops.paged_decode(*args, scale=scale, split_tokens=split_tokens, kv_rep=kv_rep, phase="plan", plan=plan)
         cache._decode_plan_owner = block_mask
         block_mask._plan_shape = shape
