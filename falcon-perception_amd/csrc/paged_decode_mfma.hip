@@ -299,12 +299,13 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
           m = m_new;
         }
       }
+      const float ms = safe_max(m);  // no key above -inf so far: its probabilities are 0
 #pragma unroll
       for (int blk = 0; blk < NB; ++blk) {
         float p[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          p[j] = fast_exp2(sc[blk][j] - m);
+          p[j] = fast_exp2(sc[blk][j] - ms);
           l += p[j];
         }
         uint32_t w[2];
@@ -329,12 +330,16 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
 
     wait_staged<0>();  // also a wavefront without a stage has its query rows in flight
 
-    // both halves of the columns together, then the wavefront's state to LDS (its ring is free again)
+    // both halves of the columns together, then the wavefront's state to LDS (its ring is free again).  Against an infinite
+    // V element what rounding left over of a probability is 0 or negative, and the sum would be NaN: the upper half stands.
     float* const acc_lds = reinterpret_cast<float*>(ring);
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[db][j] += dpp<0x128>(o[db][j]);  // row_ror:8, lane ^ 8
+      for (int j = 0; j < 4; ++j) {
+        const float rest = dpp<0x128>(o[db][j]);  // row_ror:8, lane ^ 8
+        if ((__float_as_uint(o[db][j]) & 0x7f800000u) != 0x7f800000u) o[db][j] += rest;
+      }
       if (col < G) *reinterpret_cast<f32x4*>(acc_lds + col * D + db * 16 + grp * 4) = o[db];
     }
     l += __shfl_xor(l, 16);

@@ -50,3 +50,33 @@ def test_matrix_core_decode(dtype, D, G, P, cut, spread):
     rtol, atol = TOL[dtype]
     np.testing.assert_allclose(f64(out), eo, rtol=rtol, atol=atol)
     np.testing.assert_allclose(f64(lse), el, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("D,G", [(128, 8), (64, 4)])
+@pytest.mark.parametrize("split", [512, 64])
+def test_infinite_scores_and_values(dtype, D, G, split):
+    """Keys whose score is -inf (the whole first stage of the first wavefront) weigh nothing, and an infinite V
+    element makes its element of the result infinite and no other."""
+    Hc, P, L = 2, 64, 200
+    st = PagedState(77, n_pages=8, page_size=P, max_batch=2, Hc=Hc, D=D, dtype=dtype)
+    st.add_sequence(L)
+    st.prefill_random()
+    pk, pv = st.pool_planes()
+    slots = [int(st.cache.page_table[st.slots[0], t // P]) * P + t % P for t in range(L)]
+    q = torch.ones((1, Hc * G, 1, D), dtype=dtype, device=DEV)
+    pos = torch.tensor([L - 1], dtype=torch.int32, device=DEV)
+    bidx = torch.tensor(st.slots, dtype=torch.int64, device=DEV)
+    args = (st.cache.page_table, bidx, pos, P, 256)
+    eo, el = O.decode_attention(f64(q), f64(pk[:, slots[32:]]), f64(pv[:, slots[32:]]),
+                                np.arange(L - 32).reshape(1, -1), [0], np.array([L - 33]), 1)
+    pk[:, slots[:32]] = -float("inf")
+    out, lse = ops.paged_decode(q, pk, pv, *args, split_tokens=split)
+    rtol, atol = TOL[dtype]
+    np.testing.assert_allclose(f64(out), eo, rtol=rtol, atol=atol)
+    np.testing.assert_allclose(f64(lse), el, rtol=1e-5, atol=1e-5)
+    pv[:, slots[40], 5] = float("inf")
+    got, _ = ops.paged_decode(q, pk, pv, *args, split_tokens=split)
+    assert (got[..., 5] == float("inf")).all()
+    keep = [d for d in range(D) if d != 5]
+    assert torch.equal(got[..., keep], out[..., keep])
