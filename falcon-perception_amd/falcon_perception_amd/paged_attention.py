@@ -122,6 +122,7 @@ class PagedKVCache(KVCacheBase):
         self._workspace: Tensor | None = None
         self._retired_workspaces: list[Tensor] = []  # graphs captured earlier still write to these
         self._decode_launch: dict[tuple, tuple[int, int]] = {}
+        self._decode_need: dict[tuple, int] = {}
         self._decode_plan: Tensor | None = None  # the step's plan of the decode kernel (`decode_plan`)
         self._decode_plan_owner = None           # the mask object it was made for
         self._prefill_workspace: Tensor | None = None
@@ -465,8 +466,8 @@ class PagedKVCache(KVCacheBase):
     def decode_workspace(self, B: int, Hq: int, D: int, max_context: int, Hc: int) -> Tensor | None:
         """Split-K scratch of the decode kernel, owned by the cache.
 
-        Sized on first use for the largest batch and the finest split any batch size
-        can get, so its address never changes afterwards: HIP graphs captured for
+        Sized on first use for every batch up to the largest at the split each gets,
+        so its address never changes afterwards: HIP graphs captured for
         one batch bucket stay valid when another bucket runs."""
         return self.decode_launch(B, Hq, D, max_context, Hc)[0]
 
@@ -477,22 +478,34 @@ class PagedKVCache(KVCacheBase):
         key = (B, Hq, D, max_context, Hc)
         hit = self._decode_launch.get(key)
         if hit is None:
-            # sized for the largest batch and the longest context the page table can hold, at the finest split
-            # either can get, so that later shapes fit.  Should one not (more query heads), the old buffer is
-            # kept alive: graphs captured with it go on writing to it.
+            # Sized for every batch the cache can hold at the longest context the page table can hold, so that later
+            # shapes fit, and for this launch.  Should a shape not fit (more query heads), the old buffer is kept
+            # alive: graphs captured with it go on writing to it.
             worst_b = max(B, self.max_batch_size)
-            worst_ctx = max(max_context, self.table_cols * self.page_size)
-            need = 0
-            for ctx in {max_context, worst_ctx}:
-                finest = min(self.decode_split_tokens(1, Hc, ctx), self.decode_split_tokens(worst_b, Hc, ctx))
-                need = max(need, ops.decode_workspace_bytes(worst_b, Hq, D, ctx, finest))
+            split = self.decode_split_tokens(B, Hc, max_context)
+            finest = min(self.decode_split_tokens(1, Hc, max_context), self.decode_split_tokens(worst_b, Hc, max_context))
+            need = max(ops.decode_workspace_bytes(B, Hq, D, max_context, split),
+                       ops.decode_workspace_bytes(worst_b, Hq, D, max_context, finest),
+                       self._largest_decode_need(worst_b, Hq, D, max(max_context, self.table_cols * self.page_size), Hc))
             if need and (self._workspace is None or self._workspace.numel() < need):
                 if self._workspace is not None:
                     self._retired_workspaces.append(self._workspace)
                 self._workspace = torch.empty(need, dtype=torch.uint8, device=self._kv.device)
-            hit = (need, self.decode_split_tokens(B, Hc, max_context))
+            hit = (need, split)
             self._decode_launch[key] = hit
         return (self._workspace if hit[0] else None), hit[1]
+
+    def _largest_decode_need(self, worst_b: int, Hq: int, D: int, max_context: int, Hc: int) -> int:
+        """Workspace bytes that hold the decode launch of every batch up to `worst_b`.  How finely a batch is split does
+        not run in one direction with its size, so each is asked for; 5 us a batch, once per number of heads."""
+        key = (worst_b, Hq, D, max_context, Hc)
+        need = self._decode_need.get(key)
+        if need is None:
+            splits = [self.decode_split_tokens(b, Hc, max_context) for b in range(1, worst_b + 1)]
+            need = max(ops.decode_workspace_bytes(worst_b, Hq, D, max_context, min(splits[0], splits[-1])),
+                       *(ops.decode_workspace_bytes(b, Hq, D, max_context, s) for b, s in enumerate(splits, 1)))
+            self._decode_need[key] = need
+        return need
 
     def decode_plan(self) -> Tensor:
         """Buffer of the decode step's plan (`fp_paged_decode_plan`): allocated once, so that graphs captured
