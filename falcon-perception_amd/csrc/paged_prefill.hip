@@ -40,7 +40,7 @@ constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 constexpr int kTileN = 64;  // keys per tile
 constexpr int kSlotTable = 2048;  // tiles of a run whose first pool slot is looked up ahead of the tile loop
-constexpr int kMinShareTiles = 8;  // key tiles a key share has at least
+constexpr int kMinShareTiles = 3;  // key tiles a key share has at least
 constexpr float kRowFinished = -1.f;  // in the place of share 0's denominator: the row is stored, the merge pass leaves it alone
 constexpr int kTailSlot = -2;     // table entries at or below it: a tile that ends past the run's last key
 constexpr float kMaxSlack = 6.f;  // the running maximum may lag a row's true maximum by this much (log2)
@@ -85,6 +85,7 @@ struct PrefillArgs {
   // optional (fp_paged_prefill_tile_order): the query tile workgroup row y works on, longest key range first
   const int* order;
   int order_rows;  // rows per query tile the order was made for; another tile size ignores it
+  int uncut_tiles;  // longest run of key tiles that goes without key shares
 };
 
 struct BF16 {
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     const int z = blockIdx.z;
     int n_shares = 1;
     if (gridDim.z > 1) {
-      n_shares = min(max(n_run_tiles / kMinShareTiles, 1), static_cast<int>(gridDim.z));
+      n_shares = n_run_tiles <= a.uncut_tiles ? 1 : min(n_run_tiles / kMinShareTiles, static_cast<int>(gridDim.z));
       if (z >= n_shares) {
         if (n_shares > 1 && active[0] && kg == 0 && half == 0)  // a share without keys
           *reinterpret_cast<float2*>(a.ws_ml + ((static_cast<int64_t>(z) * a.Lq + row[0]) * a.Hq + hq) * 2) =
@@ -832,9 +833,7 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(cons
 
 constexpr int kMaxKeyShares = 8;
 
-// Key shares for a launch of `wgs` workgroups, at most: the kernel makes fewer of a run without kMinShareTiles for each, down
-// to none (a share costs its partial results and the launch their merge; 613 keys of 16 heads: 28.6 us in five shares, 22.9 us
-// uncut).  bf16 / f16: a launch that would leave at least half of the
+// Key shares for a launch of `wgs` workgroups, at most (see uncut_tiles).  bf16 / f16: a launch that would leave at least half of the
 // CUs idle is cut along the keys until every CU has a workgroup.  (With about one workgroup per CU
 // already, a cut in two costs more in partial results and their merge than the shorter critical path
 // saves: 138 us against 111 us at 8 sequences x 512 rows.)  fp32: the kernel takes about eight times as
@@ -845,6 +844,17 @@ int key_shares_for(int64_t wgs, int dtype) {
   if (wgs < 1) wgs = 1;
   const int64_t n = dtype == FP_DTYPE_F32 ? (4 * fp::compute_units() + wgs / 2) / wgs : fp::compute_units() / wgs;
   return static_cast<int>(n < 1 ? 1 : n > kMaxKeyShares ? kMaxKeyShares : n);
+}
+
+// Longest run of key tiles a launch leaves uncut (`halves`: the halves of a workgroup take the tiles in turn).  Shares of
+// kMinShareTiles take tiles off a workgroup's chain and cost their partial results and the merge, which grow with rows x heads.
+// us a launch uncut without a merge / cut with it, D 128: 16 heads on 16, 32 rows over 400 keys (7 tiles) 19.7 / 19.6, 128 over 400 (9)
+// 22.4 / 21.3, 256 over 400 (11) 24.1 / 24.2, 512 over 1 and 400 (9, 15) 23.1 / 24.6, 28.4 / 26.8, 1024 over 1 and 400 (17, 23) 30.5 /
+// 30.7, 35.1 / 34.5; 32 heads on 4, without halves, 128 over 400 (9) 25.9 / 24.2, 512 over 1 and 400 27.7 / 28.2, 35.2 / 32.8.  Cutting
+// whole prompts of up to 1000 rows would also round their partial sums to the model dtype (an error of 3.3e-3 instead of 2.8e-3).
+int uncut_tiles(int Lq, int Hq, bool halves) {
+  const int64_t items = static_cast<int64_t>(Lq) * Hq;
+  return static_cast<int>(halves ? 5 + items / 1500 : 4 + items / 4000);
 }
 
 // workspace of `shares` key shares: per row and head D results of elem bytes, and two floats
@@ -889,36 +899,46 @@ void launch_merge(const PrefillArgs& a, int shares, hipStream_t st) {
                      dim3(kMergeThreads), 0, st, a, shares);
 }
 
+// How often workgroups of half the rows, whose halves take the key tiles in turn (launch_group), fit the GPU
+int64_t halves_fit(int Lq, int Hc, int g) {
+  const int rows = g > 4 ? 1 : (kWaves / 2 / g) * 32;
+  return g > 4 ? 0 : fp::compute_units() / (static_cast<int64_t>(Hc) * ((Lq + rows - 1) / rows));
+}
+
+// Key shares of a bf16 / f16 launch whose workspace holds them
+int launch_shares(int Lq, int Hq, int Hc) {
+  const int g = Hq / Hc, bm = (kWaves / g) * 32;
+  const int shares = key_shares_for(static_cast<int64_t>(Hc) * ((Lq + bm - 1) / bm), FP_DTYPE_BF16);
+  const int64_t fit = halves_fit(Lq, Hc, g);
+  return fit >= 1 && fit < shares ? static_cast<int>(fit) : shares;
+}
+
 template <typename E, int D, int G>
 void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int64_t workspace_bytes, hipStream_t st) {
   PrefillArgs a = a0;
   const bool bounded = bounded_path<E>(score_bound);
   constexpr int BM = (kWaves / G) * 32;
   a.n_tiles = (a.Lq + BM - 1) / BM;
-  int shares = workspace ? key_shares_for(static_cast<int64_t>(a.Hc) * a.n_tiles, FP_DTYPE_BF16) : 1;  // f16 alike
+  const bool halves = halves_fit(a.Lq, a.Hc, G) >= 1;
+  int shares = workspace ? launch_shares(a.Lq, a.Hq, a.Hc) : 1;
   while (shares > 1 && share_bytes(shares, a.Lq, a.Hq, D, 2) > workspace_bytes) --shares;  // what the workspace holds
-  auto set_workspace = [&] {
-    if (shares <= 1) return;
+  if (shares > 1) {
     a.ws_ml = static_cast<float*>(workspace);
     a.ws_acc = reinterpret_cast<short*>(a.ws_ml + static_cast<int64_t>(shares) * a.Lq * a.Hq * 2);
-  };
+    a.uncut_tiles = uncut_tiles(a.Lq, a.Hq, halves);
+  }
   // Launches of few rows, where a workgroup's chain of key tiles sets the time, go out as workgroups of half as many rows whose
-  // halves take the key tiles in turn: half the chain, twice the workgroups, no partial results in memory.  They have to fit the
-  // GPU in one go (K and V travel to LDS twice as often: 2700 rows, 352 workgroups, 88 us against 73 us).  us a launch, 16 q heads
-  // on 16, D 128, before (256 rows a workgroup, up to 8 key shares and their merge) and now: 59 rows 13.1 / 10.8, 170 rows
-  // 18.8 / 13.0, 613 rows 24.3 / 18.4, 1060 rows 31.8 / 25.8, 1600 rows 39.8 / 34.1; D 64 10.5 / 8.0, 13.7 / 9.4, 16.7 / 13.3,
-  // 21.0 / 17.5, 26.8 / 22.6.  Key shares go on top where four or more fit (512 rows over 2048 and 4096 cached tokens, 8 kv heads:
-  // 32.4 / 27.9 and 38.4 / 37.1); where two or three would, a caller that brings a workspace for them has long ranges, and
-  // there the staging costs more than the merge (2 x 512 rows over 4096: 52 against 58).
+  // halves take the key tiles in turn: half the chain, twice the workgroups.  They have to fit the GPU in one go (K and V travel to
+  // LDS twice as often: 2700 rows, 352 workgroups, 88 us against 73 us); key shares go on top as often as they fit.  us a launch
+  // with its merge, 16 q heads on 16, D 128, with whole workgroups in up to 8 shares / so: 128 rows over 1, 400, 1400 and 3000 cached keys
+  // 20.0 / 19.8, 21.9 / 21.3, 24.1 / 23.9 and 28.4 / 27.3; 512 rows 32.2 / 25.7, 33.2 / 29.8, 35.6 / 31.0 and 37.9 / 35.2; 1024 rows 38.8 /
+  // 32.6, 40.5 / 34.5, 44.1 / 40.3 and 52.7 / 50.9.  Short prompts without a merge, D 128 and 64: 59 rows 13.1 / 10.8 and 10.5 / 8.0,
+  // 170 rows 18.8 / 13.0 and 13.7 / 9.4, 613 rows 24.3 / 18.4 and 16.7 / 13.3.  Not the better one at 129 to 170 workgroups over 3000 keys
+  // and more, which leave no room for a second share (640 rows of 32 q / 8 kv heads: 56.5 / 61.4; over 1400 keys 44.2 / 42.1).
   if constexpr (G <= 4) {
     constexpr int BM2 = (kWaves / 2 / G) * 32;
-    const int tiles = (a.Lq + BM2 - 1) / BM2;
-    const int64_t wgs = static_cast<int64_t>(a.Hc) * tiles;
-    const int64_t fit = fp::compute_units() / (wgs < 1 ? 1 : wgs);
-    if (fit >= 4 || fit == 1 || (fit >= 1 && shares == 1)) {
-      a.n_tiles = tiles;
-      shares = shares < fit ? shares : static_cast<int>(fit);
-      set_workspace();
+    if (halves) {
+      a.n_tiles = (a.Lq + BM2 - 1) / BM2;
       a.order = nullptr;  // every workgroup starts at once
       launch_main<E, D, G, kWaves, 2>(a, dim3(a.Hc, a.n_tiles, shares), bounded, st);
       if (shares > 1) launch_merge<E, D>(a, shares, st);
@@ -943,7 +963,6 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
       return;
     }
   }
-  set_workspace();
   if (a.order_rows != BM) a.order = nullptr;
   launch_main<E, D, G, kWaves>(a, dim3(a.Hc, a.n_tiles, shares), bounded, st);
   if (shares > 1) launch_merge<E, D>(a, shares, st);
@@ -1101,7 +1120,7 @@ extern "C" int fp_paged_prefill(const void* q, int64_t q_stride_row, int64_t q_s
                 page_table, pt_row_stride, batch_idx, row_limit,
                 static_cast<char*>(out), out_stride_row * 2, out_stride_h * 2, lse, sinks,
                 Lq, Hq, Hc, fp::PageDiv(page_size), n_pages, max_batch, n_slots, scale * kLog2e, 0, nullptr, nullptr,
-                tile_order, tile_order ? tile_order_rows : 0};
+                tile_order, tile_order ? tile_order_rows : 0, 0};
   hipStream_t st = static_cast<hipStream_t>(stream);
   int rc;
   if (dtype == FP_DTYPE_BF16)

@@ -34,11 +34,11 @@ def test_sizes_around_the_tiles(dtype, D, G, P, lens, pads):
     check(st, q, bidx, lim, P, dtype, workspace=False)
 
 
-@pytest.mark.parametrize("lens", [[960], [961, 40], [1025, 20]], ids=str)
+@pytest.mark.parametrize("lens", [[256], [320], [321, 40], [385, 20], [960], [961, 40], [1025, 20]], ids=str)
 @pytest.mark.parametrize("D,G", [(128, 1), (64, 4), (128, 8)])
 def test_ranges_around_the_first_second_share(lens, D, G):
-    """15, 16 and 17 key tiles: the launch has key shares, a run of fewer than 16 tiles is not cut, and a launch holds
-    cut and uncut runs side by side.  The workspace starts as NaN: nothing that no share wrote may come through."""
+    """4 to 7 and 15 to 17 key tiles: the launch has key shares, a run of up to about five tiles is not cut, and a launch
+    holds cut and uncut runs side by side.  The workspace starts as NaN: nothing that no share wrote may come through."""
     dtype, P = torch.bfloat16, 64
     st, q, bidx, lim = make_case(dtype, D, G, P, lens=lens, pads=[5] + [0] * (len(lens) - 1))
     need = ops.prefill_workspace_bytes(q.shape[2], q.shape[1], 2, D, dtype)
