@@ -1057,6 +1057,13 @@ extern "C" int32_t fp_paged_prefill_tile_rows(int32_t Lq, int32_t Hq, int32_t Hc
   return tile_rows_for(Lq, Hq, Hc, D, dtype, workspace_bytes);
 }
 
+extern "C" int32_t fp_paged_prefill_uncut_keys(int32_t Lq, int32_t Hq, int32_t Hc, int32_t D, int dtype) {
+  const int64_t bytes = fp_paged_prefill_workspace_bytes(Lq, Hq, Hc, D, dtype);
+  if (bytes < 0) return static_cast<int32_t>(bytes);
+  if (bytes == 0 || (dtype != FP_DTYPE_F32 && launch_shares(Lq, Hq, Hc) == 1)) return INT32_MAX;
+  return dtype == FP_DTYPE_F32 ? 0 : uncut_tiles(Lq, Hq, halves_fit(Lq, Hc, Hq / Hc) >= 1) * kTileN;
+}
+
 extern "C" int fp_paged_prefill_tile_order(const int64_t* batch_idx, const int32_t* row_limit, int32_t Lq,
                                            int32_t tile_rows, int32_t* order, void* stream) {
   if (Lq < 0) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_prefill_tile_order: negative length");

@@ -131,7 +131,7 @@ class HybridPrefillMask:
         self._step_key = None  # (address, shape) of the positions whose row limits are kept below
         self._step_layer = -1  # layer that asked last: a layer id that does not grow starts a new step
         self._row_limit = None
-        self.most_keys = 0  # no row of the step sees more keys than this (host bookkeeping of the cache)
+        self.most_keys = 0  # no row of the step sees more keys than this: the longest sequence the cache holds
         self._tile_orders: dict[int, tuple[Tensor, int]] = {}  # rows per tile -> tile order of the step's limits
 
     def _limits_from_ids(self, open_spans, validate) -> Tensor:
@@ -310,7 +310,7 @@ def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, 
     pool_k, pool_v = cache._planes[step.layer_id]
     Lq, Hq, D = q.shape[2], q.shape[1], q.shape[3]
     limits = block_mask.row_limit(step.input_pos, step.layer_id)
-    workspace = cache.prefill_workspace(Lq, Hq, D, pool_k.shape[0], q.dtype)
+    workspace = cache.prefill_workspace(Lq, Hq, D, pool_k.shape[0], q.dtype, block_mask.most_keys)
     # At head_dim 64 several small workgroups share a CU and the order in which they start decides when the launch
     # ends: the step's query tiles are ranked once (first layer) and every layer starts the longest first.  At
     # head_dim 128 the order measured no difference, so no kernel is spent on it.
@@ -319,10 +319,6 @@ def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, 
         rows = cache.prefill_tile_rows(Lq, Hq, D, pool_k.shape[0], q.dtype, workspace.numel() if workspace is not False else 0)
         if rows and -(-Lq // rows) <= 4096:
             order = block_mask.tile_order(step.batch_idx, rows)
-    # Key shares and their merge pay from about 1500 keys on where two or three of them fit the GPU, and later where more
-    # do: without a workspace the 16-bit launch is not cut and has no merge pass behind it.
-    if block_mask.most_keys <= 23 * 64 and q.dtype != torch.float32:
-        workspace = False
     out, lse = ops.paged_prefill(
         q, pool_k, pool_v, cache.page_table, step.batch_idx, limits, cache.page_size, scale=scale, sinks=sinks,
         workspace=workspace, score_bound=cache.score_bound(D, scale), tile_order=order,

@@ -126,7 +126,7 @@ class PagedKVCache(KVCacheBase):
         self._decode_plan: Tensor | None = None  # the step's plan of the decode kernel (`decode_plan`)
         self._decode_plan_owner = None           # the mask object it was made for
         self._prefill_workspace: Tensor | None = None
-        self._prefill_need: dict[tuple, int] = {}
+        self._prefill_need: dict[tuple, tuple[int, int]] = {}
         self._prefill_tile_rows: dict[tuple, int] = {}
         # status word of the last prefill mask, on its way to the host (`check_prefill_masks`)
         self._mask_status_host: Tensor | None = None
@@ -530,14 +530,17 @@ class PagedKVCache(KVCacheBase):
             hit = self._prefill_tile_rows[key] = ops.prefill_tile_rows(Lq, Hq, Hc, D, dtype, workspace_bytes)
         return hit
 
-    def prefill_workspace(self, Lq: int, Hq: int, D: int, Hc: int, dtype: torch.dtype):
+    def prefill_workspace(self, Lq: int, Hq: int, D: int, Hc: int, dtype: torch.dtype, most_keys: int = 0):
         """Scratch with which the prefill kernel cuts a small launch along the keys as well, owned by the
-        cache and grown on demand (prefill steps are not captured in graphs); False when the shape needs none."""
+        cache and grown on demand (prefill steps are not captured in graphs); False when the shape needs none, or
+        when no row sees more than `most_keys` keys (0: unknown) and the launch would not be cut (same bits, no merge)."""
         key = (Lq, Hq, Hc, D, dtype)
-        need = self._prefill_need.get(key)
-        if need is None:
-            need = self._prefill_need[key] = ops.prefill_workspace_bytes(Lq, Hq, Hc, D, dtype)
-        if need == 0:
+        hit = self._prefill_need.get(key)
+        if hit is None:
+            hit = self._prefill_need[key] = (ops.prefill_workspace_bytes(Lq, Hq, Hc, D, dtype),
+                                             ops.prefill_uncut_keys(Lq, Hq, Hc, D, dtype))
+        need, uncut = hit
+        if need == 0 or 0 < most_keys <= uncut:
             return False
         if self._prefill_workspace is None or self._prefill_workspace.numel() < need:
             self._prefill_workspace = torch.empty(need, dtype=torch.uint8, device=self._kv.device)

@@ -5,10 +5,12 @@ probabilities to the dtype."""
 import numpy as np
 import pytest
 import torch
+from torch.nn.attention.flex_attention import AuxRequest
 
+from falcon_perception_amd import attention as A
 from falcon_perception_amd import ops
 from oracle import paged_kv_oracle as O
-from tests.gpu_cases import DEV, f64
+from tests.gpu_cases import DEV, PagedState, f64, randn
 from tests.test_gpu_prefill_key_shares import TOL, make_case
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +69,46 @@ def test_rows_behind_the_last_key_stay_out(dtype, rows):
     ref, _ = check(st, q, bidx, lim, P, dtype, workspace=False)
     atol, rtol = TOL[dtype]
     np.testing.assert_allclose(f64(out[:, :, -100:]), f64(ref), atol=atol, rtol=rtol)
+
+
+@pytest.mark.parametrize("D,G,rows", [(128, 1, 64), (64, 2, 300), (128, 8, 100), (128, 4, 200)])
+def test_a_launch_without_key_shares_needs_no_workspace(D, G, rows):
+    """Up to `prefill_uncut_keys` the bits are those of the launch without a workspace; four tiles on it is cut."""
+    dtype, P, Hc = torch.bfloat16, 64, 2
+    uncut = ops.prefill_uncut_keys(rows, Hc * G, Hc, D, dtype)
+    assert uncut % 64 == 0 and uncut >= rows and ops.prefill_workspace_bytes(rows, Hc * G, Hc, D, dtype) > 0
+    for keys, same in ((uncut, True), (uncut + 256, False)):
+        st, q, bidx, lim = make_case(dtype, D, G, P, lens=[keys], pads=[0])
+        q, bidx, lim = q[:, :, -rows:].to(DEV), bidx[-rows:].contiguous(), lim[-rows:].contiguous()
+        pk, pv = st.pool_planes()
+        args = (q, pk, pv, st.cache.page_table, bidx, lim, P)
+        out, lse = ops.paged_prefill(*args)
+        plain = ops.paged_prefill(*args, workspace=False)
+        assert (torch.equal(out, plain[0]) and torch.equal(lse, plain[1])) == same
+
+
+@pytest.mark.parametrize("rows", [100, 613])
+def test_a_prompt_does_not_depend_on_who_else_is_cached(rows):
+    """The drop-in leaves the workspace out where no cached sequence is long enough for key shares: a long sequence that
+    is not in the step brings the workspace back and changes no bit."""
+    dtype, Hc, D, P = torch.bfloat16, 16, 128, 128
+    results, used = [], []
+    for resident in (0, 6000):
+        st = PagedState(19, n_pages=64, page_size=P, max_batch=4, Hc=Hc, D=D, dtype=dtype)
+        cache = st.cache
+        slot = st.add_sequence(rows)
+        if resident:
+            st.add_sequence(resident)
+        L = -(-rows // 128) * 128
+        gen = torch.Generator().manual_seed(5)
+        q, k, v = (randn(gen, (1, Hc, L, D), dtype).to(DEV) for _ in range(3))
+        live = torch.arange(L, device=DEV)[None] < rows
+        bidx = torch.where(live, slot, 0)
+        pos = torch.where(live, torch.arange(L, device=DEV)[None], 0)
+        mask = cache.create_prefill_blockmask(bidx, torch.full_like(bidx, 9), 1, 2)
+        K, V = cache.insert_kv(0, k, v, input_pos=pos, batch_idx=bidx)
+        out, aux = A.compiled_flex_attn_prefill(q, K, V, block_mask=mask, return_aux=AuxRequest(lse=True))
+        results.append((out, aux.lse))
+        used.append(cache.prefill_workspace(L, Hc, D, Hc, dtype, mask.most_keys) is not False)
+    assert used == [False, True]
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
