@@ -10,9 +10,11 @@
 //   grid  = (cache heads, batch, splits); a workgroup of 4 wavefronts owns one
 //           (sequence, cache head, token range) and serves all G = Hq / Hc query
 //           heads of that cache head from a single read of K and V.  A launch
-//           larger than the GPU holds at once runs as (cache heads, chunks)
-//           instead: the contexts laid end to end and cut into equal chunks, a
-//           workgroup working through the sequences its chunk touches.
+//           larger than the GPU holds at once, or of several sequences under a
+//           limit much longer than they are (even_cut_pays), runs as (cache
+//           heads, chunks) instead: the contexts laid end to end and cut into
+//           equal chunks, a workgroup working through the sequences its chunk
+//           touches.
 //   loads = a row (D elements) is covered by TPR = D * elem / 16 lanes holding
 //           16 bytes each, so a wavefront load instruction moves 64 / TPR whole
 //           rows, contiguous inside a page; U such loads of K and of V are in
@@ -757,23 +759,72 @@ constexpr int kPhasePartial = 1;
 constexpr int kPhaseMerge = 2;
 constexpr int kPhasePlan = 4;  // alone: write the step's plan instead of launching the passes
 
-// The even cut leaves about chunks / B partial results per sequence to a merge pass of one wavefront per row, which
-// takes them eight at a time: beyond eight, a launch that fits the GPU in one go is cheaper split by split (one
-// sequence of 711 tokens 9.7 us a layer against 10.5 us, four of 5 k to 16 k tokens 22.8 against 23.7 us).
-bool few_sequences(int64_t chunks, int B) { return chunks > 8 * static_cast<int64_t>(B); }
+int n_splits_for(int max_context, int split_tokens) {
+  const int n = (max_context + split_tokens - 1) / split_tokens;
+  return n < 1 ? 1 : n;
+}
 
-// Chunks per cache head of the even cut of a launch, 0 where it goes split by split: two per CU, as many as the
-// workspace of the launch's split count has rows for (one per chunk + sequence), but at least one per CU.
-int even_cut_chunks(int Hc, int B, int n_splits, int max_context, int page_size) {
-  const int cus = fp::compute_units();
-  const int64_t wanted = 2 * cus / Hc, rows = static_cast<int64_t>(B) * (n_splits - 1);
-  const int64_t chunks = wanted < rows ? wanted : rows;
-  const bool positions_fit = static_cast<int64_t>(B) * (max_context + 64) < (1ll << 30);  // the flat axis is int
-  if (chunks < 1 || 2 * chunks < wanted || B > kFlatMaxB || !positions_fit) return 0;
-  if (few_sequences(wanted, B) && static_cast<int64_t>(Hc) * B * n_splits <= 2 * cus) return 0;
-  // a chunk's pages have to fit the page-id table
-  if ((static_cast<int64_t>(B) * (max_context + 64) / chunks + 128) / page_size + 2 > kMaxSplitPages) return 0;
-  return static_cast<int>(chunks);
+// Split length of a launch that goes split by split.  Largest split (fewest partials to merge, least per-workgroup
+// overhead) that still yields enough workgroups when every sequence is at max_context.  Enough is about 2048 (8 per CU)
+// for a batch whose sequences alone give every CU two workgroups: their lengths differ, and small pieces even that out.
+// A small batch wants larger pieces: from 512 workgroups (4 * B * Hc in between) the pass no longer gets
+// faster, and every further split is one more partial result to merge.
+int plain_split_tokens(int B, int Hc, int max_context) {
+  int64_t target = 4 * static_cast<int64_t>(B) * Hc;
+  target = target < 512 ? 512 : target > 2048 ? 2048 : target;
+  int split = 2048;
+  while (split > 128 && static_cast<int64_t>(B) * Hc * ((max_context + split - 1) / split) < target) split >>= 1;
+  return split;
+}
+
+// Chunks per cache head of the even cut: two per CU.
+int flat_chunks(int Hc) { return 2 * fp::compute_units() / Hc; }
+
+// Whether the even cut can take a launch at all: the lengths fit LDS, the flat axis is int, a chunk's pages fit the table.
+bool even_cut_fits(int Hc, int B, int max_context, int page_size) {
+  const int64_t tokens = static_cast<int64_t>(B) * (max_context + 64), chunks = flat_chunks(Hc);
+  return chunks >= 1 && B <= kFlatMaxB && tokens < (1ll << 30) && (tokens / chunks + 128) / page_size + 2 <= kMaxSplitPages;
+}
+
+// Whether a launch that the GPU holds at once is cut evenly all the same: its splits are long (1024 tokens or more, or eight
+// of 512), so that sequences much shorter than max_context leave CUs idle, and the cut makes at most eight pieces of a
+// sequence, which the merge pass (one wavefront per row) takes in one batch.  us a layer split by split / cut evenly, 16 q / 8 kv
+// heads, D 128: limit 8192, 300 to 3000 tokens, 8, 12, 16 and 24 sequences 22.4 / 19.5, 28.3 / 24.1, 35.4 / 27.1 and 43.2 / 35.8, 4000 to
+// 8000 tokens 40.4 / 39.6, 58.9 / 56.8, 69.7 / 69.2 and 107 / 100; limit 4096, 8 sequences of 64 to 300, 100 to 700 and 300 to 1500 tokens
+// 12.6 / 9.9, 14.3 / 11.6 and 14.9 / 15.8, 10 of 100 to 3900 25.7 / 22.8; the price is paid close to the limit, 8 sequences of 3500 to
+// 4000 tokens 26.6 / 30.4.  With shorter splits there is no gain: limit 1024, 16 sequences (256 tokens) 15.5 / 17.5; limit 2048, 16
+// sequences (four of 512) 29.2 / 31.4.  Nor with more pieces: one sequence of 12000 tokens 17.1 / 23.1, three of 300 to 3000 12.5 / 14.9.
+bool even_cut_pays(int Hc, int B, int max_context, int page_size) {
+  const int split = plain_split_tokens(B, Hc, max_context);
+  const int n = n_splits_for(max_context, split);
+  return n > 1 && (split >= 1024 || (split >= 512 && n >= 8)) && flat_chunks(Hc) <= 8 * static_cast<int64_t>(B) &&
+         even_cut_fits(Hc, B, max_context, page_size);
+}
+
+// Chunks per cache head of the even cut of a launch, 0 where it goes split by split.  The workspace of its splits has a row
+// per (chunk + sequence), and a launch of more workgroups than the GPU holds at once (`resident`) is always cut.
+int even_cut_chunks(int Hc, int B, int n_splits, int max_context, int page_size, int resident) {
+  const int chunks = flat_chunks(Hc);
+  if (!even_cut_fits(Hc, B, max_context, page_size) || static_cast<int64_t>(B) * (n_splits - 1) < chunks) return 0;
+  return static_cast<int64_t>(Hc) * B * n_splits > resident || even_cut_pays(Hc, B, max_context, page_size) ? chunks : 0;
+}
+
+// Workgroups of the even-cut kernel the current device holds at once (asked once per kernel and device).
+template <typename E, int D, int G, bool kAligned, bool kPerHeadK>
+int resident_workgroups() {
+  const auto kernel = paged_decode_kernel<E, D, G, false, kAligned, kPerHeadK, true>;
+  static int cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (cached[dev] == 0) {
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, 0) != hipSuccess || per_cu <= 0) {
+      (void)hipGetLastError();  // not an error of the launch that follows
+      cached[dev] = -1;
+    } else
+      cached[dev] = per_cu * fp::compute_units();
+  }
+  return cached[dev] > 0 ? cached[dev] : 0;
 }
 
 // Launches with four or more query heads per cache head in a 16-bit type run on the matrix cores: with eight the vector
@@ -805,7 +856,7 @@ void launch_decode(const DecodeArgs& a, int B, int phases, hipStream_t st) {
     // Cut evenly: the work of a workgroup then follows from the lengths of the sequences and not from max_context,
     // which an engine sets to the longest sequence it may ever hold (16 padded rows of 350 to 4620 tokens under a
     // limit of 8192, 16 q heads / 8 kv heads with shared V: 57.4 us a layer split by split, one workgroup to a CU,
-    // against 38.8 us).  Two chunks
+    // against 38.8 us; even_cut_pays has where it goes which way).  Two chunks
     // per CU, all of the same length, all resident from the start, so that every CU streams the same
     // number of rows (split by split, the CUs end up with loads 25 % apart at 64 sequences of 1 k to
     // 4 k tokens, and workgroups queue behind busy shader engines).  Measured at 64 sequences of 16 q /
@@ -816,9 +867,14 @@ void launch_decode(const DecodeArgs& a, int B, int phases, hipStream_t st) {
     // against 73.4 (the even-cut kernels are not held to 128 registers: two workgroups per CU do not need
     // it, and in fp32 it made them spill).  With the step's plan read by every workgroup the same sweep gives, in us per
     // step for 1 / 2 / 3 chunks per CU: D 128 110.4 / 111.3 / 112.2; D 64 61.7 / 61.3 / 62.1; page size 64, 32
-    // sequences 89.2 / 90.9 / 90.4: two stays.  The even cut needs the lengths of at most kFlatMaxB sequences in LDS, a workspace row per (chunk + sequence),
-    // and chunks within the page-id table.
-    const int n_chunks = even_cut_chunks(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size);
+    // sequences 89.2 / 90.9 / 90.4: two stays.
+    int resident;  // matrix cores: two to a CU, but few sequences want the third (640 / 752 / 896 workgroups, 64 q / 8 kv heads,
+                   // split by split / cut evenly: 15.1 / 17.9, 21.6 / 25.1 and 19.6 / 18.2 us)
+    if constexpr (on_matrix_cores<E, G, kPerHeadK>())
+      resident = 3 * fp::compute_units();
+    else
+      resident = aligned ? resident_workgroups<E, D, G, true, kPerHeadK>() : resident_workgroups<E, D, G, false, kPerHeadK>();
+    const int n_chunks = even_cut_chunks(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size, resident);
     DecodeArgs af = a;
     af.B = B;
     af.n_chunks = n_chunks;
@@ -871,28 +927,12 @@ int dispatch_dim(const DecodeArgs& a, int B, int D, int phases, int kv_rep, hipS
   }
 }
 
-// Largest split (fewest partials to merge, least per-workgroup overhead) that still yields enough
-// workgroups when every sequence is at max_context.  Enough is about 2048 (8 per CU) for a batch whose
-// sequences alone give every CU two workgroups: their lengths differ, and small pieces even that out.
-// A small batch wants larger pieces: from 512 workgroups (4 * B * Hc in between) the pass no longer gets
-// faster, and every further split is one more partial result to merge.
 int default_split_tokens(int B, int Hc, int max_context, int page_size) {
-  int64_t target = 4 * static_cast<int64_t>(B) * Hc;
-  target = target < 512 ? 512 : target > 2048 ? 2048 : target;
-  int split = 2048;
-  while (split > 128 && static_cast<int64_t>(B) * Hc * ((max_context + split - 1) / split) < target) split >>= 1;
-  // the workspace has B rows per split: enough of them for the even cut, where it can have them
-  const int64_t chunks = 2 * fp::compute_units() / Hc;
-  auto rows = [&](int s) { return static_cast<int64_t>(B) * ((max_context + s - 1) / s - 1); };
-  if (2 * rows(64) >= chunks && !few_sequences(chunks, B))
-    while (split > 64 && rows(split) < chunks) split >>= 1;
+  int split = plain_split_tokens(B, Hc, max_context);
+  if (even_cut_pays(Hc, B, max_context, page_size))  // the workspace has B rows per split: enough of them for the cut
+    while (split > 64 && static_cast<int64_t>(B) * (n_splits_for(max_context, split) - 1) < flat_chunks(Hc)) split >>= 1;
   while (split / page_size + 2 > kMaxSplitPages) split >>= 1;
   return split < 64 ? 64 : split;
-}
-
-int n_splits_for(int max_context, int split_tokens) {
-  const int n = (max_context + split_tokens - 1) / split_tokens;
-  return n < 1 ? 1 : n;
 }
 
 }  // namespace

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 ATOL, RTOL = 2e-2, 1e-2
 
 
-# chunks per cache head: 2 * 256 CUs / 8 heads = 64; from 8 sequences on (8 chunks each) every launch is cut evenly
+# chunks per cache head: 2 * 256 CUs / 8 heads = 64.  8 and 13 sequences (8 chunks each, eight splits of 512 tokens) are cut
+# evenly, 7 and 64 because their workgroups do not fit the GPU at once, one goes split by split
 @pytest.mark.parametrize("B", [1, 7, 8, 13, 64])
 @pytest.mark.parametrize("P", [32, 24], ids=["pages-of-32", "pages-of-24"])
 def test_short_sequences_under_a_long_limit(B, P):
@@ -34,7 +35,7 @@ def test_short_sequences_under_a_long_limit(B, P):
     plan = torch.zeros(ops.decode_plan_bytes(), dtype=torch.uint8, device=DEV)
     ops.paged_decode(*args, phase="plan", plan=plan)
     planned_batch = int(plan.view(torch.int32)[1])  # the even cut writes a plan, a launch split by split does not
-    assert planned_batch == (B if B >= 8 else 0) or 1 < B < 8
+    assert planned_batch == (B if B >= 7 else 0)
     planned = ops.paged_decode(*args, plan=plan)
     assert torch.equal(planned[0], out) and torch.equal(planned[1], lse)
     eo, el = O.decode_attention(f64(q), f64(pk), f64(pv), st.mirror.page_table, st.slots, np.array(lens) - 1, P)

@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from falcon_perception_amd import ops
+from falcon_perception_amd import _native, ops
 from falcon_perception_amd.paged_attention import PagedKVCache
 
 HEADS = [(16, 8), (64, 8), (16, 16), (8, 4), (4, 1), (32, 32)]  # query heads, workgroup heads
@@ -27,3 +27,41 @@ def test_the_caches_workspace_holds_every_batch(native_lib, max_batch, limit, ta
             if workspace is not None:  # captured graphs of other batches keep writing to it
                 address = address or workspace.data_ptr()
                 assert workspace.data_ptr() == address, (Hq, Hc, B)
+
+
+def plain_split(B, Hc, limit):
+    """The split of a launch that goes split by split: the largest power of two up to 2048 that gives the workgroups wanted."""
+    target = min(max(4 * B * Hc, 512), 2048)
+    split = 2048
+    while split > 128 and B * Hc * -(-limit // split) < target:
+        split //= 2
+    return split
+
+
+@pytest.mark.parametrize("Hc", [1, 2, 4, 8, 16, 32])
+def test_a_finer_split_only_where_the_even_cut_uses_it(native_lib, Hc):
+    """The finer split that leaves workspace rows for the even cut: never where one split covers every context, not with more
+    sequences than the cut takes, not with short splits, and without outgrowing the array of the entry point that cannot
+    allocate."""
+    finer = 0
+    for B in [*range(1, 70), 96, 128, 255, 256, 257, 512, 1024, 1025, 2048, 4096]:
+        for limit in (64, 128, 256, 512, 1024, 2048, 4096, 8192, 16384):
+            split, plain = ops.decode_split_tokens(B, Hc, limit, 128), plain_split(B, Hc, limit)
+            if split != plain:
+                finer += 1
+                assert split < plain < limit and B <= 1024 and 8 * B >= 512 // Hc
+                assert plain >= 1024 or (plain == 512 and limit > 7 * 512)
+                assert B * (-(-limit // split) - 1) >= 512 // Hc > B * (-(-limit // (2 * split)) - 1)
+            need, before = (ops.decode_workspace_bytes(B, 8 * Hc, 128, limit, s) for s in (split, plain))
+            room = _native.NOALLOC_SCRATCH_BYTES
+            assert need <= room or before > room, (B, limit)
+    assert finer > 0 or Hc > 16
+
+
+@pytest.mark.parametrize("B,Hq,Hc", [(512, 128, 16), (1024, 64, 8), (2048, 32, 8)])
+def test_large_batches_under_a_short_limit_need_no_scratch_array(native_lib, B, Hq, Hc):
+    """One split covers a limit of 1024 tokens: the call gets past the size of the array to its null pointers."""
+    rc = native_lib.fp_paged_decode_noalloc(None, 0, 0, None, None, None, 0, None, None, 0, None, 0, 0, None, None, B, Hq, Hc, 1,
+                                            128, 128, 8, B, 8192, 1024, 0, 1.0, 1, None)
+    assert rc == -1 and b"null pointer" in native_lib.fp_last_error()
+    assert ops.decode_workspace_bytes(B, Hq, 128, 1024, ops.decode_split_tokens(B, Hc, 1024, 128)) == 0
