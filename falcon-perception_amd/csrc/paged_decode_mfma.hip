@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
     for (int s = wave, buf = 0; s < n_stages; s += kWaves, buf ^= 1) {
       const int c0 = t0 + s * TS;
       const char* const k_lds = ring + buf * kStageBytes;
-      const char* const v_lds = k_lds + 4096;
+      char* const v_lds = ring + buf * kStageBytes + 4096;
       if (s + kWaves < n_stages) wait_staged<2 * NI>(); else wait_staged<0>();
       if (s == wave) {
 #pragma unroll
@@ -279,6 +279,11 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             if (c0 + blk * 16 + grp * 4 + j >= t1) sc[blk][j] = -INFINITY;
+        // their V rows, copies of the last one, become 0: a probability of 0 against an infinity would be NaN
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          if (c0 + i * RPI + lrow >= t1) *reinterpret_cast<v4u*>(v_lds + i * 1024 + lane * 16) = v4u{0, 0, 0, 0};
+        asm volatile("" : : : "memory");  // a wavefront's LDS instructions are executed in order
       }
       // Reference point of the exponentials, per column: moves only when the column's maximum has outgrown it by
       // kMaxSlack, so most stages need no exchange between the lanes of a column and no rescale.

@@ -80,3 +80,39 @@ def test_infinite_scores_and_values(dtype, D, G, split):
     assert (got[..., 5] == float("inf")).all()
     keep = [d for d in range(D) if d != 5]
     assert torch.equal(got[..., keep], out[..., keep])
+
+
+def one_sequence(dtype, D, G, L, seed=78):
+    """A sequence of L tokens; every head's query is sqrt(D) in element 0, so a key's score is its element 0."""
+    Hc, P = 2, 64
+    st = PagedState(seed, n_pages=8, page_size=P, max_batch=2, Hc=Hc, D=D, dtype=dtype)
+    st.add_sequence(L)
+    st.prefill_random()
+    pk, pv = st.pool_planes()
+    slots = [int(st.cache.page_table[st.slots[0], t // P]) * P + t % P for t in range(L)]
+    q = torch.zeros((1, Hc * G, 1, D), dtype=dtype, device=DEV)
+    q[..., 0] = D ** 0.5
+    args = (st.cache.page_table, torch.tensor(st.slots, dtype=torch.int64, device=DEV),
+            torch.tensor([L - 1], dtype=torch.int32, device=DEV), P, 256)
+    return st, q, pk, pv, slots, args
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("D,G", [(128, 8), (64, 4)])
+@pytest.mark.parametrize("L", [1, 17, 200])
+@pytest.mark.parametrize("split", [512, 64])
+@pytest.mark.parametrize("fused", [False, True], ids=["from-the-pool", "fresh-row"])
+def test_an_infinite_value_in_the_last_row(dtype, D, G, L, split, fused):
+    """The tokens a stage has room for behind the last row have no weight, and none of its infinity either."""
+    st, q, pk, pv, slots, args = one_sequence(dtype, D, G, L)
+    fresh = {}
+    if fused:
+        fresh = dict(k_new=pk[None, :, slots[-1:]].contiguous(), v_new=pv[None, :, slots[-1:]].contiguous())
+    out, lse = ops.paged_decode(q, pk, pv, *args, split_tokens=split, **fresh)
+    for v in (pv[None, :, slots[-1:]], fresh.get("v_new")):
+        if v is not None:
+            v[..., 5] = float("inf")
+    pv[:, slots[-1], 5] = float("inf")
+    got, lse2 = ops.paged_decode(q, pk, pv, *args, split_tokens=split, **fresh)
+    keep = [d for d in range(D) if d != 5]
+    assert (got[..., 5] == float("inf")).all() and torch.equal(got[..., keep], out[..., keep]) and torch.equal(lse2, lse)
