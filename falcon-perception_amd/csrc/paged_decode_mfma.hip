@@ -54,6 +54,7 @@ struct BF16 {
     const vec2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
     return __builtin_bit_cast(uint32_t, v);
   }
+  static __device__ __forceinline__ float above_zero(float p) { return p; }  // fp32's exponents: no p rounds to 0
   static __device__ __forceinline__ float low(uint32_t w) { return __uint_as_float(w << 16); }
   static __device__ __forceinline__ float high(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
   static __device__ __forceinline__ void store(char* p, float v) { *reinterpret_cast<__bf16*>(p) = static_cast<__bf16>(v); }
@@ -74,6 +75,9 @@ struct F16 {
     const vec2 v = {static_cast<_Float16>(lo), static_cast<_Float16>(hi)};
     return __builtin_bit_cast(uint32_t, v);
   }
+  // a probability that would round to 0 becomes the smallest number of the type, so that an infinite V element still meets
+  // something above 0; the other half takes it back (2^-24 - p rounds to 2^-24 again)
+  static __device__ __forceinline__ float above_zero(float p) { return fmaxf(p, fminf(p * 0x1p+102f, 0x1p-24f)); }
   static __device__ __forceinline__ float low(uint32_t w) {
     return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w & 0xffffu)));
   }
@@ -316,7 +320,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
         uint32_t w[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          w[j] = E::pack2(p[2 * j], p[2 * j + 1]);
+          w[j] = E::pack2(E::above_zero(p[2 * j]), E::above_zero(p[2 * j + 1]));
           const uint32_t rest = E::pack2(p[2 * j] - E::low(w[j]), p[2 * j + 1] - E::high(w[j]));
           if (col >= 8) w[j] = rest;
         }

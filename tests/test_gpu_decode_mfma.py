@@ -116,3 +116,22 @@ def test_an_infinite_value_in_the_last_row(dtype, D, G, L, split, fused):
     got, lse2 = ops.paged_decode(q, pk, pv, *args, split_tokens=split, **fresh)
     keep = [d for d in range(D) if d != 5]
     assert (got[..., 5] == float("inf")).all() and torch.equal(got[..., keep], out[..., keep]) and torch.equal(lse2, lse)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("D,G", [(128, 8), (64, 4)])
+@pytest.mark.parametrize("score", [-12.0, -17.5, -24.0, -60.0, -75.0])
+def test_an_infinite_value_of_a_key_that_weighs_next_to_nothing(dtype, D, G, score):
+    """A probability that the 16-bit type rounds to 0 (below 2^-33 of the largest in f16) is still above 0."""
+    st, q, pk, pv, slots, args = one_sequence(dtype, D, G, 200)
+    pk[:, slots, 0] = 0.0
+    pk[:, slots[3], 0] = score
+    out, lse = ops.paged_decode(q, pk, pv, *args, split_tokens=512)
+    pv[:, slots[3], 5] = float("-inf")
+    got, _ = ops.paged_decode(q, pk, pv, *args, split_tokens=512)
+    keep = [d for d in range(D) if d != 5]
+    assert (got[..., 5] == float("-inf")).all() and torch.equal(got[..., keep], out[..., keep])
+    eo, _ = O.decode_attention(f64(q), f64(pk), np.nan_to_num(f64(pv), neginf=0.0), st.mirror.page_table, st.slots,
+                               np.array([199]), 64)
+    rtol, atol = TOL[dtype]
+    np.testing.assert_allclose(f64(got[..., keep]), eo[..., keep], rtol=rtol, atol=atol)
