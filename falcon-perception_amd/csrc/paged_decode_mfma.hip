@@ -41,8 +41,9 @@ typedef short s16x8 __attribute__((ext_vector_type(8)));
 struct BF16 {
   typedef __bf16 vec4 __attribute__((ext_vector_type(4)));
   typedef __bf16 vec8 __attribute__((ext_vector_type(8)));
-  // added to the exponent so that what rounding leaves over of a probability stays a normal number of the type
-  static constexpr float kHeadroom = 0.f;
+  // Added to the exponents.  Here it keeps the probabilities at 1 and below although the reference point lags the maximum:
+  // a product with the largest V of the type stays in fp32.
+  static constexpr float kHeadroom = -kMaxSlack;
   static __device__ __forceinline__ f32x4 mfma_k32(const v4u& a, const v4u& b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(vec8, a), __builtin_bit_cast(vec8, b), c, 0, 0, 0);
   }
@@ -63,7 +64,8 @@ struct BF16 {
 struct F16 {
   typedef _Float16 vec4 __attribute__((ext_vector_type(4)));
   typedef _Float16 vec8 __attribute__((ext_vector_type(8)));
-  static constexpr float kHeadroom = 8.f;  // probabilities up to 2^(8 + kMaxSlack), below the largest f16
+  // what rounding leaves over of a probability stays a normal number; probabilities up to 2^(8 + kMaxSlack) are below the largest f16
+  static constexpr float kHeadroom = 8.f;
   static __device__ __forceinline__ f32x4 mfma_k32(const v4u& a, const v4u& b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(vec8, a), __builtin_bit_cast(vec8, b), c, 0, 0, 0);
   }

@@ -135,3 +135,21 @@ def test_an_infinite_value_of_a_key_that_weighs_next_to_nothing(dtype, D, G, sco
                                np.array([199]), 64)
     rtol, atol = TOL[dtype]
     np.testing.assert_allclose(f64(got[..., keep]), eo[..., keep], rtol=rtol, atol=atol)
+
+
+@pytest.mark.parametrize("D,G", [(128, 8), (64, 4)])
+@pytest.mark.parametrize("score", [1.0, 4.0])
+def test_the_largest_value_of_the_type(D, G, score):
+    """V at the largest bf16 under the key with the largest score, which comes after keys that weigh less: the reference
+    point of the exponentials lags, and no product may leave fp32."""
+    dtype = torch.bfloat16
+    st, q, pk, pv, slots, args = one_sequence(dtype, D, G, 200)
+    pk[:, slots, 0] = 0.0
+    late = slots[4 * (4096 // (2 * D)) + 2]  # in the second stage of the first wavefront
+    pk[:, late, 0] = score
+    pv[:, late, 5] = torch.finfo(dtype).max
+    pv[:, late, 6] = torch.finfo(dtype).min
+    out, _ = ops.paged_decode(q, pk, pv, *args, split_tokens=512)
+    eo, _ = O.decode_attention(f64(q), f64(pk), f64(pv), st.mirror.page_table, st.slots, np.array([199]), 64)
+    rtol, atol = TOL[dtype]
+    np.testing.assert_allclose(f64(out), eo, rtol=rtol + 2.0 ** -16, atol=atol)
