@@ -953,6 +953,18 @@ extern "C" int64_t fp_paged_decode_workspace_bytes(int32_t B, int32_t Hq, int32_
   return static_cast<int64_t>(B) * Hq * ns * (D + 2) * static_cast<int64_t>(sizeof(float));
 }
 
+extern "C" int64_t fp_paged_decode_workspace_bytes_up_to(int32_t max_B, int32_t Hq, int32_t Hc, int32_t D,
+                                                         int32_t max_context, int32_t page_size) {
+  if (max_B < 0 || Hq <= 0 || Hc <= 0 || D <= 0 || max_context < 0 || page_size <= 0)
+    return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_workspace_bytes_up_to: bad dimension");
+  int64_t rows = 0;
+  for (int B = 1; B <= max_B; ++B) {
+    const int ns = n_splits_for(max_context, default_split_tokens(B, Hc, max_context, page_size));
+    if (ns > 1 && static_cast<int64_t>(B) * ns > rows) rows = static_cast<int64_t>(B) * ns;
+  }
+  return rows * Hq * (D + 2) * static_cast<int64_t>(sizeof(float));
+}
+
 namespace {
 
 // A plan has a record per chunk of the even cut; a launch has at most two chunks per CU and cache head.

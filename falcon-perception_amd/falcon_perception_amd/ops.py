@@ -172,6 +172,13 @@ def decode_workspace_bytes(B: int, Hq: int, D: int, max_context: int, split_toke
     return n
 
 
+def decode_workspace_bytes_up_to(max_B: int, Hq: int, Hc: int, D: int, max_context: int, page_size: int) -> int:
+    """The largest `decode_workspace_bytes` of a launch with the default split over the batches 1 .. max_B."""
+    n = int(N.lib().fp_paged_decode_workspace_bytes_up_to(max_B, Hq, Hc, D, max_context, page_size))
+    N.check(n, "fp_paged_decode_workspace_bytes_up_to")
+    return n
+
+
 def _sinks_ptr(sinks: Tensor | None, Hq: int, device) -> int | None:
     if sinks is None:
         return None

@@ -122,7 +122,7 @@ class PagedKVCache(KVCacheBase):
         self._workspace: Tensor | None = None
         self._retired_workspaces: list[Tensor] = []  # graphs captured earlier still write to these
         self._decode_launch: dict[tuple, tuple[int, int]] = {}
-        self._decode_need: dict[tuple, int] = {}
+        self._decode_need: dict[tuple, int] = {}  # largest workspace over the batches, per launch shape without the batch
         self._decode_plan: Tensor | None = None  # the step's plan of the decode kernel (`decode_plan`)
         self._decode_plan_owner = None           # the mask object it was made for
         self._prefill_workspace: Tensor | None = None
@@ -484,9 +484,11 @@ class PagedKVCache(KVCacheBase):
             worst_b = max(B, self.max_batch_size)
             split = self.decode_split_tokens(B, Hc, max_context)
             finest = min(self.decode_split_tokens(1, Hc, max_context), self.decode_split_tokens(worst_b, Hc, max_context))
-            need = max(ops.decode_workspace_bytes(B, Hq, D, max_context, split),
-                       ops.decode_workspace_bytes(worst_b, Hq, D, max_context, finest),
-                       self._largest_decode_need(worst_b, Hq, D, max(max_context, self.table_cols * self.page_size), Hc))
+            all_of = (worst_b, Hq, Hc, D, max(max_context, self.table_cols * self.page_size), self.page_size)
+            if all_of not in self._decode_need:
+                self._decode_need[all_of] = ops.decode_workspace_bytes_up_to(*all_of)
+            need = max(ops.decode_workspace_bytes(B, Hq, D, max_context, split), self._decode_need[all_of],
+                       ops.decode_workspace_bytes(worst_b, Hq, D, max_context, finest))
             if need and (self._workspace is None or self._workspace.numel() < need):
                 if self._workspace is not None:
                     self._retired_workspaces.append(self._workspace)
@@ -494,18 +496,6 @@ class PagedKVCache(KVCacheBase):
             hit = (need, split)
             self._decode_launch[key] = hit
         return (self._workspace if hit[0] else None), hit[1]
-
-    def _largest_decode_need(self, worst_b: int, Hq: int, D: int, max_context: int, Hc: int) -> int:
-        """Workspace bytes that hold the decode launch of every batch up to `worst_b`.  How finely a batch is split does
-        not run in one direction with its size, so each is asked for; 5 us a batch, once per number of heads."""
-        key = (worst_b, Hq, D, max_context, Hc)
-        need = self._decode_need.get(key)
-        if need is None:
-            splits = [self.decode_split_tokens(b, Hc, max_context) for b in range(1, worst_b + 1)]
-            need = max(ops.decode_workspace_bytes(worst_b, Hq, D, max_context, min(splits[0], splits[-1])),
-                       *(ops.decode_workspace_bytes(b, Hq, D, max_context, s) for b, s in enumerate(splits, 1)))
-            self._decode_need[key] = need
-        return need
 
     def decode_plan(self) -> Tensor:
         """Buffer of the decode step's plan (`fp_paged_decode_plan`): allocated once, so that graphs captured

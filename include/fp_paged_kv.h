@@ -149,6 +149,10 @@ int32_t fp_paged_decode_default_split(int32_t B, int32_t Hc, int32_t max_context
  */
 int64_t fp_paged_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t D,
                                         int32_t max_context, int32_t split_tokens);
+/* The most of it that a launch with the default split needs over all batches of 1 .. max_B sequences: how finely a batch
+ * is split does not run in one direction with its size. */
+int64_t fp_paged_decode_workspace_bytes_up_to(int32_t max_B, int32_t Hq, int32_t Hc, int32_t D, int32_t max_context,
+                                              int32_t page_size);
 
 /*
  * Split-K paged decode attention (one query token per sequence) + cross-split merge.
