@@ -384,3 +384,42 @@ def test_the_drop_in_plans_once_per_step_mask(monkeypatch, fused):
         assert calls.count("plan") == 1 and calls[0] == "plan", calls
     rec = records(cache.decode_plan())
     assert rec[0, 0] >= 1 and rec[0, 1] == B  # the launch was large enough to be cut evenly: the plan was read
+
+
+@pytest.mark.parametrize("fused", [True, False], ids=["append-fused", "append-first"])
+def test_a_mask_kept_while_its_positions_advance_plans_every_step(fused):
+    """Sixteen sequences under a limit of 8192 tokens, cut evenly: one mask object, the positions advance in place between the
+    steps.  The plan of a step must not outlive it (its launches would also append to the slots of the step before)."""
+    dtype, B, Hc, G, D, P, ctx, layers = torch.bfloat16, 16, 8, 2, 128, 128, 8192, 3
+    lens = [60 + 97 * i for i in range(B)]
+    st = PagedState(98, n_pages=ctx // P + sum(-(-(n + 4) // P) for n in lens), page_size=P, max_batch=B + 2, Hc=Hc, D=D,
+                    dtype=dtype, n_layers=layers)
+    for n in lens:
+        st.add_sequence(n + 4)
+    st.cache.kv_cache.normal_()
+    cache = st.cache
+    cache.fuse_decode_append = fused
+    bidx = torch.tensor(st.slots, dtype=torch.int64, device=DEV)
+    pos = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    input_pos = pos.view(B, 1)
+    full = cache.create_causal_blockmask(B=1, L=ctx)
+    row, blk = torch.zeros_like(bidx), (pos // P).long()
+    logical = BlockMask.from_kv_blocks(
+        full.kv_num_blocks[row, :, blk].view(B, 1, 1), full.kv_indices[row, :, blk].view(B, 1, 1, -1),
+        full.full_kv_num_blocks[row, :, blk].view(B, 1, 1), full.full_kv_indices[row, :, blk].view(B, 1, 1, -1),
+        BLOCK_SIZE=full.BLOCK_SIZE, mask_mod=lambda b, h, q, kv: q + pos[b] >= kv, seq_lengths=(1, ctx))
+    mask = cache.convert_logical_block_mask(logical, bidx)
+    for step in range(3):
+        for layer in range(layers):
+            q, k, v = (randn(st.gen, (B, h, 1, D), dtype).to(DEV) for h in (Hc * G, Hc, Hc))
+            K, V = cache.insert_kv(layer, k, v, input_pos=input_pos, batch_idx=bidx)
+            out, aux = A.compiled_flex_attn_decode(q, K, V, block_mask=mask, return_aux=AuxRequest(lse=True))
+            pk, pv = cache.kv_cache[layer, 0, 0], cache.kv_cache[layer, 1, 0]
+            slots = cache.page_table[bidx, pos.long() // P] * P + pos.long() % P
+            assert torch.equal(pk[:, slots], k[:, :, 0].transpose(0, 1)), (step, layer)
+            eo, el = ops.paged_decode(q, pk, pv, cache.page_table, bidx, pos, P, mask.max_context,
+                                      split_tokens=cache.decode_launch(B, Hc * G, D, mask.max_context, Hc)[1])
+            torch.testing.assert_close(out, eo, rtol=2 ** -7, atol=1e-3)  # the fresh row is folded in another order
+            torch.testing.assert_close(aux.lse.view(el.shape), el, rtol=1e-5, atol=1e-5)
+        assert records(cache.decode_plan())[0, 1] == B  # the launch was planned
+        pos += 1
