@@ -827,8 +827,10 @@ int resident_workgroups() {
   return cached[dev] > 0 ? cached[dev] : 0;
 }
 
-// Launches with four or more query heads per cache head in a 16-bit type run on the matrix cores: with eight the vector
-// pipe's dot products take twice as long as the rows (142.7 us against 78.7 us at 415 MB), with four 3 % longer.
+// Launches with four or more query heads per cache head in a 16-bit type run on the matrix cores.  us a layer on the vector
+// pipe / on the matrix cores, 8 cache heads, bf16, eight query heads per cache head: one sequence of 711 tokens 15.7 / 11.1, 16 of 100
+// to 600 31.7 / 18.8, 64 of 1000 to 4000 204 / 117; four: 12.0 / 10.7, 22.6 / 17.5 and 120 / 112, at head_dim 64 11.9 / 9.5, 17.2 / 14.4
+// and 70.2 / 63.0; f16 the same.  With two the vector pipe is not the limit.
 template <typename E, int G, bool kPerHeadK>
 constexpr bool on_matrix_cores() { return sizeof(typename E::type) == 2 && !kPerHeadK && G >= 4; }
 

@@ -7,15 +7,16 @@
 //   S^T = K Q^T   v_mfma_f32_16x16x32: 16 keys x 16 columns.  Columns 0 .. 7 and 8 .. 15 both hold the heads of the group.
 //   O^T += V^T P^T  v_mfma_f32_16x16x16: P^T is in the B operand's layout as the scores leave the first product.  Columns
 //         0 .. 7 carry the probabilities rounded to the 16-bit type and columns 8 .. 15 what that rounding left over; the two
-//         halves of O^T are added at the end, so P keeps twice the mantissa bits of the type and the result is that of
-//         fp32 probabilities (bf16: 1.7e-3 of the output's norm from the float64 result either way, all of it the rounding of the output).
+//         halves of O^T are added at the end, so P keeps 16 (bf16) or 22 (f16) bits against the 24 of the vector kernel.
+//         The result's error against float64 is the rounding of the output either way: 1.648e-3 to 1.664e-3 (bf16) and 2.05e-4 to
+//         2.10e-4 (f16) over contexts of 64 to 8191 tokens, 1e-6 of that apart from the vector kernel's.
 //   K and V go straight from HBM into LDS (global_load_lds, non-temporal), row-major with the 16-byte chunks permuted
 //         against bank conflicts; V^T comes out through ds_read_b64_tr_b16.  Every wavefront has a ring of two stages of
 //         4 KB of K and 4 KB of V of its own: no barrier inside a token range, and the next stage is on its way while one
 //         is worked on.  Two workgroups to a CU keep 64 to 128 KB in flight per CU.
 // HBM-bound.  Per layer-step, merge pass included, against the vector kernel: 24 sequences of 512 to 8191 tokens, 64 q / 8 kv
-// heads, bf16 (415 MB) 78.7 us (5.3 TB/s) against 142.7 us; 96 sequences of 4352 to 16384 tokens, 32 q / 8 kv heads (4.0
-// GB) 604 us (6.7 TB/s) against 624 us.
+// heads, bf16 (415 MB) 76.8 us (5.4 TB/s) against 142.7 us; 96 sequences of 4352 to 16384 tokens, 32 q / 8 kv heads (4.0
+// GB) 626 us (6.5 TB/s) against 648 us.
 #include "decode_common.h"
 #include "paged_decode_mfma.h"
 #include "prefill_common.h"

@@ -932,7 +932,7 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   // LDS twice as often: 2700 rows, 352 workgroups, 88 us against 73 us); key shares go on top as often as they fit.  us a launch
   // with its merge, 16 q heads on 16, D 128, with whole workgroups in up to 8 shares / so: 128 rows over 1, 400, 1400 and 3000 cached keys
   // 20.0 / 19.8, 21.9 / 21.3, 24.1 / 23.9 and 28.4 / 27.3; 512 rows 32.2 / 25.7, 33.2 / 29.8, 35.6 / 31.0 and 37.9 / 35.2; 1024 rows 38.8 /
-  // 32.6, 40.5 / 34.5, 44.1 / 40.3 and 52.7 / 50.9.  Short prompts without a merge, D 128 and 64: 59 rows 13.1 / 10.8 and 10.5 / 8.0,
+  // 32.6, 40.5 / 34.5, 44.1 / 40.3 and 52.7 / 50.9.  Short prompts without a merge, back to back, D 128 and 64: 59 rows 13.1 / 10.8 and 10.5 / 8.0,
   // 170 rows 18.8 / 13.0 and 13.7 / 9.4, 613 rows 24.3 / 18.4 and 16.7 / 13.3.  Not the better one at 129 to 170 workgroups over 3000 keys
   // and more, which leave no room for a second share (640 rows of 32 q / 8 kv heads: 56.5 / 61.4; over 1400 keys 44.2 / 42.1).
   if constexpr (G <= 4) {
