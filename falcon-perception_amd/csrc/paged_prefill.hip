@@ -366,9 +366,9 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     // Every wavefront stages NI groups of RPI rows of each tile.  Where a page holds whole tiles
     // (page size a power of two, at least the tile), a tile in a mapped page is contiguous in the
     // pool: its first slot is looked up once per run into s_tslot, and a staging load is then a
-    // scalar base plus a fixed offset per lane.  In the last tile of a run the rows past the last key
-    // read that key's row again: a page behind the last key may hold anything, and these keys are masked,
-    // but 0 x inf is not 0.  (Staged row by row, every load instruction of such a tile waits for a page
+    // scalar base plus a fixed offset per lane.  In the last tile of a run the rows past the last key read
+    // slot 0: a page behind the last key may hold anything, and so may the last key's own row; these keys are
+    // masked, but 0 x inf is not 0.  (Staged row by row, every load instruction of such a tile waits for a page
     // id of its own, about 5000 cycles a run.)  Any other tile (small or odd page sizes, unmapped pages,
     // runs longer than the table) is staged row by row: a key that does not exist (past the run's
     // last key, or an unmapped page) reads slot 0, finite bytes, and every such key is masked.
@@ -423,9 +423,9 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
         load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(ts) * ROWB, is_k ? lane_k[i] : lane_v[i], lds);
       } else if (ts <= kTailSlot) {
         asm volatile("");  // once per run
-        const int past = i * ITEMS * RPI + st_row0 - tail_row;
-        const uint32_t off = (is_k ? lane_k[i] : lane_v[i]) - (past > 0 ? past : 0) * ROWB;
-        load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(kTailSlot - ts) * ROWB, off, lds);
+        const int r = i * ITEMS * RPI + st_row0;
+        const int64_t slot = r <= tail_row ? static_cast<int64_t>(kTailSlot - ts) + r : 0;
+        load_to_lds((is_k ? ksrc : vsrc) + slot * ROWB, lds);
       } else {
         asm volatile("");  // rare: keep it out of the way as a branch
         const int kpos = kt * kTileN + i * ITEMS * RPI + st_row0;

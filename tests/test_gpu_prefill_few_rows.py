@@ -71,6 +71,27 @@ def test_rows_behind_the_last_key_stay_out(dtype, rows):
     np.testing.assert_allclose(f64(out[:, :, -100:]), f64(ref), atol=atol, rtol=rtol)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("D,G", [(128, 1), (64, 4), (128, 8)])
+@pytest.mark.parametrize("L", [1, 63, 100, 700])
+@pytest.mark.parametrize("repeat", [1, 60])
+@pytest.mark.parametrize("cut", [False, True], ids=["uncut", "key-shares"])
+def test_an_infinite_value_in_the_last_key(dtype, D, G, L, repeat, cut):
+    """The rows of the last tile behind the last key have no weight, and none of its infinity either: every row sees every key,
+    so the element is infinite in every row and the others keep their bits (launches of few rows and of many)."""
+    P = 128
+    st, q, bidx, lim = make_case(dtype, D, G, P, lens=[L], pads=[0])
+    q, bidx, lim = (0.1 * q).repeat(1, 1, repeat, 1).to(DEV), bidx.repeat(repeat), torch.full_like(lim, L).repeat(repeat)
+    pk, pv = st.pool_planes()
+    last = int(st.cache.page_table[st.slots[0], (L - 1) // P]) * P + (L - 1) % P
+    args = (q, pk, pv, st.cache.page_table, bidx, lim, P)
+    out, lse = ops.paged_prefill(*args, workspace=None if cut else False)
+    pv[:, last, 5] = float("inf")
+    got, lse2 = ops.paged_prefill(*args, workspace=None if cut else False)
+    keep = [d for d in range(D) if d != 5]
+    assert (got[..., 5] == float("inf")).all() and torch.equal(got[..., keep], out[..., keep]) and torch.equal(lse2, lse)
+
+
 @pytest.mark.parametrize("D,G,rows", [(128, 1, 64), (64, 2, 300), (128, 8, 100), (128, 4, 200)])
 def test_a_launch_without_key_shares_needs_no_workspace(D, G, rows):
     """Up to `prefill_uncut_keys` the bits are those of the launch without a workspace; four tiles on it is cut."""
