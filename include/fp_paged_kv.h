@@ -457,6 +457,7 @@ int32_t fp_paged_prefill_uncut_keys(int32_t Lq, int32_t Hq, int32_t Hc, int32_t 
  * against 278 us); at head_dim 128 it changes nothing.  The ranking itself takes 5 us at 4096 rows, 21 us at 23040.  Results are bit-identical with and without.
  *   fp_paged_prefill_tile_rows   rows per query tile of the launch fp_paged_prefill makes for this shape and
  *                                workspace size (32 .. 256; 0: the launch takes no order - fp32)
+ *                                (launches of few rows, whose workgroups all start at once, leave an order aside)
  *   fp_paged_prefill_tile_order  order[ceil(Lq / tile_rows)] int32: query tiles by decreasing key range (the
  *                                largest row_limit of the tile's rows, padding rows counting as 0); at most
  *                                4096 tiles

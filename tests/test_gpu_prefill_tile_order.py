@@ -106,10 +106,12 @@ def test_a_launch_with_an_order_returns_the_bits_of_the_launch_without(dtype, D,
     torch.cuda.synchronize()
 
 
-def test_the_order_with_the_launch_cut_along_the_keys():
-    """One sequence's chunk (few workgroups): with a workspace the launch is cut along the keys and keeps the
-    eight-wavefront tile size also at head_dim 64; the order made for that size is taken, same bits."""
-    dtype, D, G, Hc, P = torch.bfloat16, 64, 2, 8, 128
+@pytest.mark.parametrize("G,Hc,tiles", [(2, 8, (128, 64)), (8, 8, (32, 32))], ids=["halves", "whole-workgroups"])
+def test_the_order_with_the_launch_cut_along_the_keys(G, Hc, tiles):
+    """One sequence's chunk (few workgroups): with a workspace the launch is cut along the keys.  With eight query heads per
+    cache head the order made for its tile size is taken; with two the workgroups of few rows all start at once and leave it
+    aside.  Same bits either way."""
+    dtype, D, P = torch.bfloat16, 64, 128
     st, bidx, lim = packed_chunks(31, 1, 512, 3000, P, Hc, D, dtype)
     Lq = bidx.numel()
     q = randn(st.gen, (1, Hc * G, Lq, D), dtype).to(DEV)
@@ -118,7 +120,7 @@ def test_the_order_with_the_launch_cut_along_the_keys():
     assert need > 0
     ws = torch.empty(need, dtype=torch.uint8, device=DEV)
     rows = ops.prefill_tile_rows(Lq, Hc * G, Hc, D, dtype, need)
-    assert rows == 128 and ops.prefill_tile_rows(Lq, Hc * G, Hc, D, dtype, 0) == 64
+    assert (rows, ops.prefill_tile_rows(Lq, Hc * G, Hc, D, dtype, 0)) == tiles
     ref = ops.paged_prefill(q, pk, pv, st.cache.page_table, bidx, lim, P, workspace=ws)
     got = ops.paged_prefill(q, pk, pv, st.cache.page_table, bidx, lim, P, workspace=ws,
                             tile_order=ops.prefill_tile_order(bidx, lim, rows))
