@@ -421,20 +421,21 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       char* lds = dst + kg * TILE_BYTES + (i * ITEMS + item) * RPI * ROWB;  // wavefront-uniform
       if (ts >= 0) {
         load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(ts) * ROWB, is_k ? lane_k[i] : lane_v[i], lds);
-      } else if (ts <= kTailSlot) {
-        asm volatile("");  // once per run
-        const int r = i * ITEMS * RPI + st_row0;
-        const int64_t slot = r <= tail_row ? static_cast<int64_t>(kTailSlot - ts) + r : 0;
-        load_to_lds((is_k ? ksrc : vsrc) + slot * ROWB, lds);
       } else {
         asm volatile("");  // rare: keep it out of the way as a branch
-        const int kpos = kt * kTileN + i * ITEMS * RPI + st_row0;
-        int blkid, off;
-        key_block(kpos, blkid, off);
-        const bool in_range = kpos < kv_max && blkid < a.n_pages;
-        const int64_t pg = pt_row[in_range ? blkid : 0];
-        const bool ok = in_range && pg >= 0 && pg < pool_pages;
-        const int slot = ok ? static_cast<int>(pg) * a.pd.page_size + off : 0;
+        const int r = i * ITEMS * RPI + st_row0;
+        int slot;
+        if (ts <= kTailSlot) {  // once per run
+          slot = r <= tail_row ? kTailSlot - ts + r : 0;
+        } else {
+          const int kpos = kt * kTileN + r;
+          int blkid, off;
+          key_block(kpos, blkid, off);
+          const bool in_range = kpos < kv_max && blkid < a.n_pages;
+          const int64_t pg = pt_row[in_range ? blkid : 0];
+          const bool ok = in_range && pg >= 0 && pg < pool_pages;
+          slot = ok ? static_cast<int>(pg) * a.pd.page_size + off : 0;
+        }
         load_to_lds((is_k ? ksrc : vsrc) + static_cast<int64_t>(slot) * ROWB, lds);
       }
     };
