@@ -900,17 +900,21 @@ void launch_merge(const PrefillArgs& a, int shares, hipStream_t st) {
                      dim3(kMergeThreads), 0, st, a, shares);
 }
 
-// How often workgroups of half the rows, whose halves take the key tiles in turn (launch_group), fit the GPU
-int64_t halves_fit(int Lq, int Hc, int g) {
-  const int rows = g > 4 ? 1 : (kWaves / 2 / g) * 32;
-  return g > 4 ? 0 : fp::compute_units() / (static_cast<int64_t>(Hc) * ((Lq + rows - 1) / rows));
+// How often workgroups of half the rows, whose halves take the key tiles in turn (launch_group), fit the GPU.  0 where a page does
+// not hold whole tiles: staging row by row is then the longer part, and they stage twice as often (us a layer with its insert, pages of
+// 32, so / with whole workgroups and key shares: 16 heads, 613 rows 45.7 / 41.2, 1024 rows over 400 keys 60.0 / 50.2; 16 q / 8 kv heads,
+// 512 rows over 1400 keys 46.8 / 42.1; with pages of 64, two chunks of 300 to 760 rows 38.4 / 45.8).
+int64_t halves_fit(int Lq, int Hc, int g, int page_size) {
+  if (g > 4 || page_size % kTileN != 0 || (page_size & (page_size - 1)) != 0) return 0;
+  const int rows = (kWaves / 2 / g) * 32;
+  return fp::compute_units() / (static_cast<int64_t>(Hc) * ((Lq + rows - 1) / rows));
 }
 
 // Key shares of a bf16 / f16 launch whose workspace holds them
-int launch_shares(int Lq, int Hq, int Hc) {
+int launch_shares(int Lq, int Hq, int Hc, int page_size) {
   const int g = Hq / Hc, bm = (kWaves / g) * 32;
   const int shares = key_shares_for(static_cast<int64_t>(Hc) * ((Lq + bm - 1) / bm), FP_DTYPE_BF16);
-  const int64_t fit = halves_fit(Lq, Hc, g);
+  const int64_t fit = halves_fit(Lq, Hc, g, page_size);
   return fit >= 1 && fit < shares ? static_cast<int>(fit) : shares;
 }
 
@@ -920,8 +924,8 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   const bool bounded = bounded_path<E>(score_bound);
   constexpr int BM = (kWaves / G) * 32;
   a.n_tiles = (a.Lq + BM - 1) / BM;
-  const bool halves = halves_fit(a.Lq, a.Hc, G) >= 1;
-  int shares = workspace ? launch_shares(a.Lq, a.Hq, a.Hc) : 1;
+  const bool halves = halves_fit(a.Lq, a.Hc, G, a.pd.page_size) >= 1;
+  int shares = workspace ? launch_shares(a.Lq, a.Hq, a.Hc, a.pd.page_size) : 1;
   while (shares > 1 && share_bytes(shares, a.Lq, a.Hq, D, 2) > workspace_bytes) --shares;  // what the workspace holds
   if (shares > 1) {
     a.ws_ml = static_cast<float*>(workspace);
@@ -1058,11 +1062,12 @@ extern "C" int32_t fp_paged_prefill_tile_rows(int32_t Lq, int32_t Hq, int32_t Hc
   return tile_rows_for(Lq, Hq, Hc, D, dtype, workspace_bytes);
 }
 
-extern "C" int32_t fp_paged_prefill_uncut_keys(int32_t Lq, int32_t Hq, int32_t Hc, int32_t D, int dtype) {
+extern "C" int32_t fp_paged_prefill_uncut_keys(int32_t Lq, int32_t Hq, int32_t Hc, int32_t D, int32_t page_size, int dtype) {
   const int64_t bytes = fp_paged_prefill_workspace_bytes(Lq, Hq, Hc, D, dtype);
   if (bytes < 0) return static_cast<int32_t>(bytes);
-  if (bytes == 0 || (dtype != FP_DTYPE_F32 && launch_shares(Lq, Hq, Hc) == 1)) return INT32_MAX;
-  return dtype == FP_DTYPE_F32 ? 0 : uncut_tiles(Lq, Hq, halves_fit(Lq, Hc, Hq / Hc) >= 1) * kTileN;
+  if (page_size <= 0) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_prefill_uncut_keys: page_size = %d", page_size);
+  if (bytes == 0 || (dtype != FP_DTYPE_F32 && launch_shares(Lq, Hq, Hc, page_size) == 1)) return INT32_MAX;
+  return dtype == FP_DTYPE_F32 ? 0 : uncut_tiles(Lq, Hq, halves_fit(Lq, Hc, Hq / Hc, page_size) >= 1) * kTileN;
 }
 
 extern "C" int fp_paged_prefill_tile_order(const int64_t* batch_idx, const int32_t* row_limit, int32_t Lq,

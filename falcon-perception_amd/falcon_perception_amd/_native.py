@@ -71,7 +71,7 @@ SIGNATURES = {
     "fp_paged_prefill_tile_rows": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int, c_int64]),
     "fp_paged_prefill_tile_order": (c_int, [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p]),
     "fp_paged_prefill_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int]),
-    "fp_paged_prefill_uncut_keys": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int]),
+    "fp_paged_prefill_uncut_keys": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int]),
 }
 
 SIGNATURES["fp_probe_mfma_softmax"] = (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_int64, c_void_p])

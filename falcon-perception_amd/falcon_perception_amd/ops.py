@@ -448,9 +448,9 @@ def prefill_workspace_bytes(Lq: int, Hq: int, Hc: int, D: int, dtype: torch.dtyp
     return n
 
 
-def prefill_uncut_keys(Lq: int, Hq: int, Hc: int, D: int, dtype: torch.dtype) -> int:
+def prefill_uncut_keys(Lq: int, Hq: int, Hc: int, D: int, page_size: int, dtype: torch.dtype) -> int:
     """Keys up to which `paged_prefill` does not cut a launch of this shape although it has its workspace: where no
     row sees more, `workspace=False` returns the same bits without a merge pass."""
-    n = int(N.lib().fp_paged_prefill_uncut_keys(Lq, Hq, Hc, D, N.dtype_code(dtype)))
+    n = int(N.lib().fp_paged_prefill_uncut_keys(Lq, Hq, Hc, D, page_size, N.dtype_code(dtype)))
     N.check(n, "fp_paged_prefill_uncut_keys")
     return n

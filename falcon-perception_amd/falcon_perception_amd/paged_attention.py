@@ -528,7 +528,7 @@ class PagedKVCache(KVCacheBase):
         hit = self._prefill_need.get(key)
         if hit is None:
             hit = self._prefill_need[key] = (ops.prefill_workspace_bytes(Lq, Hq, Hc, D, dtype),
-                                             ops.prefill_uncut_keys(Lq, Hq, Hc, D, dtype))
+                                             ops.prefill_uncut_keys(Lq, Hq, Hc, D, self.page_size, dtype))
         need, uncut = hit
         if need == 0 or 0 < most_keys <= uncut:
             return False

@@ -444,7 +444,7 @@ int fp_hybrid_row_limits(const int64_t* input_ids, const int64_t* batch_idx,
 int64_t fp_paged_prefill_workspace_bytes(int32_t Lq, int32_t Hq, int32_t Hc, int32_t D, int dtype);
 /* Keys up to which a launch of this shape is not cut although it has that workspace (INT32_MAX: never cut): a caller
  * that knows no row_limit to be larger may leave the workspace out and with it the merge pass, for the same bits. */
-int32_t fp_paged_prefill_uncut_keys(int32_t Lq, int32_t Hq, int32_t Hc, int32_t D, int dtype);
+int32_t fp_paged_prefill_uncut_keys(int32_t Lq, int32_t Hq, int32_t Hc, int32_t D, int32_t page_size, int dtype);
 
 /*
  * The order of a prefill launch's workgroups (optional; no counterpart in the reference).  The GPU hands the

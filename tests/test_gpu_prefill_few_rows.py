@@ -92,11 +92,12 @@ def test_an_infinite_value_in_the_last_key(dtype, D, G, L, repeat, cut):
     assert (got[..., 5] == float("inf")).all() and torch.equal(got[..., keep], out[..., keep]) and torch.equal(lse2, lse)
 
 
-@pytest.mark.parametrize("D,G,rows", [(128, 1, 64), (64, 2, 300), (128, 8, 100), (128, 4, 200)])
-def test_a_launch_without_key_shares_needs_no_workspace(D, G, rows):
+@pytest.mark.parametrize("P", [64, 32, 24])
+@pytest.mark.parametrize("D,G,rows", [(128, 1, 64), (64, 2, 250), (128, 8, 100), (128, 4, 200)])
+def test_a_launch_without_key_shares_needs_no_workspace(D, G, rows, P):
     """Up to `prefill_uncut_keys` the bits are those of the launch without a workspace; four tiles on it is cut."""
-    dtype, P, Hc = torch.bfloat16, 64, 2
-    uncut = ops.prefill_uncut_keys(rows, Hc * G, Hc, D, dtype)
+    dtype, Hc = torch.bfloat16, 2
+    uncut = ops.prefill_uncut_keys(rows, Hc * G, Hc, D, P, dtype)
     assert uncut % 64 == 0 and uncut >= rows and ops.prefill_workspace_bytes(rows, Hc * G, Hc, D, dtype) > 0
     for keys, same in ((uncut, True), (uncut + 256, False)):
         st, q, bidx, lim = make_case(dtype, D, G, P, lens=[keys], pads=[0])
