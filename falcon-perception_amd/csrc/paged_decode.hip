@@ -792,7 +792,9 @@ bool even_cut_fits(int Hc, int B, int max_context, int page_size) {
 // heads, D 128: limit 8192, 300 to 3000 tokens, 8, 12, 16 and 24 sequences 22.4 / 19.5, 28.3 / 24.1, 35.4 / 27.1 and 43.2 / 35.8, 4000 to
 // 8000 tokens 40.4 / 39.6, 58.9 / 56.8, 69.7 / 69.2 and 107 / 100; limit 4096, 8 sequences of 64 to 300, 100 to 700 and 300 to 1500 tokens
 // 12.6 / 9.9, 14.3 / 11.6 and 14.9 / 15.8, 10 of 100 to 3900 25.7 / 22.8; the price is paid close to the limit, 8 sequences of 3500 to
-// 4000 tokens 26.6 / 30.4.  With shorter splits there is no gain: limit 1024, 16 sequences (256 tokens) 15.5 / 17.5; limit 2048, 16
+// 4000 tokens 26.6 / 30.4, and by many short sequences with one query head per cache head: limit 8192, 32 rows, 24 of them of 239 to 459
+// tokens, 8 heads 16.5 / 16.9 (a single layer, without the step's plan, 20.1 / 22.2), 31 of 149 to 422, 4 heads 12.4 / 12.8; 8 and 16
+// of 149 to 422, 16 q / 8 kv heads 12.9 / 10.8 and 14.7 / 13.8, 48 of 300 to 1500, 8 q / 4 kv heads 29.4 / 25.0.  With shorter splits there is no gain: limit 1024, 16 sequences (256 tokens) 15.5 / 17.5; limit 2048, 16
 // sequences (four of 512) 29.2 / 31.4.  Nor with more pieces: one sequence of 12000 tokens 17.1 / 23.1, three of 300 to 3000 12.5 / 14.9.
 bool even_cut_pays(int Hc, int B, int max_context, int page_size) {
   const int split = plain_split_tokens(B, Hc, max_context);
