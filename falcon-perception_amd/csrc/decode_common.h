@@ -43,6 +43,9 @@ struct DecodeArgs {
   int B;         // sequences of the launch
   int n_chunks;  // even cut (kFlat): workgroups per cache head
   int* plan;     // optional: the step's plan of the even cut (fp_paged_decode_plan), kPlanInts ints per chunk
+  // optional [B, Hc], all 0 between launches: how many splits of a (sequence, workgroup head) have left their
+  // partial result.  The workgroup that is the last merges them, and there is no merge pass (last_to_arrive, merge_splits)
+  int* arrivals;
 };
 
 // The plan of a decode step: what every workgroup of the even cut needs before it can ask for its first K row,
@@ -174,12 +177,162 @@ __device__ __forceinline__ int flat_chunk_len(int total, int n_chunks) {
   return len < 64 ? 64 : (len + 63) & ~63;
 }
 
+// The kernel's arguments (its first parameter) read again where they are used: the merge needs a dozen of them, once, and scalar
+// registers that carried them through the loop over the rows would be spilled into vector registers.
+__device__ __forceinline__ const DecodeArgs& reread_args() {
+  auto p = (const __attribute__((address_space(4))) DecodeArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const DecodeArgs*)p;
+}
+
+// ---- splits that meet without a merge pass ----
+// A launch with `arrivals` goes split by split and has no merge pass: every workgroup leaves its partial result, counts itself
+// in, and the last of a (sequence, workgroup head) merges all of them.  Results are written and read with relaxed device-scope
+// atomics, which go past the eight L2s; a workgroup waits until its own have arrived before it counts itself in, so whoever
+// counts n - 1 others sees all rows, and no cache is written back or invalidated (a device-scope fence writes back an XCD's L2: +68 us
+// at 512 workgroups).  Nobody waits for anybody.  The last one sets its counter back to 0 for the next launch.  The three trips
+// (store, count, load) are 0.4 to 0.5 us each; a launch in a replayed graph is 1.7 us before it does anything, and a merge pass
+// 2.7 to 3.3.  What a launch of this kind is held to, and its figures: merges_itself.
+__device__ __forceinline__ void publish(float* p, float x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void publish2(float* p, float x, float y) {
+  const uint64_t w = static_cast<uint64_t>(__float_as_uint(y)) << 32 | __float_as_uint(x);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 take2(const float* p) {
+  const uint64_t w = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return float2{__uint_as_float(static_cast<uint32_t>(w)), __uint_as_float(static_cast<uint32_t>(w >> 32))};
+}
+
+// Splits of L tokens (> 0) in a launch with arrivals: the launch's length, twice that where there would be more than merge_splits
+// takes at once and half as many still give every CU a workgroup (8000 tokens, 16 q / 8 kv heads, D 128: 13.4 us a layer in 64 splits,
+// 12.3 in 32; 4 heads of 64 in fp32 9.3 and 9.5).
+__device__ __forceinline__ int split_tokens_for(const DecodeArgs& a, int L) {
+  const bool twice = a.Hc >= 8 && L > 32 * a.split_tokens && 2 * a.split_tokens / a.pd.page_size + 2 <= kMaxSplitPages;
+  return twice ? 2 * a.split_tokens : a.split_tokens;
+}
+
+// The workgroup's partial result of sequence b is on its way (publish, by any of its threads): counts it in and says whether it is
+// the last of n.  `flag`: one word of LDS.
+__device__ __forceinline__ bool last_to_arrive(int b, int n, int* flag) {
+  const DecodeArgs& a = reread_args();
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // this wavefront's stores have arrived
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int* const counter = a.arrivals + static_cast<int64_t>(b) * a.Hc + blockIdx.x;
+    const bool last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = last;
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(*flag) != 0;
+}
+
+// Merges the n partial results of sequence b's G heads (rows (b, head, split) of the workspace), normalises, gates and stores
+// them.  A wavefront takes 128 elements of the G x D (two per lane); where there are fewer of these than wavefronts, several
+// share one and take the splits in batches of kMergeBatch in turn.  Every load of two batches is in flight at once.  `s_part`: 4 * 64 * 4 floats
+// of LDS.
+constexpr int kMergeBatch = 8;
+template <typename E, int D>
+__device__ __forceinline__ void merge_splits(int b, int n, int G, float* s_part) {
+  const DecodeArgs& a = reread_args();
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // nothing in here is worked out ahead of the rows and kept in registers through them
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, hc = blockIdx.x;
+  const int n_items = (G * D + 127) / 128;        // 1 or 2 (merges_itself)
+  const int deep = 4 / n_items, turn = wave / n_items, item = wave & (n_items - 1);
+  const int e = item * 128 + lane * 2;
+  const bool on = e < G * D;
+  const int g = on ? e / D : 0, d = on ? e - g * D : 0, hq = hc * G + g;
+  const int64_t row0 = (static_cast<int64_t>(b) * a.Hq + hq) * a.n_splits;
+  const float* const ml_at = a.ws_ml + row0 * 2;
+  const float* const acc_at = a.ws_acc + row0 * D + d;
+  float m = -INFINITY, den = 0.f, num0 = 0.f, num1 = 0.f;
+  float2 ml[2][kMergeBatch], acc[2][kMergeBatch];
+  const auto load = [&](int base, float2 (&ml)[kMergeBatch], float2 (&acc)[kMergeBatch]) {
+    const float* mp = ml_at + base * 2;
+    const float* ap = acc_at + static_cast<int64_t>(base) * D;
+#pragma unroll
+    for (int s = 0; s < kMergeBatch; ++s) {  // past the last split its row again, dropped below
+      ml[s] = take2(mp);
+      acc[s] = take2(ap);
+      const int next = base + s + 1 < n ? 1 : 0;
+      mp += next * 2;
+      ap += next * D;
+    }
+  };
+  const auto fold = [&](int base, const float2 (&ml)[kMergeBatch], const float2 (&acc)[kMergeBatch]) {
+    float mn = m;
+#pragma unroll
+    for (int s = 0; s < kMergeBatch; ++s) mn = fmaxf(mn, ml[s].x);
+    const float ms = safe_max(mn), keep = fast_exp2(m - ms);
+    den *= keep;
+    num0 *= keep;
+    num1 *= keep;
+#pragma unroll
+    for (int s = 0; s < kMergeBatch; ++s) {
+      if (base + s >= n) break;
+      const float w = fast_exp2(ml[s].x - ms);
+      den += ml[s].y * w;
+      num0 += acc[s].x * w;
+      num1 += acc[s].y * w;
+    }
+    m = mn;
+  };
+  const int stride = deep * kMergeBatch;
+#pragma nounroll
+  for (int base = turn * kMergeBatch; base < n; base += 2 * stride) {
+    load(base, ml[0], acc[0]);
+    if (base + stride < n) load(base + stride, ml[1], acc[1]);
+    fold(base, ml[0], acc[0]);
+    if (base + stride < n) fold(base + stride, ml[1], acc[1]);
+  }
+  float4* const slot = reinterpret_cast<float4*>(s_part) + lane;
+  slot[wave * 64] = float4{m, den, num0, num1};
+  __syncthreads();
+  if (turn != 0) return;
+#pragma nounroll
+  for (int t = 1; t < deep; ++t) {
+    const float4 o = slot[(wave + t * n_items) * 64];
+    const float mn = fmaxf(m, o.x), ms = safe_max(mn), keep = fast_exp2(m - ms), w = fast_exp2(o.x - ms);  // w: 0 without a split
+    den = den * keep + o.y * w;
+    num0 = num0 * keep + o.z * w;
+    num1 = num1 * keep + o.w * w;
+    m = mn;
+  }
+  if (!on) return;
+  const float lse_nat = (m + log2f(den)) * kLn2;
+  char* const o = a.out + b * a.os_b + hq * a.os_h + d * sizeof(typename E::type);
+  E::store(o, sink_gate<E>(num0 / den, lse_nat, a.sinks, hq));
+  E::store(o + sizeof(typename E::type), sink_gate<E>(num1 / den, lse_nat, a.sinks, hq));
+  if (d == 0) a.lse[static_cast<int64_t>(b) * a.Hq + hq] = lse_nat;
+}
+
+// Which launches merge their splits themselves, where the caller brings the counters: up to 256 elements a merge (query heads x
+// head_dim), and not the even cut.  A single workgroup takes longer over more than a merge pass that has a wavefront per row, and the
+// even cut's workgroups end together, so that the three trips come on top of all of them.  us a layer in two passes / one launch, 8 heads: 2 x
+// 128 elements, one sequence of 300, 2000 and 8000 tokens 9.1 / 7.7, 9.7 / 8.6 and 12.9 / 12.3, 4 of 100 to 700 13.8 / 11.4; 4 x 64 (matrix cores) 8.6 /
+// 7.7, 8.7 / 7.9, 10.4 / 9.9 and 10.0 / 8.9; 4 x 128 9.5 / 8.4, 10.1 / 9.5, but 13.6 / 13.8 at 8000 tokens, and two of 8000 17.8 / 18.6; 8 x 128
+// 9.9 / 9.9, 8000 tokens 14.5 / 23.0, 4 of 100 to 700 13.7 / 12.3.  Even cut, 2 x 128: 64 of 1088 to 4096 117.3 / 118.1, 96 of 64 to 400 29.0 / 29.6,
+// 16 of 350 to 4620 38.7 / 38.2; 8 x 128: 24 of 512 to 8191 74.5 / 80.1.
+constexpr bool merges_itself(int G, int D) { return G * D <= 256; }
+
 // What a workgroup does with its cut: piece(sequence, first token, tokens, whether it is the sequence's first piece, and
-// where its partial result goes: workspace row head * part_mul + part_add; then the record and the page ids of a planned piece).
+// where its partial result goes: workspace row head * part_mul + part_add; how many pieces the sequence has in a launch with arrivals; position
+// + 1 and page-table row of the sequence; then the page ids of a planned piece).
+
+// Position + 1 of sequence b and its page-table row (-1: not a valid slot), as a piece is given them.
+__device__ __forceinline__ void load_sequence(const DecodeArgs& a, int b, int* raw, int* trow) {
+  const int64_t L = fp::load_index(a.input_pos, b, a.pos_i64) + 1;
+  const int64_t t = a.batch_idx[b];
+  *raw = static_cast<int>(L > INT32_MAX ? INT32_MAX : L < INT32_MIN ? INT32_MIN : L);
+  *trow = t < 0 || t >= a.max_batch ? -1 : static_cast<int>(t);
+}
 
 // Grid (workgroup heads, B, splits).
-template <class Piece>
-__device__ __forceinline__ void walk_split(const DecodeArgs& a, const Piece& piece) {
+template <bool kMerges, class Work>
+__device__ __forceinline__ void walk_split(const DecodeArgs& a, const Work& piece) {
   // A context of L tokens is cut into ceil(L / split_tokens) parts of equal
   // size (a multiple of 64 tokens), so the workgroups of one sequence carry the same load instead of
   // leaving a short tail split.
@@ -190,10 +343,12 @@ __device__ __forceinline__ void walk_split(const DecodeArgs& a, const Piece& pie
   // over the engines.
   const int split = blockIdx.z;
   const int b = static_cast<int>((blockIdx.y + blockIdx.z) % gridDim.y);
-  int64_t L = fp::load_index(a.input_pos, b, a.pos_i64) + 1;
-  if (L > a.max_context) L = a.max_context;
-  const int part = split_part(static_cast<int>(L < 0 ? 0 : L), a.split_tokens);
-  piece(b, split * part, part, split == 0, a.n_splits, static_cast<int64_t>(b) * a.Hq * a.n_splits + split);
+  int raw, trow;
+  load_sequence(a, b, &raw, &trow);
+  const int L = raw > a.max_context ? a.max_context : raw < 0 ? 0 : raw;
+  const int part = split_part(L, kMerges && a.arrivals ? split_tokens_for(a, L) : a.split_tokens);
+  piece(b, split * part, part, split == 0, a.n_splits, static_cast<int64_t>(b) * a.Hq * a.n_splits + split, (L + part - 1) / part,
+        raw, trow, nullptr);
 }
 
 // Grid (workgroup heads, n_chunks): every workgroup streams the same number of rows, whatever the lengths are.  `s_start`
@@ -225,7 +380,7 @@ __device__ __forceinline__ void walk_even_cut(const DecodeArgs& a, int* s_start,
         int r[6];
 #pragma unroll
         for (int j = 0; j < 6; ++j) r[j] = s_start[4 + 6 * k + j];
-        piece(r[0], r[1], r[2], false, 1, static_cast<int64_t>(c + r[0]) * a.Hq, r, s_pages + r[5]);
+        piece(r[0], r[1], r[2], false, 1, static_cast<int64_t>(c + r[0]) * a.Hq, 0, r[3], r[4], s_pages + r[5]);
         __syncthreads();  // the LDS of the piece is free again
       }
       return;
@@ -255,7 +410,9 @@ __device__ __forceinline__ void walk_even_cut(const DecodeArgs& a, int* s_start,
     if (end == begin) continue;  // a sequence without keys has no piece; the merge pass writes its zeros
     const int t0 = lo > begin ? static_cast<int>(lo - begin) : 0;
     const int t1 = static_cast<int>((hi < end ? hi : end) - begin);
-    piece(b, t0, t1 - t0, false, 1, static_cast<int64_t>(c + b) * a.Hq);
+    int raw, trow;
+    load_sequence(a, b, &raw, &trow);
+    piece(b, t0, t1 - t0, false, 1, static_cast<int64_t>(c + b) * a.Hq, 0, raw, trow, nullptr);
     __syncthreads();  // the LDS of the piece is free again
   }
 }

@@ -211,6 +211,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   constexpr int U = decode_loads_in_flight(G, kPerHeadK);  // loads of K (per K head) and of V in flight per lane
   constexpr int CH = RPW * U;           // rows per wavefront iteration
   constexpr int ROWB = D * sizeof(typename E::type);
+  constexpr bool kMerges = !kDirect && !kFlat && merges_itself(G, D);
 
   __shared__ int s_pages[kMaxSplitPages];
   __shared__ float s_acc[kWaves][G][D];
@@ -234,11 +235,9 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   // Tokens [t0, t0 + part) of sequence b; a partial result goes to row hq * part_mul + part_add of the
   // workspace.
   auto piece = [&](const int b, const int t0, const int part, const bool first, const int64_t part_mul,
-                   const int64_t part_add, const int* pre = nullptr, const int* pre_pages = nullptr) {
-  int64_t L = pre ? static_cast<int64_t>(pre[3]) : fp::load_index(a.input_pos, b, a.pos_i64) + 1;
-  const int64_t trow = pre ? static_cast<int64_t>(pre[4]) : a.batch_idx[b];
+                   const int64_t part_add, const int n_pieces, const int raw, const int trow, const int* pre_pages) {
+  int L = trow < 0 ? 0 : raw;
   const int* pages_lds = pre_pages ? pre_pages : s_pages;
-  if (trow < 0 || trow >= a.max_batch) L = 0;
   // A position at or beyond max_context is outside what the launch was sized for: the context is read
   // up to max_context from the pool, and the fresh row of a fused append is neither folded nor stored
   // (it must not land on the slot of position max_context - 1, which holds a valid row).
@@ -248,7 +247,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
     return a.lse[static_cast<int64_t>(b) * a.Hq + hq];
   };
   if (t0 >= L) {
-    if (kDirect && first) {
+    if ((kDirect || (kMerges && a.arrivals)) && first) {
       // no visible key at all: out = 0, lse = -inf
       for (int i = tid; i < G * D; i += kThreads) {
         const int g = i / D, d = i - g * D;
@@ -258,7 +257,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
     }
     return;
   }
-  const int t1 = static_cast<int>(L < t0 + part ? L : t0 + part);
+  const int t1 = L < t0 + part ? L : t0 + part;
   // Fused append: the newest token (position L - 1) is not in the pool yet.  The workgroup whose
   // range holds it reads that row from k_new / v_new, folds it in and writes it to its slot; the
   // pool is only read up to L - 2.
@@ -296,7 +295,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
     const int nblk = pre_pages ? 0 : static_cast<int>(blk_last - blk0) + 1;
     for (int i = tid; i < nblk; i += kThreads) {
       int64_t page = 0;
-      if (blk0 + i < a.n_pages) page = a.page_table[trow * a.pt_row_stride + blk0 + i];
+      if (blk0 + i < a.n_pages) page = a.page_table[static_cast<int64_t>(trow) * a.pt_row_stride + blk0 + i];
       if (page < 0 || page >= a.n_slots / a.pd.page_size) page = 0;  // not a page of the pool
       s_pages[i] = static_cast<int>(page);
     }
@@ -402,6 +401,9 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   __syncthreads();
 
   // combine the wavefronts; one thread per (head of the group, element)
+  const DecodeArgs& e = reread_args();
+  const bool merges = kMerges && e.arrivals != nullptr;
+  const bool direct = kDirect || (merges && n_pieces == 1);  // the only piece: out and lse instead of a partial result
   for (int i = tid; i < G * D; i += kThreads) {
     const int g = i / D, d = i - g * D;
     float mn = -INFINITY;
@@ -416,23 +418,33 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
       den += s_ml[w][g][1] * wgt;
     }
     const int hq = hc * G + g;
-    if (kDirect) {
+    if (direct) {
       const float lse_nat = (mn + log2f(den)) * kLn2;
-      E::store(a.out + b * a.os_b + hq * a.os_h + d * sizeof(typename E::type), sink_gate<E>(num / den, lse_nat, a.sinks, hq));
-      if (d == 0) lse_at(hq) = lse_nat;
+      E::store(e.out + b * e.os_b + hq * e.os_h + d * sizeof(typename E::type), sink_gate<E>(num / den, lse_nat, e.sinks, hq));
+      if (d == 0) e.lse[static_cast<int64_t>(b) * e.Hq + hq] = lse_nat;
     } else {
       const int64_t p = hq * part_mul + part_add;
-      a.ws_acc[p * D + d] = num;
-      if (d == 0) {
-        a.ws_ml[p * 2] = mn;
-        a.ws_ml[p * 2 + 1] = den;
+      if (merges) {
+        publish(e.ws_acc + p * D + d, num);
+        if (d == 0) publish2(e.ws_ml + p * 2, mn, den);
+      } else {
+        e.ws_acc[p * D + d] = num;
+        if (d == 0) {
+          e.ws_ml[p * 2] = mn;
+          e.ws_ml[p * 2 + 1] = den;
+        }
       }
     }
+  }
+  if constexpr (kMerges) {
+    __shared__ int s_last;
+    __shared__ __attribute__((aligned(16))) float s_part[4 * 64 * 4];
+    if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, n_pieces, G, s_part);
   }
   };  // piece
 
   if constexpr (!kFlat) {
-    walk_split(a, piece);
+    walk_split<kMerges>(a, piece);
   } else {
     __shared__ int s_start[kFlatMaxB + 1];
     walk_even_cut<kThreads>(a, s_start, s_pages, piece);
@@ -485,7 +497,7 @@ __global__ __launch_bounds__(64) void paged_decode_plan_kernel(const DecodeArgs 
       }
       int nblk = 0;
       if (t0 < L) {  // the pages of tokens t0 .. min(L, t0 + part) - 1, as the main kernel stages them
-        const int t1 = static_cast<int>(L < t0 + part ? L : t0 + part);
+        const int t1 = L < t0 + part ? L : t0 + part;
         int64_t blk0, blk_last;
         int off_unused;
         a.pd.split(t0, blk0, off_unused);
@@ -497,7 +509,7 @@ __global__ __launch_bounds__(64) void paged_decode_plan_kernel(const DecodeArgs 
         }
         for (int i = lane; i < nblk; i += 64) {
           int64_t page = 0;
-          if (blk0 + i < a.n_pages) page = a.page_table[trow * a.pt_row_stride + blk0 + i];
+          if (blk0 + i < a.n_pages) page = a.page_table[static_cast<int64_t>(trow) * a.pt_row_stride + blk0 + i];
           if (page < 0 || page >= pool_pages) page = 0;  // not a page of the pool
           pages[page_off + i] = static_cast<int>(page);
         }
@@ -837,7 +849,9 @@ template <typename E, int G, bool kPerHeadK>
 constexpr bool on_matrix_cores() { return sizeof(typename E::type) == 2 && !kPerHeadK && G >= 4; }
 
 template <typename E, int D, int G, bool kPerHeadK = false>
-void launch_decode(const DecodeArgs& a, int B, int phases, hipStream_t st) {
+void launch_decode(const DecodeArgs& a0, int B, int phases, hipStream_t st) {
+  DecodeArgs a = a0;
+  if (!merges_itself(G, D)) a.arrivals = nullptr;
   dim3 grid(a.Hc, B, a.n_splits);  // a.Hc = workgroups per sequence and split: cache heads, or groups of G heads
   // rows per wavefront iteration: the loads in flight times 64 / (D * elem / 16) rows each
   const int chunk_rows = decode_loads_in_flight(G, kPerHeadK) * 64 / (D * static_cast<int>(sizeof(typename E::type)) / 16);
@@ -893,7 +907,7 @@ void launch_decode(const DecodeArgs& a, int B, int phases, hipStream_t st) {
       else
         split_k_pass(std::false_type{}, std::false_type{}, grid, a);
     }
-    if (phases & kPhaseMerge) {
+    if ((phases & kPhaseMerge) && (n_chunks > 0 || !a.arrivals)) {
       if (n_chunks > 0)
         hipLaunchKernelGGL((paged_decode_merge_flat_kernel<E, D>), dim3(a.Hq, B), dim3(64), 0, st, af);
       else if (a.n_splits > kMergeWideSplits)
@@ -987,7 +1001,8 @@ int decode_entry(int phases, const NewRows* fresh, const void* q, int64_t q_stri
                  void* workspace, int64_t workspace_bytes, int32_t B, int32_t Hq, int32_t Hc, int32_t kv_rep,
                  int32_t D, int32_t page_size, int32_t n_pages, int32_t max_batch,
                  int64_t n_slots, int32_t max_context, int32_t split_tokens, float scale,
-                 int dtype, void* plan, int64_t plan_bytes, void* stream) {
+                 int dtype, void* plan, int64_t plan_bytes, void* stream,
+                 int32_t* arrivals = nullptr, int64_t arrivals_bytes = 0) {
   const bool plan_only = phases == kPhasePlan;  // q, out, lse and the workspace are not touched then
   const int eb = fp::elem_bytes(dtype);
   if (eb == 0) return fp::fail(FP_ERR_UNSUPPORTED, "fp_paged_decode: unknown dtype %d", dtype);
@@ -1024,6 +1039,11 @@ int decode_entry(int phases, const NewRows* fresh, const void* q, int64_t q_stri
     return fp::fail(FP_ERR_WORKSPACE, "fp_paged_decode: the plan buffer needs %lld bytes (fp_paged_decode_plan_bytes), %lld given",
                     static_cast<long long>(plan_buffer_bytes()), static_cast<long long>(plan_bytes));
 
+  const int64_t counters = static_cast<int64_t>(B) * wg_heads * 4;
+  if (arrivals && (!fp::aligned(arrivals, 4) || arrivals_bytes < counters))
+    return fp::fail(FP_ERR_WORKSPACE, "fp_paged_decode_step: %lld bytes of arrival counters needed, %lld given",
+                    static_cast<long long>(counters), static_cast<long long>(arrivals_bytes));
+
   if (split_tokens == 0) split_tokens = default_split_tokens(B, wg_heads, max_context, page_size);
   if (split_tokens % 64) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode: split_tokens must be a multiple of 64");
   if (split_tokens / page_size + 2 > kMaxSplitPages)
@@ -1038,7 +1058,7 @@ int decode_entry(int phases, const NewRows* fresh, const void* q, int64_t q_stri
                static_cast<char*>(out), out_stride_b * eb, out_stride_h * eb, lse, sinks,
                nullptr, nullptr, Hq, wg_heads, fp::PageDiv(page_size), n_pages, max_batch, n_slots,
                max_context, split_tokens, ns, scale * kLog2e,  // scores are kept in log2 units
-               nullptr, nullptr, 0, 0, 0, 0, B, 0, static_cast<int*>(plan)};
+               nullptr, nullptr, 0, 0, 0, 0, B, 0, static_cast<int*>(plan), arrivals};
   if (fresh) {
     if (!fresh->k || !fresh->v) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_append: null k_new / v_new");
     if (!fp::aligned(fresh->k, 16) || !fp::aligned(fresh->v, 16) || (fresh->k_stride_b * eb) % 16 ||
@@ -1098,6 +1118,13 @@ extern "C" int fp_paged_decode_append(const void* k_new, const void* v_new, int6
                                       int64_t v_stride_b, int64_t v_stride_h, FP_DECODE_PARAMS) {
   const NewRows fresh{k_new, v_new, k_stride_b, k_stride_h, v_stride_b, v_stride_h};
   return decode_entry(kPhasePartial | kPhaseMerge, &fresh, FP_DECODE_ARGS);
+}
+extern "C" int fp_paged_decode_step(int32_t* arrivals, int64_t arrivals_bytes, const void* k_new, const void* v_new,
+                                    int64_t k_stride_b, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_h,
+                                    FP_DECODE_PARAMS) {
+  if (B > 0 && !arrivals) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_step: null arrival counters");
+  const NewRows fresh{k_new, v_new, k_stride_b, k_stride_h, v_stride_b, v_stride_h};
+  return decode_entry(kPhasePartial | kPhaseMerge, k_new || v_new ? &fresh : nullptr, FP_DECODE_ARGS, arrivals, arrivals_bytes);
 }
 
 

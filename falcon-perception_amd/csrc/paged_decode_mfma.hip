@@ -40,6 +40,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 
 struct BF16 {
+  using type = __bf16;
   typedef __bf16 vec4 __attribute__((ext_vector_type(4)));
   typedef __bf16 vec8 __attribute__((ext_vector_type(8)));
   // Added to the exponents.  Here it keeps the probabilities at 1 and below although the reference point lags the maximum:
@@ -63,6 +64,7 @@ struct BF16 {
   static __device__ __forceinline__ float round(float v) { return static_cast<float>(static_cast<__bf16>(v)); }
 };
 struct F16 {
+  using type = _Float16;
   typedef _Float16 vec4 __attribute__((ext_vector_type(4)));
   typedef _Float16 vec8 __attribute__((ext_vector_type(8)));
   // what rounding leaves over of a probability stays a normal number; probabilities up to 2^(8 + kMaxSlack) are below the largest f16
@@ -101,7 +103,7 @@ __device__ __forceinline__ void wait_staged() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLater) : "memory");
 }
 
-template <typename E, int D>
+template <typename E, int D, bool kFlat>
 __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const DecodeArgs a, const Cut cut) {
   constexpr int ROWB = D * 2;             // bytes of a row
   constexpr int CPR = ROWB / 16;          // 16-byte chunks per row
@@ -112,12 +114,12 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
   constexpr int NB = TS / 16;             // 16-key blocks per stage
   constexpr int KK = D / 32;              // k-steps of the score product
   constexpr int DB = D / 16;              // 16-row blocks of O^T
+  constexpr bool kMerges = !kFlat && merges_itself(4, D);  // a launch of eight heads comes without arrival counters
   constexpr int NQ = kMaxGroup * ROWB / 1024;  // load instructions of the query rows
 
   __shared__ __attribute__((aligned(1024))) char s_ring[kWaves * kStages * kStageBytes];
   __shared__ __attribute__((aligned(1024))) char s_q[kMaxGroup * ROWB];
   __shared__ int s_pages[kMaxSplitPages];
-  __shared__ int s_start[kFlatMaxB + 1];
   __shared__ float s_ml[kWaves][kMaxGroup][2];
 
   const int hc = blockIdx.x;
@@ -148,15 +150,13 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
 
   // Tokens [t0, t0 + part) of sequence b; a partial result goes to row hq * part_mul + part_add of the workspace.
   auto piece = [&](const int b, const int t0, const int part, const bool first, const int64_t part_mul,
-                   const int64_t part_add, const int* pre = nullptr, const int* pre_pages = nullptr) {
-    int64_t L = pre ? static_cast<int64_t>(pre[3]) : fp::load_index(a.input_pos, b, a.pos_i64) + 1;
-    const int64_t trow = pre ? static_cast<int64_t>(pre[4]) : a.batch_idx[b];
+                   const int64_t part_add, const int n_pieces, const int raw, const int trow, const int* pre_pages) {
+    int L = trow < 0 ? 0 : raw;
     const int* pages_lds = pre_pages ? pre_pages : s_pages;
-    if (trow < 0 || trow >= a.max_batch) L = 0;
     const bool beyond = L > a.max_context;  // as in paged_decode_kernel: read up to max_context, no fresh row
     if (beyond) L = a.max_context;
     if (t0 >= L) {
-      if (cut.direct && first) {  // no visible key at all: out = 0, lse = -inf
+      if ((cut.direct || (kMerges && a.arrivals)) && first) {  // no visible key at all: out = 0, lse = -inf
         for (int i = tid; i < G * D; i += kThreads) {
           const int g = i / D, d = i - g * D;
           E::store(a.out + b * a.os_b + (hc * G + g) * a.os_h + d * 2, 0.f);
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
       }
       return;
     }
-    const int t1 = static_cast<int>(L < t0 + part ? L : t0 + part);
+    const int t1 = L < t0 + part ? L : t0 + part;
     // fused append: the newest token (position L - 1) is read from k_new / v_new by the workgroup whose range ends with
     // it, and written to its slot
     const bool owns_new = a.k_new != nullptr && !beyond && t1 == L;
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
       if (!pre_pages) {
         for (int i = tid; i <= static_cast<int>(blk_last - blk0); i += kThreads) {
           int64_t page = 0;
-          if (blk0 + i < a.n_pages) page = a.page_table[trow * a.pt_row_stride + blk0 + i];
+          if (blk0 + i < a.n_pages) page = a.page_table[static_cast<int64_t>(trow) * a.pt_row_stride + blk0 + i];
           if (page < 0 || page >= a.n_slots / a.pd.page_size) page = 0;  // not a page of the pool
           s_pages[i] = static_cast<int>(page);
         }
@@ -371,6 +371,9 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
     __syncthreads();
 
     // combine the wavefronts; one thread per (head of the group, element)
+    const DecodeArgs& e = reread_args();
+    const bool merges = kMerges && e.arrivals != nullptr;
+    const bool direct = cut.direct || (merges && n_pieces == 1);  // the only piece: out and lse, no partial result
     for (int i = tid; i < G * D; i += kThreads) {
       const int g = i / D, d = i - g * D;
       float mn = -INFINITY;
@@ -385,33 +388,52 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
         den += s_ml[w][g][1] * wgt;
       }
       const int hq = hc * G + g;
-      if (cut.direct) {
+      if (direct) {
         const float lse_nat = (mn + log2f(den)) * kLn2;
-        E::store(a.out + b * a.os_b + hq * a.os_h + d * 2, sink_gate<E>(num / den, lse_nat, a.sinks, hq));
-        if (d == 0) a.lse[static_cast<int64_t>(b) * a.Hq + hq] = lse_nat;
+        E::store(e.out + b * e.os_b + hq * e.os_h + d * 2, sink_gate<E>(num / den, lse_nat, e.sinks, hq));
+        if (d == 0) e.lse[static_cast<int64_t>(b) * e.Hq + hq] = lse_nat;
       } else {
         const int64_t p = hq * part_mul + part_add;
-        a.ws_acc[p * D + d] = num;
-        if (d == 0) {
-          a.ws_ml[p * 2] = mn;
-          a.ws_ml[p * 2 + 1] = den;
+        if (merges) {
+          publish(e.ws_acc + p * D + d, num);
+          if (d == 0) publish2(e.ws_ml + p * 2, mn, den);
+        } else {
+          e.ws_acc[p * D + d] = num;
+          if (d == 0) {
+            e.ws_ml[p * 2] = mn;
+            e.ws_ml[p * 2 + 1] = den;
+          }
         }
       }
     }
+    if constexpr (kMerges) {  // the rings are free behind the barrier inside
+      __shared__ int s_last;
+      if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, n_pieces, G, reinterpret_cast<float*>(s_ring));
+    }
   };  // piece
 
-  if (cut.flat)
+  if constexpr (kFlat) {
+    __shared__ int s_start[kFlatMaxB + 1];
     walk_even_cut<kThreads>(a, s_start, s_pages, piece);
+  } else {
+    walk_split<kMerges>(a, piece);
+  }
+}
+
+template <typename E, int D>
+void launch(const DecodeArgs& a, const Cut& cut, dim3 grid, hipStream_t st) {
+  if (cut.flat)
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<E, D, true>), grid, dim3(kThreads), 0, st, a, cut);
   else
-    walk_split(a, piece);
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<E, D, false>), grid, dim3(kThreads), 0, st, a, cut);
 }
 
 template <typename E>
 int dispatch(const DecodeArgs& a, int D, const Cut& cut, dim3 grid, hipStream_t st) {
   if (D == 64)
-    hipLaunchKernelGGL((paged_decode_mfma_kernel<E, 64>), grid, dim3(kThreads), 0, st, a, cut);
+    launch<E, 64>(a, cut, grid, st);
   else
-    hipLaunchKernelGGL((paged_decode_mfma_kernel<E, 128>), grid, dim3(kThreads), 0, st, a, cut);
+    launch<E, 128>(a, cut, grid, st);
   return FP_OK;
 }
 

@@ -283,7 +283,7 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
         block_mask._plan_shape = shape
     block_mask._plan_layer = step.layer_id
     out, lse = ops.paged_decode(*args, scale=scale, workspace=workspace, split_tokens=split_tokens, sinks=sinks,
-                                kv_rep=kv_rep, k_new=k_new, v_new=v_new, plan=plan)
+                                kv_rep=kv_rep, k_new=k_new, v_new=v_new, plan=plan, arrivals=cache._decode_arrivals)
     return _result(out, lse, return_aux, return_lse)
 
 

@@ -193,7 +193,8 @@ def paged_decode(q: Tensor, pool_k: Tensor, pool_v: Tensor, page_table: Tensor, 
                  split_tokens: int = 0, workspace: Tensor | None = None,
                  out: Tensor | None = None, lse: Tensor | None = None, phase: str = "both",
                  k_new: Tensor | None = None, v_new: Tensor | None = None,
-                 sinks: Tensor | None = None, kv_rep: int = 1, plan: Tensor | None = None) -> tuple[Tensor, Tensor]:
+                 sinks: Tensor | None = None, kv_rep: int = 1, plan: Tensor | None = None,
+                 arrivals: Tensor | None = None) -> tuple[Tensor, Tensor]:
     """Single-query paged attention.  q [B, Hq, 1, D]; pools [Hc, N, D]; returns out [B, Hq, 1, D], lse [B, Hq, 1].
 
     `kv_rep` > 1 declares a cache with one head per query head whose V heads are `kv_rep` identical
@@ -212,7 +213,11 @@ def paged_decode(q: Tensor, pool_k: Tensor, pool_v: Tensor, page_table: Tensor, 
     `plan`: a uint8 tensor of `decode_plan_bytes()` bytes.  Written by a `phase="plan"` call with the
     arguments of the step (once per step: the positions and page tables of all layers are the same), it lets
     the workgroups of a large launch start from one load instead of positions -> cut -> page table; results
-    are bit-identical with and without."""
+    are bit-identical with and without.
+
+    `arrivals`: an int32 tensor of B * Hc / kv_rep entries or more, all 0, which every launch leaves all 0: a launch
+    that goes split by split is then one launch without a merge pass (`fp_paged_decode_step`).  Like the workspace it serves one
+    launch at a time."""
     N.require_cuda(q, pool_k, pool_v, page_table, batch_idx, input_pos, workspace, out, lse)
     B, Hq, Sq, D = q.shape
     if Sq != 1:
@@ -262,6 +267,14 @@ def paged_decode(q: Tensor, pool_k: Tensor, pool_v: Tensor, page_table: Tensor, 
         k_new, v_new = _rows(k_new), _rows(v_new)
         entry = "fp_paged_decode_append"
         fresh = (k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1))
+    if arrivals is not None:
+        N.require_cuda(arrivals)
+        if phase != "both":
+            raise RuntimeError("arrival counters serve the call that runs both passes")
+        if arrivals.dtype != torch.int32 or not arrivals.is_contiguous():
+            raise RuntimeError("arrivals must be a contiguous int32 tensor")
+        entry = "fp_paged_decode_step"
+        fresh = (arrivals.data_ptr(), arrivals.numel() * 4, *(fresh or (None, None, 0, 0, 0, 0)))
     rc = getattr(N.lib(), entry)(
         *fresh,
         q.data_ptr(), q.stride(0), q.stride(1), pool_k.data_ptr(), pool_v.data_ptr(),

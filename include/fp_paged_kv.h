@@ -44,7 +44,7 @@
 extern "C" {
 #endif
 
-#define FP_ABI_VERSION 8
+#define FP_ABI_VERSION 9
 
 /* element types of pool / q / k / v */
 #define FP_DTYPE_F32 0
@@ -308,6 +308,35 @@ int fp_paged_decode_append(const void* k_new, const void* v_new,
                            float scale, int dtype,
                            void* plan, int64_t plan_bytes,
                            void* stream);
+
+/*
+ * fp_paged_decode_append, or fp_paged_decode where k_new and v_new are NULL, for callers that keep counters: a launch that goes
+ * split by split is then ONE launch, in which the workgroup that is the last to leave its partial result of a (sequence, cache
+ * head) merges them.  Launches that are cut evenly, or with more than 256 elements per sequence and cache head (Hq / Hc * D, or
+ * kv_rep * D), keep their merge pass, which is faster there; they do not touch the counters.
+ *   arrivals   [B, Hc / kv_rep] int32 device memory of the caller, arrivals_bytes long: all 0 before the first launch that
+ *              uses it and never written by anybody else.  Every launch leaves it all 0.  Like the workspace it belongs
+ *              to one launch at a time: launches that overlap need a workspace and counters of their own.
+ * Results equal those of the two passes up to the order of the sums over the splits.  All other arguments as fp_paged_decode_append.
+ */
+int fp_paged_decode_step(int32_t* arrivals, int64_t arrivals_bytes,
+                         const void* k_new, const void* v_new,
+                         int64_t k_stride_b, int64_t k_stride_h,
+                         int64_t v_stride_b, int64_t v_stride_h,
+                         const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                         const void* pool_k, const void* pool_v,
+                         const int64_t* page_table, int64_t pt_row_stride,
+                         const int64_t* batch_idx,
+                         const void* input_pos, int pos_index_type,
+                         void* out, int64_t out_stride_b, int64_t out_stride_h,
+                         float* lse, const float* sinks,
+                         void* workspace, int64_t workspace_bytes,
+                         int32_t B, int32_t Hq, int32_t Hc, int32_t kv_rep, int32_t D,
+                         int32_t page_size, int32_t n_pages, int32_t max_batch,
+                         int64_t n_slots, int32_t max_context, int32_t split_tokens,
+                         float scale, int dtype,
+                         void* plan, int64_t plan_bytes,
+                         void* stream);
 
 /*
  * fp_paged_decode without a workspace argument, for callers that cannot allocate device memory:

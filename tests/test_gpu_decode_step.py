@@ -1,0 +1,116 @@
+"""GPU parity: the decode step as one launch (fp_paged_decode_step).
+
+The last workgroup to leave a partial result merges them, so that a launch has no merge pass.  The pieces and their partial
+results are those of the two passes (which the other decode tests hold against the float64 oracle), only the sums over the pieces
+run in another order: in fp32 that moves a result by less than n * 2^-23 of the largest term for n pieces (n <= 64 here, and
+the weights add up to 1), and the type's rounding comes on top.
+"""
+
+import pytest
+import torch
+
+from falcon_perception_amd import ops
+from tests.gpu_cases import DEV, randn
+from tests.test_gpu_decode_plan import decode, flat_state, new_plan
+
+pytestmark = pytest.mark.gpu
+
+STEP = {torch.bfloat16: 2.0**-7, torch.float16: 2.0**-10, torch.float32: 0.0}  # distance of two neighbours, relative
+
+
+def close(got, ref, dtype, n):
+    (out, lse), (ro, rl) = got, ref
+    bound = 2 * n * 2.0**-23
+    assert not (out.isnan() ^ ro.isnan()).any()
+    tol = STEP[dtype] * ro.float().abs() + bound * (1 + ro.float().abs().amax(-1, keepdim=True))
+    assert ((out.float() - ro.float()).abs() <= tol).all()
+    same = torch.isneginf(lse) == torch.isneginf(rl)
+    assert same.all() and ((lse - rl).abs().nan_to_num(0.0) <= bound * (1 + rl.abs().nan_to_num(0.0, 0.0, 0.0))).all()
+
+
+def inputs(st, B, Hc, G, D, dtype, rep):
+    q = randn(st.gen, (B, Hc * G, 1, D), dtype).to(DEV)
+    k_new = randn(st.gen, (B, Hc * rep, 1, D), dtype).to(DEV)
+    v_new = randn(st.gen, (B, Hc, 1, D), dtype).repeat_interleave(rep, dim=1).to(DEV)
+    return q, k_new, v_new
+
+
+# split by split: one sequence of 64 splits (8 heads: of 32 twice as long ones), of 33, of 17 and of 1, a few of different
+# lengths; cut evenly, where the merge pass stays
+@pytest.mark.parametrize("cut", ["all", "33", "17", "one", "few", "even"])
+@pytest.mark.parametrize("dtype,D,P,G,rep", [
+    (torch.bfloat16, 128, 64, 2, 1), (torch.bfloat16, 64, 24, 4, 1), (torch.float32, 64, 16, 1, 1), (torch.float32, 128, 32, 8, 1),
+    (torch.float16, 128, 48, 8, 1), (torch.bfloat16, 128, 64, 2, 2), (torch.float16, 64, 64, 1, 1), (torch.bfloat16, 64, 16, 4, 4)],
+    ids=str)
+def test_one_launch_gives_what_the_two_passes_give(cut, dtype, D, P, G, rep):
+    B, Hc, split, ctx = {"all": (1, 8, 64, 4096), "33": (1, 8, 64, 64 * 33), "17": (1, 8, 64, 64 * 17), "one": (1, 8, 64, 128),
+                         "few": (7, 4, 128, 1536), "even": (96, 4, 64, 512)}[cut]
+    lens = {"all": [4090], "33": [64 * 33 - 1], "17": [64 * 16], "one": [63], "few": [1535, 0, 700, 127, 128, 1, 900], "even": None}[cut]
+    st = flat_state(17 + D + G, B, Hc, D, P, ctx, dtype, rep, lens)
+    q, k_new, v_new = inputs(st, B, Hc, G, D, dtype, rep)
+    pos = torch.tensor(st.lens, dtype=torch.int32, device=DEV)
+    bidx = torch.tensor(st.slots, dtype=torch.int64, device=DEV)
+    if B > 20:
+        pos[5], bidx[9], bidx[11], pos[13] = -1, B + 40, -3, ctx + 7  # no key, foreign slots, beyond the launch's limit
+    elif B > 1:
+        pos[1], bidx[6] = -1, B + 40
+    arrivals = torch.zeros(B * Hc, dtype=torch.int32, device=DEV)
+    before = st.cache.kv_cache.clone()
+    sinks = torch.linspace(-2, 3, Hc * G, device=DEV)
+    for gate in (None, sinks):
+        kw = dict(max_context=ctx, split_tokens=split, kv_rep=rep, bidx=bidx, sinks=gate)
+        st.cache.kv_cache.copy_(before)
+        ref = decode(st, q, pos, k_new=k_new, v_new=v_new, **kw)
+        pool = st.cache.kv_cache.clone()
+        plan = new_plan()
+        decode(st, q, pos, phase="plan", plan=plan, **kw)
+        for p in (None, plan, new_plan(0xA5)):
+            st.cache.kv_cache.copy_(before)
+            got = decode(st, q, pos, k_new=k_new, v_new=v_new, plan=p, arrivals=arrivals, **kw)
+            close(got, ref, dtype, 64)
+            assert torch.equal(st.cache.kv_cache, pool)
+            assert not arrivals.any()
+            again = decode(st, q, pos, plan=p, arrivals=arrivals, **kw)  # the rows are in the pool now
+            close(again, ref, dtype, 64)
+            assert not arrivals.any()
+
+
+def test_counters_too_small_are_refused():
+    st = flat_state(6, 4, 2, 64, 32, 256, torch.float32)
+    q, *_ = inputs(st, 4, 2, 1, 64, torch.float32, 1)
+    pos = torch.tensor(st.lens, dtype=torch.int32, device=DEV)
+    with pytest.raises(RuntimeError, match="arrival counters"):
+        decode(st, q, pos, max_context=256, split_tokens=64, arrivals=torch.zeros(8 - 1, dtype=torch.int32, device=DEV))
+    with pytest.raises(RuntimeError, match="int32"):
+        decode(st, q, pos, max_context=256, split_tokens=64, arrivals=torch.zeros(8, dtype=torch.int64, device=DEV))
+    with pytest.raises(RuntimeError, match="both passes"):
+        decode(st, q, pos, max_context=256, split_tokens=64, phase="merge", arrivals=torch.zeros(8, dtype=torch.int32, device=DEV))
+
+
+def test_replays_of_a_captured_step():
+    """Layers that share workspace and counters, replayed with the positions advancing in place."""
+    dtype, B, Hc, G, D, P, split, ctx = torch.bfloat16, 6, 8, 2, 128, 32, 128, 1024
+    st = flat_state(8, B, Hc, D, P, ctx - 40, dtype)
+    q, *_ = inputs(st, B, Hc, G, D, dtype, 1)
+    pos = torch.tensor(st.lens, dtype=torch.int32, device=DEV)
+    arrivals = torch.zeros(B * Hc, dtype=torch.int32, device=DEV)
+    ws = torch.empty(ops.decode_workspace_bytes(B, Hc * G, D, ctx, split), dtype=torch.uint8, device=DEV)
+    outs = [(torch.empty_like(q), torch.empty((B, Hc * G, 1), device=DEV)) for _ in range(3)]
+    bidx = torch.tensor(st.slots, dtype=torch.int64, device=DEV)
+
+    def layers():
+        for o, l in outs:
+            decode(st, q, pos, bidx=bidx, max_context=ctx, split_tokens=split, workspace=ws, arrivals=arrivals, out=o, lse=l)
+
+    layers()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layers()
+    for _ in range(6):
+        ref = decode(st, q, pos, bidx=bidx, max_context=ctx, split_tokens=split)
+        graph.replay()
+        for got in outs:
+            close(got, ref, dtype, 64)
+        assert not arrivals.any()
+        pos -= 13
