@@ -837,13 +837,16 @@ constexpr int kMaxKeyShares = 8;
 // Key shares for a launch of `wgs` workgroups, at most (see uncut_tiles).  bf16 / f16: a launch that would leave at least half of the
 // CUs idle is cut along the keys until every CU has a workgroup.  (With about one workgroup per CU
 // already, a cut in two costs more in partial results and their merge than the shorter critical path
-// saves: 138 us against 111 us at 8 sequences x 512 rows.)  fp32: the kernel takes about eight times as
-// long over the same partial results, so the cut pays until there are about four workgroups per CU to
-// even out sequences of different lengths and the last, partly filled round of workgroups (8 sequences
-// x 512 rows: 962 us uncut, 838 us in four shares; one sequence of 4608 rows: 1992 us and 1315 us).
+// saves: 138 us against 111 us at 8 sequences x 512 rows.)  fp32: the kernel takes about four times as long over twice the partial
+// results.  Up to a workgroup for every other CU the same rule (16 heads, D 128, us with 1 / 2 / 3 / 4 / 6 / 8 shares: 512 rows over 4096
+// keys, 32 workgroups, 613 / 326 / 226 / 179 / 130 / 114; 1100 rows, 80 workgroups, 148 / 93 / 75 / 96 / 93 / 108).  Beyond that up to
+// four workgroups per CU even out sequences of different lengths and the last, partly filled round of workgroups: 160 workgroups 565 / 413 /
+// 349 / 339 / 335 / 345 (5: 333), 256 594 / 567 / 526 / 507 / 526 / 562, 336 463 / 431 / 436 / 462 / 508 / 562, 448 640 / 575 / 598 / 635 / 694 / 751, 1120
+// 1873 / 2002 / 2075 / 2184 / 2366 / 2518.
 int key_shares_for(int64_t wgs, int dtype) {
   if (wgs < 1) wgs = 1;
-  const int64_t n = dtype == FP_DTYPE_F32 ? (4 * fp::compute_units() + wgs / 2) / wgs : fp::compute_units() / wgs;
+  const int64_t cus = fp::compute_units();
+  const int64_t n = dtype == FP_DTYPE_F32 && 2 * wgs > cus ? 4 * cus / wgs : cus / wgs;
   return static_cast<int>(n < 1 ? 1 : n > kMaxKeyShares ? kMaxKeyShares : n);
 }
 
