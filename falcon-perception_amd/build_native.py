@@ -1,9 +1,9 @@
-"""Build libfp_paged_kv.so (the gfx950 kernels + C ABI) with hipcc, in-tree.
+"""Build libfp_paged_kv.so (the gfx950 kernels + C ABI) with hipcc, and fp_host.so (its calls from PyTorch tensors) with g++, in-tree.
 
     python falcon-perception_amd/build_native.py
 
-hipcc cross-compiles for gfx950 without a GPU.  The shared library has no torch
-or Python dependency; the host package loads it with ctypes.
+hipcc cross-compiles for gfx950 without a GPU.  The kernels' library has no torch
+or Python dependency; the host package loads it with ctypes.  fp_host.so is a Python module on top of it.
 """
 
 from __future__ import annotations
@@ -14,6 +14,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -21,6 +22,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 OUT_DIR = os.path.join(HERE, "falcon_perception_amd", "_lib")
 LIB_PATH = os.path.join(OUT_DIR, "libfp_paged_kv.so")
+HOST_PATH = os.path.join(OUT_DIR, "fp_host.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 # packed-FP32 VALU forms are switched off for every kernel of this library
@@ -80,12 +82,40 @@ def resource_usage() -> dict[str, dict[str, int]]:
     return out
 
 
+def _compile_host() -> str:
+    import torch
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(OBJ_DIR, "host.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
+           "-I", sysconfig.get_paths()["include"]]
+    for path in cpp_extension.include_paths():
+        cmd += ["-isystem", path]
+    res = subprocess.run([*cmd, "-c", os.path.join(CSRC, "host.cpp"), "-o", obj], capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{res.stdout}\n{res.stderr}")
+    return obj
+
+
+def _link_host(obj: str) -> None:
+    import torch
+
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = HOST_PATH + ".tmp"
+    res = subprocess.run(["g++", "-shared", obj, "-o", tmp, "-L", OUT_DIR, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN",
+                          "-L", libs, "-ltorch_python", "-ltorch_cpu", "-lc10"], capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link of fp_host.so failed:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build_library(verbose: bool = True) -> str:
-    """Compile every csrc/*.hip for gfx950 and link libfp_paged_kv.so. Returns its path."""
+    """Compile every csrc/*.hip for gfx950 and link libfp_paged_kv.so, and fp_host.so on top of it. Returns the library's path."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(OUT_DIR, exist_ok=True)
     srcs = sources()
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        host = ex.submit(_compile_host)
         objs = list(ex.map(_compile, srcs))
     tmp = LIB_PATH + ".tmp"
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", tmp]
@@ -93,6 +123,7 @@ def build_library(verbose: bool = True) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _link_host(host.result())
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources", file=sys.stderr)
     return LIB_PATH

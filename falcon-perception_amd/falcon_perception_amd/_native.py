@@ -7,6 +7,8 @@ fallback.  If it is missing, `lib()` raises and so does every operator.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_void_p
 
@@ -14,6 +16,7 @@ import torch
 
 _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib")
 LIB_PATH = os.path.join(_LIB_DIR, "libfp_paged_kv.so")
+HOST_PATH = os.path.join(_LIB_DIR, "fp_host.so")
 
 FP_ABI_VERSION = 9
 NOALLOC_SCRATCH_BYTES = 64 << 20  # FP_NOALLOC_SCRATCH_BYTES
@@ -109,6 +112,23 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The module of csrc/host.cpp, which calls the same library from tensors; raises if it has not been built."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python falcon-perception_amd/build_native.py`.")
+        loader = importlib.machinery.ExtensionFileLoader("fp_host", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("fp_host", loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     if rc < 0:
         msg = lib().fp_last_error().decode("utf-8", "replace")
@@ -117,6 +137,11 @@ def check(rc: int, what: str) -> None:
 
 def stream_ptr(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def raw_stream(t: torch.Tensor) -> int:
+    """Handle of the stream that is current on the device of `t` (0 for a tensor that is not on the GPU)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device()) if t.is_cuda else 0
 
 
 def require_cuda(*tensors) -> None:

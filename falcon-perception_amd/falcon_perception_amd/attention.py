@@ -20,10 +20,13 @@ The mask-mod factories and `create_attention_mask` keep the reference's names
 
 from __future__ import annotations
 
+import math
+
 import torch
 from torch import Tensor
 from torch.nn.attention.flex_attention import AuxOutput, BlockMask, and_masks, or_masks
 
+from . import _native as N
 from . import ops
 
 __all__ = [
@@ -251,8 +254,10 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
             f"the mask was converted for {tuple(block_mask.batch_idx.shape)} sequences but the last insert_kv of this "
             f"cache appended {tuple(step.batch_idx.shape)}: attention must follow the insert_kv of its own step")
     kv_rep = getattr(cache, "kv_rep", 1)
-    wg_heads = k.shape[1] // kv_rep  # workgroups per sequence and split
-    workspace, split_tokens = cache.decode_launch(q.shape[0], q.shape[1], q.shape[3], block_mask.max_context, wg_heads)
+    B, Hq, _, D = q.shape
+    Hc = k.shape[1]
+    max_context = block_mask.max_context
+    workspace, split_tokens = cache.decode_launch(B, Hq, D, max_context, Hc // kv_rep)  # workgroups per sequence and split
     # the pool views insert_kv returned, as planes [H, N, D]: the cache keeps both forms of every layer
     pools = cache._pools[step.layer_id]
     own = k is pools[0] and v is pools[1]
@@ -262,9 +267,9 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
         # the append of this step was left to this launch (`PagedKVCache.fuse_decode_append`): the kernel
         # appends the rows and attends over them.  Any other k, v than the pool views of the step's layer
         # means the caller is not the model's insert -> attend pair, and the plain append runs first.
-        if own and step.k_new.shape[0] == q.shape[0]:
+        if own and step.k_new.shape[0] == B:
             k_new, v_new = step.k_new, step.v_new
-            cache.last_decode_step = step._replace(k_new=None, v_new=None)
+            cache.last_decode_step = type(step)(step.layer_id, step.input_pos, step.batch_idx)
         else:
             cache.flush()
     # The plan of the step: the reference converts its mask once per step and every layer consumes it
@@ -273,18 +278,23 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
     # several steps, whose positions tensor advances in place, plans again where the layers start over.
     # (The plan saves a layer 1.3 to 2.5 us and takes 4 to 5 us: a model of one or two layers goes without.)
     plan = cache.decode_plan() if len(cache._planes) > 2 else None
-    args = (q, pool_k, pool_v, cache.page_table, block_mask.batch_idx, step.input_pos, cache.page_size,
-            block_mask.max_context)
-    shape = (q.shape[0], q.shape[1], q.shape[3], k.shape[1], kv_rep, split_tokens, step.input_pos.data_ptr())
-    if plan is not None and (cache._decode_plan_owner is not block_mask or block_mask._plan_shape != shape
-                             or step.layer_id <= block_mask._plan_layer):
-        ops.paged_decode(*args, scale=scale, split_tokens=split_tokens, kv_rep=kv_rep, phase="plan", plan=plan)
-        cache._decode_plan_owner = block_mask
-        block_mask._plan_shape = shape
+    args = (q, pool_k, pool_v, cache.page_table, block_mask.batch_idx, step.input_pos, cache.page_size, max_context)
+    if plan is not None:
+        shape = (B, Hq, D, Hc, kv_rep, split_tokens, step.input_pos.data_ptr())
+        if (cache._decode_plan_owner is not block_mask or block_mask._plan_shape != shape
+                or step.layer_id <= block_mask._plan_layer):
+            ops.paged_decode(*args, scale=scale, split_tokens=split_tokens, kv_rep=kv_rep, phase="plan", plan=plan)
+            cache._decode_plan_owner = block_mask
+            block_mask._plan_shape = shape
     block_mask._plan_layer = step.layer_id
-    out, lse = ops.paged_decode(*args, scale=scale, workspace=workspace, split_tokens=split_tokens, sinks=sinks,
-                                kv_rep=kv_rep, k_new=k_new, v_new=v_new, plan=plan, arrivals=cache._decode_arrivals)
-    return _result(out, lse, return_aux, return_lse)
+    got = None
+    if q.is_cuda:
+        got = N.host().decode(*args, 1.0 / math.sqrt(D) if scale is None else scale, split_tokens, workspace, sinks, kv_rep,
+                              k_new, v_new, plan, cache._decode_arrivals, N.raw_stream(q))
+    if got is None:
+        got = ops.paged_decode(*args, scale=scale, workspace=workspace, split_tokens=split_tokens, sinks=sinks,
+                               kv_rep=kv_rep, k_new=k_new, v_new=v_new, plan=plan, arrivals=cache._decode_arrivals)
+    return _result(*got, return_aux, return_lse)
 
 
 def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, block_mask=None,
@@ -323,11 +333,15 @@ def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, 
         rows = cache.prefill_tile_rows(Lq, Hq, D, pool_k.shape[0], q.dtype, workspace.numel() if workspace is not False else 0)
         if rows and -(-Lq // rows) <= 4096:
             order = block_mask.tile_order(step.batch_idx, rows)
-    out, lse = ops.paged_prefill(
-        q, pool_k, pool_v, cache.page_table, step.batch_idx, limits, cache.page_size, scale=scale, sinks=sinks,
-        workspace=workspace, score_bound=cache.score_bound(D, scale), tile_order=order,
-    )
-    return _result(out, lse, return_aux, return_lse)
+    args = (q, pool_k, pool_v, cache.page_table, step.batch_idx, limits, cache.page_size)
+    bound = cache.score_bound(D, scale)
+    got = None
+    if q.is_cuda:
+        got = N.host().prefill(*args, 1.0 / math.sqrt(D) if scale is None else scale, sinks, None if workspace is False else workspace,
+                               bound, *((None, 0) if order is None else order), N.raw_stream(q))
+    if got is None:
+        got = ops.paged_prefill(*args, scale=scale, sinks=sinks, workspace=workspace, score_bound=bound, tile_order=order)
+    return _result(*got, return_aux, return_lse)
 
 
 # --------------------------------------------------------------------------

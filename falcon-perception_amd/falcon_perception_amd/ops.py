@@ -28,6 +28,9 @@ def kv_append(pool_k: Tensor, pool_v: Tensor, k: Tensor, v: Tensor, page_table: 
     `packed`: k, v are the prefill layout [1, H, L, D] with batch_idx, input_pos [1, L]; they are read as
     L row groups of one token each through their strides.
     """
+    if k.is_cuda and N.host().append(pool_k, pool_v, k, v, page_table, batch_idx, input_pos, page_size, clamp_negative, packed,
+                                     N.raw_stream(k)):
+        return
     N.require_cuda(pool_k, pool_v, k, v, page_table, batch_idx, input_pos)
     if v.shape != k.shape:
         raise RuntimeError(f"k {tuple(k.shape)} and v {tuple(v.shape)} must have the same shape")
