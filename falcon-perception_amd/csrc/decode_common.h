@@ -30,7 +30,7 @@ struct DecodeArgs {
   float* ws_ml;   // [B, Hq, n_splits, 2]
   int Hq, Hc;
   fp::PageDiv pd;
-  int n_pages, max_batch;
+  int n_pages, max_batch, pool_pages;  // pool_pages = n_slots / page_size
   int64_t n_slots;
   int max_context;
   int split_tokens;
@@ -41,7 +41,7 @@ struct DecodeArgs {
   const char* v_new;
   int64_t kn_b, kn_h, vn_b, vn_h;  // bytes
   int B;         // sequences of the launch
-  int n_chunks;  // even cut (kFlat): workgroups per cache head
+  int n_chunks;  // even cut (kFlat): workgroups per cache head; walk_pieces: splits of all sequences together, about
   int* plan;     // optional: the step's plan of the even cut (fp_paged_decode_plan), kPlanInts ints per chunk
   // optional [B, Hc], all 0 between launches: how many splits of a (sequence, workgroup head) have left their
   // partial result.  The workgroup that is the last merges them, and there is no merge pass (last_to_arrive, merge_splits)
@@ -116,13 +116,17 @@ __device__ __forceinline__ void row_sum(float (&x)[kN]) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float safe_max(float m) { return m == -INFINITY ? 0.f : m; }
 
+// ceil(L / part) for L > 0; unsigned, which is two thirds of the instructions of the signed division in front of the first row
+__device__ __forceinline__ int pieces_of(int L, int part) {
+  return static_cast<int>((static_cast<uint32_t>(L) + part - 1) / static_cast<uint32_t>(part));
+}
+
 // tokens per split of a context of L tokens: L is divided evenly over ceil(L / split_tokens)
 // splits, rounded up to 64 tokens (so every split starts on a wavefront-iteration boundary)
 __device__ __forceinline__ int split_part(int L, int split_tokens) {
   if (L <= 0) return split_tokens;
-  const int n = (L + split_tokens - 1) / split_tokens;
-  const int even = (L + n - 1) / n;
-  return (even + 63) & ~63;
+  const int n = pieces_of(L, split_tokens);
+  return (pieces_of(L, n) + 63) & ~63;
 }
 
 // Even cut of a launch (kFlat): the contexts of the launch, each rounded up to 64 tokens, are laid end
@@ -205,11 +209,30 @@ __device__ __forceinline__ float2 take2(const float* p) {
   return float2{__uint_as_float(static_cast<uint32_t>(w)), __uint_as_float(static_cast<uint32_t>(w >> 32))};
 }
 
+// x / d for 0 <= x < 2^23, d >= 1 and a quotient below 2^21, in half the instructions of an integer division: it is in front of the
+// first row.  The product's error is below x / d * 2^-22 + 1, so a step up or down is all there is to mend.
+__device__ __forceinline__ int quotient(int x, int d) {
+  const int q = static_cast<int>(static_cast<float>(x) * __builtin_amdgcn_rcpf(static_cast<float>(d)));
+  const int rest = x - q * d;
+  return q + (rest >= d ? 1 : rest < 0 ? -1 : 0);
+}
+
+// Inclusive sum over the lanes up to this one, without a trip through LDS.
+__device__ __forceinline__ int scan_lanes(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8, then row_bcast:15, 31
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true);
+  return x;
+}
+
 // Splits of L tokens (> 0) in a launch with arrivals: the launch's length, twice that where there would be more than merge_splits
 // takes at once and half as many still give every CU a workgroup (8000 tokens, 16 q / 8 kv heads, D 128: 13.4 us a layer in 64 splits,
 // 12.3 in 32; 4 heads of 64 in fp32 9.3 and 9.5).
 __device__ __forceinline__ int split_tokens_for(const DecodeArgs& a, int L) {
-  const bool twice = a.Hc >= 8 && L > 32 * a.split_tokens && 2 * a.split_tokens / a.pd.page_size + 2 <= kMaxSplitPages;
+  const bool twice = a.Hc >= 8 && L > 32 * a.split_tokens && 2 * a.split_tokens < (kMaxSplitPages - 1) * a.pd.page_size;  // pages fit LDS
   return twice ? 2 * a.split_tokens : a.split_tokens;
 }
 
@@ -229,13 +252,13 @@ __device__ __forceinline__ bool last_to_arrive(int b, int n, int* flag) {
   return __builtin_amdgcn_readfirstlane(*flag) != 0;
 }
 
-// Merges the n partial results of sequence b's G heads (rows (b, head, split) of the workspace), normalises, gates and stores
-// them.  A wavefront takes 128 elements of the G x D (two per lane); where there are fewer of these than wavefronts, several
+// Merges the n partial results of sequence b's G heads (rows hq * row_mul + row_add + split of the workspace), normalises, gates and
+// stores them.  A wavefront takes 128 elements of the G x D (two per lane); where there are fewer of these than wavefronts, several
 // share one and take the splits in batches of kMergeBatch in turn.  Every load of two batches is in flight at once.  `s_part`: 4 * 64 * 4 floats
 // of LDS.
 constexpr int kMergeBatch = 8;
 template <typename E, int D>
-__device__ __forceinline__ void merge_splits(int b, int n, int G, float* s_part) {
+__device__ __forceinline__ void merge_splits(int b, int64_t row_mul, int64_t row_add, int n, int G, float* s_part) {
   const DecodeArgs& a = reread_args();
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));  // nothing in here is worked out ahead of the rows and kept in registers through them
@@ -245,7 +268,7 @@ __device__ __forceinline__ void merge_splits(int b, int n, int G, float* s_part)
   const int e = item * 128 + lane * 2;
   const bool on = e < G * D;
   const int g = on ? e / D : 0, d = on ? e - g * D : 0, hq = hc * G + g;
-  const int64_t row0 = (static_cast<int64_t>(b) * a.Hq + hq) * a.n_splits;
+  const int64_t row0 = hq * row_mul + row_add;
   const float* const ml_at = a.ws_ml + row0 * 2;
   const float* const acc_at = a.ws_acc + row0 * D + d;
   float m = -INFINITY, den = 0.f, num0 = 0.f, num1 = 0.f;
@@ -310,7 +333,8 @@ __device__ __forceinline__ void merge_splits(int b, int n, int G, float* s_part)
 }
 
 // Which launches merge their splits themselves, where the caller brings the counters: up to 256 elements a merge (query heads x
-// head_dim), and not the even cut.  A single workgroup takes longer over more than a merge pass that has a wavefront per row, and the
+// head_dim), and not the even cut (merged_pieces: which of these go piece by piece).  A single workgroup takes longer over more than a merge
+// pass that has a wavefront per row, and the
 // even cut's workgroups end together, so that the three trips come on top of all of them.  us a layer in two passes / one launch, 8 heads: 2 x
 // 128 elements, one sequence of 300, 2000 and 8000 tokens 9.1 / 7.7, 9.7 / 8.6 and 12.9 / 12.3, 4 of 100 to 700 13.8 / 11.4; 4 x 64 (matrix cores) 8.6 /
 // 7.7, 8.7 / 7.9, 10.4 / 9.9 and 10.0 / 8.9; 4 x 128 9.5 / 8.4, 10.1 / 9.5, but 13.6 / 13.8 at 8000 tokens, and two of 8000 17.8 / 18.6; 8 x 128
@@ -318,15 +342,37 @@ __device__ __forceinline__ void merge_splits(int b, int n, int G, float* s_part)
 // 16 of 350 to 4620 38.7 / 38.2; 8 x 128: 24 of 512 to 8191 74.5 / 80.1.
 constexpr bool merges_itself(int G, int D) { return G * D <= 256; }
 
-// What a workgroup does with its cut: piece(sequence, first token, tokens, whether it is the sequence's first piece, and
+// What a workgroup does with its cut: piece(sequence, first token, tokens, which of the sequence's pieces it is (of the even cut only: not the first), and
 // where its partial result goes: workspace row head * part_mul + part_add; how many pieces the sequence has in a launch with arrivals; position
 // + 1 and page-table row of the sequence; then the page ids of a planned piece).
 
+// tokens a split has at least there, by the bytes of a row: what the wavefronts ask for at once
+// (16 sequences of 64 to 500 tokens, head_dim 64, 2 query heads, f16: 10.1 us a layer from 128 on, 9.6 from 256)
+constexpr int min_part(int row_bytes) { return row_bytes < 256 ? 256 : 128; }
+constexpr int kMostPieces = 16;  // splits a sequence has at most there: what merge_splits asks for at once with two query heads
+
+// One trip to memory for the arguments up to the first row: each is otherwise asked for where it is first used, and a line of 64
+// bytes that no load before it touched is a trip of its own.
+__device__ __forceinline__ void ask_for_arguments(const DecodeArgs& a) {
+  asm volatile("" : : "s"(a.q), "s"(a.batch_idx), "s"(a.input_pos), "s"(a.Hq), "s"(a.Hc), "s"(a.n_slots), "s"(a.n_splits),
+               "s"(a.k_new), "s"(a.vn_h), "s"(a.B), "s"(a.arrivals));
+}
+
 // Position + 1 of sequence b and its page-table row (-1: not a valid slot), as a piece is given them.
+template <bool kUniform>
 __device__ __forceinline__ void load_sequence(const DecodeArgs& a, int b, int* raw, int* trow) {
-  const int64_t L = fp::load_index(a.input_pos, b, a.pos_i64) + 1;
-  const int64_t t = a.batch_idx[b];
-  *raw = static_cast<int>(L > INT32_MAX ? INT32_MAX : L < INT32_MIN ? INT32_MIN : L);
+  // one trip to memory: both words of an int64 position or an int32 one twice, so that neither its type nor the slot waits for a load
+  const int at = a.pos_i64 ? 2 * b : b;
+  const auto pos = (const __attribute__((address_space(4))) int*)a.input_pos;  // no launch writes them: scalar loads
+  int lo = pos[at];
+  int hi = pos[a.pos_i64 ? at + 1 : at];
+  int64_t t = ((const __attribute__((address_space(4))) int64_t*)a.batch_idx)[b];
+  if constexpr (kUniform)
+    asm volatile("" : "+s"(lo), "+s"(hi), "+s"(t));
+  else
+    asm volatile("" : "+v"(lo), "+v"(hi), "+v"(t));
+  if (a.pos_i64 && hi != lo >> 31) lo = hi < 0 ? INT32_MIN : INT32_MAX;
+  *raw = lo == INT32_MAX ? lo : lo + 1;
   *trow = t < 0 || t >= a.max_batch ? -1 : static_cast<int>(t);
 }
 
@@ -342,13 +388,54 @@ __device__ __forceinline__ void walk_split(const DecodeArgs& a, const Work& piec
   // sequences of 1 k to 4 k tokens).  Rotating the sequences by the split index spreads each sequence
   // over the engines.
   const int split = blockIdx.z;
-  const int b = static_cast<int>((blockIdx.y + blockIdx.z) % gridDim.y);
+  ask_for_arguments(a);
+  int b = blockIdx.y + blockIdx.z;
+  b = static_cast<int>(static_cast<uint32_t>(b) % static_cast<uint32_t>(a.B));
   int raw, trow;
-  load_sequence(a, b, &raw, &trow);
+  load_sequence<true>(a, b, &raw, &trow);
   const int L = raw > a.max_context ? a.max_context : raw < 0 ? 0 : raw;
   const int part = split_part(L, kMerges && a.arrivals ? split_tokens_for(a, L) : a.split_tokens);
-  piece(b, split * part, part, split == 0, a.n_splits, static_cast<int64_t>(b) * a.Hq * a.n_splits + split, (L + part - 1) / part,
+  piece(b, split * part, part, split, a.n_splits, static_cast<int64_t>(b) * a.Hq * a.n_splits + split, L > 0 ? pieces_of(L, part) : 0,
         raw, trow, nullptr);
+}
+
+// Grid (workgroup heads, n_chunks + B) of a launch with arrivals, up to 64 sequences: the splits of all sequences have one length, as long
+// as n_chunks of them need to be, and what a workgroup does follows from the lengths of the sequences.  Split by split it follows
+// from max_context, and a workgroup that finds nothing to do costs the launch 3 ns: 4 sequences of 300 tokens under a limit of 4096, 1024
+// workgroups 10.9 us a layer, 512 9.4, 256 8.1.  Every wavefront works the cut out by itself, a sequence to a lane, without LDS or a barrier; that
+// is 0.3 us in front of the first row, which is why launches that gain nothing else go split by split (merged_pieces).
+template <int kMinPart, class Work>
+__device__ __forceinline__ void walk_pieces(const DecodeArgs& a, const Work& piece) {
+  ask_for_arguments(a);
+  const int lane = threadIdx.x & 63, c = blockIdx.y, pieces = a.n_chunks;
+  int lane_raw, lane_trow;
+  load_sequence<false>(a, lane < a.B ? lane : 0, &lane_raw, &lane_trow);
+  int L = lane_trow < 0 || lane_raw < 0 || lane >= a.B ? 0 : lane_raw;
+  L = L > a.max_context ? a.max_context : L;
+  const int total = __builtin_amdgcn_readlane(scan_lanes(L), 63);
+  int part = total <= kMinPart * pieces ? kMinPart : (quotient(total, pieces) + 64) & ~63;
+  int count, upto;
+  for (int tries = 0;; ++tries) {
+    count = quotient(L + part - 1, part);
+    count = count < 1 ? 1 : count < kMostPieces ? count : kMostPieces;
+    upto = scan_lanes(lane < a.B ? count : 0);
+    // with the remainders there are up to B more than `pieces`, which would run behind the others: somewhat longer, then
+    if (__builtin_amdgcn_readlane(upto, 63) <= pieces || part == kMinPart || tries == 4) break;
+    part += 64 + (part >> 4 & ~63);
+  }
+  // the splits of a sequence are equal, too, and may be fewer for it (every lane its own)
+  int own = (quotient(L + count - 1, count) + 63) & ~63;
+  own = own < 64 ? 64 : own;
+  const int n_own = quotient(L + own - 1, own);
+  const unsigned long long behind = __ballot(upto > c);
+  if (behind == 0) return;
+  const int b = __builtin_ctzll(behind);
+  const int raw = __builtin_amdgcn_readlane(lane_raw, b), trow = __builtin_amdgcn_readlane(lane_trow, b);
+  const int n = __builtin_amdgcn_readlane(n_own, b);
+  part = __builtin_amdgcn_readlane(own, b);
+  const int split = c - __builtin_amdgcn_readlane(upto - count, b);
+  if (split > 0 && split >= n) return;
+  piece(b, split * part, part, split, pieces + a.B, c, n, raw, trow, nullptr);
 }
 
 // Grid (workgroup heads, n_chunks): every workgroup streams the same number of rows, whatever the lengths are.  `s_start`
@@ -380,7 +467,7 @@ __device__ __forceinline__ void walk_even_cut(const DecodeArgs& a, int* s_start,
         int r[6];
 #pragma unroll
         for (int j = 0; j < 6; ++j) r[j] = s_start[4 + 6 * k + j];
-        piece(r[0], r[1], r[2], false, 1, static_cast<int64_t>(c + r[0]) * a.Hq, 0, r[3], r[4], s_pages + r[5]);
+        piece(r[0], r[1], r[2], 1, 1, static_cast<int64_t>(c + r[0]) * a.Hq, 0, r[3], r[4], s_pages + r[5]);
         __syncthreads();  // the LDS of the piece is free again
       }
       return;
@@ -411,8 +498,8 @@ __device__ __forceinline__ void walk_even_cut(const DecodeArgs& a, int* s_start,
     const int t0 = lo > begin ? static_cast<int>(lo - begin) : 0;
     const int t1 = static_cast<int>((hi < end ? hi : end) - begin);
     int raw, trow;
-    load_sequence(a, b, &raw, &trow);
-    piece(b, t0, t1 - t0, false, 1, static_cast<int64_t>(c + b) * a.Hq, 0, raw, trow, nullptr);
+    load_sequence<false>(a, b, &raw, &trow);
+    piece(b, t0, t1 - t0, 1, 1, static_cast<int64_t>(c + b) * a.Hq, 0, raw, trow, nullptr);
     __syncthreads();  // the LDS of the piece is free again
   }
 }

@@ -202,7 +202,7 @@ constexpr int decode_waves_per_simd() {
   return (!kFlat && !kPerHeadK && (G == 1 || (G == 2 && sizeof(typename E::type) == 4))) ? 4 : 1;
 }
 
-template <typename E, int D, int G, bool kDirect, bool kAligned, bool kPerHeadK = false, bool kFlat = false>
+template <typename E, int D, int G, bool kDirect, bool kAligned, bool kPerHeadK = false, bool kFlat = false, bool kPieces = false>
 __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK, kFlat>())) void paged_decode_kernel(const DecodeArgs a) {
   constexpr int EPL = E::kEpl;          // elements per lane
   constexpr int TPR = D / EPL;          // lanes per row
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
 
   // Tokens [t0, t0 + part) of sequence b; a partial result goes to row hq * part_mul + part_add of the
   // workspace.
-  auto piece = [&](const int b, const int t0, const int part, const bool first, const int64_t part_mul,
+  auto piece = [&](const int b, const int t0, const int part, const int split, const int64_t part_mul,
                    const int64_t part_add, const int n_pieces, const int raw, const int trow, const int* pre_pages) {
   int L = trow < 0 ? 0 : raw;
   const int* pages_lds = pre_pages ? pre_pages : s_pages;
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
     return a.lse[static_cast<int64_t>(b) * a.Hq + hq];
   };
   if (t0 >= L) {
-    if ((kDirect || (kMerges && a.arrivals)) && first) {
+    if ((kDirect || (kMerges && a.arrivals)) && split == 0) {
       // no visible key at all: out = 0, lse = -inf
       for (int i = tid; i < G * D; i += kThreads) {
         const int g = i / D, d = i - g * D;
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
     for (int i = tid; i < nblk; i += kThreads) {
       int64_t page = 0;
       if (blk0 + i < a.n_pages) page = a.page_table[static_cast<int64_t>(trow) * a.pt_row_stride + blk0 + i];
-      if (page < 0 || page >= a.n_slots / a.pd.page_size) page = 0;  // not a page of the pool
+      if (page < 0 || page >= a.pool_pages) page = 0;  // not a page of the pool
       s_pages[i] = static_cast<int>(page);
     }
   }
@@ -439,11 +439,13 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   if constexpr (kMerges) {
     __shared__ int s_last;
     __shared__ __attribute__((aligned(16))) float s_part[4 * 64 * 4];
-    if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, n_pieces, G, s_part);
+    if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, part_mul, part_add - split, n_pieces, G, s_part);
   }
   };  // piece
 
-  if constexpr (!kFlat) {
+  if constexpr (kPieces) {
+    walk_pieces<min_part(ROWB)>(a, piece);
+  } else if constexpr (!kFlat) {
     walk_split<kMerges>(a, piece);
   } else {
     __shared__ int s_start[kFlatMaxB + 1];
@@ -465,7 +467,7 @@ __global__ __launch_bounds__(64) void paged_decode_plan_kernel(const DecodeArgs 
   const int64_t lo = static_cast<int64_t>(c) * len;
   const int64_t hi = lo + len < total ? lo + len : total;
   const int lane = threadIdx.x;
-  const int64_t pool_pages = a.n_slots / a.pd.page_size;
+  const int64_t pool_pages = a.pool_pages;
   int n = 0, page_off = 0;
   bool ok = true;
   if (lo < total) {
@@ -823,6 +825,34 @@ int even_cut_chunks(int Hc, int B, int n_splits, int max_context, int page_size,
   return static_cast<int64_t>(Hc) * B * n_splits > resident || even_cut_pays(Hc, B, max_context, page_size) ? chunks : 0;
 }
 
+// Splits of all sequences together, about, of a launch with arrival counters that goes piece by piece (walk_pieces): two workgroups to a
+// CU.  0 where it goes another way.  us a layer split by split or, with its plan, cut evenly / piece by piece:
+//                                              16 q / 8 kv, D 128   16 K and shared V heads   D 64, f16    4 x 8 q / 8 kv, D 64   8 heads, D 64, f32
+//   limit 8192, 4 of 100 to 700                     11.5 / 8.8            12.8 / 9.3          10.0 / 8.7        8.6 / 7.9             9.3 / 7.3
+//   limit 8192, 5 of 3000 to 8000                   28.4 / 23.9           36.4 / 31.4         18.3 / 16.0      18.9 / 15.6           25.2 / 21.9
+//   limit 4096, 8 of 300 to 1500                    15.9 / 12.4           18.0 / 13.9         14.5 / 10.9      14.2 / 10.8           13.2 / 10.8
+//   limit 8192, 16 of 350 to 4620                   33.4 / 30.3           44.1 / 41.1         22.4 / 19.5      22.1 / 18.3           30.4 / 28.4
+//   limit 1024, 48 of 64 to 500                     20.6 / 16.2           25.4 / 20.4         18.5 / 13.0      17.7 / 14.4           17.1 / 14.5
+// The price is paid where the lengths are close to the limit and fill the grid split by split anyway: limit 8192, 4 of 8000 26.6 / 27.4,
+// 36.3 / 36.5, 17.3 / 18.1, 16.5 / 17.3 and 24.7 / 25.6.  The lines: with fewer workgroup heads x sequences the merge is on fewer
+// workgroups than there are rows to hide it behind (8 heads, one of 711 tokens 8.0 / 8.0, two of 300 to 6000 11.6 / 12.1); a grid of up to four splits that the
+// CUs hold at once has few idle workgroups (limit 1024, 16 of 900 to 1000 16.9 / 18.1, of 100 to 900 13.2 / 13.4); and with more
+// tokens or sequences the remainders, up to B pieces, run behind the others (limit 8192, 24 of 4000 to 8000 96.7 / 99.8, 60 of these 228 / 261; limit 4096, 24 of
+// 64 to 4000 41.2 / 37.9, 32 of 300 to 4000 51.1 / 51.3; limit 2048, 32 of 300 to 2000 33.7 / 31.4; limit 1024, 60 of 100 to 1000 31.8 / 31.8
+// and in a step of 28 layers 908 / 920 us).  The step's plan does not know which way its launches go: one that goes piece by piece reads none.
+int merged_pieces(int Hc, int B, int n_splits, int max_context, int page_size) {
+  const int64_t groups = static_cast<int64_t>(Hc) * B, tokens = static_cast<int64_t>(B) * (max_context + 64), two = 2 * fp::compute_units();
+  if (B < 3 || B > 48 || groups < 32 || n_splits < 2 || (n_splits <= 4 && groups * n_splits <= two) || tokens >= 1 << 22 ||
+      groups * max_context > (B <= 24 ? 1 << 20 : 1 << 19))
+    return 0;
+  int64_t pieces = two / Hc;
+  if (pieces > kMostPieces * B) pieces = kMostPieces * B;
+  if (pieces > static_cast<int64_t>(B) * (n_splits - 1)) pieces = static_cast<int64_t>(B) * (n_splits - 1);  // a row per (piece + sequence)
+  if (pieces < 4) return 0;
+  const int64_t longest = tokens / pieces * 3 / 2 + 512;  // walk_pieces: (x + 64) * 17 / 16 + 64, four times
+  return longest / page_size + 2 <= kMaxSplitPages ? static_cast<int>(pieces) : 0;
+}
+
 // Workgroups of the even-cut kernel the current device holds at once (asked once per kernel and device).
 template <typename E, int D, int G, bool kAligned, bool kPerHeadK>
 int resident_workgroups() {
@@ -857,19 +887,19 @@ void launch_decode(const DecodeArgs& a0, int B, int phases, hipStream_t st) {
   const int chunk_rows = decode_loads_in_flight(G, kPerHeadK) * 64 / (D * static_cast<int>(sizeof(typename E::type)) / 16);
   const bool aligned = a.pd.shift >= 0 && a.pd.page_size % chunk_rows == 0;
   // the split-K pass, by the kernel that serves this instance
-  auto split_k_pass = [&](auto direct, auto flat, dim3 g, const DecodeArgs& args) {
-    constexpr bool kDirect = decltype(direct)::value, kFlat = decltype(flat)::value;
+  auto split_k_pass = [&](auto direct, auto flat, auto pieces, dim3 g, const DecodeArgs& args) {
+    constexpr bool kDirect = decltype(direct)::value, kFlat = decltype(flat)::value, kPieces = decltype(pieces)::value;
     if constexpr (on_matrix_cores<E, G, kPerHeadK>())
-      launch_mfma(args, std::is_same<E, BF16>::value ? FP_DTYPE_BF16 : FP_DTYPE_F16, D, Cut{kDirect, kFlat}, g, st);
+      launch_mfma(args, std::is_same<E, BF16>::value ? FP_DTYPE_BF16 : FP_DTYPE_F16, D, Cut{kDirect, kFlat, kPieces}, g, st);
     else if (aligned)
-      hipLaunchKernelGGL((paged_decode_kernel<E, D, G, kDirect, true, kPerHeadK, kFlat>), g, dim3(kThreads), 0, st, args);
+      hipLaunchKernelGGL((paged_decode_kernel<E, D, G, kDirect, true, kPerHeadK, kFlat, kPieces>), g, dim3(kThreads), 0, st, args);
     else
-      hipLaunchKernelGGL((paged_decode_kernel<E, D, G, kDirect, false, kPerHeadK, kFlat>), g, dim3(kThreads), 0, st, args);
+      hipLaunchKernelGGL((paged_decode_kernel<E, D, G, kDirect, false, kPerHeadK, kFlat, kPieces>), g, dim3(kThreads), 0, st, args);
   };
   if (a.n_splits == 1) {
     // one split covers every context: the partial pass writes out and lse itself
     if (!(phases & kPhasePartial)) return;  // also the plan phase: such a launch has no even cut
-    split_k_pass(std::true_type{}, std::false_type{}, grid, a);
+    split_k_pass(std::true_type{}, std::false_type{}, std::false_type{}, grid, a);
   } else {
     // Cut evenly: the work of a workgroup then follows from the lengths of the sequences and not from max_context,
     // which an engine sets to the longest sequence it may ever hold (16 padded rows of 350 to 4620 tokens under a
@@ -892,7 +922,10 @@ void launch_decode(const DecodeArgs& a0, int B, int phases, hipStream_t st) {
       resident = 3 * fp::compute_units();
     else
       resident = aligned ? resident_workgroups<E, D, G, true, kPerHeadK>() : resident_workgroups<E, D, G, false, kPerHeadK>();
-    const int n_chunks = even_cut_chunks(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size, resident);
+    const int pieces = a.arrivals ? merged_pieces(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size) : 0;
+    DecodeArgs ap = a;
+    ap.n_chunks = pieces;
+    const int n_chunks = pieces > 0 ? 0 : even_cut_chunks(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size, resident);
     DecodeArgs af = a;
     af.B = B;
     af.n_chunks = n_chunks;
@@ -903,9 +936,11 @@ void launch_decode(const DecodeArgs& a0, int B, int phases, hipStream_t st) {
     }
     if (phases & kPhasePartial) {
       if (n_chunks > 0)
-        split_k_pass(std::false_type{}, std::true_type{}, dim3(a.Hc, n_chunks), af);
-      else
-        split_k_pass(std::false_type{}, std::false_type{}, grid, a);
+        split_k_pass(std::false_type{}, std::true_type{}, std::false_type{}, dim3(a.Hc, n_chunks), af);
+      else if (pieces == 0)
+        split_k_pass(std::false_type{}, std::false_type{}, std::false_type{}, grid, a);
+      else if constexpr (merges_itself(G, D))
+        split_k_pass(std::false_type{}, std::false_type{}, std::true_type{}, dim3(a.Hc, pieces + B), ap);
     }
     if ((phases & kPhaseMerge) && (n_chunks > 0 || !a.arrivals)) {
       if (n_chunks > 0)
@@ -959,6 +994,16 @@ extern "C" int32_t fp_paged_decode_default_split(int32_t B, int32_t Hc, int32_t 
   if (B <= 0 || Hc <= 0 || max_context < 0 || page_size <= 0)
     return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_default_split: bad dimension");
   return default_split_tokens(B, Hc, max_context, page_size);
+}
+
+extern "C" int32_t fp_paged_decode_step_pieces(int32_t B, int32_t Hq, int32_t Hc, int32_t kv_rep, int32_t D, int32_t max_context,
+                                               int32_t page_size, int32_t split_tokens) {
+  if (B <= 0 || Hc <= 0 || Hq < Hc || kv_rep <= 0 || D <= 0 || max_context < 0 || page_size <= 0 || split_tokens < 0)
+    return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_step_pieces: bad dimension");
+  const int wg_heads = kv_rep > 1 ? Hq / kv_rep : Hc;
+  const int split = split_tokens ? split_tokens : default_split_tokens(B, wg_heads, max_context, page_size);
+  if (!merges_itself(Hq / wg_heads, D)) return 0;
+  return merged_pieces(wg_heads, B, n_splits_for(max_context, split), max_context, page_size);
 }
 
 extern "C" int64_t fp_paged_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t D, int32_t max_context,
@@ -1056,7 +1101,8 @@ int decode_entry(int phases, const NewRows* fresh, const void* q, int64_t q_stri
                static_cast<const char*>(pool_k), static_cast<const char*>(pool_v),
                page_table, pt_row_stride, batch_idx, input_pos, pos_index_type == FP_INDEX_I64,
                static_cast<char*>(out), out_stride_b * eb, out_stride_h * eb, lse, sinks,
-               nullptr, nullptr, Hq, wg_heads, fp::PageDiv(page_size), n_pages, max_batch, n_slots,
+               nullptr, nullptr, Hq, wg_heads, fp::PageDiv(page_size), n_pages, max_batch,
+               static_cast<int>(n_slots / page_size > INT32_MAX ? INT32_MAX : n_slots / page_size), n_slots,
                max_context, split_tokens, ns, scale * kLog2e,  // scores are kept in log2 units
                nullptr, nullptr, 0, 0, 0, 0, B, 0, static_cast<int*>(plan), arrivals};
   if (fresh) {

@@ -5,10 +5,12 @@
 
 namespace fp_decode {
 
-// How a launch is cut: grid (heads, B, splits), with one split storing its results itself, or grid (heads, chunks).
+// How a launch is cut: grid (heads, B, splits), with one split storing its results itself, grid (heads, chunks) or grid
+// (heads, pieces + B).
 struct Cut {
   bool direct;
   bool flat;
+  bool pieces;
 };
 
 // The split-K pass of a bf16 or f16 launch with up to 8 query heads per cache head.

@@ -103,7 +103,7 @@ __device__ __forceinline__ void wait_staged() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLater) : "memory");
 }
 
-template <typename E, int D, bool kFlat>
+template <typename E, int D, bool kFlat, bool kPieces = false>
 __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const DecodeArgs a, const Cut cut) {
   constexpr int ROWB = D * 2;             // bytes of a row
   constexpr int CPR = ROWB / 16;          // 16-byte chunks per row
@@ -149,14 +149,14 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
   const char* const vplane = a.pool_v + static_cast<int64_t>(hc) * a.n_slots * ROWB;
 
   // Tokens [t0, t0 + part) of sequence b; a partial result goes to row hq * part_mul + part_add of the workspace.
-  auto piece = [&](const int b, const int t0, const int part, const bool first, const int64_t part_mul,
+  auto piece = [&](const int b, const int t0, const int part, const int split, const int64_t part_mul,
                    const int64_t part_add, const int n_pieces, const int raw, const int trow, const int* pre_pages) {
     int L = trow < 0 ? 0 : raw;
     const int* pages_lds = pre_pages ? pre_pages : s_pages;
     const bool beyond = L > a.max_context;  // as in paged_decode_kernel: read up to max_context, no fresh row
     if (beyond) L = a.max_context;
     if (t0 >= L) {
-      if ((cut.direct || (kMerges && a.arrivals)) && first) {  // no visible key at all: out = 0, lse = -inf
+      if ((cut.direct || (kMerges && a.arrivals)) && split == 0) {  // no visible key at all: out = 0, lse = -inf
         for (int i = tid; i < G * D; i += kThreads) {
           const int g = i / D, d = i - g * D;
           E::store(a.out + b * a.os_b + (hc * G + g) * a.os_h + d * 2, 0.f);
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
         for (int i = tid; i <= static_cast<int>(blk_last - blk0); i += kThreads) {
           int64_t page = 0;
           if (blk0 + i < a.n_pages) page = a.page_table[static_cast<int64_t>(trow) * a.pt_row_stride + blk0 + i];
-          if (page < 0 || page >= a.n_slots / a.pd.page_size) page = 0;  // not a page of the pool
+          if (page < 0 || page >= a.pool_pages) page = 0;  // not a page of the pool
           s_pages[i] = static_cast<int>(page);
         }
         __syncthreads();
@@ -408,13 +408,15 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
     }
     if constexpr (kMerges) {  // the rings are free behind the barrier inside
       __shared__ int s_last;
-      if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, n_pieces, G, reinterpret_cast<float*>(s_ring));
+      if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, part_mul, part_add - split, n_pieces, G, reinterpret_cast<float*>(s_ring));
     }
   };  // piece
 
   if constexpr (kFlat) {
     __shared__ int s_start[kFlatMaxB + 1];
     walk_even_cut<kThreads>(a, s_start, s_pages, piece);
+  } else if constexpr (kPieces) {
+    walk_pieces<min_part(ROWB)>(a, piece);
   } else {
     walk_split<kMerges>(a, piece);
   }
@@ -424,6 +426,8 @@ template <typename E, int D>
 void launch(const DecodeArgs& a, const Cut& cut, dim3 grid, hipStream_t st) {
   if (cut.flat)
     hipLaunchKernelGGL((paged_decode_mfma_kernel<E, D, true>), grid, dim3(kThreads), 0, st, a, cut);
+  else if (merges_itself(4, D) && cut.pieces)
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<E, D, false, merges_itself(4, D)>), grid, dim3(kThreads), 0, st, a, cut);
   else
     hipLaunchKernelGGL((paged_decode_mfma_kernel<E, D, false>), grid, dim3(kThreads), 0, st, a, cut);
 }

@@ -42,6 +42,7 @@ SIGNATURES = {
         c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
         c_int32, c_int32, c_int32, c_int32, c_int32, c_void_p]),
     "fp_paged_decode_default_split": (c_int32, [c_int32, c_int32, c_int32, c_int32]),
+    "fp_paged_decode_step_pieces": (c_int32, [c_int32] * 8),
     "fp_paged_decode_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32]),
     "fp_paged_decode_workspace_bytes_up_to": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "fp_paged_decode": (c_int, [

@@ -169,6 +169,13 @@ def decode_split_tokens(B: int, Hc: int, max_context: int, page_size: int) -> in
     return int(N.lib().fp_paged_decode_default_split(B, Hc, max_context, page_size))
 
 
+def decode_step_pieces(B: int, Hq: int, Hc: int, kv_rep: int, D: int, max_context: int, page_size: int, split_tokens: int) -> int:
+    """About how many pieces `paged_decode(arrivals=...)` cuts a launch of this shape into; 0: as without counters."""
+    n = int(N.lib().fp_paged_decode_step_pieces(B, Hq, Hc, kv_rep, D, max_context, page_size, split_tokens))
+    N.check(n, "fp_paged_decode_step_pieces")
+    return n
+
+
 def decode_workspace_bytes(B: int, Hq: int, D: int, max_context: int, split_tokens: int) -> int:
     n = int(N.lib().fp_paged_decode_workspace_bytes(B, Hq, D, max_context, split_tokens))
     N.check(n, "fp_paged_decode_workspace_bytes")

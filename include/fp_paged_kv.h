@@ -141,6 +141,13 @@ int fp_convert_block_ids(const int32_t* kv_indices, int32_t* out,
 int32_t fp_paged_decode_default_split(int32_t B, int32_t Hc, int32_t max_context, int32_t page_size);
 
 /*
+ * About how many pieces of one length fp_paged_decode_step cuts all sequences of a launch into, or 0 where the launch goes split by
+ * split or is cut evenly as without counters.  A launch that goes piece by piece reads no plan.  Arguments as fp_paged_decode.
+ */
+int32_t fp_paged_decode_step_pieces(int32_t B, int32_t Hq, int32_t Hc, int32_t kv_rep, int32_t D, int32_t max_context,
+                                    int32_t page_size, int32_t split_tokens);
+
+/*
  * Bytes of workspace fp_paged_decode needs for the given launch shape
  * (split-K partial results: B * Hq * ceil(max_context / split_tokens) * (D + 2) floats;
  * nothing when one split covers max_context).  max_context bounds input_pos + 1,
@@ -312,12 +319,13 @@ int fp_paged_decode_append(const void* k_new, const void* v_new,
 /*
  * fp_paged_decode_append, or fp_paged_decode where k_new and v_new are NULL, for callers that keep counters: a launch that goes
  * split by split is then ONE launch, in which the workgroup that is the last to leave its partial result of a (sequence, cache
- * head) merges them.  Launches that are cut evenly, or with more than 256 elements per sequence and cache head (Hq / Hc * D, or
+ * head) merges them.  With counters a launch may also be cut into pieces of one length (fp_paged_decode_step_pieces), whatever split_tokens
+ * says; the workspace is that of its splits.  Launches that are cut evenly, or with more than 256 elements per sequence and cache head (Hq / Hc * D, or
  * kv_rep * D), keep their merge pass, which is faster there; they do not touch the counters.
  *   arrivals   [B, Hc / kv_rep] int32 device memory of the caller, arrivals_bytes long: all 0 before the first launch that
  *              uses it and never written by anybody else.  Every launch leaves it all 0.  Like the workspace it belongs
  *              to one launch at a time: launches that overlap need a workspace and counters of their own.
- * Results equal those of the two passes up to the order of the sums over the splits.  All other arguments as fp_paged_decode_append.
+ * Results equal those of the two passes up to the order of the sums over the keys.  All other arguments as fp_paged_decode_append.
  */
 int fp_paged_decode_step(int32_t* arrivals, int64_t arrivals_bytes,
                          const void* k_new, const void* v_new,

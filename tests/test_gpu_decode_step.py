@@ -114,3 +114,55 @@ def test_replays_of_a_captured_step():
             close(got, ref, dtype, 64)
         assert not arrivals.any()
         pos -= 13
+
+
+# piece by piece: the fewest sequences and few of them, more than 16 pieces' worth of one, some without keys, all shorter than a
+# piece, the most sequences; page sizes that are no power of two; the first shapes on the other side of each line
+PIECES = {"three": (3, 16, 2048, [1, 2047, 300]), "uneven": (9, 8, 8192, [8190, 0, 63, 64, 127, 4000, 65, 1, 700]),
+          "empty": (8, 8, 1536, [-1, 1535, -1, 200, 0, 0, 129, 999]), "short": (40, 8, 1024, None), "most": (48, 4, 1100, None)}
+
+
+@pytest.mark.parametrize("case", PIECES)
+@pytest.mark.parametrize("dtype,D,P,G,rep", [
+    (torch.bfloat16, 128, 64, 2, 1), (torch.bfloat16, 64, 24, 4, 1), (torch.float32, 64, 16, 1, 1), (torch.float32, 128, 32, 2, 1),
+    (torch.bfloat16, 128, 48, 2, 2), (torch.float16, 64, 128, 1, 1), (torch.bfloat16, 64, 16, 4, 4)], ids=str)
+def test_piece_by_piece_gives_what_the_two_passes_give(case, dtype, D, P, G, rep):
+    B, Hc, ctx, lens = PIECES[case]
+    if lens is None:
+        lens = [(37 * i * i + 11 * i) % (250 if case == "short" else ctx - 2) for i in range(B)]
+    split = ops.decode_split_tokens(B, Hc, ctx, P)
+    assert ops.decode_step_pieces(B, Hc * G, Hc * rep, rep, D, ctx, P, split) > 0
+    st = flat_state(31 + D + G, B, Hc, D, P, ctx, dtype, rep, [max(n, 0) for n in lens])
+    q, k_new, v_new = inputs(st, B, Hc, G, D, dtype, rep)
+    bidx = torch.tensor(st.slots, dtype=torch.int64, device=DEV)
+    if B > 20:
+        lens[5], lens[13], bidx[9], bidx[11] = -1, ctx + 7, B + 40, -3  # no key, beyond the launch's limit, foreign slots
+    before = st.cache.kv_cache.clone()
+    arrivals = torch.zeros(B * Hc, dtype=torch.int32, device=DEV)
+    kw = dict(max_context=ctx, split_tokens=split, kv_rep=rep, bidx=bidx)
+    # the pieces are others than the splits, so the sums over the keys run in another order: n = keys in `close`
+    for pos_type in (torch.int32, torch.int64):
+        pos = torch.tensor(lens, dtype=pos_type, device=DEV)
+        if pos_type is torch.int64 and B > 20:
+            pos[13], pos[5] = 2**40, -(2**40)
+        st.cache.kv_cache.copy_(before)
+        ref = decode(st, q, pos, k_new=k_new, v_new=v_new, **kw)
+        pool = st.cache.kv_cache.clone()
+        st.cache.kv_cache.copy_(before)
+        got = decode(st, q, pos, k_new=k_new, v_new=v_new, arrivals=arrivals, **kw)
+        close(got, ref, dtype, ctx)
+        assert torch.equal(st.cache.kv_cache, pool) and not arrivals.any()
+
+
+def test_which_launches_go_piece_by_piece():
+    def pieces(B, Hc, limit, G=2, D=128, P=64, rep=1):
+        return ops.decode_step_pieces(B, Hc * G, Hc * rep, rep, D, limit, P, 0)
+
+    assert [pieces(B, 8, 8192) > 0 for B in (1, 3, 4, 16, 17, 63, 64)] == [False, False, True, True, False, False, False]
+    assert pieces(48, 8, 1024) > 0 and pieces(49, 8, 1024) == 0
+    assert pieces(2, 16, 8192) == 0 and pieces(3, 16, 8192) > 0 and pieces(7, 4, 8192) == 0 and pieces(8, 4, 8192) > 0
+    assert pieces(16, 8, 1024) == 0 and pieces(17, 8, 1024) > 0  # the splits fill the CUs as it is
+    assert pieces(8, 8, 8192, G=4) == 0 and pieces(8, 8, 8192, G=4, D=64) > 0  # more than 256 elements a merge
+    assert pieces(8, 8, 128) == 0 and pieces(8, 8, 0) == 0  # one split
+    with pytest.raises(RuntimeError):
+        pieces(0, 8, 8192)
