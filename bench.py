@@ -685,6 +685,7 @@ def prefill_rate(steps: int = 10, name: str = "cfg3", bounded: bool = True, both
         res["paged_prefill_ms_no_tile_order"] = ms_no_order
     if case.q.dtype == torch.float32:
         res["frac_of_f32_mfma_peak"] = tf / MFMA_F32_PEAK_TFLOPS
+        res["frac_of_bf16_mfma_peak_six_products"] = 6 * tf / MFMA_BF16_PEAK_TFLOPS  # what the kernel runs: six bf16 products each
     else:
         res["frac_of_bf16_mfma_peak"] = tf / MFMA_BF16_PEAK_TFLOPS
     if ms_unbounded is not None:
