@@ -46,6 +46,7 @@ struct DecodeArgs {
   // optional [B, Hc], all 0 between launches: how many splits of a (sequence, workgroup head) have left their
   // partial result.  The workgroup that is the last merges them, and there is no merge pass (last_to_arrive, merge_splits)
   int* arrivals;
+  int arrivals_step;  // ints from counter to counter
 };
 
 // The plan of a decode step: what every workgroup of the even cut needs before it can ask for its first K row,
@@ -243,7 +244,7 @@ __device__ __forceinline__ bool last_to_arrive(int b, int n, int* flag) {
   asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // this wavefront's stores have arrived
   __syncthreads();
   if (threadIdx.x == 0) {
-    int* const counter = a.arrivals + static_cast<int64_t>(b) * a.Hc + blockIdx.x;
+    int* const counter = a.arrivals + (static_cast<int64_t>(b) * a.Hc + blockIdx.x) * a.arrivals_step;
     const bool last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
     if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *flag = last;

@@ -323,7 +323,8 @@ int fp_paged_decode_append(const void* k_new, const void* v_new,
  * says; the workspace is that of its splits.  Launches that are cut evenly, or with more than 256 elements per sequence and cache head (Hq / Hc * D, or
  * kv_rep * D), keep their merge pass, which is faster there; they do not touch the counters.
  *   arrivals   [B, Hc / kv_rep] int32 device memory of the caller, arrivals_bytes long: all 0 before the first launch that
- *              uses it and never written by anybody else.  Every launch leaves it all 0.  Like the workspace it belongs
+ *              uses it and never written by anybody else; 32 times that many bytes give every counter a line of its own, which few
+ *              sequences of many tokens want.  Every launch leaves it all 0.  Like the workspace it belongs
  *              to one launch at a time: launches that overlap need a workspace and counters of their own.
  * Results equal those of the two passes up to the order of the sums over the keys.  All other arguments as fp_paged_decode_append.
  */

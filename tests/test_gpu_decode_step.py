@@ -138,7 +138,7 @@ def test_piece_by_piece_gives_what_the_two_passes_give(case, dtype, D, P, G, rep
     if B > 20:
         lens[5], lens[13], bidx[9], bidx[11] = -1, ctx + 7, B + 40, -3  # no key, beyond the launch's limit, foreign slots
     before = st.cache.kv_cache.clone()
-    arrivals = torch.zeros(B * Hc, dtype=torch.int32, device=DEV)
+    arrivals = torch.zeros(B * Hc * 5 + 3, dtype=torch.int32, device=DEV)  # counters five words apart
     kw = dict(max_context=ctx, split_tokens=split, kv_rep=rep, bidx=bidx)
     # the pieces are others than the splits, so the sums over the keys run in another order: n = keys in `close`
     for pos_type in (torch.int32, torch.int64):
