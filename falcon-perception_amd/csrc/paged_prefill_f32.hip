@@ -19,8 +19,8 @@
 //   S^T = K Q^T : a lane holds the scores of ONE query (softmax reductions stay in registers plus
 //                 one exchange between the lane halves); Q is scaled when it is loaded.
 //   O^T = V^T P^T : P^T is the B operand as it leaves the softmax; V^T comes out of LDS through ds_read_b64_tr_b16.
-// A run with an infinity, a NaN, or a number too large or too small for the split (from the largest bf16 on, below 2^-100) in a tile or in
-// a row of Q is done again on the fp32 matrix instruction.
+// A run with an infinity, a NaN, or a number too large or too small for the split (from the largest bf16 on, in K and Q from 2^60 on; below
+// 2^-100) in a tile or in a row of Q is done again on the fp32 matrix instruction.
 #include "fp_common.h"
 #include "prefill_common.h"
 
@@ -121,9 +121,10 @@ __device__ __forceinline__ Split split(const float (&x)[8]) {
   return r;
 }
 // Whether one of the numbers is out of the split's range, by its first part: an infinity or a NaN, or below 2^-100 and not 0 (what
-// rounds to 0 is below 2^-134).
-constexpr uint32_t kTooLarge = 0x7f80u, kTooSmall = 0x0d80u;
-__device__ __forceinline__ bool out_of_range(const Split& s) {
+// rounds to 0 is below 2^-134).  K and Q also from 2^60 on (kScoreTooLarge): below, no sum of up to 128 products leaves fp32.  Beyond, the
+// large and the small products of a score may overflow to opposite infinities, a NaN where plain fp32 has -inf and no weight.
+constexpr uint32_t kTooLarge = 0x7f80u, kScoreTooLarge = (127u + 60u) << 7, kTooSmall = 0x0d80u;
+__device__ __forceinline__ bool out_of_range(const Split& s, uint32_t too_large) {
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
   const u16x2 one = {1, 1};
   u16x2 most = {0, 0}, least = {0xffff, 0xffff};
@@ -134,7 +135,7 @@ __device__ __forceinline__ bool out_of_range(const Split& s) {
     most = __builtin_elementwise_max(most, b);
     least = __builtin_elementwise_min(least, static_cast<u16x2>(b - one));  // 0 comes out above everything
   }
-  return max(most.x, most.y) >= kTooLarge || min(least.x, least.y) < kTooSmall - 1u;
+  return max(most.x, most.y) >= too_large || min(least.x, least.y) < kTooSmall - 1u;
 }
 
 // LDS layout of a plane of a tile: unpadded rows of D bf16, whose 16-byte chunks are permuted against bank conflicts as in the
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_prefill_f32_kernel(const Ar
                         (is_k ? (at.chunk ^ SW::kswz(at.row)) * 16
                               : (((at.chunk >> 1) + SW::vrot(at.row)) % R32) * 32 + (at.chunk & 1) * 16);
       const Split s = split(x);
-      if (out_of_range(s)) s_bad[word] = 1;
+      if (out_of_range(s, is_k ? kScoreTooLarge : kTooLarge)) s_bad[word] = 1;
 #pragma unroll
       for (int n = 0; n < 3; ++n) *reinterpret_cast<v4u*>(dst + n * PLANE) = s.p[n];
     };
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_prefill_f32_kernel(const Ar
         load_q(16 * ds + 8 * half, x);
         load_q(16 * ds + 8 * half + 4, x + 4);
         qreg[ds] = split(x);
-        if (out_of_range(qreg[ds])) s_bad[1] = 1;
+        if (out_of_range(qreg[ds], kScoreTooLarge)) s_bad[1] = 1;
       }
       __builtin_amdgcn_sched_barrier(0);  // not before: Q as it came and split fills the registers
       m_run = -INFINITY;

@@ -108,3 +108,24 @@ def test_query_rows_it_does_not_hold(D, G):
     assert out[:, 20].isnan().all() and not lse[:, 20].isfinite().any()
     q[:, 20, 1] = 0.0
     check((out, lse), q, k, v, skip=[(0, None, 20)])
+
+
+@pytest.mark.parametrize("shares", [1, 3])
+@pytest.mark.parametrize("D,G,P", [(128, 1, 64), (128, 2, 24), (64, 4, 16)])
+def test_a_score_that_overflows_takes_its_own_key_only(D, G, P, shares):
+    """Finite numbers whose product is beyond fp32: the score is -inf and its key has no weight, whatever the signs of the products
+    of their smaller parts are.  Each factor comes as itself and with another lowest part, so that these have either sign."""
+    st, q, k, v = build(D, G, P)
+    q[..., 0] = 0.0
+    k[..., 0] = 0.0
+    big = torch.tensor([3.01e22, 3.0e22, 2.97e22, 1.0e21, 2.0**61, 9.99e30])
+    first, third = slice(0, LENS[0]), slice(sum(LENS[:2]), sum(LENS[:3]))
+    for rows in (first, third):
+        n = rows.stop - rows.start
+        k[:, rows.start + 5 : rows.start + 5 + len(big), 0] = big
+        q[:, rows, 0] = -(big * 1.001)[torch.arange(n) % len(big)].clamp(min=1e21)
+    got = run(st, q, k, v, shares)
+    qc, kc = q.clone(), k.clone()  # the same with products that fp32 holds: at -180 and below a key has no weight either
+    qc[..., 0] = (q[..., 0] != 0) * -32.0
+    kc[..., 0] = (k[..., 0] != 0) * 64.0 * math.sqrt(D / 128)
+    check(got, qc, kc, v)
