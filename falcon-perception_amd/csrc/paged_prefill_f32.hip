@@ -187,8 +187,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_prefill_f32_kernel(const Ar
   const int tile0 = tile * BM;
 
   // Everything the set-up needs from global memory is requested at once: the sequence of each row
-  // of the tile, then this wavefront's row limit and Q row.  Rows outside a run keep their Q values:
-  // what such a row computes is never stored.
+  // of the tile, then this wavefront's row limit and Q row.
   const int bi_row = tile0 + tid;
   const int64_t bx_raw = (tid < BM && bi_row < a.Lq) ? a.batch_idx[bi_row] : 0;
   if (tid < BM) {
@@ -351,11 +350,12 @@ __global__ __launch_bounds__(kThreads, 2) void paged_prefill_f32_kernel(const Ar
       }
       return r;
     };
-    // 4 numbers of this lane's query row from head_dim element d on, scaled
+    // 4 numbers of this lane's query row from head_dim element d on, scaled.  Rows of other sequences count as 0: what they hold neither
+    // sends this run through the fp32 instruction nor moves its reference points.
     auto load_q = [&](int d, float* x) {
       f32x4 w = {0, 0, 0, 0};
-      const int r = tile0 + rblock * 32 + (thread() & 31);
-      if (r < a.Lq) w = *reinterpret_cast<const f32x4*>(a.q + r * a.qs_row + hq * a.qs_h + d * 4);
+      const int tr = rblock * 32 + (thread() & 31), r = tile0 + tr;
+      if (tr >= run0 && tr < run1 && r < a.Lq) w = *reinterpret_cast<const f32x4*>(a.q + r * a.qs_row + hq * a.qs_h + d * 4);
 #pragma unroll
       for (int t = 0; t < 4; ++t) x[t] = w[t] * a.qscale;
     };

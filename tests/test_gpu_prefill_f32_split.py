@@ -129,3 +129,19 @@ def test_a_score_that_overflows_takes_its_own_key_only(D, G, P, shares):
     qc[..., 0] = (q[..., 0] != 0) * -32.0
     kc[..., 0] = (k[..., 0] != 0) * 64.0 * math.sqrt(D / 128)
     check(got, qc, kc, v)
+
+
+@pytest.mark.parametrize("D,G,P", [(128, 1, 64), (128, 4, 24), (64, 2, 16)])
+def test_queries_of_one_sequence_leave_the_others_alone(D, G, P):
+    """The rows of several sequences share a workgroup; what the queries of one hold changes no bit of the others."""
+    rows = slice(sum(LENS[:2]), sum(LENS[:3]))
+    others = torch.ones(sum(LENS), dtype=torch.bool)
+    others[rows] = False
+    results = []
+    for value in (1.0, math.nan, math.inf, 2.0**-110, 1e30):
+        st, q, k, v = build(D, G, P)
+        q[:, rows] *= value
+        out, lse = run(st, q, k, v, 1)
+        results.append((out[:, others], lse[:, others]))
+    for out, lse in results[1:]:
+        assert torch.equal(out, results[0][0]) and torch.equal(lse, results[0][1])
