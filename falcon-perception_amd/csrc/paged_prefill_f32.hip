@@ -290,7 +290,8 @@ __global__ __launch_bounds__(kThreads, 2) void paged_prefill_f32_kernel(const Ar
     // tiles (page size a power of two, at least the tile), a tile that lies before the run's last key in a
     // mapped page is contiguous in the pool: its first slot is looked up once per run into s_tslot.  Any other tile (the
     // last one of a run, small or odd page sizes, unmapped pages, runs longer than the table) looks its rows up one by
-    // one: a key that does not exist (past the run's last key, or an unmapped page) is 0, and masked.
+    // one: a row past the run's last key is 0, and masked; a key below it on a page that is not mapped reads slot 0 of the
+    // pool, here and on the fp32 matrix instruction.
     const int64_t* pt_row = a.page_table + static_cast<int64_t>(sq) * a.pt_row_stride;
     const int64_t pool_pages = a.pool_pages;
     // first pool slots of tiles lo .. hi - 1 of n keys each -> s_tslot
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_prefill_f32_kernel(const Ar
         off = kpos - blkid * page_size;
       }
     };
-    // Byte offset of this lane's row of tile kt in a plane of the pool, or -1: the key does not exist.
+    // Byte offset of this lane's row of tile kt in a plane of the pool, or -1: past the run's last key.
     auto row_offset = [&](int kt) -> int64_t {
       const int ts = tile_slot(kt, kt_lo, n_kv_tiles);
       const Place at = staged();
@@ -334,10 +335,10 @@ __global__ __launch_bounds__(kThreads, 2) void paged_prefill_f32_kernel(const Ar
       const int kpos = kt * kTileN + at.row;
       int blkid, off;
       key_block(kpos, blkid, off);
-      if (kpos >= kv_max || blkid >= a.n_pages) return -1;
-      const int64_t pg = pt_row[blkid];
-      if (pg < 0 || pg >= pool_pages) return -1;
-      return (pg * a.pd.page_size + off) * ROWB + at.chunk * 32;
+      if (kpos >= kv_max) return -1;
+      const int64_t pg = blkid < a.n_pages ? pt_row[blkid] : -1;
+      const int64_t slot = pg >= 0 && pg < pool_pages ? pg * a.pd.page_size + off : 0;
+      return slot * ROWB + at.chunk * 32;
     };
     struct Raw {
       f32x4 lo, hi;

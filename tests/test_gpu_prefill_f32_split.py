@@ -145,3 +145,29 @@ def test_queries_of_one_sequence_leave_the_others_alone(D, G, P):
         results.append((out[:, others], lse[:, others]))
     for out, lse in results[1:]:
         assert torch.equal(out, results[0][0]) and torch.equal(lse, results[0][1])
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["split", "instruction"])
+@pytest.mark.parametrize("D,P", [(128, 32), (128, 24), (64, 64), (64, 8)])
+def test_a_key_without_a_page_reads_slot_0(D, P, exact):
+    """A limit beyond the pages a sequence has, and beyond the table: every key there is the first row of the pool, on either matrix instruction."""
+    Hc, n, more = 2, 75, 30
+    mapped = -(-n // P) * P
+    st = PagedState(5, n_pages=16, page_size=P, max_batch=3, Hc=Hc, D=D, dtype=torch.float32, max_blocks_per_seq=mapped // P + 1)
+    st.add_sequence(n)
+    k, v = (torch.randn((Hc, mapped + more, D), generator=st.gen) for _ in range(2))
+    q = torch.randn((Hc, n, D), generator=st.gen)
+    if exact:
+        v[:, 3, 0] = 2.0**-105  # sends the run to the fp32 instruction
+    k[:, mapped:], v[:, mapped:] = k[:, mapped : mapped + 1], v[:, mapped : mapped + 1]
+    pk, pv = st.pool_planes()
+    slots = (st.cache.page_table[st.slots[0], : mapped // P, None] * P + torch.arange(P, device=DEV)).reshape(-1)
+    for pool, x in ((pk, k), (pv, v)):
+        pool[:, slots], pool[:, 0] = x[:, :mapped].to(DEV), x[:, mapped].to(DEV)
+    bidx = torch.full((n,), st.slots[0], dtype=torch.int64, device=DEV)
+    limit = torch.full((n,), mapped + more, dtype=torch.int32, device=DEV)
+    out, _ = ops.paged_prefill(q[None].to(DEV), pk, pv, st.cache.page_table, bidx, limit, P, workspace=False)
+    s = q.double() @ k.double().transpose(1, 2) / math.sqrt(D)
+    p = torch.softmax(s, -1)
+    weight = 12 / math.sqrt(D) * (q.abs() @ k.abs().transpose(1, 2)).amax(-1, keepdim=True) + 2 * k.shape[1] + 16
+    assert ((out[0].cpu().double() - p @ v.double()).abs() <= weight * 2.0**-24 * (p @ v.double().abs())).all()
