@@ -1000,6 +1000,9 @@ extern "C" int32_t fp_paged_decode_step_pieces(int32_t B, int32_t Hq, int32_t Hc
                                                int32_t page_size, int32_t split_tokens) {
   if (B <= 0 || Hc <= 0 || Hq < Hc || kv_rep <= 0 || D <= 0 || max_context < 0 || page_size <= 0 || split_tokens < 0)
     return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_step_pieces: bad dimension");
+  if (Hq % Hc || (kv_rep > 1 && (Hc != Hq || Hq % kv_rep)) || split_tokens % 64)  // as the launch itself asks
+    return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_step_pieces: Hq = %d, Hc = %d, kv_rep = %d, split_tokens = %d is no launch",
+                    Hq, Hc, kv_rep, split_tokens);
   const int wg_heads = kv_rep > 1 ? Hq / kv_rep : Hc;
   const int split = split_tokens ? split_tokens : default_split_tokens(B, wg_heads, max_context, page_size);
   if (!merges_itself(Hq / wg_heads, D)) return 0;

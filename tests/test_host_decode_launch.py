@@ -65,3 +65,10 @@ def test_large_batches_under_a_short_limit_need_no_scratch_array(native_lib, B, 
                                             128, 128, 8, B, 8192, 1024, 0, 1.0, 1, None)
     assert rc == -1 and b"null pointer" in native_lib.fp_last_error()
     assert ops.decode_workspace_bytes(B, Hq, 128, 1024, ops.decode_split_tokens(B, Hc, 1024, 128)) == 0
+
+
+@pytest.mark.parametrize("Hq,Hc,kv_rep,split", [(1, 1, 2, 128), (4, 4, 8, 128), (6, 6, 4, 128), (8, 4, 2, 128), (9, 4, 1, 128), (8, 4, 1, 100)])
+def test_pieces_of_a_launch_that_cannot_be(native_lib, Hq, Hc, kv_rep, split):
+    """More copies than heads would leave no workgroup heads to divide by."""
+    with pytest.raises(RuntimeError, match="is no launch"):
+        ops.decode_step_pieces(4, Hq, Hc, kv_rep, 64, 8192, 64, split)
