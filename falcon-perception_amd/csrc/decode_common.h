@@ -47,6 +47,7 @@ struct DecodeArgs {
   // partial result.  The workgroup that is the last merges them, and there is no merge pass (last_to_arrive, merge_splits)
   int* arrivals;
   int arrivals_step;  // ints from counter to counter
+  int* next_arrivals;  // optional, laid out alike: counters of a launch after this one, which this one sets to 0 (clear_next_counter)
 };
 
 // The plan of a decode step: what every workgroup of the even cut needs before it can ask for its first K row,
@@ -251,6 +252,15 @@ __device__ __forceinline__ bool last_to_arrive(int b, int n, int* flag) {
   }
   __syncthreads();
   return __builtin_amdgcn_readfirstlane(*flag) != 0;
+}
+
+// Counters are 0 behind a launch because its last workgroups say so; where one was not (launches that overlapped on the same counters, positions
+// written while a launch read them), every launch to come would merge too early or never.  A launch that is given the counters of a later one
+// sets these to 0, by the workgroup of the first split, so that such a fault does not outlast the next launch.
+__device__ __forceinline__ void clear_next_counter(const DecodeArgs& a, int b) {
+  if (threadIdx.x != 0 || a.next_arrivals == nullptr) return;
+  __hip_atomic_store(a.next_arrivals + (static_cast<int64_t>(b) * a.Hc + blockIdx.x) * a.arrivals_step, 0, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Merges the n partial results of sequence b's G heads (rows hq * row_mul + row_add + split of the workspace), normalises, gates and

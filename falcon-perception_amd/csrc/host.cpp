@@ -127,7 +127,7 @@ PyObject* append_unguarded(PyObject* const* args) {
 }
 
 // q, pool_k, pool_v, page_table, batch_idx, input_pos, page_size, max_context, scale, split_tokens, workspace, sinks, kv_rep,
-// k_new, v_new, plan, arrivals, stream -> (out, lse)
+// k_new, v_new, plan, arrivals, next_arrivals, stream -> (out, lse)
 PyObject* decode_unguarded(PyObject* const* args) {
   Args a{args};
   const at::Tensor *q = a.tensor(), *pk = a.tensor(), *pv = a.tensor(), *table = a.tensor(), *bidx = a.tensor(), *pos = a.tensor();
@@ -136,7 +136,8 @@ PyObject* decode_unguarded(PyObject* const* args) {
   const int64_t split_tokens = a.integer();
   const at::Tensor *ws = a.maybe_tensor(), *sinks = a.maybe_tensor();
   const int64_t kv_rep = a.integer();
-  const at::Tensor *kn = a.maybe_tensor(), *vn = a.maybe_tensor(), *plan = a.maybe_tensor(), *arrivals = a.tensor();
+  const at::Tensor *kn = a.maybe_tensor(), *vn = a.maybe_tensor(), *plan = a.maybe_tensor(), *arrivals = a.tensor(),
+                   *after = a.maybe_tensor();
   const int64_t stream = a.integer();
   if (!a.ok) Py_RETURN_NONE;
   const int dt = dtype_code(*q), it = index_code(*pos);
@@ -147,6 +148,7 @@ PyObject* decode_unguarded(PyObject* const* args) {
   const int64_t B = q->size(0), Hq = q->size(1), D = q->size(3), Hc = pk->size(0);
   if (!is_indices(*bidx, B) || pos->numel() != B || !pos->is_contiguous() || (ws && !is_bytes(*ws)) || (plan && !is_bytes(*plan)) ||
       arrivals->scalar_type() != at::kInt || !arrivals->is_contiguous() ||
+      (after && (after->scalar_type() != at::kInt || !after->is_contiguous() || after->numel() != arrivals->numel())) ||
       (sinks && (sinks->scalar_type() != at::kFloat || sinks->dim() != 1 || sinks->size(0) != Hq || !sinks->is_contiguous() ||
                  sinks->device() != q->device())))
     Py_RETURN_NONE;
@@ -159,7 +161,7 @@ PyObject* decode_unguarded(PyObject* const* args) {
   }
   const at::Tensor out = at::empty({B, Hq, 1, D}, q->options()), lse = at::empty({B, Hq, 1}, q->options().dtype(at::kFloat));
   const int rc = fp_paged_decode_step(
-      static_cast<int32_t*>(arrivals->data_ptr()), arrivals->numel() * 4, kn ? kn->data_ptr() : nullptr, vn ? vn->data_ptr() : nullptr,
+      static_cast<int32_t*>(arrivals->data_ptr()), after ? static_cast<int32_t*>(after->data_ptr()) : nullptr, arrivals->numel() * 4, kn ? kn->data_ptr() : nullptr, vn ? vn->data_ptr() : nullptr,
       kn ? kn->stride(0) : 0, kn ? kn->stride(1) : 0, vn ? vn->stride(0) : 0, vn ? vn->stride(1) : 0, q->data_ptr(), q->stride(0),
       q->stride(1), pk->data_ptr(), pv->data_ptr(), static_cast<const int64_t*>(table->data_ptr()), table->stride(0),
       static_cast<const int64_t*>(bidx->data_ptr()), pos->data_ptr(), it, out.data_ptr(), out.stride(0), out.stride(1),
@@ -222,7 +224,7 @@ PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 #define FP_METHOD(name, call, n) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<call, n>)), METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {FP_METHOD("append", append_unguarded, 11), FP_METHOD("decode", decode_unguarded, 18),
+PyMethodDef kMethods[] = {FP_METHOD("append", append_unguarded, 11), FP_METHOD("decode", decode_unguarded, 19),
                           FP_METHOD("prefill", prefill_unguarded, 14), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "fp_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -254,6 +254,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
         E::store(a.out + b * a.os_b + (hc * G + g) * a.os_h + d * sizeof(typename E::type), 0.f);
       }
       if (tid < G) lse_at(hc * G + tid) = -INFINITY;
+      if constexpr (kMerges) clear_next_counter(a, b);
     }
     return;
   }
@@ -437,6 +438,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
     }
   }
   if constexpr (kMerges) {
+    if (merges && split == 0) clear_next_counter(e, b);
     __shared__ int s_last;
     __shared__ __attribute__((aligned(16))) float s_part[4 * 64 * 4];
     if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, part_mul, part_add - split, n_pieces, G, s_part);
@@ -1050,7 +1052,7 @@ int decode_entry(int phases, const NewRows* fresh, const void* q, int64_t q_stri
                  int32_t D, int32_t page_size, int32_t n_pages, int32_t max_batch,
                  int64_t n_slots, int32_t max_context, int32_t split_tokens, float scale,
                  int dtype, void* plan, int64_t plan_bytes, void* stream,
-                 int32_t* arrivals = nullptr, int64_t arrivals_bytes = 0) {
+                 int32_t* arrivals = nullptr, int32_t* next_arrivals = nullptr, int64_t arrivals_bytes = 0) {
   const bool plan_only = phases == kPhasePlan;  // q, out, lse and the workspace are not touched then
   const int eb = fp::elem_bytes(dtype);
   if (eb == 0) return fp::fail(FP_ERR_UNSUPPORTED, "fp_paged_decode: unknown dtype %d", dtype);
@@ -1091,6 +1093,9 @@ int decode_entry(int phases, const NewRows* fresh, const void* q, int64_t q_stri
   if (arrivals && (!fp::aligned(arrivals, 4) || arrivals_bytes < counters))
     return fp::fail(FP_ERR_WORKSPACE, "fp_paged_decode_step: %lld bytes of arrival counters needed, %lld given",
                     static_cast<long long>(counters), static_cast<long long>(arrivals_bytes));
+  const char *const now = reinterpret_cast<const char*>(arrivals), *const later = reinterpret_cast<const char*>(next_arrivals);
+  if (later && (!fp::aligned(later, 4) || (later < now + arrivals_bytes && now < later + arrivals_bytes)))
+    return fp::fail(FP_ERR_WORKSPACE, "fp_paged_decode_step: the counters of the next launch overlap those of this one");
 
   if (split_tokens == 0) split_tokens = default_split_tokens(B, wg_heads, max_context, page_size);
   if (split_tokens % 64) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode: split_tokens must be a multiple of 64");
@@ -1112,7 +1117,7 @@ int decode_entry(int phases, const NewRows* fresh, const void* q, int64_t q_stri
                nullptr, nullptr, Hq, wg_heads, fp::PageDiv(page_size), n_pages, max_batch,
                static_cast<int>(n_slots / page_size > INT32_MAX ? INT32_MAX : n_slots / page_size), n_slots,
                max_context, split_tokens, ns, scale * kLog2e,  // scores are kept in log2 units
-               nullptr, nullptr, 0, 0, 0, 0, B, 0, static_cast<int*>(plan), arrivals, arrivals_step};
+               nullptr, nullptr, 0, 0, 0, 0, B, 0, static_cast<int*>(plan), arrivals, arrivals_step, next_arrivals};
   if (fresh) {
     if (!fresh->k || !fresh->v) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_append: null k_new / v_new");
     if (!fp::aligned(fresh->k, 16) || !fp::aligned(fresh->v, 16) || (fresh->k_stride_b * eb) % 16 ||
@@ -1173,12 +1178,12 @@ extern "C" int fp_paged_decode_append(const void* k_new, const void* v_new, int6
   const NewRows fresh{k_new, v_new, k_stride_b, k_stride_h, v_stride_b, v_stride_h};
   return decode_entry(kPhasePartial | kPhaseMerge, &fresh, FP_DECODE_ARGS);
 }
-extern "C" int fp_paged_decode_step(int32_t* arrivals, int64_t arrivals_bytes, const void* k_new, const void* v_new,
+extern "C" int fp_paged_decode_step(int32_t* arrivals, int32_t* next_arrivals, int64_t arrivals_bytes, const void* k_new, const void* v_new,
                                     int64_t k_stride_b, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_h,
                                     FP_DECODE_PARAMS) {
   if (B > 0 && !arrivals) return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_decode_step: null arrival counters");
   const NewRows fresh{k_new, v_new, k_stride_b, k_stride_h, v_stride_b, v_stride_h};
-  return decode_entry(kPhasePartial | kPhaseMerge, k_new || v_new ? &fresh : nullptr, FP_DECODE_ARGS, arrivals, arrivals_bytes);
+  return decode_entry(kPhasePartial | kPhaseMerge, k_new || v_new ? &fresh : nullptr, FP_DECODE_ARGS, arrivals, next_arrivals, arrivals_bytes);
 }
 
 

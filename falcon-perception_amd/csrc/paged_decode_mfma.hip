@@ -162,6 +162,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
           E::store(a.out + b * a.os_b + (hc * G + g) * a.os_h + d * 2, 0.f);
         }
         if (tid < G) a.lse[static_cast<int64_t>(b) * a.Hq + hc * G + tid] = -INFINITY;
+        if (kMerges && a.arrivals) clear_next_counter(a, b);
       }
       return;
     }
@@ -407,6 +408,7 @@ __global__ __launch_bounds__(kThreads, 2) void paged_decode_mfma_kernel(const De
       }
     }
     if constexpr (kMerges) {  // the rings are free behind the barrier inside
+      if (merges && split == 0) clear_next_counter(e, b);
       __shared__ int s_last;
       if (merges && !direct && last_to_arrive(b, n_pieces, &s_last)) merge_splits<E, D>(b, part_mul, part_add - split, n_pieces, G, reinterpret_cast<float*>(s_ring));
     }

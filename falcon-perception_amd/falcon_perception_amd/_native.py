@@ -18,7 +18,7 @@ _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib")
 LIB_PATH = os.path.join(_LIB_DIR, "libfp_paged_kv.so")
 HOST_PATH = os.path.join(_LIB_DIR, "fp_host.so")
 
-FP_ABI_VERSION = 9
+FP_ABI_VERSION = 10
 NOALLOC_SCRATCH_BYTES = 64 << 20  # FP_NOALLOC_SCRATCH_BYTES
 FP_DTYPE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 FP_INDEX = {torch.int32: 0, torch.int64: 1}
@@ -57,7 +57,7 @@ SIGNATURES = {
     "fp_paged_decode_partial": None,
     "fp_paged_decode_merge": None,
     "fp_paged_decode_append": None,  # two row pointers and four strides in front of the same list
-    "fp_paged_decode_step": None,  # the arrival counters and their size in front of that
+    "fp_paged_decode_step": None,  # two sets of arrival counters and their size in front of that
     "fp_paged_decode_noalloc": None,  # the same list without the workspace pair
     "fp_qkv_norm_rope_append": (c_int, [
         c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
@@ -87,7 +87,7 @@ _d = SIGNATURES["fp_paged_decode"][1]
 SIGNATURES["fp_paged_decode_noalloc"] = (c_int, _d[:15] + _d[17:-3] + _d[-1:])  # no workspace and no plan (pointer, size)
 SIGNATURES["fp_paged_decode_append"] = (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64]
                                         + SIGNATURES["fp_paged_decode"][1])
-SIGNATURES["fp_paged_decode_step"] = (c_int, [c_void_p, c_int64] + SIGNATURES["fp_paged_decode_append"][1])
+SIGNATURES["fp_paged_decode_step"] = (c_int, [c_void_p, c_void_p, c_int64] + SIGNATURES["fp_paged_decode_append"][1])
 
 _lib = None
 

@@ -287,13 +287,15 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
             cache._decode_plan_owner = block_mask
             block_mask._plan_shape = shape
     block_mask._plan_layer = step.layer_id
+    arrivals, after = cache._decode_arrivals
+    cache._decode_arrivals = after, arrivals
     got = None
     if q.is_cuda:
         got = N.host().decode(*args, 1.0 / math.sqrt(D) if scale is None else scale, split_tokens, workspace, sinks, kv_rep,
-                              k_new, v_new, plan, cache._decode_arrivals, N.raw_stream(q))
+                              k_new, v_new, plan, arrivals, after, N.raw_stream(q))
     if got is None:
-        got = ops.paged_decode(*args, scale=scale, workspace=workspace, split_tokens=split_tokens, sinks=sinks,
-                               kv_rep=kv_rep, k_new=k_new, v_new=v_new, plan=plan, arrivals=cache._decode_arrivals)
+        got = ops.paged_decode(*args, scale=scale, workspace=workspace, split_tokens=split_tokens, sinks=sinks, kv_rep=kv_rep,
+                               k_new=k_new, v_new=v_new, plan=plan, arrivals=arrivals, next_arrivals=after)
     return _result(*got, return_aux, return_lse)
 
 

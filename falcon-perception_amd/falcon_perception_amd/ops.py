@@ -204,7 +204,7 @@ def paged_decode(q: Tensor, pool_k: Tensor, pool_v: Tensor, page_table: Tensor, 
                  out: Tensor | None = None, lse: Tensor | None = None, phase: str = "both",
                  k_new: Tensor | None = None, v_new: Tensor | None = None,
                  sinks: Tensor | None = None, kv_rep: int = 1, plan: Tensor | None = None,
-                 arrivals: Tensor | None = None) -> tuple[Tensor, Tensor]:
+                 arrivals: Tensor | None = None, next_arrivals: Tensor | None = None) -> tuple[Tensor, Tensor]:
     """Single-query paged attention.  q [B, Hq, 1, D]; pools [Hc, N, D]; returns out [B, Hq, 1, D], lse [B, Hq, 1].
 
     `kv_rep` > 1 declares a cache with one head per query head whose V heads are `kv_rep` identical
@@ -227,7 +227,8 @@ def paged_decode(q: Tensor, pool_k: Tensor, pool_v: Tensor, page_table: Tensor, 
 
     `arrivals`: an int32 tensor of B * Hc / kv_rep entries or more, all 0, which every launch leaves all 0: a launch
     that goes split by split is then one launch without a merge pass (`fp_paged_decode_step`).  Like the workspace it serves one
-    launch at a time."""
+    launch at a time.  `next_arrivals`: a second tensor like it, for the launch after this one, which this one sets to 0 as far
+    as its sequences go; two that are given in turn recover from launches that overlapped on them."""
     N.require_cuda(q, pool_k, pool_v, page_table, batch_idx, input_pos, workspace, out, lse)
     B, Hq, Sq, D = q.shape
     if Sq != 1:
@@ -283,8 +284,12 @@ def paged_decode(q: Tensor, pool_k: Tensor, pool_v: Tensor, page_table: Tensor, 
             raise RuntimeError("arrival counters serve the call that runs both passes")
         if arrivals.dtype != torch.int32 or not arrivals.is_contiguous():
             raise RuntimeError("arrivals must be a contiguous int32 tensor")
+        if next_arrivals is not None:
+            N.require_cuda(next_arrivals)
+            if next_arrivals.dtype != torch.int32 or not next_arrivals.is_contiguous() or next_arrivals.numel() != arrivals.numel():
+                raise RuntimeError("next_arrivals must be like arrivals")
         entry = "fp_paged_decode_step"
-        fresh = (arrivals.data_ptr(), arrivals.numel() * 4, *(fresh or (None, None, 0, 0, 0, 0)))
+        fresh = (arrivals.data_ptr(), None if next_arrivals is None else next_arrivals.data_ptr(), arrivals.numel() * 4, *(fresh or (None, None, 0, 0, 0, 0)))
     rc = getattr(N.lib(), entry)(
         *fresh,
         q.data_ptr(), q.stride(0), q.stride(1), pool_k.data_ptr(), pool_v.data_ptr(),

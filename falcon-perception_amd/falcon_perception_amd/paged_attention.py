@@ -120,9 +120,10 @@ class PagedKVCache(KVCacheBase):
         self.last_decode_step: StepMeta | None = None
         self.last_prefill_step: StepMeta | None = None
         self._workspace: Tensor | None = None
-        # counters of the decode launch, all 0 between launches (`fp_paged_decode_step`).  Made here and not at first use, which
-        # may lie inside a graph capture: the zeros would be written by a replay only.
-        self._decode_arrivals = torch.zeros(max(max_batch_size * n_heads, 8192), dtype=torch.int32, device=device)
+        # counters of the decode launch, all 0 between launches (`fp_paged_decode_step`): two sets that the attention calls use in
+        # turn, each launch setting the next one's to 0.  Made here and not at first use, which may lie inside a graph capture: the
+        # zeros would be written by a replay only.
+        self._decode_arrivals = torch.zeros(2, max(max_batch_size * n_heads, 8192), dtype=torch.int32, device=device).unbind()
         self._retired_workspaces: list[Tensor] = []  # graphs captured earlier still write to these
         self._decode_launch: dict[tuple, tuple[int, int]] = {}
         self._decode_need: dict[tuple, int] = {}  # largest workspace over the batches, per launch shape without the batch

@@ -44,7 +44,7 @@
 extern "C" {
 #endif
 
-#define FP_ABI_VERSION 9
+#define FP_ABI_VERSION 10
 
 /* element types of pool / q / k / v */
 #define FP_DTYPE_F32 0
@@ -326,9 +326,12 @@ int fp_paged_decode_append(const void* k_new, const void* v_new,
  *              uses it and never written by anybody else; 32 times that many bytes give every counter a line of its own, which few
  *              sequences of many tokens want.  Every launch leaves it all 0.  Like the workspace it belongs
  *              to one launch at a time: launches that overlap need a workspace and counters of their own.
+ *   next_arrivals  optional: counters of the same size, elsewhere, that a launch after this one will be given (a caller with two
+ *              sets gives them in turn): the launch sets those of its (sequence, cache head)s to 0.  Counters that are not 0
+ *              although they should be, because launches overlapped on them after all, then spoil one launch and not all to come.
  * Results equal those of the two passes up to the order of the sums over the keys.  All other arguments as fp_paged_decode_append.
  */
-int fp_paged_decode_step(int32_t* arrivals, int64_t arrivals_bytes,
+int fp_paged_decode_step(int32_t* arrivals, int32_t* next_arrivals, int64_t arrivals_bytes,
                          const void* k_new, const void* v_new,
                          int64_t k_stride_b, int64_t k_stride_h,
                          int64_t v_stride_b, int64_t v_stride_h,

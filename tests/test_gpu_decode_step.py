@@ -8,9 +8,11 @@ the weights add up to 1), and the type's rounding comes on top.
 
 import pytest
 import torch
+from torch.nn.attention.flex_attention import AuxRequest, BlockMask
 
+from falcon_perception_amd import attention as A
 from falcon_perception_amd import ops
-from tests.gpu_cases import DEV, randn
+from tests.gpu_cases import DEV, PagedState, randn
 from tests.test_gpu_decode_plan import decode, flat_state, new_plan
 
 pytestmark = pytest.mark.gpu
@@ -166,3 +168,65 @@ def test_which_launches_go_piece_by_piece():
     assert pieces(8, 8, 128) == 0 and pieces(8, 8, 0) == 0  # one split
     with pytest.raises(RuntimeError):
         pieces(0, 8, 8192)
+
+
+def drop_in_state(B, Hc, D, P, ctx, dtype, layers, lens):
+    """A cache with `lens` tokens per sequence in every layer, and the positions and mask of the step after them."""
+    st = PagedState(57, n_pages=ctx // P + sum(-(-(n + 4) // P) for n in lens), page_size=P, max_batch=B + 2, Hc=Hc, D=D, dtype=dtype,
+                    n_layers=layers)
+    for n in lens:
+        st.add_sequence(n + 4)
+    st.cache.kv_cache.normal_()
+    bidx, pos = torch.tensor(st.slots, dtype=torch.int64, device=DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+    full = st.cache.create_causal_blockmask(B=1, L=ctx)
+    row, blk = torch.zeros_like(bidx), (pos // P).long()
+    logical = BlockMask.from_kv_blocks(
+        full.kv_num_blocks[row, :, blk].view(B, 1, 1), full.kv_indices[row, :, blk].view(B, 1, 1, -1),
+        full.full_kv_num_blocks[row, :, blk].view(B, 1, 1), full.full_kv_indices[row, :, blk].view(B, 1, 1, -1),
+        BLOCK_SIZE=full.BLOCK_SIZE, mask_mod=lambda b, h, q, kv: q + pos[b] >= kv, seq_lengths=(1, ctx))
+    return st, st.cache.convert_logical_block_mask(logical, bidx), bidx, pos
+
+
+# split by split; piece by piece; on the matrix cores
+@pytest.mark.parametrize("layers", [2, 3])
+@pytest.mark.parametrize("B,G,D,dtype", [(2, 2, 128, torch.bfloat16), (9, 1, 64, torch.float32), (9, 4, 64, torch.float16)], ids=str)
+def test_counters_that_are_not_zero_spoil_one_launch(B, G, D, dtype, layers):
+    """Launches that overlapped on one cache, against its contract, may leave counters behind; the layers after the next one and
+    every later step are right again."""
+    Hc, P, ctx = 8, 64, 4096
+    lens = [4000 - 431 * i for i in range(B)]
+    lens[1] = 0
+    st, mask, bidx, pos = drop_in_state(B, Hc, D, P, ctx, dtype, layers, lens)
+    cache = st.cache
+    for left_over in (1, 3, 1000):
+        sets = cache._decode_arrivals if isinstance(cache._decode_arrivals, tuple) else (cache._decode_arrivals,)
+        for t in sets:
+            t.fill_(left_over)
+        for step in range(2):
+            for layer in range(layers):
+                q, k, v = (randn(st.gen, (B, h, 1, D), dtype).to(DEV) for h in (Hc * G, Hc, Hc))
+                K, V = cache.insert_kv(layer, k, v, input_pos=pos.view(B, 1), batch_idx=bidx)
+                out, aux = A.compiled_flex_attn_decode(q, K, V, block_mask=mask, return_aux=AuxRequest(lse=True))
+                if step == 0 and layer == 0:
+                    continue
+                eo, el = ops.paged_decode(q, K[0], V[0], cache.page_table, bidx, pos, P, mask.max_context)
+                torch.testing.assert_close(out, eo, rtol=max(2 * STEP[dtype], 1e-5), atol=1e-5)
+                torch.testing.assert_close(aux.lse.view(el.shape), el, rtol=1e-5, atol=1e-5)
+
+
+def test_counters_of_the_next_launch():
+    """They are set to 0 for the sequences of the launch, whether a sequence has splits to merge or not, and lie elsewhere."""
+    B, Hc, ctx = 4, 2, 256
+    st = flat_state(6, B, Hc, 64, 32, ctx, torch.float32, 1, [255, 0, 60, 130])
+    q, *_ = inputs(st, B, Hc, 1, 64, torch.float32, 1)
+    pos = torch.tensor([255, -1, 60, 130], dtype=torch.int32, device=DEV)
+    sets = torch.zeros(3, 24, dtype=torch.int32, device=DEV)  # counters three words apart
+    sets[1:] = 7
+    kw = dict(max_context=ctx, split_tokens=64, bidx=torch.tensor(st.slots, dtype=torch.int64, device=DEV))
+    ref = decode(st, q, pos, **kw)
+    got = decode(st, q, pos, arrivals=sets[0], next_arrivals=sets[1], **kw)
+    close(got, ref, torch.float32, 64)
+    assert not sets[0].any() and not sets[1, ::3].any() and (sets[1].view(8, 3)[:, 1:] == 7).all() and (sets[2] == 7).all()
+    for after, match in ((sets[0], "overlap"), (sets.view(-1)[20:44], "overlap"), (sets[1, :8], "like arrivals"), (sets[1].float(), "like arrivals")):
+        with pytest.raises(RuntimeError, match=match):
+            decode(st, q, pos, arrivals=sets[0], next_arrivals=after, **kw)
