@@ -46,6 +46,14 @@ bool is_indices(const at::Tensor& t, int64_t n) { return t.scalar_type() == at::
 bool is_bytes(const at::Tensor& t) { return t.scalar_type() == at::kByte && t.is_contiguous(); }
 bool dense_rows(const at::Tensor& t) { return t.stride(t.dim() - 1) == 1; }
 
+// Other Python threads run while this one allocates and launches, which may wait (for a full queue, or for memory).
+struct Unlocked {
+  PyThreadState* const thread = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(thread); }
+};
+
 PyObject* fail(const char* what, int rc) {
   PyErr_Format(PyExc_RuntimeError, "%s failed (%d): %s", what, rc, fp_last_error());
   return nullptr;
@@ -118,10 +126,14 @@ PyObject* append_unguarded(PyObject* const* args) {
     for (int i = 0; i < 3; ++i) ks[i] = k->stride(i), vs[i] = v->stride(i);
   }
   if (!is_indices(*bidx, T)) Py_RETURN_NONE;
-  const int rc = fp_kv_append(pk->data_ptr(), pv->data_ptr(), k->data_ptr(), v->data_ptr(), ks[0], ks[1], ks[2], vs[0], vs[1], vs[2],
-                              static_cast<const int64_t*>(table->data_ptr()), table->stride(0),
-                              static_cast<const int64_t*>(bidx->data_ptr()), pos->data_ptr(), it, T, H, S, D, page_size,
-                              table->size(1), table->size(0), pk->size(1), dt, clamp ? 1 : 0, reinterpret_cast<void*>(stream));
+  int rc;
+  {
+    const Unlocked others;
+    rc = fp_kv_append(pk->data_ptr(), pv->data_ptr(), k->data_ptr(), v->data_ptr(), ks[0], ks[1], ks[2], vs[0], vs[1], vs[2],
+                      static_cast<const int64_t*>(table->data_ptr()), table->stride(0),
+                      static_cast<const int64_t*>(bidx->data_ptr()), pos->data_ptr(), it, T, H, S, D, page_size,
+                      table->size(1), table->size(0), pk->size(1), dt, clamp ? 1 : 0, reinterpret_cast<void*>(stream));
+  }
   if (rc < 0) return fail("fp_kv_append", rc);
   Py_RETURN_TRUE;
 }
@@ -159,15 +171,22 @@ PyObject* decode_unguarded(PyObject* const* args) {
         vn->scalar_type() != q->scalar_type() || !dense_rows(*kn) || !dense_rows(*vn))
       Py_RETURN_NONE;
   }
-  const at::Tensor out = at::empty({B, Hq, 1, D}, q->options()), lse = at::empty({B, Hq, 1}, q->options().dtype(at::kFloat));
-  const int rc = fp_paged_decode_step(
-      static_cast<int32_t*>(arrivals->data_ptr()), after ? static_cast<int32_t*>(after->data_ptr()) : nullptr, arrivals->numel() * 4, kn ? kn->data_ptr() : nullptr, vn ? vn->data_ptr() : nullptr,
-      kn ? kn->stride(0) : 0, kn ? kn->stride(1) : 0, vn ? vn->stride(0) : 0, vn ? vn->stride(1) : 0, q->data_ptr(), q->stride(0),
-      q->stride(1), pk->data_ptr(), pv->data_ptr(), static_cast<const int64_t*>(table->data_ptr()), table->stride(0),
-      static_cast<const int64_t*>(bidx->data_ptr()), pos->data_ptr(), it, out.data_ptr(), out.stride(0), out.stride(1),
-      static_cast<float*>(lse.data_ptr()), sinks ? static_cast<const float*>(sinks->data_ptr()) : nullptr, ws ? ws->data_ptr() : nullptr,
-      ws ? ws->numel() : 0, B, Hq, Hc, kv_rep, D, page_size, table->size(1), table->size(0), pk->size(1), max_context, split_tokens,
-      static_cast<float>(scale), dt, plan ? plan->data_ptr() : nullptr, plan ? plan->numel() : 0, reinterpret_cast<void*>(stream));
+  at::Tensor out, lse;
+  int rc;
+  {
+    const Unlocked others;
+    out = at::empty({B, Hq, 1, D}, q->options());
+    lse = at::empty({B, Hq, 1}, q->options().dtype(at::kFloat));
+    rc = fp_paged_decode_step(
+        static_cast<int32_t*>(arrivals->data_ptr()), after ? static_cast<int32_t*>(after->data_ptr()) : nullptr,
+        arrivals->numel() * 4, kn ? kn->data_ptr() : nullptr, vn ? vn->data_ptr() : nullptr,
+        kn ? kn->stride(0) : 0, kn ? kn->stride(1) : 0, vn ? vn->stride(0) : 0, vn ? vn->stride(1) : 0, q->data_ptr(), q->stride(0),
+        q->stride(1), pk->data_ptr(), pv->data_ptr(), static_cast<const int64_t*>(table->data_ptr()), table->stride(0),
+        static_cast<const int64_t*>(bidx->data_ptr()), pos->data_ptr(), it, out.data_ptr(), out.stride(0), out.stride(1),
+        static_cast<float*>(lse.data_ptr()), sinks ? static_cast<const float*>(sinks->data_ptr()) : nullptr, ws ? ws->data_ptr() : nullptr,
+        ws ? ws->numel() : 0, B, Hq, Hc, kv_rep, D, page_size, table->size(1), table->size(0), pk->size(1), max_context, split_tokens,
+        static_cast<float>(scale), dt, plan ? plan->data_ptr() : nullptr, plan ? plan->numel() : 0, reinterpret_cast<void*>(stream));
+  }
   if (rc < 0) return fail("fp_paged_decode_step", rc);
   return pair(out, lse);
 }
@@ -197,16 +216,22 @@ PyObject* prefill_unguarded(PyObject* const* args) {
       (order && (order_rows <= 0 || order->scalar_type() != at::kInt || !order->is_contiguous() ||
                  order->numel() != (Lq + order_rows - 1) / order_rows)))
     Py_RETURN_NONE;
-  const at::Tensor out = at::empty_like(*q);
+  at::Tensor out, lse;
+  int rc = FP_OK;
+  {
+    const Unlocked others;
+    out = at::empty_like(*q);
+    lse = at::empty({1, Hq, Lq}, q->options().dtype(at::kFloat));
+    if (dense_rows(out))
+      rc = fp_paged_prefill(
+          q->data_ptr(), q->stride(2), q->stride(1), pk->data_ptr(), pv->data_ptr(), static_cast<const int64_t*>(table->data_ptr()),
+          table->stride(0), static_cast<const int64_t*>(bidx->data_ptr()), static_cast<const int32_t*>(limit->data_ptr()), out.data_ptr(),
+          out.stride(2), out.stride(1), static_cast<float*>(lse.data_ptr()), sinks ? static_cast<const float*>(sinks->data_ptr()) : nullptr,
+          Lq, Hq, Hc, D, page_size, table->size(1), table->size(0), pk->size(1), static_cast<float>(scale), static_cast<float>(bound), dt,
+          ws ? ws->data_ptr() : nullptr, ws ? ws->numel() : 0, order ? static_cast<const int32_t*>(order->data_ptr()) : nullptr,
+          order ? order_rows : 0, reinterpret_cast<void*>(stream));
+  }
   if (!dense_rows(out)) Py_RETURN_NONE;
-  const at::Tensor lse = at::empty({1, Hq, Lq}, q->options().dtype(at::kFloat));
-  const int rc = fp_paged_prefill(
-      q->data_ptr(), q->stride(2), q->stride(1), pk->data_ptr(), pv->data_ptr(), static_cast<const int64_t*>(table->data_ptr()),
-      table->stride(0), static_cast<const int64_t*>(bidx->data_ptr()), static_cast<const int32_t*>(limit->data_ptr()), out.data_ptr(),
-      out.stride(2), out.stride(1), static_cast<float*>(lse.data_ptr()), sinks ? static_cast<const float*>(sinks->data_ptr()) : nullptr,
-      Lq, Hq, Hc, D, page_size, table->size(1), table->size(0), pk->size(1), static_cast<float>(scale), static_cast<float>(bound), dt,
-      ws ? ws->data_ptr() : nullptr, ws ? ws->numel() : 0, order ? static_cast<const int32_t*>(order->data_ptr()) : nullptr,
-      order ? order_rows : 0, reinterpret_cast<void*>(stream));
   if (rc < 0) return fail("fp_paged_prefill", rc);
   return pair(out, lse);
 }

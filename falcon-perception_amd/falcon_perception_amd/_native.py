@@ -140,9 +140,8 @@ def stream_ptr(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def raw_stream(t: torch.Tensor) -> int:
-    """Handle of the stream that is current on the device of `t` (0 for a tensor that is not on the GPU)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device()) if t.is_cuda else 0
+# device index -> handle of the stream that is current there (None: a torch without GPUs)
+raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def require_cuda(*tensors) -> None:

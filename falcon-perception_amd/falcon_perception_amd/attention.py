@@ -292,7 +292,7 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
     got = None
     if q.is_cuda:
         got = N.host().decode(*args, 1.0 / math.sqrt(D) if scale is None else scale, split_tokens, workspace, sinks, kv_rep,
-                              k_new, v_new, plan, arrivals, after, N.raw_stream(q))
+                              k_new, v_new, plan, arrivals, after, N.raw_stream(q.get_device()))
     if got is None:
         got = ops.paged_decode(*args, scale=scale, workspace=workspace, split_tokens=split_tokens, sinks=sinks, kv_rep=kv_rep,
                                k_new=k_new, v_new=v_new, plan=plan, arrivals=arrivals, next_arrivals=after)
@@ -340,7 +340,7 @@ def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, 
     got = None
     if q.is_cuda:
         got = N.host().prefill(*args, 1.0 / math.sqrt(D) if scale is None else scale, sinks, None if workspace is False else workspace,
-                               bound, *((None, 0) if order is None else order), N.raw_stream(q))
+                               bound, *((None, 0) if order is None else order), N.raw_stream(q.get_device()))
     if got is None:
         got = ops.paged_prefill(*args, scale=scale, sinks=sinks, workspace=workspace, score_bound=bound, tile_order=order)
     return _result(*got, return_aux, return_lse)

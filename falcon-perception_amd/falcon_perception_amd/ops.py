@@ -29,7 +29,7 @@ def kv_append(pool_k: Tensor, pool_v: Tensor, k: Tensor, v: Tensor, page_table: 
     L row groups of one token each through their strides.
     """
     if k.is_cuda and N.host().append(pool_k, pool_v, k, v, page_table, batch_idx, input_pos, page_size, clamp_negative, packed,
-                                     N.raw_stream(k)):
+                                     N.raw_stream(k.get_device())):
         return
     N.require_cuda(pool_k, pool_v, k, v, page_table, batch_idx, input_pos)
     if v.shape != k.shape:
