@@ -14,6 +14,7 @@
 
 #include <ATen/ATen.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <exception>
 
@@ -260,5 +261,7 @@ PyMODINIT_FUNC PyInit_fp_host() {
     PyErr_Format(PyExc_RuntimeError, "libfp_paged_kv.so has ABI %d, fp_host was built for %d", fp_abi_version(), FP_ABI_VERSION);
     return nullptr;
   }
-  return PyModule_Create(&kModule);
+  PyObject* const module = PyModule_Create(&kModule);
+  if (module) PyModule_AddStringConstant(module, "torch_version", TORCH_VERSION);
+  return module;
 }

@@ -10,6 +10,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import re
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_void_p
 
 import torch
@@ -126,6 +127,10 @@ def host():
         loader = importlib.machinery.ExtensionFileLoader("fp_host", HOST_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("fp_host", loader))
         loader.exec_module(module)
+        # it reads tensors as the headers it was compiled with lay them out, which another release of torch need not do
+        if re.match(r"\d+\.\d+\.\d+", torch.__version__).group() != module.torch_version:
+            raise RuntimeError(f"{HOST_PATH} was built for torch {module.torch_version} and this is {torch.__version__}: build it "
+                               "again with `python falcon-perception_amd/build_native.py`.")
         _host = module
     return _host
 

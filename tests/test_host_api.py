@@ -37,6 +37,15 @@ def test_library_exports_every_declared_symbol(native_lib):
     assert native_lib.fp_abi_version() == _native.FP_ABI_VERSION
 
 
+def test_calls_built_for_another_torch_are_refused(native_lib, monkeypatch):
+    monkeypatch.setattr(_native, "_host", None)
+    assert _native.host().decode
+    monkeypatch.setattr(_native, "_host", None)
+    monkeypatch.setattr(torch, "__version__", "9.9.0+rocm")
+    with pytest.raises(RuntimeError, match="was built for torch"):
+        _native.host()
+
+
 def header_declarations():
     """name -> number of parameters, from the C declarations of the header."""
     text = open(os.path.join(ROOT, "include", "fp_paged_kv.h")).read()
