@@ -30,6 +30,32 @@ def close(got, ref, dtype, n):
     assert same.all() and ((lse - rl).abs().nan_to_num(0.0) <= bound * (1 + rl.abs().nan_to_num(0.0, 0.0, 0.0))).all()
 
 
+def holds(got, st, q, pos, bidx, ctx, dtype, split_p):
+    """`got` against float64 over the pool as it is, each sequence within what its own keys can be off by: a score by 12 roundings of
+    sum |q k|, the sums of a lane over n / 16 of n keys by two roundings a key, and as many for pieces, wavefronts and the last
+    division as 64 cover; `split_p`: probabilities in two 16-bit parts, 2^-16 of each is left over in bf16.  A key that is missing or
+    counted twice, or a piece a few per cent off in weight, is more than that."""
+    (out, lse), (pk, pv) = got, st.pool_planes()
+    B, Hq, _, D = q.shape
+    scale = D**-0.5
+    table = st.cache.page_table
+    for b in range(B):
+        slot, n = int(bidx[b]), min(int(pos[b]) + 1, ctx)
+        if n <= 0 or not 0 <= slot < table.shape[0]:
+            assert not out[b].any() and torch.isneginf(lse[b]).all(), b
+            continue
+        t = torch.arange(n, device=DEV)
+        slots = table[slot, t // st.P].clamp(min=0) * st.P + t % st.P  # without a page: page 0
+        K, V = (x[:, slots].double().repeat_interleave(Hq // x.shape[0], 0) for x in (pk, pv))
+        Q = q[b].double()
+        s = Q @ K.transpose(1, 2) * scale
+        p = torch.softmax(s, -1)
+        off = (12 * scale * (Q.abs() @ K.abs().transpose(1, 2)).amax(-1) + n / 8 + 64) * 2.0**-24 + split_p * 2.0**-16
+        ref, size = p @ V, p @ V.abs()
+        assert ((out[b].double() - ref).abs() <= off[..., None] * size + STEP[dtype] / 2 * ref.abs() + 2.0**-25 * (dtype == torch.float16)).all(), b
+        assert ((lse[b].double() - torch.logsumexp(s, -1)).abs() <= 2 * off).all(), b
+
+
 def inputs(st, B, Hc, G, D, dtype, rep):
     q = randn(st.gen, (B, Hc * G, 1, D), dtype).to(DEV)
     k_new = randn(st.gen, (B, Hc * rep, 1, D), dtype).to(DEV)
@@ -142,7 +168,8 @@ def test_piece_by_piece_gives_what_the_two_passes_give(case, dtype, D, P, G, rep
     before = st.cache.kv_cache.clone()
     arrivals = torch.zeros(B * Hc * 5 + 3, dtype=torch.int32, device=DEV)  # counters five words apart
     kw = dict(max_context=ctx, split_tokens=split, kv_rep=rep, bidx=bidx)
-    # the pieces are others than the splits, so the sums over the keys run in another order: n = keys in `close`
+    # the pieces are others than the splits, so the sums over the keys run in another order: n = keys in `close`, which says little of
+    # a long sequence; `holds` bounds each by itself
     for pos_type in (torch.int32, torch.int64):
         pos = torch.tensor(lens, dtype=pos_type, device=DEV)
         if pos_type is torch.int64 and B > 20:
@@ -154,6 +181,7 @@ def test_piece_by_piece_gives_what_the_two_passes_give(case, dtype, D, P, G, rep
         got = decode(st, q, pos, k_new=k_new, v_new=v_new, arrivals=arrivals, **kw)
         close(got, ref, dtype, ctx)
         assert torch.equal(st.cache.kv_cache, pool) and not arrivals.any()
+        holds(got, st, q, pos, bidx, ctx, dtype, G >= 4 and dtype == torch.bfloat16)
 
 
 def test_which_launches_go_piece_by_piece():
@@ -230,3 +258,42 @@ def test_counters_of_the_next_launch():
     for after, match in ((sets[0], "overlap"), (sets.view(-1)[20:44], "overlap"), (sets[1, :8], "like arrivals"), (sets[1].float(), "like arrivals")):
         with pytest.raises(RuntimeError, match=match):
             decode(st, q, pos, arrivals=sets[0], next_arrivals=after, **kw)
+
+
+@pytest.mark.parametrize("case", [*PIECES, "splits"])
+@pytest.mark.parametrize("dtype,D,P,G,rep", [
+    (torch.bfloat16, 128, 64, 2, 1), (torch.float32, 64, 16, 1, 1), (torch.float16, 64, 24, 4, 1), (torch.bfloat16, 128, 48, 2, 2)], ids=str)
+def test_every_key_counts_once(case, dtype, D, P, G, rep):
+    """Keys of equal weight: lse is the logarithm of their number, and element d of a head whose V is 4096 at one key and 0 elsewhere is
+    4096 over their number, if that key counts once.  The keys marked are those at multiples of 64 and in front of them, where pieces
+    end, the first and the last, then some of the others."""
+    B, Hc, ctx, lens = PIECES[case] if case != "splits" else (2, 8, 4096, [4095, 1000])
+    if lens is None:
+        lens = [(37 * i * i + 11 * i) % (ctx - 2) for i in range(B)]
+    split = ops.decode_split_tokens(B, Hc, ctx, P)
+    assert (ops.decode_step_pieces(B, Hc * G, Hc * rep, rep, D, ctx, P, split) > 0) == (case != "splits")
+    st = flat_state(77, B, Hc, D, P, ctx, dtype, rep, [max(n, 0) for n in lens])
+    _, pv = st.pool_planes()
+    pv.zero_()
+    v_new = torch.zeros(B, Hc * rep, 1, D, dtype=dtype, device=DEV)
+    for b, n in enumerate(lens):
+        if n < 0:
+            continue
+        edges = {0, n, *range(64, n + 1, 64), *range(63, n + 1, 64)}
+        keys = [*sorted(edges), *(i * 7919 % (n + 1) for i in range(Hc * D))][: Hc * D]
+        keys = torch.tensor(keys, device=DEV).view(Hc, D).repeat_interleave(rep, 0)
+        slots = st.cache.page_table[st.slots[b], keys // P] * P + keys % P
+        h, d = torch.meshgrid(torch.arange(Hc * rep, device=DEV), torch.arange(D, device=DEV), indexing="ij")
+        pool_has = keys < n
+        pv[h[pool_has], slots[pool_has], d[pool_has]] = 4096.0
+        v_new[b, :, 0] = torch.where(pool_has, 0.0, 4096.0)
+    q = torch.zeros(B, Hc * G, 1, D, dtype=dtype, device=DEV)
+    k_new = randn(st.gen, v_new.shape, dtype).to(DEV)
+    pos = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    arrivals = torch.zeros(B * Hc, dtype=torch.int32, device=DEV)
+    out, lse = decode(st, q, pos, k_new=k_new, v_new=v_new, max_context=ctx, split_tokens=split, kv_rep=rep, arrivals=arrivals)
+    n = (pos + 1).double().view(B, 1, 1, 1)
+    want = torch.where(n > 0, 4096.0 / n, 0.0)
+    assert ((out.double() - want).abs() <= (STEP[dtype] / 2 + 2.0**-21) * want).all()
+    assert torch.equal(torch.isneginf(lse), (n[..., 0] <= 0).expand_as(lse))
+    assert ((lse.double() - n[..., 0].clamp(min=1).log()).abs() <= 2.0**-20 * (1 + n[..., 0].clamp(min=1).log()))[pos >= 0].all()
