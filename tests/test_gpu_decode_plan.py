@@ -386,11 +386,15 @@ def test_the_drop_in_plans_once_per_step_mask(monkeypatch, fused):
     assert rec[0, 0] >= 1 and rec[0, 1] == B  # the launch was large enough to be cut evenly: the plan was read
 
 
+@pytest.mark.parametrize("B", [16, 24])
 @pytest.mark.parametrize("fused", [True, False], ids=["append-fused", "append-first"])
-def test_a_mask_kept_while_its_positions_advance_plans_every_step(fused):
-    """Sixteen sequences under a limit of 8192 tokens, cut evenly: one mask object, the positions advance in place between the
-    steps.  The plan of a step must not outlive it (its launches would also append to the slots of the step before)."""
-    dtype, B, Hc, G, D, P, ctx, layers = torch.bfloat16, 16, 8, 2, 128, 128, 8192, 3
+def test_a_mask_kept_while_its_positions_advance_plans_every_step(fused, B):
+    """Sequences under a limit of 8192 tokens: one mask object, the positions advance in place between the steps.  24 are cut evenly
+    and read the step's plan, which must not outlive it (its launches would also append to the slots of the step before); 16 go
+    piece by piece and read none, so that only the cut has to follow."""
+    dtype, Hc, G, D, P, ctx, layers = torch.bfloat16, 8, 2, 128, 128, 8192, 3
+    pieces = ops.decode_step_pieces(B, Hc * G, Hc, 1, D, ctx, P, 0)
+    assert (pieces > 0) == (B == 16)
     lens = [60 + 97 * i for i in range(B)]
     st = PagedState(98, n_pages=ctx // P + sum(-(-(n + 4) // P) for n in lens), page_size=P, max_batch=B + 2, Hc=Hc, D=D,
                     dtype=dtype, n_layers=layers)
