@@ -98,6 +98,7 @@ class DecodeCase:
     lse: torch.Tensor | None = None
     plan: torch.Tensor | None = None  # the step's plan (fp_paged_decode_plan), read by the launches while `planned`
     planned: bool = True
+    arrivals: torch.Tensor | None = None  # arrival counters: the step in one launch where that serves (fp_paged_decode_step)
     layer_steps: int = 0              # layer-steps run through `run_step` so far
     extra: dict = field(default_factory=dict)
 
@@ -166,7 +167,7 @@ class DecodeCase:
                                 self.input_pos, self.page_size, self.max_context,
                                 split_tokens=self.split_tokens, workspace=self.workspace,
                                 out=self.out, lse=self.lse, k_new=self.k_new, v_new=self.v_new,
-                                kv_rep=self.cfg.get("kv_rep", 1), plan=self._plan)
+                                kv_rep=self.cfg.get("kv_rep", 1), plan=self._plan, arrivals=self.arrivals)
 
     def run_fused_gated(self):
         """run_fused plus the caller's post-attention sink gate (reference model.py:122-127) inside the
@@ -508,7 +509,7 @@ def model_depth_graph_ms(case: "DecodeCase", steps: int, layers: int = MODEL_LAY
             ops.paged_decode(case.q, pools[layer, 0], pools[layer, 1], case.cache.page_table, case.batch_idx,
                              case.input_pos, case.page_size, case.max_context, split_tokens=case.split_tokens,
                              workspace=case.workspace, out=case.out, lse=case.lse, k_new=case.k_new, v_new=case.v_new,
-                             kv_rep=c.get("kv_rep", 1), plan=case._plan)
+                             kv_rep=c.get("kv_rep", 1), plan=case._plan, arrivals=case.arrivals)
 
     ms = graph_ms(all_layers, max(steps // 10, 5))
     del pools
@@ -796,19 +797,23 @@ def decode_drop_in(case: "DecodeCase", steps: int, model_layers: bool = False) -
 
 
 def small_batch_decode(steps: int = 200) -> dict:
-    """The decode step (append + split-K pass + merge pass) of a few long sequences, replayed from a HIP
-    graph: the regime of one or a few requests, where the split length and the merge pass set the time."""
+    """The decode step (append, attention and merge) of a few long sequences, replayed from a HIP graph: the regime of one or a
+    few requests, with the arrival counters an engine's cache keeps (`fp_paged_decode_step`), so that the launch merges its splits
+    itself, and in two passes without them."""
     out = {}
     for B, L in ((1, 8192), (1, 32768), (4, 8192), (16, 8192)):
         name = f"small_B{B}_L{L}"
         DECODE_WORKLOADS[name] = dict(seed=7, dtype="bf16", B=B, Hq=16, Hc=8, D=128, P=128,
                                       n_pages=B * (L // 128 + 2) + 8, prefix=L - 64, lo=0, hi=63)
         case = make_decode_case(name)
+        ms_two = graph_ms(case.run_fused, steps)
+        case.arrivals = torch.zeros(B * case.cfg["Hc"] * 32, dtype=torch.int32, device="cuda")
         ms = graph_ms(case.run_fused, steps)
         # one step per replay pays the replay's own launch cost (about 5 us) on a 12 us step; the engine replays a
         # graph of the model's depth, so the same step is also timed as one of 28 layers (own K/V planes each)
         ms_model = model_depth_graph_ms(case, steps)
         out[f"batch {B}, context ~{L}"] = {"split_tokens": case.split_tokens, "ms_per_step_hip_graph": ms,
+                                          "ms_per_step_hip_graph_in_two_passes": ms_two,
                                           "gbps": case.bytes_decode() / (ms * 1e-3) / 1e9,
                                           "ms_per_layer_in_a_graph_of_all_layers": ms_model / MODEL_LAYERS if ms_model else None}
         if (B, L) == (1, 8192):  # the same step through the callables an unedited engine binds
