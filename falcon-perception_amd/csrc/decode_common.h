@@ -410,7 +410,7 @@ __device__ __forceinline__ void walk_split(const DecodeArgs& a, const Work& piec
         raw, trow, nullptr);
 }
 
-// Grid (workgroup heads, n_chunks + B) of a launch with arrivals, up to 64 sequences: the splits of all sequences have one length, as long
+// Grid (workgroup heads, n_chunks + B) of a launch with arrivals, up to 48 sequences (merged_pieces; a lane of a wavefront each): the splits of all sequences have one length, as long
 // as n_chunks of them need to be, and what a workgroup does follows from the lengths of the sequences.  Split by split it follows
 // from max_context, and a workgroup that finds nothing to do costs the launch 3 ns: 4 sequences of 300 tokens under a limit of 4096, 1024
 // workgroups 10.9 us a layer, 512 9.4, 256 8.1.  Every wavefront works the cut out by itself, a sequence to a lane, without LDS or a barrier; that

@@ -57,7 +57,7 @@ struct PageDiv {
   }
 };
 
-// fp32 chunked-prefill attention on the fp32 matrix instruction (paged_prefill_f32.hip)
+// fp32 chunked-prefill attention (paged_prefill_f32.hip)
 int prefill_mfma_f32(const void* q, int64_t q_stride_row, int64_t q_stride_h, const void* pool_k, const void* pool_v,
                      const int64_t* page_table, int64_t pt_row_stride, const int64_t* batch_idx,
                      const int32_t* row_limit, void* out, int64_t out_stride_row, int64_t out_stride_h, float* lse,

@@ -3,8 +3,8 @@
 //
 // Bound by the host: a layer of a small eager step is shorter on the GPU than its calls are in Python, where every pointer, size
 // and stride is an attribute look-up and the foreign call converts forty arguments one by one.  Here they are read from the tensors in C++:
-// four short fp32 sequences, 28 layers, without graphs 760 -> 380 us a step (27 -> 13.5 us a layer, of which the GPU works 7), one prompt
-// of 613 rows 910 -> 700 us (32 -> 25 us a layer, now the GPU's).
+// four short fp32 sequences, 28 layers, without graphs 818 -> 380 us a step (29 -> 13.5 us a layer, of which the GPU works 7), one prompt
+// of 613 rows 911 -> 700 us (33 -> 25 us a layer, now the GPU's).
 //
 // The functions take the tensors as ops.py would hand them to the library.  What they do not recognise at once (a tensor
 // subclass, another device or type, rows that are not dense, shapes that do not match) they leave alone and return None: ops.py

@@ -14,7 +14,9 @@
 //           limit much longer than they are (even_cut_pays), runs as (cache
 //           heads, chunks) instead: the contexts laid end to end and cut into
 //           equal chunks, a workgroup working through the sequences its chunk
-//           touches.
+//           touches.  With arrival counters (fp_paged_decode_step) few
+//           sequences run as (cache heads, pieces), all pieces of one length
+//           (merged_pieces).
 //   loads = a row (D elements) is covered by TPR = D * elem / 16 lanes holding
 //           16 bytes each, so a wavefront load instruction moves 64 / TPR whole
 //           rows, contiguous inside a page; U such loads of K and of V are in
@@ -22,7 +24,9 @@
 //   math  = each lane group keeps its own online-softmax state (m, l, acc) in
 //           log2 space; q.k partial sums are combined across the TPR lanes with
 //           DPP adds; lane groups, then wavefronts (through LDS), then splits
-//           (through the workspace, by the merge kernel) are combined at the end.
+//           (through the workspace) are combined at the end: by the merge
+//           kernel, or by the last workgroup of a (sequence, cache head) to
+//           leave its result where the caller keeps arrival counters.
 #include "decode_common.h"
 #include "paged_decode_mfma.h"
 
@@ -841,7 +845,9 @@ int even_cut_chunks(int Hc, int B, int n_splits, int max_context, int page_size,
 // CUs hold at once has few idle workgroups (limit 1024, 16 of 900 to 1000 16.9 / 18.1, of 100 to 900 13.2 / 13.4); and with more
 // tokens or sequences the remainders, up to B pieces, run behind the others (limit 8192, 24 of 4000 to 8000 96.7 / 99.8, 60 of these 228 / 261; limit 4096, 24 of
 // 64 to 4000 41.2 / 37.9, 32 of 300 to 4000 51.1 / 51.3; limit 2048, 32 of 300 to 2000 33.7 / 31.4; limit 1024, 60 of 100 to 1000 31.8 / 31.8
-// and in a step of 28 layers 908 / 920 us).  The step's plan does not know which way its launches go: one that goes piece by piece reads none.
+// and in a step of 28 layers 908 / 920 us).  The line at limit 8192 is that of the long ones; shorter sequences would gain on its other side, too (cut evenly /
+// piece by piece, a layer of 28: 17 of 64 to 500 14.9 / 11.1, of 300 to 3000 27.0 / 24.8, of 64 to 8000 51.2 / 48.7; 24 of these 15.4 / 12.0, 34.4 / 32.9 and 69.4 / 70.5,
+// D 64, f16 13.9 / 10.7 and 23.7 / 21.0; limit 16384, 12 of 64 to 500 11.5 / 9.4).  The step's plan does not know which way its launches go: one that goes piece by piece reads none.
 int merged_pieces(int Hc, int B, int n_splits, int max_context, int page_size) {
   const int64_t groups = static_cast<int64_t>(Hc) * B, tokens = static_cast<int64_t>(B) * (max_context + 64), two = 2 * fp::compute_units();
   if (B < 3 || B > 48 || groups < 32 || n_splits < 2 || (n_splits <= 4 && groups * n_splits <= two) || tokens >= 1 << 22 ||

@@ -839,10 +839,14 @@ constexpr int kMaxKeyShares = 8;
 // already, a cut in two costs more in partial results and their merge than the shorter critical path
 // saves: 138 us against 111 us at 8 sequences x 512 rows.)  fp32: the kernel takes about four times as long over twice the partial
 // results.  Up to a workgroup for every other CU the same rule (16 heads, D 128, us with 1 / 2 / 3 / 4 / 6 / 8 shares: 512 rows over 4096
-// keys, 32 workgroups, 613 / 326 / 226 / 179 / 130 / 114; 1100 rows, 80 workgroups, 148 / 93 / 75 / 96 / 93 / 108).  Beyond that up to
-// four workgroups per CU even out sequences of different lengths and the last, partly filled round of workgroups: 160 workgroups 565 / 413 /
+// keys, 32 workgroups, 613 / 326 / 226 / 179 / 130 / 114; 1100 rows, 80 workgroups, 148 / 93 / 75 / 96 / 93 / 108; 1536 rows, 96, 210 / 134 / 170 /
+// 141 / 157 / 144; 1792, 112, 242 / 157 / 191 / 161 / 178 / 194; 2048, 128, 281 / 189 / 228 / 199 / 213 / 227; chunks of 512 rows over 256 to 4096
+// keys, 96 and 128 workgroups, 577 / 318 / 234 / 283 / 244 / 255 and 577 / 324 / 322 / 295 / 299 / 297).  Beyond that up to
+// four workgroups per CU even out sequences of different lengths and the last, partly filled round of workgroups: 144 workgroups (2176 rows of
+// one sequence) 288 / 284 / 236 / 252 / 256 / 258 (5: 237, 7: 246), 160 565 / 413 /
 // 349 / 339 / 335 / 345 (5: 333), 256 594 / 567 / 526 / 507 / 526 / 562, 336 463 / 431 / 436 / 462 / 508 / 562, 448 640 / 575 / 598 / 635 / 694 / 751, 1120
-// 1873 / 2002 / 2075 / 2184 / 2366 / 2518.
+// 1873 / 2002 / 2075 / 2184 / 2366 / 2518.  Many short sequences pay for it: 8 of 80 to 500 rows, 176 workgroups, 67 / 87 / 88 / 105 / 124 / 155
+// (5: 117).
 int key_shares_for(int64_t wgs, int dtype) {
   if (wgs < 1) wgs = 1;
   const int64_t cus = fp::compute_units();
@@ -1116,7 +1120,7 @@ extern "C" int fp_paged_prefill(const void* q, int64_t q_stride_row, int64_t q_s
   if (workspace && (!fp::aligned(workspace, 16) || workspace_bytes < 0))
     return fp::fail(FP_ERR_WORKSPACE, "fp_paged_prefill: the workspace must be 16-byte aligned");
   if (dtype == FP_DTYPE_F32) {
-    // fp32 has a kernel of its own on the fp32 matrix instruction
+    // fp32 has a kernel of its own: six bf16 products of three-part numbers, the fp32 matrix instruction where these do not do
     if (!fp::aligned(q, 16) || !fp::aligned(pool_k, 16) || !fp::aligned(pool_v, 16) || !fp::aligned(out, 4) ||
         (q_stride_row * 4) % 16 || (q_stride_h * 4) % 16)
       return fp::fail(FP_ERR_INVALID_ARGUMENT, "fp_paged_prefill: q rows must be 16-byte aligned");

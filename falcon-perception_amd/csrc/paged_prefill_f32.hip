@@ -7,9 +7,10 @@
 //
 // MFMA-bound.  The fp32 matrix instruction does a sixteenth of the bf16 one's work per cycle.  An fp32 number is exactly the sum of three
 // bf16 numbers, each the rounding of what the ones before leave (x = x1 + x2 + x3), so a product of two is six bf16 products
-// and a rest of 2^-26: k1 q1 + (k1 q2 + k2 q1) + (k1 q3 + k2 q2 + k3 q1), 6 / 16 of the cycles.  Sums stay in the instruction's
+// and a rest of 2^-26: k1 q1 + (k1 q2 + k2 q1) + (k1 q3 + k2 q2 + k3 q1), 6 / 16 of the cycles (the method of G. Henry, P. T. P. Tang and
+// A. Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations", 2019).  Sums stay in the instruction's
 // fp32 accumulators; in the scores the five small products have accumulators of their own, so that the large one is rounded
-// D / 16 times.  K, V, Q and the probabilities are all kept to their 24 bits.
+// D / 16 times.  K, V and Q are all kept to their 24 bits, and so are probabilities from 2^-100 on; of a smaller one less than 2^-125 is lost.
 // us a launch with its merge on the fp32 instruction / so, 16 heads, D 128: whole sequences of 5376 rows 681 / 488, of 17920 2909 /
 // 1924 (126 / 190 TFLOP/s: 1.14 PFLOP/s of bf16 products, the rate of a large matrix product here, 1.18 to 1.23), 8 chunks of 512 rows on 8
 // cache heads 823 / 570, D 64 390 / 284; relative error against float64 5.7e-7 / 4.6e-7, 8.6e-7 / 6.9e-7, 5.2e-7 / 3.9e-7 and 4.9e-7 / 4.5e-7.
@@ -20,7 +21,8 @@
 //                 one exchange between the lane halves); Q is scaled when it is loaded.
 //   O^T = V^T P^T : P^T is the B operand as it leaves the softmax; V^T comes out of LDS through ds_read_b64_tr_b16.
 // A run with an infinity, a NaN, or a number too large or too small for the split (from the largest bf16 on, in K and Q from 2^60 on; below
-// 2^-100) in a tile or in a row of Q is done again on the fp32 matrix instruction.
+// 2^-100) in a tile or in a row of Q is done again on the fp32 matrix instruction, from the start of the run (a V of 2^-110 in the first / last tile
+// of every sequence, all heads: whole sequences of 5376 rows 501 us without, 574 / 588 with it, 8 chunks 536, 577 / 780, D 64 264, 290 / 324).
 #include "fp_common.h"
 #include "prefill_common.h"
 
