@@ -289,6 +289,8 @@ def compiled_flex_attn_decode(q: Tensor, k: Tensor, v: Tensor, score_mod=None, b
     block_mask._plan_layer = step.layer_id
     arrivals, after = cache._decode_arrivals
     cache._decode_arrivals = after, arrivals
+    if (B > cache.max_batch_size or not own) and B * Hc > arrivals.numel():
+        arrivals = after = None  # more rows or heads than the cache has counters for: in two passes
     got = None
     if q.is_cuda:
         got = N.host().decode(*args, 1.0 / math.sqrt(D) if scale is None else scale, split_tokens, workspace, sinks, kv_rep,

@@ -297,3 +297,25 @@ def test_every_key_counts_once(case, dtype, D, P, G, rep):
     assert ((out.double() - want).abs() <= (STEP[dtype] / 2 + 2.0**-21) * want).all()
     assert torch.equal(torch.isneginf(lse), (n[..., 0] <= 0).expand_as(lse))
     assert ((lse.double() - n[..., 0].clamp(min=1).log()).abs() <= 2.0**-20 * (1 + n[..., 0].clamp(min=1).log()))[pos >= 0].all()
+
+
+def test_more_rows_than_the_cache_has_counters_for():
+    """A batch padded far beyond the cache's slots goes in two passes, as does one over pools of another cache."""
+    dtype, live, B, Hc, G, D, P, ctx = torch.float16, 3, 1030, 8, 2, 64, 64, 4096
+    st, mask, bidx, pos = drop_in_state(live, Hc, D, P, ctx, dtype, 1, [4000, 70, 1500])
+    assert B * Hc > max(len(t) for t in st.cache._decode_arrivals)
+    logical = mask.logical
+    rows = torch.arange(B, device=DEV).clamp(max=live - 1)
+    many = BlockMask.from_kv_blocks(*(getattr(logical, n)[rows] for n in ("kv_num_blocks", "kv_indices", "full_kv_num_blocks", "full_kv_indices")),
+                                    BLOCK_SIZE=logical.BLOCK_SIZE, mask_mod=logical.mask_mod, seq_lengths=(1, ctx))
+    wide = torch.zeros(B, dtype=torch.int64, device=DEV)
+    wide[:live] = bidx
+    pos = torch.cat([pos, torch.zeros(B - live, dtype=torch.int32, device=DEV)])
+    q, k, v = (randn(st.gen, (B, h, 1, D), dtype).to(DEV) for h in (Hc * G, Hc, Hc))
+    k[live:], v[live:] = k[live].clone(), v[live].clone()  # all of them the same padding row
+    K, V = st.cache.insert_kv(0, k, v, input_pos=pos.view(B, 1), batch_idx=wide)
+    for kk, vv in ((K, V), (K.clone(), V.clone())):
+        out, aux = A.compiled_flex_attn_decode(q, kk, vv, block_mask=A.PagedDecodeMask(st.cache, many, wide), return_aux=AuxRequest(lse=True))
+        eo, el = ops.paged_decode(q, K[0], V[0], st.cache.page_table, wide, pos, P, ctx)
+        torch.testing.assert_close(out, eo, rtol=2 * STEP[dtype], atol=1e-5)
+        torch.testing.assert_close(aux.lse.view(el.shape), el, rtol=1e-5, atol=1e-5)
