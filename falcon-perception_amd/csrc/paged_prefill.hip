@@ -74,8 +74,9 @@ struct PrefillArgs {
   fp::PageDiv pd;
   int n_pages, max_batch;
   int64_t n_slots;
-  float qscale;  // scale * log2(e)
-  int n_tiles;   // query tiles
+  int pool_pages;  // n_slots / page_size
+  float qscale;    // scale * log2(e)
+  int n_tiles;     // query tiles
   // key split: grid z = n_key_splits workgroups share a query tile, each taking an equal share of every
   // run's key tiles and leaving unnormalised partial results for the merge pass
   // key shares: a share's result for a row, normalised by its own denominator, in the model dtype (half
@@ -183,10 +184,10 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   __shared__ __attribute__((aligned(1024))) char s_k1[KG * TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) char s_v0[KG * TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) char s_v1[KG * TILE_BYTES];
-  __shared__ int s_bidx[BM];
-  __shared__ int s_red[W];
   __shared__ int s_tslot[kSlotTable];
 
+  // one trip to memory for the arguments: a line of them that no load before has touched is a trip of its own
+  asm volatile("" : : "s"(a.q), "s"(a.batch_idx), "s"(a.Lq), "s"(a.order));
   // linear id = cache head + Hc * tile: all tiles that read one cache head run on the XCD that
   // already holds its K/V in L2
   const int hc = blockIdx.x;
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   // rows see more keys) but not across a packed row of several.
   int tile = a.n_tiles - 1 - blockIdx.y;
   if (a.order) {
-    tile = a.order[blockIdx.y];
+    tile = ((const __attribute__((address_space(4))) int*)a.order)[blockIdx.y];
     tile = tile < 0 ? 0 : tile >= a.n_tiles ? a.n_tiles - 1 : tile;  // whatever the buffer holds, no row outside the launch
   }
   const int tid = threadIdx.x;
@@ -212,42 +213,59 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   const int tile0 = tile * BM;
 
   // Everything the set-up needs from global memory is requested at once, so the loads travel
-  // together: the sequence of each row of the tile, then this wavefront's row limits and Q rows.
-  // Rows outside a run keep their Q values: what such a row computes is never stored.
-  int64_t bx_raw[(BM + kThreads - 1) / kThreads];
+  // together: sequence and limit of every row of the tile (by every wavefront for itself: what follows from them needs no LDS and
+  // no barrier), then this wavefront's row limits and Q rows.  What is in front of the first key tile is a chain of trips to memory and
+  // of scalar instructions, 4 to 8 cycles each, that nothing on the CU hides: 6.9 us a workgroup with limits that went through LDS,
+  // loads under conditions and 64-bit divisions, 5.2 us so (613 rows 20.2 -> 19.2 us a launch, 8 chunks of 512 rows 125 -> 121).
+  // Rows outside a run keep their Q values: what such a row computes is never stored.  Rows past the last one read that one's (a load
+  // under a condition is followed by a wait where the compiler finds something to do with what it brought).
+  constexpr int RJ = (BM + 63) / 64;
+  int row_seq[RJ], row_lim[RJ];  // of tile row j * 64 + lane
+  auto load_rows = [&] {
+    int64_t bx[RJ];
 #pragma unroll
-  for (int j = 0; j < (BM + kThreads - 1) / kThreads; ++j) {
-    const int r = tile0 + j * kThreads + tid;
-    bx_raw[j] = (j * kThreads + tid < BM && r < a.Lq) ? a.batch_idx[r] : 0;
-  }
+    for (int j = 0; j < RJ; ++j) {
+      const int r = min(tile0 + j * 64 + lane, a.Lq - 1);
+      bx[j] = a.batch_idx[r];
+      row_lim[j] = a.row_limit[r];
+    }
+#pragma unroll
+    for (int j = 0; j < RJ; ++j) {
+      const bool in = (BM >= 64 || lane < BM) && tile0 + j * 64 + lane < a.Lq;
+      row_seq[j] = !in || bx[j] < 0 || bx[j] >= a.max_batch ? 0 : static_cast<int>(bx[j]);
+    }
+  };
+  load_rows();
   int row[MB], lim_raw[MB];
   s16x8 qreg[MB][DS];  // Q^T operands: lane (query ln, half) holds d = 16*ds + 8*half .. +8 for every k-step
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     row[mb] = tile0 + (rblock * MB + mb) * 32 + ln;
-    const bool in = row[mb] < a.Lq;
-    lim_raw[mb] = in ? a.row_limit[row[mb]] : 0;
+    const int r = min(row[mb], a.Lq - 1);
+    lim_raw[mb] = a.row_limit[r];
+    const char* const q = a.q + r * a.qs_row + hq * a.qs_h + half * 16;
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) {
-      v4u w = {0, 0, 0, 0};
-      if (in) w = *reinterpret_cast<const v4u*>(a.q + row[mb] * a.qs_row + hq * a.qs_h + (16 * ds + 8 * half) * 2);
-      if constexpr (kBounded) {
-        // bounded scores: Q carries scale * log2(e), so that the matrix product leaves the exponent itself
+    for (int ds = 0; ds < DS; ++ds) qreg[mb][ds] = __builtin_bit_cast(s16x8, *reinterpret_cast<const v4u*>(q + ds * 32));
+  }
+  __builtin_amdgcn_sched_barrier(0);  // all of them are on their way before the first is waited for
+  if constexpr (kBounded) {
+    // page ids of the first run, in the caches by the time Q is there and scaled
+    const int seq0 = __builtin_amdgcn_readlane(row_seq[0], 0);
+    const int64_t page = a.page_table[static_cast<int64_t>(seq0) * a.pt_row_stride + min(lane, a.n_pages - 1)];
+    // bounded scores: Q carries scale * log2(e), so that the matrix product leaves the exponent itself
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int ds = 0; ds < DS; ++ds) {
+        v4u w = __builtin_bit_cast(v4u, qreg[mb][ds]);
 #pragma unroll
         for (int c = 0; c < 4; ++c)
           w[c] = E::pack2(E::to_float(static_cast<short>(w[c] & 0xffffu)) * a.qscale,
                           E::to_float(static_cast<short>(w[c] >> 16)) * a.qscale);
+        qreg[mb][ds] = __builtin_bit_cast(s16x8, w);
       }
-      qreg[mb][ds] = __builtin_bit_cast(s16x8, w);
-    }
+    asm volatile("" : : "v"(page));
   }
-#pragma unroll
-  for (int j = 0; j < (BM + kThreads - 1) / kThreads; ++j) {
-    int64_t bx = bx_raw[j];
-    if (bx < 0 || bx >= a.max_batch) bx = 0;
-    if (j * kThreads + tid < BM) s_bidx[j * kThreads + tid] = static_cast<int>(bx);
-  }
-  __syncthreads();
 
   const char* kplane = a.pool_k + static_cast<int64_t>(hc) * a.n_slots * ROWB;
   const char* vplane = a.pool_v + static_cast<int64_t>(hc) * a.n_slots * ROWB;
@@ -269,18 +287,16 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   while (run0 < BM) {
     // values every lane agrees on are moved to scalar registers so the control flow that
     // depends on them stays uniform
-    const int sq = __builtin_amdgcn_readfirstlane(s_bidx[run0]);
-    // end of the run: the first row of another sequence, found 64 rows at a time
-    int run1 = BM;
-    for (int base = run0; base < BM; base += 64) {
-      const int idx = base + lane;
-      const unsigned long long other = __ballot(idx < BM && s_bidx[idx] != sq);
-      if (other != 0) {
-        run1 = base + __builtin_ctzll(other);
-        break;
-      }
+    int sq = 0, run1 = BM;  // the run's sequence; its end, the first row of another one
+#pragma unroll
+    for (int j = 0; j < RJ; ++j)
+      if (j == run0 >> 6) sq = __builtin_amdgcn_readlane(row_seq[j], run0 & 63);
+#pragma unroll
+    for (int j = RJ - 1; j >= 0; --j) {
+      const int idx = j * 64 + lane;
+      const unsigned long long other = __ballot(idx > run0 && idx < BM && row_seq[j] != sq);
+      if (other != 0) run1 = j * 64 + __builtin_ctzll(other);
     }
-    run1 = __builtin_amdgcn_readfirstlane(run1);
 
     // rows of this wavefront: tile rows rblock * 32 + ln
     int lim[MB];
@@ -313,26 +329,21 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       continue;
     }
 
-    // key range of the run: wavefront maximum, then workgroup maximum
-    int wave_max = my_max;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) wave_max = max(wave_max, __shfl_xor(wave_max, off));
-    wave_max = __builtin_amdgcn_readfirstlane(wave_max);
-    int wave_min = 0x7fffffff;  // smallest limit among the active rows (tiles below it need no masking)
+    // key range of the wavefront's rows (tiles below the smallest limit among them need no masking) and of the run
+    int wave_max = my_max, wave_min = 0x7fffffff, kv_max = 0;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
       if (active[mb]) wave_min = min(wave_min, lim[mb]);
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) wave_min = min(wave_min, __shfl_xor(wave_min, off));
-    wave_min = __builtin_amdgcn_readfirstlane(wave_min);
-    __syncthreads();  // s_red and the LDS tiles of the previous run are free
-    if (lane == 0) s_red[wave] = wave_max;
-    __syncthreads();
-    int kv_max = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) kv_max = max(kv_max, s_red[w]);
-    kv_max = __builtin_amdgcn_readfirstlane(kv_max);
-    const int n_run_tiles = (kv_max + kTileN - 1) / kTileN;
+    for (int j = 0; j < RJ; ++j) {
+      const int idx = j * 64 + lane;
+      if (idx >= run0 && idx < run1) kv_max = max(kv_max, row_lim[j]);
+    }
+    wave_max = fp::wave_max(wave_max);
+    wave_min = -fp::wave_max(-wave_min);
+    kv_max = fp::wave_max(kv_max);
+    const int n_run_tiles = (kv_max + kTileN - 1) >> 6;
+    static_assert(kTileN == 64, "the shift above");
     // Key shares of the run: the grid has as many as may pay, but only the kernel knows how long the run's range is
     const int z = blockIdx.z;
     int n_shares = 1;
@@ -346,9 +357,12 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
         continue;
       }
     }
-    // this workgroup's share of the run's key tiles: [kt_lo, n_kv_tiles)
-    const int kt_lo = static_cast<int>(static_cast<int64_t>(n_run_tiles) * z / n_shares);
-    const int n_kv_tiles = static_cast<int>(static_cast<int64_t>(n_run_tiles) * (z + 1) / n_shares);
+    // this workgroup's share of the run's key tiles: [kt_lo, n_kv_tiles)  (at most 2^25 tiles and 8 shares)
+    int kt_lo = 0, n_kv_tiles = n_run_tiles;
+    if (n_shares > 1) {
+      kt_lo = static_cast<int>(static_cast<uint32_t>(n_run_tiles) * z / n_shares);
+      n_kv_tiles = static_cast<int>(static_cast<uint32_t>(n_run_tiles) * (z + 1) / n_shares);
+    }
     const int n_my = (n_kv_tiles - kt_lo + KG - 1) / KG;  // steps
     const int kt_my = kt_lo + kg;                           // step i of this wavefront works on key tile kt_my + KG * i
 
@@ -373,25 +387,24 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     // runs longer than the table) is staged row by row: a key that does not exist (past the run's
     // last key, or an unmapped page) reads slot 0, finite bytes, and every such key is masked.
     const int64_t* pt_row = a.page_table + static_cast<int64_t>(sq) * a.pt_row_stride;
-    const int64_t pool_pages = a.n_slots / a.pd.page_size;
-    const bool page_holds_tile = kPow2 && a.pd.page_size % kTileN == 0;
+    const bool page_holds_tile = a.pd.page_size % kTileN == 0;
     const int tail_row = (kv_max - 1) % kTileN;  // row of the last key in the last tile
-    for (int t = kt_lo + tid; t < n_kv_tiles && t - kt_lo < kSlotTable; t += kThreads) {
+    auto look_up = [&](int t) {
       int slot = -1;
       if (page_holds_tile) {
         const int key0 = t * kTileN;
         const int blk = key0 >> a.pd.shift;
         if (blk < a.n_pages) {
           const int64_t pg = pt_row[blk];
-          if (pg >= 0 && pg < pool_pages) slot = static_cast<int>(pg) * a.pd.page_size + (key0 & (a.pd.page_size - 1));
+          if (pg >= 0 && pg < a.pool_pages) slot = static_cast<int>(pg) * a.pd.page_size + (key0 & (a.pd.page_size - 1));
           if (slot >= 0 && key0 + kTileN > kv_max) slot = kTailSlot - slot;
         }
       }
-      s_tslot[t - kt_lo] = slot;
-    }
-    __syncthreads();
+      return slot;
+    };
     // first pool slot of tile kt, kTailSlot minus it for the tile with the last key, or -1: wavefront-uniform
     auto tile_slot = [&](int kt) {
+      if constexpr (!kPow2) return -1;
       return __builtin_amdgcn_readfirstlane((kt >= kt_lo && kt < n_kv_tiles && kt - kt_lo < kSlotTable) ? s_tslot[kt - kt_lo] : -1);
     };
 
@@ -433,12 +446,22 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
           key_block(kpos, blkid, off);
           const bool in_range = kpos < kv_max && blkid < a.n_pages;
           const int64_t pg = pt_row[in_range ? blkid : 0];
-          const bool ok = in_range && pg >= 0 && pg < pool_pages;
+          const bool ok = in_range && pg >= 0 && pg < a.pool_pages;
           slot = ok ? static_cast<int>(pg) * a.pd.page_size + off : 0;
         }
         load_to_lds((is_k ? ksrc : vsrc) + static_cast<int64_t>(slot) * ROWB, lds);
       }
     };
+
+    // K of the first tile, whose slot every wavefront looks up for itself, travels while the table is made
+    {
+      const int ts0 = __builtin_amdgcn_readfirstlane(kPow2 && kt_my < n_kv_tiles ? look_up(kt_my) : -1);
+#pragma unroll
+      for (int piece = NI; piece < 2 * NI; ++piece) fetch_piece(piece, kt_my, ts0, s_k0);
+    }
+    if constexpr (kPow2)
+      for (int t = kt_lo + tid; t < n_kv_tiles && t - kt_lo < kSlotTable; t += kThreads) s_tslot[t - kt_lo] = look_up(t);
+    __syncthreads();
 
     // per-lane LDS offsets of the operand reads, the same for every tile and buffer
     int kofs[DS], vofs[DB];
@@ -459,11 +482,6 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     // everywhere, and every wavefront has waited for its loads before B(i + 1), after which M(i + 1)
     // begins.  (A second barrier between the two parts of the interval kept the halves in step more
     // strictly and cost 2 %.)  K(i) lives in K buffer i % 2, V(i) in V buffer i % 2.
-    {
-      const int ts0 = tile_slot(kt_my);
-#pragma unroll
-      for (int piece = NI; piece < 2 * NI; ++piece) fetch_piece(piece, kt_my, ts0, s_k0);  // K of the first tile
-    }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's rows have landed in LDS
 
     s16x8 p_op[MB][4];  // P^T as B operands of the 4 k-steps (16 keys each), from X(i) to M(i + 1)
@@ -771,6 +789,10 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       }
     }
     run0 = run1;
+    if (run0 < BM) {
+      load_rows();
+      __syncthreads();  // the table and the tiles of this run are free
+    }
   }
 }
 
@@ -1139,7 +1161,7 @@ extern "C" int fp_paged_prefill(const void* q, int64_t q_stride_row, int64_t q_s
                 static_cast<const char*>(pool_k), static_cast<const char*>(pool_v),
                 page_table, pt_row_stride, batch_idx, row_limit,
                 static_cast<char*>(out), out_stride_row * 2, out_stride_h * 2, lse, sinks,
-                Lq, Hq, Hc, fp::PageDiv(page_size), n_pages, max_batch, n_slots, scale * kLog2e, 0, nullptr, nullptr,
+                Lq, Hq, Hc, fp::PageDiv(page_size), n_pages, max_batch, n_slots, static_cast<int>(n_slots / page_size), scale * kLog2e, 0, nullptr, nullptr,
                 tile_order, tile_order ? tile_order_rows : 0, 0};
   hipStream_t st = static_cast<hipStream_t>(stream);
   int rc;

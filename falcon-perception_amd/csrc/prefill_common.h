@@ -49,5 +49,15 @@ __device__ __forceinline__ float max_across_lane_halves(float x) {
   return fmaxf(lo, hi);
 }
 
+// Largest x of the wavefront, in scalar registers: lane exchanges inside rows of 16, then one lane of each, no trip through LDS.
+__device__ __forceinline__ int wave_max(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xf, 0xf, true));   // quad_perm [1,0,3,2]
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x4E, 0xf, 0xf, true));   // quad_perm [2,3,0,1]
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x141, 0xf, 0xf, true));  // row_half_mirror
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x140, 0xf, 0xf, true));  // row_mirror
+  return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
+             max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
+}
+
 }  // namespace fp
 #endif
