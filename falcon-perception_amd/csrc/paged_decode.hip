@@ -29,6 +29,7 @@
 //           leave its result where the caller keeps arrival counters.
 #include "decode_common.h"
 #include "paged_decode_mfma.h"
+#include "prefill_common.h"
 
 #include <atomic>
 
@@ -220,6 +221,9 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   __shared__ int s_pages[kMaxSplitPages];
   __shared__ float s_acc[kWaves][G][D];
   __shared__ float s_ml[kWaves][G][2];
+  constexpr int NR = (2 * GK + RPW - 1) / RPW;  // load instructions for the fresh rows, a row to a lane group
+  constexpr bool kEarly = !kFlat && !kPieces;
+  __shared__ __attribute__((aligned(1024))) char s_fresh[kEarly ? NR * 1024 : 16];
 
   // Workgroups are dealt to the 8 XCDs round-robin by linear id.  Heads run fastest:
   // every head of a sequence has the same amount of work, so each XCD gets an equal
@@ -266,8 +270,8 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   // Fused append: the newest token (position L - 1) is not in the pool yet.  The workgroup whose
   // range holds it reads that row from k_new / v_new, folds it in and writes it to its slot; the
   // pool is only read up to L - 2.
-  const bool owns_new = a.k_new != nullptr && !beyond && L - 1 >= t0;  // t1 == L whenever L - 1 lies in this split
-  const int t1_pool = (owns_new && t1 == L) ? t1 - 1 : t1;
+  const bool owns_new = a.k_new != nullptr && !beyond && t1 == L;
+  const int t1_pool = owns_new ? t1 - 1 : t1;
 
   // this lane's 16 bytes of the query row of every head of the group
   typename E::Q q[G];
@@ -289,6 +293,26 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   const int64_t head_stride = a.n_slots * ROWB;
   const char* kbase = a.pool_k + static_cast<int64_t>(kPerHeadK ? hc * G : hc) * head_stride + col * 16;
   const char* vbase = a.pool_v + static_cast<int64_t>(kPerHeadK ? hc * G : hc) * head_stride + col * 16;
+
+  // GK fresh rows of K, then as many of V: V is written to every copy so that the pool stays what the reference's append leaves (the
+  // copies are read by the prefill kernel and by other callers).  Split by split they travel to LDS beside the page ids (kEarly): asked for
+  // behind the other rows they are a trip to memory at the end of a short launch's last splits (one sequence of 711 tokens 8.0 -> 7.6 us a
+  // layer).  Pieces and chunks of many lengths end one after the other anyway, and are no faster for it (16 sequences of 350 to
+  // 4620 tokens 36.7 / 36.9 us, 64 of 1088 to 4096 117.1 / 117.4).
+  const int h0 = kPerHeadK ? hc * G : hc;  // first cache head of this workgroup
+  const auto fresh_row = [&](int r) {
+    return r < GK ? a.k_new + b * a.kn_b + (h0 + r) * a.kn_h : a.v_new + b * a.vn_b + (h0 + r - GK) * a.vn_h;
+  };
+  const bool takes_new = owns_new && wave == (kEarly ? kWaves - 1 : 0);
+  if constexpr (kEarly) {
+    if (takes_new) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) {
+        const int r = grp + j * RPW < 2 * GK ? grp + j * RPW : 2 * GK - 1;
+        fp::load_to_lds(fresh_row(r) + col * 16, s_fresh + j * 1024);
+      }
+    }
+  }
 
   // page ids of the split -> LDS, then the rows
   int64_t blk0;
@@ -343,64 +367,83 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
       fold_rows<E, TPR, G, GK, U, RPW, true>(kreg, vreg, q, a.qscale, c0 + grp, c_end, m, l, acc);
   }
 
-  if (t1_pool != t1 && wave == 0) {
-    // the newest token: one row, held by lane group 0; every other row of this pass is masked
-    v4u kreg[GK][U], vreg[U];
-    const int h0 = kPerHeadK ? hc * G : hc;  // first cache head of this workgroup
-    v4u kn[GK];
+  if (takes_new) {
+    int at = lane;
+    if constexpr (kFlat) asm volatile("" : "+v"(at));  // here and below: what only the end of a piece needs is not kept in registers from piece to piece
+    const int byte = at % TPR * 16;
+    // the newest token: one row, held by lane group 0; the other groups' is masked
+    v4u kreg[GK][1], vreg[1];
+    if constexpr (kEarly) {
+      asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // the fresh rows have landed in LDS
 #pragma unroll
-    for (int gk = 0; gk < GK; ++gk)
-      kn[gk] = *reinterpret_cast<const v4u*>(a.k_new + b * a.kn_b + (h0 + gk) * a.kn_h + col * 16);
-    const v4u vn = *reinterpret_cast<const v4u*>(a.v_new + b * a.vn_b + h0 * a.vn_h + col * 16);
+      for (int gk = 0; gk < GK; ++gk) kreg[gk][0] = *reinterpret_cast<const v4u*>(s_fresh + gk * ROWB + byte);
+      vreg[0] = *reinterpret_cast<const v4u*>(s_fresh + GK * ROWB + byte);
+    } else {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int gk = 0; gk < GK; ++gk) kreg[gk][u] = kn[gk];
-      vreg[u] = vn;
+      for (int gk = 0; gk < GK; ++gk) kreg[gk][0] = *reinterpret_cast<const v4u*>(fresh_row(gk) + byte);
+      vreg[0] = *reinterpret_cast<const v4u*>(fresh_row(GK) + byte);
     }
-    fold_rows<E, TPR, G, GK, U, RPW, true>(kreg, vreg, q, a.qscale, t1 - 1 + grp, t1, m, l, acc);
-    if (grp == 0) {
+    fold_rows<E, TPR, G, GK, 1, RPW, true>(kreg, vreg, q, a.qscale, t1 - 1 + at / TPR, t1, m, l, acc);
+    if (at < TPR) {
       int64_t blk;
       int off;
       a.pd.split(t1 - 1, blk, off);
       const int64_t slot = static_cast<int64_t>(pages_lds[blk - blk0]) * a.pd.page_size + off;
 #pragma unroll
       for (int gk = 0; gk < GK; ++gk) {
-        // every cached head gets its K row; V is written to every copy so the pool stays what the
-        // reference's append leaves (the copies are read by the prefill kernel and by other callers)
-        __builtin_nontemporal_store(kn[gk], reinterpret_cast<v4u*>(const_cast<char*>(kbase) + gk * head_stride + slot * ROWB));
-        const v4u vrow = kPerHeadK ? *reinterpret_cast<const v4u*>(a.v_new + b * a.vn_b + (h0 + gk) * a.vn_h + col * 16) : vn;
+        __builtin_nontemporal_store(kreg[gk][0], reinterpret_cast<v4u*>(const_cast<char*>(kbase) + gk * head_stride + slot * ROWB));
+        v4u vrow = vreg[0];
+        if constexpr (kEarly && GK > 1)
+          vrow = *reinterpret_cast<const v4u*>(s_fresh + (GK + gk) * ROWB + byte);
+        else if constexpr (GK > 1)
+          vrow = *reinterpret_cast<const v4u*>(fresh_row(GK + gk) + byte);
         __builtin_nontemporal_store(vrow, reinterpret_cast<v4u*>(const_cast<char*>(vbase) + gk * head_stride + slot * ROWB));
       }
     }
   }
 
-  // combine the lane groups of this wavefront
+  // combine the lane groups of this wavefront: every state at the common maximum, then the sums.  Each exchange between the lane
+  // halves, and between rows of 16 lanes, adds up two elements at once and leaves one of them in either part, so that a lane
+  // ends with a part of the elements.  (An exchange through LDS for every element and group was 0.8 us at the end of every piece; 0.2 us so.)
+  constexpr int N = G * EPL;
+  float sum[N];
 #pragma unroll
-  for (int off = TPR; off < 64; off <<= 1) {
+  for (int g = 0; g < G; ++g) {
+    float mx = m[g];
+    if (TPR <= 8) mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror:8
+    if (TPR <= 16) mx = max_across_rows(mx);
+    if (TPR <= 32) mx = max_across_halves(mx);
+    const float w = fast_exp2(m[g] - safe_max(mx));
+    m[g] = mx;
+    l[g] *= w;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const float mo = __shfl_xor(m[g], off);
-      const float lo = __shfl_xor(l[g], off);
-      const float mn = fmaxf(m[g], mo);
-      const float ms = safe_max(mn);
-      const float wa = fast_exp2(m[g] - ms);
-      const float wb = fast_exp2(mo - ms);
-      l[g] = l[g] * wa + lo * wb;
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) acc[g][e] = acc[g][e] * wa + __shfl_xor(acc[g][e], off) * wb;
-      m[g] = mn;
-    }
+    for (int e = 0; e < EPL; ++e) sum[g * EPL + e] = acc[g][e] * w;
   }
-  if (lane < TPR) {
+  if (TPR <= 8) {
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
+    for (int i = 0; i < N; ++i) sum[i] += dpp<0x128>(sum[i]);
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) s_acc[wave][g][col * EPL + e] = acc[g][e];
-      if (lane == 0) {
-        s_ml[wave][g][0] = m[g];
-        s_ml[wave][g][1] = l[g];
-      }
+    for (int g = 0; g < G; ++g) l[g] += dpp<0x128>(l[g]);
+  }
+  if (TPR <= 32) add_across_halves<N>(sum);
+  if (TPR <= 16) add_across_rows<N / 2>(sum);
+  constexpr int NL = TPR <= 16 ? N / 4 : TPR <= 32 ? N / 2 : N;  // elements this lane ends with, from `held` on
+  int at = lane;
+  if constexpr (kFlat) asm volatile("" : "+v"(at));
+  const int held = (TPR <= 32 ? (at >> 5) * (N / 2) : 0) + (TPR <= 16 ? (at >> 4 & 1) * (N / 4) : 0);
+  static_assert(NL % EPL == 0 || EPL % NL == 0, "either whole heads or a part of one");
+  float* const to = &s_acc[wave][held / EPL][at % TPR * EPL + held % EPL];
+  if (TPR > 8 || (at & 8) == 0) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) to[i / EPL * D + i % EPL] = sum[i];
+  }
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    if (TPR <= 16) l[g] = sum_across_rows(l[g]);
+    if (TPR <= 32) l[g] = sum_across_halves(l[g]);
+    if (lane == 0) {
+      s_ml[wave][g][0] = m[g];
+      s_ml[wave][g][1] = l[g];
     }
   }
   __syncthreads();
@@ -861,22 +904,13 @@ int merged_pieces(int Hc, int B, int n_splits, int max_context, int page_size) {
   return longest / page_size + 2 <= kMaxSplitPages ? static_cast<int>(pieces) : 0;
 }
 
-// Workgroups of the even-cut kernel the current device holds at once (asked once per kernel and device).
-template <typename E, int D, int G, bool kAligned, bool kPerHeadK>
-int resident_workgroups() {
-  const auto kernel = paged_decode_kernel<E, D, G, false, kAligned, kPerHeadK, true>;
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cached[dev] == 0) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, 0) != hipSuccess || per_cu <= 0) {
-      (void)hipGetLastError();  // not an error of the launch that follows
-      cached[dev] = -1;
-    } else
-      cached[dev] = per_cu * fp::compute_units();
-  }
-  return cached[dev] > 0 ? cached[dev] : 0;
+// Workgroups to a CU beyond which a launch is always cut evenly: as many as the even-cut kernel's registers let a CU hold when the
+// sweeps at even_cut_pays and merged_pieces were made.  Numbers, so that a kernel that needs fewer registers does not move the line.
+template <typename E, int D, int G, bool kPerHeadK>
+constexpr int workgroups_held(bool aligned) {
+  const bool narrow = sizeof(typename E::type) == 2;
+  if (kPerHeadK) return narrow ? (G == 2 && !aligned ? 3 : 2) : (D == 128 && aligned ? 2 : 3);
+  return G == 1 ? 4 : G == 2 ? 3 : G == 4 || (D == 64 && aligned) ? 2 : 1;
 }
 
 // Launches with four or more query heads per cache head in a 16-bit type run on the matrix cores.  us a layer on the vector
@@ -929,7 +963,7 @@ void launch_decode(const DecodeArgs& a0, int B, int phases, hipStream_t st) {
     if constexpr (on_matrix_cores<E, G, kPerHeadK>())
       resident = 3 * fp::compute_units();
     else
-      resident = aligned ? resident_workgroups<E, D, G, true, kPerHeadK>() : resident_workgroups<E, D, G, false, kPerHeadK>();
+      resident = workgroups_held<E, D, G, kPerHeadK>(aligned) * fp::compute_units();
     const int pieces = a.arrivals ? merged_pieces(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size) : 0;
     DecodeArgs ap = a;
     ap.n_chunks = pieces;
