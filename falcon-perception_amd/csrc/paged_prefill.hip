@@ -272,11 +272,15 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
 
   // ---- per-lane constants of the staging loads and of the operand reads ----
   // load instruction i of this wavefront fills LDS rows (i * ITEMS + item) * RPI .. + RPI; this lane
-  // fills position lp of row lrow in that group.  kswz / vrot of the row do not depend on i.
+  // fills position lp of row lrow in that group.
   const int lrow = lane / CPR;
   const int lp = lane % CPR;
   const int st_row0 = item * RPI + lrow;  // row of load instruction 0; instruction i adds i * ITEMS * RPI
+  // kswz of the row does not depend on i where an instruction of all staging wavefronts is 16 rows or more; where it is 8, every
+  // second one flips the chunk's highest bit.  vrot has a period of 4 rows.
+  static_assert(ITEMS * RPI % 16 == 0 || (ITEMS * RPI == 8 && CPR == 16), "the permutation of a lane's rows");
   const int k_src_off = (lp ^ SW::kswz(st_row0)) * 16;
+  const auto k_flip = [](int i) { return ITEMS * RPI == 8 ? (i & 1) * 128 : 0; };
   const int v_src_off = ((((lp >> 1) + R32 - SW::vrot(st_row0)) % R32) * 2 + (lp & 1)) * 16;
   // K operand: row kb * 32 + ln, chunk 2 * ds + half at position (2 * ds) ^ ksel
   const int ksel = half ^ SW::kswz(ln);
@@ -417,12 +421,11 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
         off = kpos - blkid * a.pd.page_size;
       }
     };
-    const char* ksrc = kplane + k_src_off;
     const char* vsrc = vplane + v_src_off;
     uint32_t lane_k[NI], lane_v[NI];  // byte offset of this lane's 16 bytes from the first row of a tile
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      lane_k[i] = (i * ITEMS * RPI + st_row0) * ROWB + k_src_off;
+      lane_k[i] = (i * ITEMS * RPI + st_row0) * ROWB + (k_src_off ^ k_flip(i));
       lane_v[i] = (i * ITEMS * RPI + st_row0) * ROWB + v_src_off;
     }
     // One staging load of tile kt, whose table entry is ts: pieces 0 .. NI - 1 are the V loads
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
           const bool ok = in_range && pg >= 0 && pg < a.pool_pages;
           slot = ok ? static_cast<int>(pg) * a.pd.page_size + off : 0;
         }
-        load_to_lds((is_k ? ksrc : vsrc) + static_cast<int64_t>(slot) * ROWB, lds);
+        load_to_lds((is_k ? kplane + (k_src_off ^ k_flip(i)) : vsrc) + static_cast<int64_t>(slot) * ROWB, lds);
       }
     };
 
@@ -969,6 +972,20 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   // 32.6, 40.5 / 34.5, 44.1 / 40.3 and 52.7 / 50.9.  Short prompts without a merge, back to back, D 128 and 64: 59 rows 13.1 / 10.8 and 10.5 / 8.0,
   // 170 rows 18.8 / 13.0 and 13.7 / 9.4, 613 rows 24.3 / 18.4 and 16.7 / 13.3.  Not the better one at 129 to 170 workgroups over 3000 keys
   // and more, which leave no room for a second share (640 rows of 32 q / 8 kv heads: 56.5 / 61.4; over 1400 keys 44.2 / 42.1).
+  // With one query head per cache head, head_dim 128 and bounded scores workgroups of half as many rows again (four wavefronts, each
+  // alone on its SIMD) are the better ones where these, too, fit the GPU in one go: a step is shorter without a second wavefront's
+  // matrix instructions, and a tile holds fewer runs.  us a layer with its insert, eight wavefronts / four: 613 rows 24.0 / 23.2, three prompts
+  // of 120 to 260 rows 20.5 / 18.3, 1000 rows on 8 heads 27.6 / 27.7.  Two query heads to a cache head 22.7 / 23.2, the running maximum
+  // 24.7 / 25.2: the tiles are staged twice as often, and there is less time to hide it in.
+  if constexpr (G == 1 && D == 128 && std::is_same<E, BF16>::value) {
+    constexpr int BM4 = 64;
+    if (shares == 1 && halves && bounded && static_cast<int64_t>(a.Hc) * ((a.Lq + BM4 - 1) / BM4) <= fp::compute_units()) {
+      a.n_tiles = (a.Lq + BM4 - 1) / BM4;
+      a.order = nullptr;
+      launch_instance<E, D, G, true, 4, true, 2>(a, dim3(a.Hc, a.n_tiles, 1), st);  // halves: pages hold whole tiles
+      return;
+    }
+  }
   if constexpr (G <= 4) {
     constexpr int BM2 = (kWaves / 2 / G) * 32;
     if (halves) {
