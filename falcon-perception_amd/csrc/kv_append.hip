@@ -48,9 +48,25 @@ struct AppendArgs {
   int64_t n_slots;
   int clamp_negative;
   int64_t item0;  // first item of this launch: a launch holds fewer than 2^32 lanes, a larger append is several
+  int tok_shift;    // lanes per token (token-major: H * chunks, else chunks) and per row as powers of two, or -1
+  int chunk_shift;
 };
 
 constexpr int kThreads = 256;
+
+// Slot of position pos of slot row b, or -1: none.
+__device__ __forceinline__ int64_t slot_of(const AppendArgs& a, int64_t b, int64_t pos) {
+  if (b < 0 || b >= a.max_batch || pos < 0) return -1;
+  int64_t blk;
+  int off;
+  a.pd.split(pos, blk, off);
+  if (blk >= a.n_pages) return -1;
+  int64_t page = a.page_table[b * a.pt_row_stride + blk];
+  if (a.clamp_negative && page < 0) page = 0;
+  int64_t slot = page * a.pd.page_size + off;
+  if (slot < 0) slot += a.n_slots;  // negative index counts from the end of the slot axis
+  return slot < a.n_slots ? slot : -1;
+}
 
 // One 16-byte vector of K and one of V per lane.  kTokenMajor: lanes run over (token, head, chunk), the
 // order of a [T, H, D] source, so a load instruction reads consecutive source bytes and every row leaves
@@ -59,16 +75,29 @@ constexpr int kThreads = 256;
 // the item count allows (one division per lane instead of a 64-bit one).
 template <typename Vec, bool kTokenMajor, typename Idx>
 __global__ __launch_bounds__(kThreads) void kv_append_kernel(const AppendArgs a, int H) {
+  // A launch of few rows is bound by what is in front of its stores (613 rows x 16 heads in front of their attention launch, 28 layers: 655 -> 648 us a step): one trip to memory
+  // for the arguments (each is otherwise asked for where it is first used, and a line of 64 bytes that no load before it touched is a trip of its
+  // own) and shifts in the place of divisions.
+  asm volatile("" : : "s"(a.pool_k), "s"(a.vs_t), "s"(a.max_batch), "s"(a.item0), "s"(a.chunk_shift));
   const Idx per_tok = kTokenMajor ? static_cast<Idx>(H) * a.chunks : static_cast<Idx>(a.chunks);
   const Idx items = static_cast<Idx>(a.n_tok) * per_tok;
   const Idx i = static_cast<Idx>(a.item0) + static_cast<Idx>(blockIdx.x) * kThreads + threadIdx.x;
   if (i >= items) return;
-  const int tok = static_cast<int>(i / per_tok);
-  int c = static_cast<int>(i - static_cast<Idx>(tok) * per_tok);
-  int h = blockIdx.y;
-  if (kTokenMajor) {
-    h = c / a.chunks;
-    c -= h * a.chunks;
+  int tok, c, h = blockIdx.y;
+  if (a.tok_shift >= 0) {
+    tok = static_cast<int>(i >> a.tok_shift);
+    c = static_cast<int>(i) & ((1 << a.tok_shift) - 1);
+    if (kTokenMajor) {
+      h = c >> a.chunk_shift;
+      c &= (1 << a.chunk_shift) - 1;
+    }
+  } else {
+    tok = static_cast<int>(i / per_tok);
+    c = static_cast<int>(i - static_cast<Idx>(tok) * per_tok);
+    if (kTokenMajor) {
+      h = c / a.chunks;
+      c -= h * a.chunks;
+    }
   }
   int t = tok, s = 0;
   if (a.S != 1) {
@@ -80,18 +109,8 @@ __global__ __launch_bounds__(kThreads) void kv_append_kernel(const AppendArgs a,
   const Vec kreg = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(a.k + ko));
   const Vec vreg = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(a.v + vo));
 
-  const int64_t b = a.batch_idx[t];
-  const int64_t pos = fp::load_index(a.input_pos, tok, a.pos_i64);
-  if (b < 0 || b >= a.max_batch || pos < 0) return;
-  int64_t blk;
-  int off;
-  a.pd.split(pos, blk, off);
-  if (blk >= a.n_pages) return;
-  int64_t page = a.page_table[b * a.pt_row_stride + blk];
-  if (a.clamp_negative && page < 0) page = 0;
-  int64_t slot = page * a.pd.page_size + off;
-  if (slot < 0) slot += a.n_slots;  // negative index counts from the end of the slot axis
-  if (slot < 0 || slot >= a.n_slots) return;
+  const int64_t slot = slot_of(a, a.batch_idx[t], fp::load_index(a.input_pos, tok, a.pos_i64));
+  if (slot < 0) return;
   const int64_t dst = (static_cast<int64_t>(h) * a.n_slots + slot) * a.row_bytes + static_cast<int64_t>(c) * sizeof(Vec);
   __builtin_nontemporal_store(kreg, reinterpret_cast<Vec*>(a.pool_k + dst));
   __builtin_nontemporal_store(vreg, reinterpret_cast<Vec*>(a.pool_v + dst));
@@ -109,6 +128,10 @@ int launch(const AppendArgs& a0, int H, hipStream_t stream) {
   const int64_t blocks = (per_grid_row + kThreads - 1) / kThreads;
   const bool narrow = per_grid_row + kThreads < (1ll << 32);
   AppendArgs a = a0;
+  const int64_t per_tok = static_cast<int64_t>(a.chunks) * (token_major ? H : 1);
+  const auto shift_of = [](int64_t n) { return (n & (n - 1)) == 0 && n < (1 << 30) ? __builtin_ctzll(n) : -1; };
+  a.chunk_shift = shift_of(a.chunks);
+  a.tok_shift = a.chunk_shift >= 0 ? shift_of(per_tok) : -1;
   for (int64_t b0 = 0; b0 < blocks; b0 += kLaunchBlocks) {
     a.item0 = b0 * kThreads;
     const int64_t nb = blocks - b0 < kLaunchBlocks ? blocks - b0 : kLaunchBlocks;
@@ -159,7 +182,7 @@ extern "C" int fp_kv_append(void* pool_k, void* pool_v, const void* k, const voi
                v_stride_t * eb, v_stride_h * eb, v_stride_s * eb,
                page_table, pt_row_stride, batch_idx, input_pos,
                pos_index_type == FP_INDEX_I64, T * S, S, 0, D * eb, fp::PageDiv(page_size),
-               n_pages, max_batch, n_slots, clamp_negative, 0};
+               n_pages, max_batch, n_slots, clamp_negative, 0, -1, -1};
 
   // widest vector every row address is a multiple of
   int vec = 16;
