@@ -32,6 +32,7 @@
 #include <hip/hip_fp16.h>
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -890,6 +891,9 @@ int uncut_tiles(int Lq, int Hq, bool halves) {
   return static_cast<int>(halves ? 5 + items / 1500 : 4 + items / 4000);
 }
 
+// Key tiles up to which workgroups of 64 rows may be the better ones (launch_group)
+constexpr int kShortRange = 13;
+
 // workspace of `shares` key shares: per row and head D results of elem bytes, and two floats
 int64_t share_bytes(int shares, int Lq, int Hq, int D, int elem) {
   return shares <= 1 ? 0 : static_cast<int64_t>(shares) * Lq * Hq * (static_cast<int64_t>(D) * elem + 8);
@@ -973,13 +977,21 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   // 170 rows 18.8 / 13.0 and 13.7 / 9.4, 613 rows 24.3 / 18.4 and 16.7 / 13.3.  Not the better one at 129 to 170 workgroups over 3000 keys
   // and more, which leave no room for a second share (640 rows of 32 q / 8 kv heads: 56.5 / 61.4; over 1400 keys 44.2 / 42.1).
   // With one query head per cache head, head_dim 128 and bounded scores workgroups of half as many rows again (four wavefronts, each
-  // alone on its SIMD) are the better ones where these, too, fit the GPU in one go: a step is shorter without a second wavefront's
-  // matrix instructions, and a tile holds fewer runs.  us a layer with its insert, eight wavefronts / four: 613 rows 24.0 / 23.2, three prompts
-  // of 120 to 260 rows 20.5 / 18.3, 1000 rows on 8 heads 27.6 / 27.7.  Two query heads to a cache head 22.7 / 23.2, the running maximum
-  // 24.7 / 25.2: the tiles are staged twice as often, and there is less time to hide it in.
+  // alone on its SIMD) are the better ones where these, too, fit the GPU in one go and no row sees more keys than kShortRange and
+  // uncut_tiles say (what the table has columns for: a caller that knows the longest sequence passes no more): their set-up is
+  // shorter and a tile holds fewer runs, but a pair of key tiles takes longer (1.9 us instead of 1.6: no second wavefront on the SIMD hides a
+  // wavefront's softmax).  us a launch, 16 heads, eight wavefronts / four: 64 rows over 64, 320, 576 and 1400 keys 9.9 / 8.9, 13.0 / 12.5,
+  // 15.9 / 16.2 and 26.0 / 29.2; 200 over 200, 448 and 704 12.7 / 11.0, 15.5 / 15.0 and 18.2 / 18.6; 400 over 400 and 832 15.3 / 14.2 and 21.0 / 20.3;
+  // 613 over 613, 704, 832 and 4600 17.9 / 16.8, 18.8 / 18.8, 20.1 / 20.4 and 64.0 / 74.3; 1000 over 1000 and 1216 22.8 / 22.5 and 24.7 / 26.1;
+  // four of 75, of 153 and of 250 rows 22.2 / 14.7, 19.0 / 16.5 and 19.0 / 17.0; at the end of the range eight of 100 over 822 48.8 / 37.0, two and four of 100 to 200
+  // over 566 26.9 / 27.4 and 28.6 / 28.9, past it eight of 125 over 950 38.4 / 39.8.  Eight and four heads the same.  Two query heads to a
+  // cache head (us a layer with its insert) 22.7 / 23.2, the running maximum 24.7 / 25.2: the tiles are staged twice as often, and there is less time
+  // to hide it in.  Head_dim 64 is not compiled so; a trial gave 64, 200 and 613 rows 6.9 / 6.6, 8.9 / 8.0 and 12.5 / 11.3, 64 over 1400 keys 18.4 / 18.7.
   if constexpr (G == 1 && D == 128 && std::is_same<E, BF16>::value) {
     constexpr int BM4 = 64;
-    if (shares == 1 && halves && bounded && static_cast<int64_t>(a.Hc) * ((a.Lq + BM4 - 1) / BM4) <= fp::compute_units()) {
+    const int short_tiles = std::min(uncut_tiles(a.Lq, a.Hq, true), kShortRange);
+    if (shares == 1 && halves && bounded && static_cast<int64_t>(a.Hc) * ((a.Lq + BM4 - 1) / BM4) <= fp::compute_units() &&
+        static_cast<int64_t>(a.n_pages) * a.pd.page_size <= short_tiles * kTileN) {
       a.n_tiles = (a.Lq + BM4 - 1) / BM4;
       a.order = nullptr;
       launch_instance<E, D, G, true, 4, true, 2>(a, dim3(a.Hc, a.n_tiles, 1), st);  // halves: pages hold whole tiles

@@ -136,6 +136,7 @@ class HybridPrefillMask:
         self._step_layer = -1  # layer that asked last: a layer id that does not grow starts a new step
         self._row_limit = None
         self.most_keys = 0  # no row of the step sees more keys than this: the longest sequence the cache holds
+        self._short_table = None  # the columns of the page table that hold so many, where `short_table` was asked for them
         self._tile_orders: dict[int, tuple[Tensor, int]] = {}  # rows per tile -> tile order of the step's limits
 
     def _limits_from_ids(self, open_spans, validate) -> Tensor:
@@ -182,8 +183,17 @@ class HybridPrefillMask:
             self._step_key = key
             self._tile_orders = {}
             self.most_keys = max(self.cache.capacity)
+            self._short_table = None
         self._step_layer = layer_id
         return self._row_limit
+
+    def short_table(self) -> Tensor:
+        """The page table with no more columns than the longest sequence of the step's cache has pages, made by the first layer that
+        asks after `row_limit`: the width of the table is what a launch knows of the key ranges of its rows."""
+        if self._short_table is None:
+            table, pages = self.cache.page_table, -(-self.most_keys // self.cache.page_size)
+            self._short_table = table[:, :pages] if 0 < pages < table.shape[1] else table
+        return self._short_table
 
     def tile_order(self, batch_idx: Tensor, tile_rows: int) -> tuple[Tensor, int]:
         """Query tiles of the step by decreasing key range (`ops.prefill_tile_order`), made by the first layer
@@ -337,8 +347,10 @@ def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, 
         rows = cache.prefill_tile_rows(Lq, Hq, D, pool_k.shape[0], q.dtype, workspace.numel() if workspace is not False else 0)
         if rows and -(-Lq // rows) <= 4096:
             order = block_mask.tile_order(step.batch_idx, rows)
-    args = (q, pool_k, pool_v, cache.page_table, step.batch_idx, limits, cache.page_size)
     bound = cache.score_bound(D, scale)
+    # head_dim 128, a bound and no workspace: launches of few rows over few keys have workgroups of their own
+    table = block_mask.short_table() if bound and D == 128 and workspace is False else cache.page_table
+    args = (q, pool_k, pool_v, table, step.batch_idx, limits, cache.page_size)
     got = None
     if q.is_cuda:
         got = N.host().prefill(*args, 1.0 / math.sqrt(D) if scale is None else scale, sinks, None if workspace is False else workspace,

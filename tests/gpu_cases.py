@@ -80,3 +80,15 @@ class PagedState:
 def check_tables_match(state: PagedState):
     assert state.cache.page_table.cpu().numpy().tolist() == state.mirror.page_table.tolist()
     assert state.cache.physical_to_logical.cpu().numpy().tolist() == state.mirror.physical_to_logical.tolist()
+
+
+def kernels(run) -> list[str]:
+    """Names of the library's kernels that `run` launches, as the profiler sees them: which way a launch goes."""
+    from torch.profiler import ProfilerActivity, profile
+
+    run()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA], acc_events=True) as seen:
+        run()
+        torch.cuda.synchronize()
+    return [e.name.replace("(anonymous namespace)::", "") for e in seen.events() if "paged_" in e.name]

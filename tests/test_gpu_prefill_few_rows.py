@@ -10,7 +10,7 @@ from torch.nn.attention.flex_attention import AuxRequest
 from falcon_perception_amd import attention as A
 from falcon_perception_amd import ops
 from oracle import paged_kv_oracle as O
-from tests.gpu_cases import DEV, PagedState, f64, randn
+from tests.gpu_cases import DEV, PagedState, f64, kernels, randn
 from tests.test_gpu_prefill_key_shares import TOL, make_case
 
 pytestmark = pytest.mark.gpu
@@ -133,4 +133,59 @@ def test_a_prompt_does_not_depend_on_who_else_is_cached(rows):
         results.append((out, aux.lse))
         used.append(cache.prefill_workspace(L, Hc, D, Hc, dtype, mask.most_keys) is not False)
     assert used == [False, True]
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
+FOUR, EIGHT = ("paged_prefill_kernel<BF16, 128, 1, true, %d, true, 2>" % w for w in (4, 8))
+
+
+@pytest.mark.parametrize("lens,pages,rows", [
+    ([320], 5, 64), ([320], 6, 64), ([1464], 23, 64), ([613], 11, 613), ([613], 12, 613), ([704], 11, 613), ([1400], 22, 613),
+    ([832], 13, 832), ([832], 14, 832), ([500, 500], 13, 1000), ([500, 500], 14, 1000), ([1000], 16, 1000)], ids=str)
+def test_workgroups_of_64_rows_are_for_short_ranges(lens, pages, rows):
+    """What a launch knows of the rows' key ranges is the width of the page table.  Over long ranges workgroups of 64 rows are the
+    slower ones (64 rows over 1400 keys 29.2 us instead of 26.0), also without a workspace; the bits are the same."""
+    dtype, P, heads = torch.bfloat16, 64, 8
+    st, q, bidx, lim = make_case(dtype, 128, 1, P, lens=lens, pads=[0] * len(lens))
+    q, bidx, lim = (q[:, :, -rows:] / 3).repeat(1, heads, 1, 1).to(DEV), bidx[-rows:].contiguous(), lim[-rows:].contiguous()
+    pk, pv = (x.repeat(heads, 1, 1) for x in st.pool_planes())
+    table = st.cache.page_table
+    wide = torch.cat([table, torch.full_like(table, -1), torch.full_like(table, -1)], 1)
+    short = 64 * min(5 + rows * 16 // 1500, 13)
+
+    def run(columns):
+        return ops.paged_prefill(q, pk, pv, wide[:, :columns], bidx, lim, P, workspace=False, score_bound=39.0)
+
+    assert wide.shape[1] * P > short and pages <= wide.shape[1]
+    ways = [kernels(lambda c=c: run(c)) for c in (pages, wide.shape[1])]
+    assert [len(w) for w in ways] == [1, 1]
+    assert (FOUR if pages * P <= short else EIGHT) in ways[0][0] and EIGHT in ways[1][0]
+    (out, lse), (out2, lse2) = run(pages), run(wide.shape[1])
+    assert torch.equal(out, out2) and torch.equal(lse, lse2)
+
+
+def test_the_drop_in_says_how_long_its_sequences_are():
+    """A prompt in a cache whose table has columns for 8192 tokens; the same prompt once a sequence of 6000 tokens is cached."""
+    dtype, Hc, D, P, rows = torch.bfloat16, 16, 128, 128, 613
+    st = PagedState(19, n_pages=64, page_size=P, max_batch=4, Hc=Hc, D=D, dtype=dtype)
+    cache, L = st.cache, 640
+    cache.qk_normalised = True
+    slot, results = st.add_sequence(rows), []
+    q, k, v = (randn(st.gen, (1, Hc, L, D), dtype).to(DEV) for _ in range(3))
+    q = q / 3
+    live = torch.arange(L, device=DEV)[None] < rows
+    bidx, pos = torch.where(live, slot, 0), torch.where(live, torch.arange(L, device=DEV)[None], 0)
+    for way in ([FOUR], [EIGHT, "paged_prefill_merge_kernel"]):
+
+        def run():
+            mask = cache.create_prefill_blockmask(bidx, torch.full_like(bidx, 9), 1, 2)
+            K, V = cache.insert_kv(0, k, v, input_pos=pos, batch_idx=bidx)
+            return A.compiled_flex_attn_prefill(q, K, V, block_mask=mask, return_aux=AuxRequest(lse=True))
+
+        seen = [n for n in kernels(run) if "paged_prefill" in n]
+        assert len(seen) == len(way) and all(w in n for w, n in zip(way, seen))
+        out, aux = run()
+        results.append((out, aux.lse))
+        if len(results) == 1:
+            st.add_sequence(6000)
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
