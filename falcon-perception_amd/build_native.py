@@ -65,7 +65,7 @@ def _compile(src: str) -> str:
 
 def resource_usage() -> dict[str, dict[str, int]]:
     """Per kernel of the last build: {"vgprs", "agprs", "scratch" (bytes per lane), "lds" (bytes per workgroup),
-    "occupancy" (wavefronts per SIMD)}, keyed by the mangled kernel name; builds first if nothing has been
+    "occupancy" (wavefronts per SIMD), "sgprs_moved" (scalar registers kept in lanes of vector registers)}, keyed by the mangled kernel name; builds first if nothing has been
     built.  A kernel with scratch > 0 spills registers to memory; the first launch of such a kernel makes the
     runtime set that memory up, which it cannot do while a stream is being captured into a graph."""
     names = [os.path.join(OBJ_DIR, os.path.basename(s)[:-4] + ".resources.txt") for s in sources()]
@@ -73,7 +73,8 @@ def resource_usage() -> dict[str, dict[str, int]]:
         build_library(verbose=False)
     out: dict[str, dict[str, int]] = {}
     fields = {"vgprs": r"VGPRs: (\d+)", "agprs": r"AGPRs: (\d+)", "scratch": r"ScratchSize \[bytes/lane\]: (\d+)",
-              "lds": r"LDS Size \[bytes/block\]: (\d+)", "occupancy": r"Occupancy \[waves/SIMD\]: (\d+)"}
+              "lds": r"LDS Size \[bytes/block\]: (\d+)", "occupancy": r"Occupancy \[waves/SIMD\]: (\d+)",
+              "sgprs_moved": r"SGPRs Spill: (\d+)"}
     for n in names:
         with open(n) as f:
             text = f.read()

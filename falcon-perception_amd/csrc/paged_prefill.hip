@@ -186,6 +186,8 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   __shared__ __attribute__((aligned(1024))) char s_v0[KG * TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) char s_v1[KG * TILE_BYTES];
   __shared__ int s_tslot[kSlotTable];
+  const uint32_t lds_k0 = fp::lds_address(s_k0), lds_k1 = fp::lds_address(s_k1);
+  const uint32_t lds_v0 = fp::lds_address(s_v0), lds_v1 = fp::lds_address(s_v1);
 
   // one trip to memory for the arguments: a line of them that no load before has touched is a trip of its own
   asm volatile("" : : "s"(a.q), "s"(a.batch_idx), "s"(a.Lq), "s"(a.order));
@@ -222,11 +224,20 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   // under a condition is followed by a wait where the compiler finds something to do with what it brought).
   constexpr int RJ = (BM + 63) / 64;
   int row_seq[RJ], row_lim[RJ];  // of tile row j * 64 + lane
+  // What only the beginning or the end of a run needs is worked out there: the addresses, two registers each, would be kept through
+  // the tile loop (at head_dim 64, where three workgroups share a CU, in scratch memory: 20 to 44 bytes a lane).  Together with the
+  // buffers' addresses in LDS as numbers, us a launch with bounded scores: 256 rows of 16 heads over 16000 keys, D 128, without a workspace
+  // 201 -> 184, 600 over 4000 64.4 -> 59.4; D 64, 24 prompts of 100 to 700 rows 29.7 -> 28.0; 8 chunks of 512 rows over 256 to 4096 72.1 -> 70.1.
+  const auto anew = [](int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+  };
   auto load_rows = [&] {
     int64_t bx[RJ];
+    const int at = anew(lane);
 #pragma unroll
     for (int j = 0; j < RJ; ++j) {
-      const int r = min(tile0 + j * 64 + lane, a.Lq - 1);
+      const int r = min(tile0 + j * 64 + at, a.Lq - 1);
       bx[j] = a.batch_idx[r];
       row_lim[j] = a.row_limit[r];
     }
@@ -321,13 +332,14 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         if (!active[mb] || kg != 0 || blockIdx.z != 0) continue;
+        const int r = anew(row[mb]);
         // a row is 2 * D bytes; each lane half clears D of them
-        char* o = a.out + row[mb] * a.os_row + hq * a.os_h + half * D;
+        char* o = a.out + r * a.os_row + hq * a.os_h + half * D;
 #pragma unroll
         for (int c = 0; c < D / 8; ++c) *reinterpret_cast<uint2*>(o + c * 8) = uint2{0, 0};
         if (half == 0) {
-          a.lse[static_cast<int64_t>(hq) * a.Lq + row[mb]] = -INFINITY;
-          if (gridDim.z > 1) a.ws_ml[(static_cast<int64_t>(row[mb]) * a.Hq + hq) * 2 + 1] = kRowFinished;
+          a.lse[static_cast<int64_t>(hq) * a.Lq + r] = -INFINITY;
+          if (gridDim.z > 1) a.ws_ml[(static_cast<int64_t>(r) * a.Hq + hq) * 2 + 1] = kRowFinished;
         }
       }
       run0 = run1;
@@ -356,7 +368,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       n_shares = n_run_tiles <= a.uncut_tiles ? 1 : min(n_run_tiles / kMinShareTiles, static_cast<int>(gridDim.z));
       if (z >= n_shares) {
         if (n_shares > 1 && active[0] && kg == 0 && half == 0)  // a share without keys
-          *reinterpret_cast<float2*>(a.ws_ml + ((static_cast<int64_t>(z) * a.Lq + row[0]) * a.Hq + hq) * 2) =
+          *reinterpret_cast<float2*>(a.ws_ml + ((static_cast<int64_t>(z) * a.Lq + anew(row[0])) * a.Hq + hq) * 2) =
               float2{-INFINITY, 0.f};
         run0 = run1;
         continue;
@@ -431,11 +443,12 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     }
     // One staging load of tile kt, whose table entry is ts: pieces 0 .. NI - 1 are the V loads
     // of the row groups, NI .. 2 NI - 1 the K loads.  Tiles past the run's last one are not staged.
-    auto fetch_piece = [&](int piece, int kt, int ts, char* dst) {
+    // `dst`: the buffer's address in LDS.
+    auto fetch_piece = [&](int piece, int kt, int ts, uint32_t dst) {
       if (kt >= n_kv_tiles) return;
       const int i = piece % NI;
       const bool is_k = piece >= NI;
-      char* lds = dst + kg * TILE_BYTES + (i * ITEMS + item) * RPI * ROWB;  // wavefront-uniform
+      const uint32_t lds = dst + kg * TILE_BYTES + (i * ITEMS + item) * RPI * ROWB;  // wavefront-uniform
       if (ts >= 0) {
         load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(ts) * ROWB, is_k ? lane_k[i] : lane_v[i], lds);
       } else {
@@ -461,7 +474,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     {
       const int ts0 = __builtin_amdgcn_readfirstlane(kPow2 && kt_my < n_kv_tiles ? look_up(kt_my) : -1);
 #pragma unroll
-      for (int piece = NI; piece < 2 * NI; ++piece) fetch_piece(piece, kt_my, ts0, s_k0);
+      for (int piece = NI; piece < 2 * NI; ++piece) fetch_piece(piece, kt_my, ts0, lds_k0);
     }
     if constexpr (kPow2)
       for (int t = kt_lo + tid; t < n_kv_tiles && t - kt_lo < kSlotTable; t += kThreads) s_tslot[t - kt_lo] = look_up(t);
@@ -506,8 +519,8 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       constexpr int kBuf = decltype(parity)::value;
       const char* kcur = kBuf ? s_k1 : s_k0;   // K(i)
       const char* vprev = kBuf ? s_v0 : s_v1;  // V(i - 1)
-      char* knext = kBuf ? s_k0 : s_k1;        // K(i + 1) goes here
-      char* vcur = kBuf ? s_v1 : s_v0;         // V(i) goes here
+      const uint32_t knext = kBuf ? lds_k0 : lds_k1;  // K(i + 1) goes here
+      const uint32_t vcur = kBuf ? lds_v1 : lds_v0;   // V(i) goes here
       const int key0 = (kt_my + KG * i) * kTileN;
       const bool work_cur = (KG == 1 ? i < n_my : kt_my + KG * i < n_kv_tiles) && key0 < wave_max;
       const bool work_prev = i > 0 && (KG == 1 || kt_my + KG * (i - 1) < n_kv_tiles) && key0 - KG * kTileN < wave_max;
@@ -597,7 +610,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
 #pragma unroll
         for (int piece = 0; piece < 2 * NI; ++piece)
           fetch_piece(piece, piece < NI ? kt_k - KG : kt_k, piece < NI ? ts_v : ts_k,
-                      const_cast<char*>(piece < NI ? vprev : kcur));
+                      piece < NI ? (kBuf ? lds_v0 : lds_v1) : (kBuf ? lds_k1 : lds_k0));
       }
 
       // ---- X(i): online softmax of tile i, one query per lane ----
@@ -695,7 +708,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
         const int ts1 = tile_slot(kt_my + KG), ts0 = tile_slot(kt_my);
 #pragma unroll
         for (int piece = 0; piece < 2 * NI; ++piece)
-          fetch_piece(piece, piece < NI ? kt_my : kt_my + KG, piece < NI ? ts0 : ts1, piece < NI ? s_v0 : s_k1);
+          fetch_piece(piece, piece < NI ? kt_my : kt_my + KG, piece < NI ? ts0 : ts1, piece < NI ? lds_v0 : lds_k1);
       }
       for (int i = 0; i <= n_my; i += 2) {
         step(IntC<1>{}, IntC<0>{}, i);
@@ -755,9 +768,10 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     if (active[0]) {
       const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
       const bool writes_ml = half == 0 && kg == 0;
+      const int r = anew(row[0]);
       if (n_shares > 1) {
         // one of several key shares: the state goes to the merge pass
-        const int64_t p = (static_cast<int64_t>(z) * a.Lq + row[0]) * a.Hq + hq;
+        const int64_t p = (static_cast<int64_t>(z) * a.Lq + r) * a.Hq + hq;
         short* po = a.ws_acc + p * D + d0;
 #pragma unroll
         for (int db = 0; db < PB; ++db)
@@ -768,7 +782,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
                       E::pack2(o_acc[0][db][i4 * 4 + 2] * inv, o_acc[0][db][i4 * 4 + 3] * inv)};
         if (writes_ml) *reinterpret_cast<float2*>(a.ws_ml + p * 2) = float2{m_tot, l_tot};
       } else {
-        char* o = a.out + row[0] * a.os_row + hq * a.os_h + d0 * 2;
+        char* o = a.out + r * a.os_row + hq * a.os_h + d0 * 2;
         const float lse_nat = l_tot > 0.f ? (m_tot + log2f(l_tot)) * kLn2 : -INFINITY;
         // attention-sink gate of the caller's post-attention step (model.py:122-128): the output,
         // rounded to the model dtype, times sigmoid(lse - sinks[h]) in fp32, rounded again
@@ -787,8 +801,8 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
           }
         }
         if (writes_ml) {
-          a.lse[static_cast<int64_t>(hq) * a.Lq + row[0]] = lse_nat;
-          if (gridDim.z > 1) a.ws_ml[(static_cast<int64_t>(row[0]) * a.Hq + hq) * 2 + 1] = kRowFinished;
+          a.lse[static_cast<int64_t>(hq) * a.Lq + r] = lse_nat;
+          if (gridDim.z > 1) a.ws_ml[(static_cast<int64_t>(r) * a.Hq + hq) * 2 + 1] = kRowFinished;
         }
       }
     }
@@ -979,14 +993,15 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   // With one query head per cache head, head_dim 128 and bounded scores workgroups of half as many rows again (four wavefronts, each
   // alone on its SIMD) are the better ones where these, too, fit the GPU in one go and no row sees more keys than kShortRange and
   // uncut_tiles say (what the table has columns for: a caller that knows the longest sequence passes no more): their set-up is
-  // shorter and a tile holds fewer runs, but a pair of key tiles takes longer (1.9 us instead of 1.6: no second wavefront on the SIMD hides a
-  // wavefront's softmax).  us a launch, 16 heads, eight wavefronts / four: 64 rows over 64, 320, 576 and 1400 keys 9.9 / 8.9, 13.0 / 12.5,
-  // 15.9 / 16.2 and 26.0 / 29.2; 200 over 200, 448 and 704 12.7 / 11.0, 15.5 / 15.0 and 18.2 / 18.6; 400 over 400 and 832 15.3 / 14.2 and 21.0 / 20.3;
-  // 613 over 613, 704, 832 and 4600 17.9 / 16.8, 18.8 / 18.8, 20.1 / 20.4 and 64.0 / 74.3; 1000 over 1000 and 1216 22.8 / 22.5 and 24.7 / 26.1;
-  // four of 75, of 153 and of 250 rows 22.2 / 14.7, 19.0 / 16.5 and 19.0 / 17.0; at the end of the range eight of 100 over 822 48.8 / 37.0, two and four of 100 to 200
-  // over 566 26.9 / 27.4 and 28.6 / 28.9, past it eight of 125 over 950 38.4 / 39.8.  Eight and four heads the same.  Two query heads to a
-  // cache head (us a layer with its insert) 22.7 / 23.2, the running maximum 24.7 / 25.2: the tiles are staged twice as often, and there is less time
-  // to hide it in.  Head_dim 64 is not compiled so; a trial gave 64, 200 and 613 rows 6.9 / 6.6, 8.9 / 8.0 and 12.5 / 11.3, 64 over 1400 keys 18.4 / 18.7.
+  // shorter and a tile holds fewer runs, but a pair of key tiles takes longer: no second wavefront on the SIMD hides a wavefront's
+  // softmax.  us a launch, 16 heads, eight wavefronts / four: 64 rows over 64, 192 and 320 keys 8.7 / 8.3, 10.4 / 10.0 and 11.8 / 11.7, 200 over 200
+  // and 448 11.8 / 10.4 and 13.9 / 13.8, 400 over 400 and 576 13.5 / 13.1 and 16.4 / 15.5, 613 over 613 and 704 16.4 / 15.5 and 17.3 / 17.3, 800 over 800 and
+  // 832 18.0 / 18.3 and 19.2 / 18.9; four of 75, of 153 and of 250 rows 20.8 / 13.5, 17.2 / 15.5 and 17.9 / 16.4; at the end of the range eight of 100 over
+  // 822 45.9 / 34.0, eight of 125 over 832 32.8 / 32.6, two of 200 and four of 100 over 566 24.9 / 25.0 and 26.1 / 26.7, four of 250 over 832 30.0 / 30.7.  Past it,
+  // before the tile loops lost a tenth: 64 rows over 576 and 1400 15.9 / 16.2 and 26.0 / 29.2, 613 over 832 and 4600 20.1 / 20.4 and 64.0 / 74.3, eight
+  // of 125 over 950 38.4 / 39.8.  Eight and four heads the same.  Two query heads to a cache head (us a layer with its insert) 22.7 / 23.2, the running
+  // maximum 24.7 / 25.2: the tiles are staged twice as often, and there is less time to hide it in.  Head_dim 64 is not compiled so; a trial gave
+  // 64, 200 and 613 rows 6.9 / 6.6, 8.9 / 8.0 and 12.5 / 11.3, 64 over 1400 keys 18.4 / 18.7.
   if constexpr (G == 1 && D == 128 && std::is_same<E, BF16>::value) {
     constexpr int BM4 = 64;
     const int short_tiles = std::min(uncut_tiles(a.Lq, a.Hq, true), kShortRange);
@@ -1013,7 +1028,7 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   // cheap, the softmax (which does not shrink with head_dim) is what a step waits for, and independent
   // workgroups on a CU fill each other's barrier and set-up gaps: 8 x 512-row chunks 85 us against 91 us, the
   // same 8 sequences whole 350 us against 370 us with two per CU and 316 us with three (the instance is
-  // compiled for 168 registers, a handful of values spilled outside the tile loop); 6 chunks 85 us against
+  // compiled for 168 registers; where it spills, 20 bytes, that is in front of and behind the tile loop); 6 chunks 85 us against
   // 91 us, and where no workspace allows the cut along the keys, 1 / 4 chunks 59 / 72 us against 74 / 90 us.
   // At head_dim 128 the same split is slower (whole sequences 564 us against 485 us): the staging path is
   // the limit there, and its 242 registers allow two wavefronts per SIMD at most.

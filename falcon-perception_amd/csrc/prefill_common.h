@@ -26,6 +26,20 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, c
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(m0v), "v"(offset), "s"(base) : "memory");
 }
 
+// Both forms with the place in LDS as a number, `lds` = lds_address(array) + bytes: a pointer that a loop keeps is 64 bits of scalar
+// registers, and a test for null at every load.
+__device__ __forceinline__ uint32_t lds_address(const char* array) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)array));
+}
+__device__ __forceinline__ void load_to_lds(const char* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               : : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src) : "memory");
+}
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               : : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(offset), "s"(base) : "memory");
+}
+
 // Both forms for rows that are read once (non-temporal, so that they do not displace what the caches hold).
 __device__ __forceinline__ void load_to_lds_nt(const char* src, char* lds) {
   const uint32_t base = __builtin_amdgcn_readfirstlane(

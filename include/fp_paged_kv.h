@@ -16,8 +16,8 @@
  *    launched once on the device BEFORE a capture, because its first launch makes the
  *    runtime set that memory up, which it cannot do while a stream is being captured.
  *    The only such kernels here are those fp_paged_prefill launches at head_dim 64 for a
- *    launch that is not cut along the keys (bf16 and f16, 20 to 44 bytes per lane); every
- *    kernel behind the other entry points, and the rest of fp_paged_prefill, uses none
+ *    launch that is not cut along the keys (bf16 and f16, 20 bytes per lane: one or four query
+ *    heads per cache head, no score bound, a page size that is a power of two); every kernel behind the other entry points, and the rest of fp_paged_prefill, uses none
  *    (the build writes every kernel's figure to build/<source>.resources.txt and a test
  *    holds the list to exactly this).  The reference's engine captures decode steps only
  *    (paged_inference.py:916-935).
