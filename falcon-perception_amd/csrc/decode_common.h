@@ -3,6 +3,7 @@
 #pragma once
 
 #include "fp_common.h"
+#include "prefill_common.h"
 
 #include <math.h>
 
@@ -115,14 +116,8 @@ __device__ __forceinline__ void row_sum(float (&x)[kN]) {
   for (int i = 0; i < kN; ++i) if (kLanes >= 64) x[i] += __shfl_xor(x[i], 32);
 }
 
-// v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second, v_permlane16_swap the odd rows
-// of 16 lanes of its first with the even rows of its second.  Of one value twice, both operands hold both parts' values
-// afterwards, in every lane; of two values, the sum of the operands is the first value's total in the lower half (the even rows) and the
-// second's in the other.  (Inline assembly: the compiler's builtin returned the first operand for both.  The no-ops are the wait states
-// between a vector write, the swap and the next vector read.)
-__device__ __forceinline__ void swap_halves(float& a, float& b) {
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
+// v_permlane16_swap exchanges the odd rows of 16 lanes of its first operand with the even rows of its second, as
+// fp::swap_lane_halves does with the halves of the wavefront (inline assembly for the reason given there).
 __device__ __forceinline__ void swap_rows(float& a, float& b) {
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
 }
@@ -132,11 +127,6 @@ __device__ __forceinline__ void swap_halves(float& a, float& b, float& c, float&
 __device__ __forceinline__ void swap_rows(float& a, float& b, float& c, float& d) {
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
 }
-__device__ __forceinline__ float max_across_halves(float x) {
-  float y = x;
-  swap_halves(x, y);
-  return fmaxf(x, y);
-}
 __device__ __forceinline__ float max_across_rows(float x) {
   float y = x;
   swap_rows(x, y);
@@ -144,7 +134,7 @@ __device__ __forceinline__ float max_across_rows(float x) {
 }
 __device__ __forceinline__ float sum_across_halves(float x) {
   float y = x;
-  swap_halves(x, y);
+  fp::swap_lane_halves(x, y);
   return x + y;
 }
 __device__ __forceinline__ float sum_across_rows(float x) {
@@ -161,7 +151,7 @@ __device__ __forceinline__ void add_across_halves(float (&x)[M]) {
     for (int i = 0; i < N / 2; i += 2) swap_halves(x[i], x[i + N / 2], x[i + 1], x[i + 1 + N / 2]);
   } else {
 #pragma unroll
-    for (int i = 0; i < N / 2; ++i) swap_halves(x[i], x[i + N / 2]);
+    for (int i = 0; i < N / 2; ++i) fp::swap_lane_halves(x[i], x[i + N / 2]);
   }
 #pragma unroll
   for (int i = 0; i < N / 2; ++i) x[i] += x[i + N / 2];

@@ -29,7 +29,6 @@
 //           leave its result where the caller keeps arrival counters.
 #include "decode_common.h"
 #include "paged_decode_mfma.h"
-#include "prefill_common.h"
 
 #include <atomic>
 
@@ -412,7 +411,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
     float mx = m[g];
     if (TPR <= 8) mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror:8
     if (TPR <= 16) mx = max_across_rows(mx);
-    if (TPR <= 32) mx = max_across_halves(mx);
+    if (TPR <= 32) mx = fp::max_across_lane_halves(mx);
     const float w = fast_exp2(m[g] - safe_max(mx));
     m[g] = mx;
     l[g] *= w;

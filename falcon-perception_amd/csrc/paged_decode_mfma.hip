@@ -19,7 +19,6 @@
 // GB) 626 us (6.5 TB/s) against 648 us.
 #include "decode_common.h"
 #include "paged_decode_mfma.h"
-#include "prefill_common.h"
 
 #include <type_traits>
 

@@ -1,5 +1,5 @@
-// Shared by the prefill kernels: loads from global memory straight into LDS (no staging registers)
-// and an exchange between the two halves of a wavefront.
+// Shared by the prefill and the decode kernels: loads from global memory straight into LDS (no staging registers)
+// and exchanges between the lanes of a wavefront.
 #ifndef FP_PREFILL_COMMON_H
 #define FP_PREFILL_COMMON_H
 
@@ -52,15 +52,18 @@ __device__ __forceinline__ void load_to_lds_nt(const char* base, uint32_t offset
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" : : "s"(m0v), "v"(offset), "s"(base) : "memory");
 }
 
-// max(x of lane l, x of lane l ^ 32) in both lanes, without the trip through LDS a shuffle takes:
-// v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second, so
-// from (x, x) it leaves the lower halves' values in one register and the upper halves' in the other.
-// (Inline assembly: the compiler's builtin returned the first register for both results.)  The no-ops
-// cover the wait states between a vector write, the swap and the next vector read.
+// v_permlane32_swap exchanges the upper half of its first operand with the lower half of its second.  Of one value twice, both
+// operands hold both halves' values afterwards, in every lane; of two values, the sum of the operands is the first value's total in the
+// lower half and the second's in the upper.  No trip through LDS as a shuffle takes it.  (Inline assembly: the compiler's builtin returned
+// the first operand for both.  The no-ops are the wait states between a vector write, the swap and the next vector read.)
+__device__ __forceinline__ void swap_lane_halves(float& a, float& b) {
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+// max(x of lane l, x of lane l ^ 32) in both lanes
 __device__ __forceinline__ float max_across_lane_halves(float x) {
-  float lo = x, hi = x;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lo), "+v"(hi));
-  return fmaxf(lo, hi);
+  float y = x;
+  swap_lane_halves(x, y);
+  return fmaxf(x, y);
 }
 
 // Largest x of the wavefront, in scalar registers: lane exchanges inside rows of 16, then one lane of each, no trip through LDS.
