@@ -10,8 +10,9 @@
 //   grid  = (cache heads, batch, splits); a workgroup of 4 wavefronts owns one
 //           (sequence, cache head, token range) and serves all G = Hq / Hc query
 //           heads of that cache head from a single read of K and V.  A launch
-//           larger than the GPU holds at once, or of several sequences under a
-//           limit much longer than they are (even_cut_pays), runs as (cache
+//           of more than one to four workgroups to a CU (even_cut_line), or of
+//           several sequences under a limit much longer than they are
+//           (even_cut_pays), runs as (cache
 //           heads, chunks) instead: the contexts laid end to end and cut into
 //           equal chunks, a workgroup working through the sequences its chunk
 //           touches.  With arrival counters (fp_paged_decode_step) few
@@ -848,7 +849,7 @@ bool even_cut_fits(int Hc, int B, int max_context, int page_size) {
   return chunks >= 1 && B <= kFlatMaxB && tokens < (1ll << 30) && (tokens / chunks + 128) / page_size + 2 <= kMaxSplitPages;
 }
 
-// Whether a launch that the GPU holds at once is cut evenly all the same: its splits are long (1024 tokens or more, or eight
+// Whether a launch on this side of even_cut_line is cut evenly all the same: its splits are long (1024 tokens or more, or eight
 // of 512), so that sequences much shorter than max_context leave CUs idle, and the cut makes at most eight pieces of a
 // sequence, which the merge pass (one wavefront per row) takes in one batch.  us a layer split by split / cut evenly, 16 q / 8 kv
 // heads, D 128: limit 8192, 300 to 3000 tokens, 8, 12, 16 and 24 sequences 22.4 / 19.5, 28.3 / 24.1, 35.4 / 27.1 and 43.2 / 35.8, 4000 to
@@ -866,11 +867,11 @@ bool even_cut_pays(int Hc, int B, int max_context, int page_size) {
 }
 
 // Chunks per cache head of the even cut of a launch, 0 where it goes split by split.  The workspace of its splits has a row
-// per (chunk + sequence), and a launch of more workgroups than the GPU holds at once (`resident`) is always cut.
-int even_cut_chunks(int Hc, int B, int n_splits, int max_context, int page_size, int resident) {
+// per (chunk + sequence), and a launch of more than `line` workgroups is always cut.
+int even_cut_chunks(int Hc, int B, int n_splits, int max_context, int page_size, int line) {
   const int chunks = flat_chunks(Hc);
   if (!even_cut_fits(Hc, B, max_context, page_size) || static_cast<int64_t>(B) * (n_splits - 1) < chunks) return 0;
-  return static_cast<int64_t>(Hc) * B * n_splits > resident || even_cut_pays(Hc, B, max_context, page_size) ? chunks : 0;
+  return static_cast<int64_t>(Hc) * B * n_splits > line || even_cut_pays(Hc, B, max_context, page_size) ? chunks : 0;
 }
 
 // Splits of all sequences together, about, of a launch with arrival counters that goes piece by piece (walk_pieces): two workgroups to a
@@ -903,10 +904,18 @@ int merged_pieces(int Hc, int B, int n_splits, int max_context, int page_size) {
   return longest / page_size + 2 <= kMaxSplitPages ? static_cast<int>(pieces) : 0;
 }
 
-// Workgroups to a CU beyond which a launch is always cut evenly: as many as the even-cut kernel's registers let a CU hold when the
-// sweeps at even_cut_pays and merged_pieces were made.  Numbers, so that a kernel that needs fewer registers does not move the line.
+// Workgroups to a CU beyond which a launch is always cut evenly.  Numbers, so that a kernel that needs fewer registers does not move
+// the line: as many as the even-cut kernels' registers let a CU hold when the sweeps at even_cut_pays and merged_pieces were made.  Since
+// then a CU holds one more of the 16-bit kernels for a cache of one K head per query head with V in pairs and whole pages, and in fp32 of most with two
+// and four heads (at head_dim 64 and two heads a fourth).  Between the two numbers, cut evenly / split by split, us a layer in a graph of the
+// plan and four layers (about 1 us of it the plan): bf16, V in pairs, D 128: limit 4096, 8 heads, 5 sequences of 200 to 1600, 400 to
+// 4096 and 3500 to 4096 tokens 14.5 / 12.2, 21.7 / 22.2 and 28.1 / 26.7; limit 512, 24 of 25 to 200 and of 50 to 500 12.5 / 11.0 and 17.0 / 15.3; limit
+// 8192, 3 of 800 to 8192, 16 and 4 heads 27.9 / 27.9 and 18.1 / 12.4.  fp32 the same 19.7 / 17.1, 29.6 / 35.2 and 44.8 / 45.9; 14.6 / 14.9 and 22.5 /
+// 23.4; 43.8 / 47.3 and 23.4 / 17.8.  fp32, four heads: limit 8192, 16 heads, 3 of 400 to 3200 21.0 / 23.1; limit 512, 12 of 50 to 500 20.6 / 18.1.
+// fp32, D 64, two heads: limit 512, 8 heads, 30 of 50 to 500 15.3 / 12.5; limit 8192, 4 heads, 7 of 800 to 8192 20.2 / 17.5.  In fp32 at D 128 either side is
+// the better one somewhere; in 16 bits and at D 64 split by split mostly is, and a line one higher there would be worth these figures.
 template <typename E, int D, int G, bool kPerHeadK>
-constexpr int workgroups_held(bool aligned) {
+constexpr int even_cut_line(bool aligned) {
   const bool narrow = sizeof(typename E::type) == 2;
   if (kPerHeadK) return narrow ? (G == 2 && !aligned ? 3 : 2) : (D == 128 && aligned ? 2 : 3);
   return G == 1 ? 4 : G == 2 ? 3 : G == 4 || (D == 64 && aligned) ? 2 : 1;
@@ -957,16 +966,16 @@ void launch_decode(const DecodeArgs& a0, int B, int phases, hipStream_t st) {
     // it, and in fp32 it made them spill).  With the step's plan read by every workgroup the same sweep gives, in us per
     // step for 1 / 2 / 3 chunks per CU: D 128 110.4 / 111.3 / 112.2; D 64 61.7 / 61.3 / 62.1; page size 64, 32
     // sequences 89.2 / 90.9 / 90.4: two stays.
-    int resident;  // matrix cores: two to a CU, but few sequences want the third (640 / 752 / 896 workgroups, 64 q / 8 kv heads,
-                   // split by split / cut evenly: 15.1 / 17.9, 21.6 / 25.1 and 19.6 / 18.2 us)
+    int line;  // matrix cores: two to a CU, but few sequences want the third (640 / 752 / 896 workgroups, 64 q / 8 kv heads,
+               // split by split / cut evenly: 15.1 / 17.9, 21.6 / 25.1 and 19.6 / 18.2 us)
     if constexpr (on_matrix_cores<E, G, kPerHeadK>())
-      resident = 3 * fp::compute_units();
+      line = 3 * fp::compute_units();
     else
-      resident = workgroups_held<E, D, G, kPerHeadK>(aligned) * fp::compute_units();
+      line = even_cut_line<E, D, G, kPerHeadK>(aligned) * fp::compute_units();
     const int pieces = a.arrivals ? merged_pieces(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size) : 0;
     DecodeArgs ap = a;
     ap.n_chunks = pieces;
-    const int n_chunks = pieces > 0 ? 0 : even_cut_chunks(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size, resident);
+    const int n_chunks = pieces > 0 ? 0 : even_cut_chunks(a.Hc, B, a.n_splits, a.max_context, a.pd.page_size, line);
     DecodeArgs af = a;
     af.B = B;
     af.n_chunks = n_chunks;
