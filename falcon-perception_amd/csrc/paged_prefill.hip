@@ -226,8 +226,8 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   int row_seq[RJ], row_lim[RJ];  // of tile row j * 64 + lane
   // What only the beginning or the end of a run needs is worked out there: the addresses, two registers each, would be kept through
   // the tile loop (at head_dim 64, where three workgroups share a CU, in scratch memory: 20 to 44 bytes a lane).  Together with the
-  // buffers' addresses in LDS as numbers, us a launch with bounded scores: 256 rows of 16 heads over 16000 keys, D 128, without a workspace
-  // 201 -> 184, 600 over 4000 64.4 -> 59.4; D 64, 24 prompts of 100 to 700 rows 29.7 -> 28.0; 8 chunks of 512 rows over 256 to 4096 72.1 -> 70.1.
+  // loads' places in LDS as numbers summed at the load, us a launch with bounded scores: 256 rows of 16 heads over 16000 keys, D 128, without a
+  // workspace 201 -> 178, 600 over 4000 64.4 -> 57.8; D 64, 24 prompts of 100 to 700 rows 29.7 -> 28.0, 8 chunks of 512 rows over 256 to 4096 72.1 -> 70.1.
   const auto anew = [](int x) {
     asm volatile("" : "+v"(x));
     return x;
@@ -291,6 +291,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   // kswz of the row does not depend on i where an instruction of all staging wavefronts is 16 rows or more; where it is 8, every
   // second one flips the chunk's highest bit.  vrot has a period of 4 rows.
   static_assert(ITEMS * RPI % 16 == 0 || (ITEMS * RPI == 8 && CPR == 16), "the permutation of a lane's rows");
+  const uint32_t lds_own = kg * TILE_BYTES + item * RPI * ROWB;  // where this wavefront's rows begin in a buffer
   const int k_src_off = (lp ^ SW::kswz(st_row0)) * 16;
   const auto k_flip = [](int i) { return ITEMS * RPI == 8 ? (i & 1) * 128 : 0; };
   const int v_src_off = ((((lp >> 1) + R32 - SW::vrot(st_row0)) % R32) * 2 + (lp & 1)) * 16;
@@ -448,9 +449,9 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
       if (kt >= n_kv_tiles) return;
       const int i = piece % NI;
       const bool is_k = piece >= NI;
-      const uint32_t lds = dst + kg * TILE_BYTES + (i * ITEMS + item) * RPI * ROWB;  // wavefront-uniform
+      const uint32_t lds = dst + i * ITEMS * RPI * ROWB;
       if (ts >= 0) {
-        load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(ts) * ROWB, is_k ? lane_k[i] : lane_v[i], lds);
+        load_to_lds((is_k ? kplane : vplane) + static_cast<int64_t>(ts) * ROWB, is_k ? lane_k[i] : lane_v[i], lds_own, lds);
       } else {
         asm volatile("");  // rare: keep it out of the way as a branch
         const int r = i * ITEMS * RPI + st_row0;
@@ -466,7 +467,7 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
           const bool ok = in_range && pg >= 0 && pg < a.pool_pages;
           slot = ok ? static_cast<int>(pg) * a.pd.page_size + off : 0;
         }
-        load_to_lds((is_k ? kplane + (k_src_off ^ k_flip(i)) : vsrc) + static_cast<int64_t>(slot) * ROWB, lds);
+        load_to_lds((is_k ? kplane + (k_src_off ^ k_flip(i)) : vsrc) + static_cast<int64_t>(slot) * ROWB, lds_own, lds);
       }
     };
 
@@ -994,10 +995,10 @@ void launch_group(const PrefillArgs& a0, float score_bound, void* workspace, int
   // alone on its SIMD) are the better ones where these, too, fit the GPU in one go and no row sees more keys than kShortRange and
   // uncut_tiles say (what the table has columns for: a caller that knows the longest sequence passes no more): their set-up is
   // shorter and a tile holds fewer runs, but a pair of key tiles takes longer: no second wavefront on the SIMD hides a wavefront's
-  // softmax.  us a launch, 16 heads, eight wavefronts / four: 64 rows over 64, 192 and 320 keys 8.7 / 8.3, 10.4 / 10.0 and 11.8 / 11.7, 200 over 200
-  // and 448 11.8 / 10.4 and 13.9 / 13.8, 400 over 400 and 576 13.5 / 13.1 and 16.4 / 15.5, 613 over 613 and 704 16.4 / 15.5 and 17.3 / 17.3, 800 over 800 and
-  // 832 18.0 / 18.3 and 19.2 / 18.9; four of 75, of 153 and of 250 rows 20.8 / 13.5, 17.2 / 15.5 and 17.9 / 16.4; at the end of the range eight of 100 over
-  // 822 45.9 / 34.0, eight of 125 over 832 32.8 / 32.6, two of 200 and four of 100 over 566 24.9 / 25.0 and 26.1 / 26.7, four of 250 over 832 30.0 / 30.7.  Past it,
+  // softmax.  us a launch, 16 heads, eight wavefronts / four: 64 rows over 64, 192 and 320 keys 8.5 / 8.0, 10.3 / 9.7 and 11.6 / 11.3, 200 over 200
+  // and 448 11.6 / 10.0 and 13.8 / 13.5, 400 over 400 and 576 13.4 / 12.6 and 16.1 / 15.1, 613 over 613 and 704 16.2 / 15.0 and 17.1 / 16.7, 800 over 800 and
+  // 832 17.9 / 17.6 and 18.9 / 18.1; four of 75, of 153 and of 250 rows 20.7 / 13.3, 17.3 / 15.4 and 17.8 / 16.1; at the end of the range eight of 100 over
+  // 822 45.0 / 32.8, eight of 125 over 832 32.3 / 31.6, two of 200 and four of 100 over 566 24.6 / 24.1 and 25.8 / 25.9, four of 250 over 832 29.5 / 29.6.  Past it,
   // before the tile loops lost a tenth: 64 rows over 576 and 1400 15.9 / 16.2 and 26.0 / 29.2, 613 over 832 and 4600 20.1 / 20.4 and 64.0 / 74.3, eight
   // of 125 over 950 38.4 / 39.8.  Eight and four heads the same.  Two query heads to a cache head (us a layer with its insert) 22.7 / 23.2, the running
   // maximum 24.7 / 25.2: the tiles are staged twice as often, and there is less time to hide it in.  Head_dim 64 is not compiled so; a trial gave

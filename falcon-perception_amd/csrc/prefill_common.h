@@ -26,18 +26,18 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, c
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(m0v), "v"(offset), "s"(base) : "memory");
 }
 
-// Both forms with the place in LDS as a number, `lds` = lds_address(array) + bytes: a pointer that a loop keeps is 64 bits of scalar
-// registers, and a test for null at every load.
+// Both forms with the place in LDS as a number in two parts, a wavefront's own and a constant (lds_address of an array, plus bytes): a pointer
+// that a loop keeps is 64 bits of scalar registers and a test for null at every load, and a sum for every load of a loop a register each.
 __device__ __forceinline__ uint32_t lds_address(const char* array) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)array));
 }
-__device__ __forceinline__ void load_to_lds(const char* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               : : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src) : "memory");
+__device__ __forceinline__ void load_to_lds(const char* src, uint32_t own, uint32_t constant) {
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off"
+               : : "s"(own), "s"(constant), "v"(src) : "memory", "scc");
 }
-__device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               : : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(offset), "s"(base) : "memory");
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, uint32_t own, uint32_t constant) {
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+               : : "s"(own), "s"(constant), "v"(offset), "s"(base) : "memory", "scc");
 }
 
 // Both forms for rows that are read once (non-temporal, so that they do not displace what the caches hold).

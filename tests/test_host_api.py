@@ -439,8 +439,8 @@ def test_only_the_documented_kernels_use_scratch_memory():
 
 def test_the_prefill_kernels_keep_their_tile_loops_registers():
     """What a tile loop keeps for the code around it costs the loop: at head_dim 64 scratch memory (44 bytes a lane with the addresses of
-    a run's rows kept), in launches of few rows scalar registers that every step moves back from vector lanes (80 and more with
-    the addresses of the buffers in LDS as pointers).  The compiler's report of the last build."""
+    a run's rows kept), in launches of few rows scalar registers that every step moves back from vector lanes (80 to 93 with
+    the loads' places in LDS as pointers or as a sum each).  The compiler's report of the last build."""
     import importlib.util
     import re
 
@@ -449,6 +449,6 @@ def test_the_prefill_kernels_keep_their_tile_loops_registers():
     spec.loader.exec_module(mod)
     usage = mod.resource_usage()
     narrow = [u for n, u in usage.items() if re.search(r"paged_prefill_kernelINS_\d?(BF16|F16)ELi64ELi\dELb[01]ELi4E", n)]
-    halves = [u for n, u in usage.items() if re.search(r"paged_prefill_kernelINS_\d?(BF16|F16)ELi\d+ELi\dELb[01]ELi8ELb[01]ELi2E", n)]
-    assert len(narrow) == 18 and len(halves) == 36
-    assert max(u["scratch"] for u in narrow) <= 20 and max(u["sgprs_moved"] for u in halves) <= 64
+    halves = [u for n, u in usage.items() if re.search(r"paged_prefill_kernelINS_\d?(BF16|F16)ELi\d+ELi\dELb[01]ELi[48]ELb[01]ELi2E", n)]
+    assert len(narrow) == 18 and len(halves) == 37
+    assert max(u["scratch"] for u in narrow) <= 20 and max(u["sgprs_moved"] for u in halves) <= 48
