@@ -10,7 +10,9 @@
 //
 // MFMA-bound.  A workgroup of 8 wavefronts owns one cache head and 256 / G consecutive packed
 // query rows of each of its G query heads; a wavefront owns 32 rows of one query head.  (Large launches
-// at head_dim 64 use workgroups of 4 wavefronts and 128 / G rows, three to a CU.)
+// at head_dim 64 use workgroups of 4 wavefronts and 128 / G rows, three to a CU.  In launches of few
+// rows the two halves of a workgroup have the same rows and take the key tiles in turn: 8 wavefronts and
+// 128 / G rows, or 4 and 64, a wavefront to a SIMD.  launch_group has which goes out how.)
 //   S^T = K Q^T  (v_mfma_f32_32x32x16): keys are the M rows, queries the N columns, so a
 //         lane holds scores of ONE query and softmax row reductions stay in registers
 //         (plus one exchange between the two lane halves).
@@ -20,9 +22,9 @@
 //   (16 bytes per lane, no staging registers), into double buffers whose rows are
 //   chunk-permuted against bank conflicts; the first pool slot of every tile of a run is
 //   looked up once, so a staging load is a scalar base plus a fixed lane offset.
-//   The two wavefronts that share a SIMD run half a step apart (two barriers per tile): one is
-//   in its MFMA phase (O^T of the previous tile, S^T of the current one) while the other is in
-//   its softmax.
+//   The halves of a workgroup run half a step apart (one barrier per step).  With eight wavefronts two
+//   of them share a SIMD, one of each half: one is in its MFMA phase (O^T of the previous tile, S^T of
+//   the current one) while the other is in its softmax.
 // Rows of one tile may belong to several sequences: the tile is processed one
 // run of equal batch_idx at a time; rows of slot 0 are padding (out 0, lse -inf).
 #include "fp_common.h"
@@ -162,6 +164,9 @@ struct Swizzle {
 //
 // KG = 2: the two halves of the workgroup have the same query rows (half as many) and take the key tiles in turn, each half from
 // buffers of its own; their states meet in LDS at the end.  See launch_group for the launches that go out so.
+//
+// The workgroups of four wavefronts and 64 rows are built for two wavefronts to a SIMD, too, though their LDS allows one: asked for one
+// the compiler moves the accumulators to the other half of the register file, and the times are the same (613 rows 15.6 / 15.5 us).
 template <typename E, int D, int G, bool kPow2, int W = kWaves, bool kBounded = false, int KG = 1>
 __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_prefill_kernel(const PrefillArgs a) {
   constexpr int kThreads = W * 64;  // shadows the file-scope constant: W wavefronts per workgroup
@@ -500,6 +505,11 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     // everywhere, and every wavefront has waited for its loads before B(i + 1), after which M(i + 1)
     // begins.  (A second barrier between the two parts of the interval kept the halves in step more
     // strictly and cost 2 %.)  K(i) lives in K buffer i % 2, V(i) in V buffer i % 2.
+    // With four wavefronts no two of a workgroup share a SIMD.  At head_dim 64 a SIMD has one wavefront each of three workgroups, which
+    // fill each other's phases.  In the workgroups of 64 rows (KG = 2) a wavefront is alone on its SIMD: the half step hides
+    // nothing there, matrix phase, softmax and staging follow one another, and a step is 3700 to 4300 cycles, of which 1024 are matrix
+    // instructions (613 rows, 16 heads: 3100 until Q is scaled, 4500 until K of the first tile is on its way and the table is made, five steps, 1200 for
+    // the last tile's O^T, 3800 for the halves to meet and the results to leave).
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's rows have landed in LDS
 
     s16x8 p_op[MB][4];  // P^T as B operands of the 4 k-steps (16 keys each), from X(i) to M(i + 1)
