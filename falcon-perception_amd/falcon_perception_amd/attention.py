@@ -136,7 +136,7 @@ class HybridPrefillMask:
         self._step_layer = -1  # layer that asked last: a layer id that does not grow starts a new step
         self._row_limit = None
         self.most_keys = 0  # no row of the step sees more keys than this: the longest sequence the cache holds
-        self._short_table = None  # the columns of the page table that hold so many, where `short_table` was asked for them
+        self.table = cache.page_table  # with columns for so many
         self._tile_orders: dict[int, tuple[Tensor, int]] = {}  # rows per tile -> tile order of the step's limits
 
     def _limits_from_ids(self, open_spans, validate) -> Tensor:
@@ -183,17 +183,9 @@ class HybridPrefillMask:
             self._step_key = key
             self._tile_orders = {}
             self.most_keys = max(self.cache.capacity)
-            self._short_table = None
+            self.table = self.cache.table_for(self.most_keys)
         self._step_layer = layer_id
         return self._row_limit
-
-    def short_table(self) -> Tensor:
-        """The page table with no more columns than the longest sequence of the step's cache has pages, made by the first layer that
-        asks after `row_limit`: the width of the table is what a launch knows of the key ranges of its rows."""
-        if self._short_table is None:
-            table, pages = self.cache.page_table, -(-self.most_keys // self.cache.page_size)
-            self._short_table = table[:, :pages] if 0 < pages < table.shape[1] else table
-        return self._short_table
 
     def tile_order(self, batch_idx: Tensor, tile_rows: int) -> tuple[Tensor, int]:
         """Query tiles of the step by decreasing key range (`ops.prefill_tile_order`), made by the first layer
@@ -348,8 +340,8 @@ def compiled_flex_attn_prefill(q: Tensor, k: Tensor, v: Tensor, score_mod=None, 
         if rows and -(-Lq // rows) <= 4096:
             order = block_mask.tile_order(step.batch_idx, rows)
     bound = cache.score_bound(D, scale)
-    # head_dim 128, a bound and no workspace: launches of few rows over few keys have workgroups of their own
-    table = block_mask.short_table() if bound and D == 128 and workspace is False else cache.page_table
+    # launches of few rows over few keys have workgroups of their own at head_dim 128
+    table = block_mask.table if workspace is False and D == 128 else cache.page_table
     args = (q, pool_k, pool_v, table, step.batch_idx, limits, cache.page_size)
     got = None
     if q.is_cuda:

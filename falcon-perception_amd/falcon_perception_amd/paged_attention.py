@@ -130,6 +130,7 @@ class PagedKVCache(KVCacheBase):
         self._decode_plan: Tensor | None = None  # the step's plan of the decode kernel (`decode_plan`)
         self._decode_plan_owner = None           # the mask object it was made for
         self._prefill_workspace: Tensor | None = None
+        self._table_view: tuple[Tensor, int, Tensor] | None = None  # of `table_for`
         self._prefill_need: dict[tuple, tuple[int, int]] = {}
         self._prefill_tile_rows: dict[tuple, int] = {}
         # status word of the last prefill mask, on its way to the host (`check_prefill_masks`)
@@ -508,6 +509,16 @@ class PagedKVCache(KVCacheBase):
         if self._decode_plan is None:
             self._decode_plan = torch.zeros(ops.decode_plan_bytes(), dtype=torch.uint8, device=self._kv.device)
         return self._decode_plan
+
+    def table_for(self, keys: int) -> Tensor:
+        """The page table with no more columns than `keys` keys have pages (0: unknown): its width is what a prefill launch knows of
+        the key ranges of its rows.  The view of the last call is kept: making one is a tenth of a short prompt's host time."""
+        table, pages = self.page_table, -(-keys // self.page_size)
+        if not 0 < pages < table.shape[1]:
+            return table
+        if self._table_view is None or self._table_view[0] is not table or self._table_view[1] != pages:
+            self._table_view = (table, pages, table[:, :pages])
+        return self._table_view[2]
 
     def score_bound(self, head_dim: int, scale: float | None) -> float:
         """Bound of |scale * q.k| the prefill kernel may rely on: 0 (unknown) unless q and k are normalised;
