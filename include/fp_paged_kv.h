@@ -473,6 +473,9 @@ int fp_hybrid_row_limits(const int64_t* input_ids, const int64_t* batch_idx,
  *              fixed point 0.  Results agree with the unbounded path within bf16 rounding.  A bound
  *              the data breaks gives wrong results only once exp2(score * log2 e) leaves fp32's
  *              range.  f16 and fp32 ignore the argument.
+ *   n_pages    columns of page_table that a row's keys may lie in.  A caller that knows its longest
+ *              sequence may pass no more than that one has pages (the row stride stays): launches of
+ *              few rows over few keys go out as smaller workgroups, for the same bits.
  *   workspace  NULL, or workspace_bytes bytes of device memory, 16-byte aligned (no need to clear it).
  *              A launch with fewer workgroups than the GPU needs (few query rows, few heads) is then
  *              also cut along the keys: up to 8 workgroups share a query tile, each takes an equal part
