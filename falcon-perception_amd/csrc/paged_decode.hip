@@ -223,6 +223,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   __shared__ float s_ml[kWaves][G][2];
   constexpr int NR = (2 * GK + RPW - 1) / RPW;  // load instructions for the fresh rows, a row to a lane group
   constexpr bool kEarly = !kFlat && !kPieces;
+  constexpr bool kFull = kFlat && G * D >= 1024;  // the registers of a row's loop are all taken (fp32, eight heads, D 128)
   __shared__ __attribute__((aligned(1024))) char s_fresh[kEarly ? NR * 1024 : 16];
 
   // Workgroups are dealt to the 8 XCDs round-robin by linear id.  Heads run fastest:
@@ -369,7 +370,7 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
 
   if (takes_new) {
     int at = lane;
-    if constexpr (kFlat) asm volatile("" : "+v"(at));  // here and below: what only the end of a piece needs is not kept in registers from piece to piece
+    if constexpr (kFlat && !kFull) asm volatile("" : "+v"(at));  // here and below: what only the end of a piece needs is not kept in registers from piece to piece
     const int byte = at % TPR * 16;
     // the newest token: one row, held by lane group 0; the other groups' is masked
     v4u kreg[GK][1], vreg[1];
@@ -405,45 +406,74 @@ __global__ __launch_bounds__(kThreads, (decode_waves_per_simd<E, D, G, kPerHeadK
   // combine the lane groups of this wavefront: every state at the common maximum, then the sums.  Each exchange between the lane
   // halves, and between rows of 16 lanes, adds up two elements at once and leaves one of them in either part, so that a lane
   // ends with a part of the elements.  (An exchange through LDS for every element and group was 0.8 us at the end of every piece; 0.2 us so.)
-  constexpr int N = G * EPL;
-  float sum[N];
+  // Where the loop in front has no register left the exchange through LDS is the better one, which changes the states in place: with
+  // the sums beside them the compiler's loop is 3 % slower (64 sequences of 1024 to 4096 tokens, fp32, eight heads on 8, D 128: 358 / 346 us a layer).
+  if constexpr (kFull) {
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float mx = m[g];
-    if (TPR <= 8) mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror:8
-    if (TPR <= 16) mx = max_across_rows(mx);
-    if (TPR <= 32) mx = fp::max_across_lane_halves(mx);
-    const float w = fast_exp2(m[g] - safe_max(mx));
-    m[g] = mx;
-    l[g] *= w;
+    for (int off = TPR; off < 64; off <<= 1) {
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) sum[g * EPL + e] = acc[g][e] * w;
-  }
-  if (TPR <= 8) {
+      for (int g = 0; g < G; ++g) {
+        const float mo = __shfl_xor(m[g], off), lo = __shfl_xor(l[g], off);
+        const float mx = fmaxf(m[g], mo), ms = safe_max(mx);
+        const float wa = fast_exp2(m[g] - ms), wb = fast_exp2(mo - ms);
+        l[g] = l[g] * wa + lo * wb;
 #pragma unroll
-    for (int i = 0; i < N; ++i) sum[i] += dpp<0x128>(sum[i]);
+        for (int e = 0; e < EPL; ++e) acc[g][e] = acc[g][e] * wa + __shfl_xor(acc[g][e], off) * wb;
+        m[g] = mx;
+      }
+    }
+    if (lane < TPR) {
 #pragma unroll
-    for (int g = 0; g < G; ++g) l[g] += dpp<0x128>(l[g]);
-  }
-  if (TPR <= 32) add_across_halves<N>(sum);
-  if (TPR <= 16) add_across_rows<N / 2>(sum);
-  constexpr int NL = TPR <= 16 ? N / 4 : TPR <= 32 ? N / 2 : N;  // elements this lane ends with, from `held` on
-  int at = lane;
-  if constexpr (kFlat) asm volatile("" : "+v"(at));
-  const int held = (TPR <= 32 ? (at >> 5) * (N / 2) : 0) + (TPR <= 16 ? (at >> 4 & 1) * (N / 4) : 0);
-  static_assert(NL % EPL == 0 || EPL % NL == 0, "either whole heads or a part of one");
-  float* const to = &s_acc[wave][held / EPL][at % TPR * EPL + held % EPL];
-  if (TPR > 8 || (at & 8) == 0) {
+      for (int g = 0; g < G; ++g) {
 #pragma unroll
-    for (int i = 0; i < NL; ++i) to[i / EPL * D + i % EPL] = sum[i];
-  }
+        for (int e = 0; e < EPL; ++e) s_acc[wave][g][col * EPL + e] = acc[g][e];
+        if (lane == 0) {
+          s_ml[wave][g][0] = m[g];
+          s_ml[wave][g][1] = l[g];
+        }
+      }
+    }
+  } else {
+    constexpr int N = G * EPL;
+    float sum[N];
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    if (TPR <= 16) l[g] = sum_across_rows(l[g]);
-    if (TPR <= 32) l[g] = sum_across_halves(l[g]);
-    if (lane == 0) {
-      s_ml[wave][g][0] = m[g];
-      s_ml[wave][g][1] = l[g];
+    for (int g = 0; g < G; ++g) {
+      float mx = m[g];
+      if (TPR <= 8) mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror:8
+      if (TPR <= 16) mx = max_across_rows(mx);
+      if (TPR <= 32) mx = fp::max_across_lane_halves(mx);
+      const float w = fast_exp2(m[g] - safe_max(mx));
+      m[g] = mx;
+      l[g] *= w;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) sum[g * EPL + e] = acc[g][e] * w;
+    }
+    if (TPR <= 8) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) sum[i] += dpp<0x128>(sum[i]);
+#pragma unroll
+      for (int g = 0; g < G; ++g) l[g] += dpp<0x128>(l[g]);
+    }
+    if (TPR <= 32) add_across_halves<N>(sum);
+    if (TPR <= 16) add_across_rows<N / 2>(sum);
+    constexpr int NL = TPR <= 16 ? N / 4 : TPR <= 32 ? N / 2 : N;  // elements this lane ends with, from `held` on
+    int at = lane;
+    if constexpr (kFlat) asm volatile("" : "+v"(at));
+    const int held = (TPR <= 32 ? (at >> 5) * (N / 2) : 0) + (TPR <= 16 ? (at >> 4 & 1) * (N / 4) : 0);
+    static_assert(NL % EPL == 0 || EPL % NL == 0, "either whole heads or a part of one");
+    float* const to = &s_acc[wave][held / EPL][at % TPR * EPL + held % EPL];
+    if (TPR > 8 || (at & 8) == 0) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) to[i / EPL * D + i % EPL] = sum[i];
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (TPR <= 16) l[g] = sum_across_rows(l[g]);
+      if (TPR <= 32) l[g] = sum_across_halves(l[g]);
+      if (lane == 0) {
+        s_ml[wave][g][0] = m[g];
+        s_ml[wave][g][1] = l[g];
+      }
     }
   }
   __syncthreads();
