@@ -266,9 +266,6 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   }
   __builtin_amdgcn_sched_barrier(0);  // all of them are on their way before the first is waited for
   if constexpr (kBounded) {
-    // page ids of the first run, in the caches by the time Q is there and scaled
-    const int seq0 = __builtin_amdgcn_readlane(row_seq[0], 0);
-    const int64_t page = a.page_table[static_cast<int64_t>(seq0) * a.pt_row_stride + min(lane, a.n_pages - 1)];
     // bounded scores: Q carries scale * log2(e), so that the matrix product leaves the exponent itself
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -281,7 +278,6 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
                           E::to_float(static_cast<short>(w[c] >> 16)) * a.qscale);
         qreg[mb][ds] = __builtin_bit_cast(s16x8, w);
       }
-    asm volatile("" : : "v"(page));
   }
 
   const char* kplane = a.pool_k + static_cast<int64_t>(hc) * a.n_slots * ROWB;
