@@ -224,7 +224,9 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
   // together: sequence and limit of every row of the tile (by every wavefront for itself: what follows from them needs no LDS and
   // no barrier), then this wavefront's row limits and Q rows.  What is in front of the first key tile is a chain of trips to memory and
   // of scalar instructions, 4 to 8 cycles each, that nothing on the CU hides: 6.9 us a workgroup with limits that went through LDS,
-  // loads under conditions and 64-bit divisions, 5.2 us so (613 rows 20.2 -> 19.2 us a launch, 8 chunks of 512 rows 125 -> 121).
+  // loads under conditions and 64-bit divisions, 5.2 us so (613 rows 20.2 -> 19.2 us a launch, 8 chunks of 512 rows 125 -> 121); 3.5 us, in the
+  // workgroups of 64 rows 2.8, without the registers that were kept for the code around the loop and without the first run's page ids asked for
+  // and waited for before Q is scaled.
   // Rows outside a run keep their Q values: what such a row computes is never stored.  Rows past the last one read that one's (a load
   // under a condition is followed by a wait where the compiler finds something to do with what it brought).
   constexpr int RJ = (BM + 63) / 64;
@@ -503,9 +505,9 @@ __global__ __launch_bounds__(W * 64, (W == 4 && D == 64 ? 3 : 2)) void paged_pre
     // strictly and cost 2 %.)  K(i) lives in K buffer i % 2, V(i) in V buffer i % 2.
     // With four wavefronts no two of a workgroup share a SIMD.  At head_dim 64 a SIMD has one wavefront each of three workgroups, which
     // fill each other's phases.  In the workgroups of 64 rows (KG = 2) a wavefront is alone on its SIMD: the half step hides
-    // nothing there, matrix phase, softmax and staging follow one another, and a step is 3700 to 4300 cycles, of which 1024 are matrix
-    // instructions (613 rows, 16 heads: 3100 until Q is scaled, 4500 until K of the first tile is on its way and the table is made, five steps, 1200 for
-    // the last tile's O^T, 3800 for the halves to meet and the results to leave).
+    // nothing there, matrix phase, softmax and staging follow one another, and a step is 3600 to 4300 cycles, of which 1024 are matrix
+    // instructions (613 rows, 16 heads, at 2.3 GHz: 6400 cycles until Q is scaled and the first tile is there, five steps, 1200 for the last tile's
+    // O^T, 3600 for the halves to meet and the results to leave: 13.5 us).
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's rows have landed in LDS
 
     s16x8 p_op[MB][4];  // P^T as B operands of the 4 k-steps (16 keys each), from X(i) to M(i + 1)
